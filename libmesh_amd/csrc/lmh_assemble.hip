@@ -20,12 +20,6 @@ namespace lmh {
 typedef double double4_t __attribute__((ext_vector_type(4)));
 typedef float float4_t __attribute__((ext_vector_type(4)));
 
-__device__ inline double forcing(int f_kind, double x, double y, double z) {
-  if (f_kind == 0) return 1.0;
-  const double pi = 3.14159265358979323846264338327950288;
-  return 3.0 * pi * pi * sin(pi * x) * sin(pi * y) * sin(pi * z);
-}
-
 // Geometry at one quadrature point from LDS coordinates X[a*3+c] and the
 // reference derivative table dref[(a*nq+q)*3+r].  Writes M (9, symmetric,
 // scaled by JxW*kappa) and JxW (which is negative for the negative-weight tet
@@ -543,6 +537,21 @@ __global__ void k_add_vec_gather(const int32_t *__restrict__ inc_ptr, const int3
   }
 }
 
+// v[r] = sum of Fe over DoF r's incidences in ascending order (v overwritten);
+// MASK: 0 on constrained DoFs
+template <bool MASK>
+__global__ __launch_bounds__(256) void k_sum_vec_gather(const int32_t *__restrict__ inc_ptr,
+                                                        const int32_t *__restrict__ inc,
+                                                        const uint8_t *__restrict__ cons, int64_t n_rows,
+                                                        const double *__restrict__ Fe, double *__restrict__ v) {
+  for (int64_t r = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; r < n_rows; r += (int64_t)gridDim.x * blockDim.x) {
+    const int32_t k0 = inc_ptr[r], k1 = inc_ptr[r + 1];
+    double s = 0.0;
+    for (int32_t k = k0; k < k1; ++k) s += Fe[inc[k]];
+    v[r] = MASK && cons[r] ? 0.0 : s;
+  }
+}
+
 // Element residuals of the Poisson physics, R_e = K_e u_e - F_e from the
 // unconstrained element matrices, with C^T applied for empty constraint rows
 // (a constrained DoF's entry is 0); written over Fe.  One wave per element:
@@ -619,11 +628,6 @@ __global__ __launch_bounds__(64) void k_qoi_box(const double *__restrict__ tab, 
   }
 }
 
-__global__ void k_zero_constrained(double *__restrict__ v, const uint8_t *__restrict__ cons, int64_t n) {
-  for (int64_t r = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; r < n; r += (int64_t)gridDim.x * blockDim.x)
-    if (cons[r]) v[r] = 0.0;
-}
-
 // ---------------------------------------------------------------------------
 // Adjoint backward kernel: dJ/dkappa_e = -lambda_e^T (dKc_e/dkappa_e) u_e.
 // Kc_e is linear in kappa_e on free rows/columns and kappa-independent on
@@ -679,6 +683,16 @@ __global__ __launch_bounds__(64) void k_adjoint_kappa(const double *__restrict__
     }
     __syncthreads();
   }
+}
+
+// Kernels that need no element matrix or table in LDS, by element and rule:
+// 1 the HEX27 tensor kernels (their points are the 3^3 rule's), 2 one element
+// per thread (TET4, TET10, HEX8: at most 10 nodes fit a thread's registers,
+// any rule), 0 the general one-element-per-wavefront kernels (HEX27 with
+// another rule).
+static int matrix_free_path(int type, int npts) {
+  if (type == LMH_HEX27) return npts == 3 ? 1 : 0;
+  return type == LMH_TET4 || type == LMH_TET10 || type == LMH_HEX8 ? 2 : 0;
 }
 
 static int read_flag(lmh_context *ctx, const char *what) {
@@ -899,15 +913,24 @@ int lmh_assemble_residual_poisson(lmh_matrix *A, const lmh_mesh *m, const lmh_do
   lmh_context *ctx = A->ctx;
   const int64_t ne = m->n_elem, dd = (int64_t)dm->dpe * dm->dpe;
   if (!A->Fe) LMH_HIP(hipMalloc((void **)&A->Fe, sizeof(double) * ne * dm->dpe));
-  if (!A->Ke) LMH_HIP(hipMalloc((void **)&A->Ke, sizeof(double) * ne * dd));
+  LMH_CHECK(dm->nv == 1, LMH_ERR_UNSUPPORTED, "Poisson assembly needs one variable");
+  const FETable *t = nullptr;
+  LMH_TRY(fe_table(ctx, m->type, npts, &t));
   LMH_HIP(hipMemsetAsync(ctx->d_flags, 0, sizeof(int), ctx->stream));
-  LMH_TRY(element_poisson_impl<double>(ctx, m, dm, npts, kappa_d, f_kind, 0, A->Ke, A->Fe));
-  LMH_LAUNCH(ctx, "element_residual", k_elem_residual, dim3(grid_for((ne + 3) / 4, 1, ctx->cu_count * 8)), dim3(256),
-             sizeof(double) * 4 * ((size_t)dm->dpe * dm->dpe + dm->dpe), (const double *)A->Ke, A->Fe, dm->edofs,
-             dm->cons, u_d, dm->dpe, ne);
-  LMH_LAUNCH(ctx, "fill", k_fill<double>, dim3(grid_for(dm->n_dofs, 256, 8192)), dim3(256), 0, R_d, dm->n_dofs, 0.0);
-  LMH_LAUNCH(ctx, "add_element_vectors", k_add_vec_gather, dim3(grid_for(dm->n_dofs, 256, 8192)), dim3(256), 0,
-             dm->inc_ptr, dm->inc, dm->n_dofs, (const double *)A->Fe, R_d);
+  const int path = matrix_free_path(m->type, npts);
+  if (path == 1) {
+    LMH_TRY(hex27_residual(ctx, m, dm, kappa_d, f_kind, u_d, A->Fe));
+  } else if (path == 2) {
+    LMH_TRY(thread_residual(ctx, t, m, dm, kappa_d, f_kind, u_d, A->Fe));
+  } else {
+    if (!A->Ke) LMH_HIP(hipMalloc((void **)&A->Ke, sizeof(double) * ne * dd));
+    LMH_TRY(element_poisson_impl<double>(ctx, m, dm, npts, kappa_d, f_kind, 0, A->Ke, A->Fe));
+    LMH_LAUNCH(ctx, "element_residual", k_elem_residual, dim3(grid_for((ne + 3) / 4, 1, ctx->cu_count * 8)), dim3(256),
+               sizeof(double) * 4 * ((size_t)dm->dpe * dm->dpe + dm->dpe), (const double *)A->Ke, A->Fe, dm->edofs,
+               dm->cons, u_d, dm->dpe, ne);
+  }
+  LMH_LAUNCH(ctx, "add_element_vectors", k_sum_vec_gather<true>, dim3(grid_for(dm->n_dofs, 256, 8192)), dim3(256), 0,
+             dm->inc_ptr, dm->inc, dm->cons, dm->n_dofs, (const double *)A->Fe, R_d);
   LMH_TRY(check_launch("residual"));
   LMH_TRY(read_flag(ctx, "lmh_assemble_residual_poisson"));
   // general rows: u holds the enforced values (C u + H), so the summed element
@@ -924,15 +947,19 @@ int lmh_qoi_box_derivative(const lmh_mesh *m, const lmh_dofmap *dm, int npts, do
   double *Q = nullptr;
   LMH_HIP(hipMallocAsync((void **)&Q, sizeof(double) * m->n_elem * t->n, ctx->stream));
   LMH_HIP(hipMemsetAsync(ctx->d_flags, 0, sizeof(int), ctx->stream));
-  const size_t shm = sizeof(double) * (t->nq + (size_t)t->n * t->nq * 4 + 81 + t->nq);
-  LMH_LAUNCH(ctx, "qoi_box", k_qoi_box, dim3(grid_for(m->n_elem, 1, ctx->cu_count * 8)), dim3(64), shm, t->d_data,
-             t->n, t->nq, m->xyz, m->conn, m->n_elem, lo, hi, Q, ctx->d_flags);
-  LMH_TRY(check_launch("k_qoi_box"));
-  LMH_LAUNCH(ctx, "fill", k_fill<double>, dim3(grid_for(dm->n_dofs, 256, 8192)), dim3(256), 0, dq_d, dm->n_dofs, 0.0);
-  LMH_LAUNCH(ctx, "add_element_vectors", k_add_vec_gather, dim3(grid_for(dm->n_dofs, 256, 8192)), dim3(256), 0,
-             dm->inc_ptr, dm->inc, dm->n_dofs, (const double *)Q, dq_d);
-  LMH_LAUNCH(ctx, "zero_constrained", k_zero_constrained, dim3(grid_for(dm->n_dofs, 256, 8192)), dim3(256), 0, dq_d,
-             dm->cons, dm->n_dofs);
+  const int path = matrix_free_path(m->type, npts);
+  if (path == 1) {
+    LMH_TRY(hex27_qoi(ctx, m, lo, hi, Q));
+  } else if (path == 2) {
+    LMH_TRY(thread_qoi(ctx, t, m, lo, hi, Q));
+  } else {
+    const size_t shm = sizeof(double) * (t->nq + (size_t)t->n * t->nq * 4 + 81 + t->nq);
+    LMH_LAUNCH(ctx, "qoi_box", k_qoi_box, dim3(grid_for(m->n_elem, 1, ctx->cu_count * 8)), dim3(64), shm, t->d_data,
+               t->n, t->nq, m->xyz, m->conn, m->n_elem, lo, hi, Q, ctx->d_flags);
+    LMH_TRY(check_launch("k_qoi_box"));
+  }
+  LMH_LAUNCH(ctx, "add_element_vectors", k_sum_vec_gather<true>, dim3(grid_for(dm->n_dofs, 256, 8192)), dim3(256), 0,
+             dm->inc_ptr, dm->inc, dm->cons, dm->n_dofs, (const double *)Q, dq_d);
   LMH_TRY(check_launch("qoi"));
   LMH_HIP(hipFreeAsync(Q, ctx->stream));
   LMH_TRY(read_flag(ctx, "lmh_qoi_box_derivative"));
@@ -954,6 +981,12 @@ int lmh_adjoint_kappa_gradient(const lmh_mesh *m, const lmh_dofmap *dm, int npts
   LMH_TRY(fe_table(ctx, m->type, npts, &t));
   LMH_CHECK(t->nq <= 64 && t->n <= 27, LMH_ERR_UNSUPPORTED, "element too large");
   LMH_HIP(hipMemsetAsync(ctx->d_flags, 0, sizeof(int), ctx->stream));
+  const int path = matrix_free_path(m->type, npts);
+  if (path != 0) {
+    LMH_TRY(path == 1 ? hex27_adjoint(ctx, m, dm, u_d, lambda_d, grad_d)
+                      : thread_adjoint(ctx, t, m, dm, u_d, lambda_d, grad_d));
+    return read_flag(ctx, "lmh_adjoint_kappa_gradient");
+  }
   const size_t shm = sizeof(double) * (t->nq + (size_t)t->n * t->nq * 4 + 81 + 27 + 27 + 64);
   LMH_LAUNCH(ctx, "adjoint_kappa", k_adjoint_kappa, dim3(grid_for(m->n_elem, 1, ctx->cu_count * 8)), dim3(64), shm,
              t->d_data, t->n, t->nq, m->xyz, m->conn, dm->edofs, dm->cons, u_d, lambda_d, m->n_elem, grad_d,
@@ -1024,9 +1057,8 @@ int lmh_matrix_scatter_elements(lmh_matrix *A, const double *Ke_d, const double 
   if (R_d) {
     // residual only: the DoF map's incidence lists hold (element, local) in
     // ascending order, so each entry sums in element order
-    LMH_LAUNCH(ctx, "fill", k_fill<double>, dim3(grid_for(A->rows, 256, 8192)), dim3(256), 0, R_d, A->rows, 0.0);
-    LMH_LAUNCH(ctx, "add_element_vectors", k_add_vec_gather, dim3(grid_for(A->rows, 256, 8192)), dim3(256), 0,
-               dm->inc_ptr, dm->inc, A->rows, Fe_d, R_d);
+    LMH_LAUNCH(ctx, "add_element_vectors", k_sum_vec_gather<false>, dim3(grid_for(A->rows, 256, 8192)), dim3(256), 0,
+               dm->inc_ptr, dm->inc, dm->cons, A->rows, Fe_d, R_d);
   }
   return check_launch("lmh_matrix_scatter_elements");
 }

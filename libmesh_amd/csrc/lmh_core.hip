@@ -209,13 +209,19 @@ int fe_table(lmh_context *ctx, int type, int arg, const FETable **out) {
     std::unique_ptr<FETable> t(new FETable);
     LMH_CHECK(build_fe_table(type, arg, *t), LMH_ERR_UNSUPPORTED, "no quadrature/shape table for type %d arg %d",
               type, arg);
-    const size_t cnt = t->w.size() + t->phi.size() + t->dref.size();
+    const size_t cnt = t->w.size() * 2 + (t->phi.size() + t->dref.size()) * 2;
     LMH_HIP(hipMalloc(&t->d_data, cnt * sizeof(double)));
     std::vector<double> flat;
     flat.reserve(cnt);
     flat.insert(flat.end(), t->w.begin(), t->w.end());
     flat.insert(flat.end(), t->phi.begin(), t->phi.end());
     flat.insert(flat.end(), t->dref.begin(), t->dref.end());
+    for (int q = 0; q < t->nq; ++q) {
+      flat.push_back(t->w[q]);
+      for (int a = 0; a < t->n; ++a) flat.push_back(t->phi[(size_t)a * t->nq + q]);
+      for (int a = 0; a < t->n; ++a)
+        for (int r = 0; r < 3; ++r) flat.push_back(t->dref[((size_t)a * t->nq + q) * 3 + r]);
+    }
     LMH_HIP(hipMemcpy(t->d_data, flat.data(), cnt * sizeof(double), hipMemcpyHostToDevice));
     it = ctx->tables.emplace(key, std::move(t)).first;
   }

@@ -1,0 +1,319 @@
+// lmh_hex27.hip -- HEX27 element kernels on the tensor-product evaluation of
+// lmh_hex27.h: residual of the Poisson physics, QoI derivative and adjoint
+// gradient, none of which needs an element matrix.
+//
+// What bounds them: the element data are small (27 nodes, a few fields), so the
+// kernels are FP64-instruction and LDS-read bound.  With one element per
+// wavefront and a lane per point, 27 of 64 lanes worked and every point summed
+// 27 nodes against a 17 KB table in LDS (three workgroups per CU).  Here seven
+// elements share a wavefront, each lane forms three points by sum factorisation
+// and no table is read.  64,000 elements (40^3), before -> now: residual
+// element stage 555 (element matrices, then K_e u_e) -> 35 us, QoI 290 -> 21 us,
+// adjoint gradient 326 -> 52 us; the three calls with their gathers and host
+// waits 1288 -> 240 us.
+#include <algorithm>
+
+#include "lmh_hex27.h"
+
+namespace lmh {
+
+// Nodal data of the wavefront's seven elements: ids of the next group are
+// fetched while the current one is computed.
+struct H27Slots {
+  int el[3], lat[3];
+  bool live[3];
+  __device__ explicit H27Slots(int lane) {
+#pragma unroll
+    for (int m = 0; m < 3; ++m) {
+      const int k = lane + 64 * m;
+      live[m] = k < 27 * kH27PerWave;
+      const int kk = live[m] ? k : 0;
+      el[m] = kk / 27;
+      lat[m] = kH27Lat[kk - 27 * el[m]];
+    }
+  }
+  // entries t = e0 * 27 + lane + 64 m of an n_elem x 27 table (clamped to the last)
+  __device__ inline void ids(const int32_t *__restrict__ tab, int64_t e0, int64_t total, int lane,
+                             int32_t (&id)[3]) const {
+#pragma unroll
+    for (int m = 0; m < 3; ++m) {
+      const int64_t t = e0 * 27 + lane + 64 * m;
+      id[m] = tab[t < total ? t : total - 1];
+    }
+  }
+};
+
+// Element vectors R_e = K_e u_e - F_e without K_e: at each point the reference
+// flux M grad u (M = JxW kappa G G^T) and f JxW, contracted with the test
+// functions direction 3 first (in registers), then directions 1 and 2 through
+// LDS, lane l owning the test functions (i1, i2) = (l % 3, l / 3).
+template <int FK>
+__global__ __launch_bounds__(64) void k_hex27_residual(const double *__restrict__ xyz, const int32_t *__restrict__ conn,
+                                                       const int32_t *__restrict__ edofs,
+                                                       const double *__restrict__ kappa, const double *__restrict__ u,
+                                                       int64_t ne, double *__restrict__ Fe, int *__restrict__ err) {
+  constexpr int NF = 4, ST = 27 * NF + 1;  // odd stride: the elements' broadcasts fall in different banks
+  __shared__ double s_f[kH27PerWave * ST];
+  __shared__ double s_h[kH27PerWave * 81];
+  const int lane = threadIdx.x;
+  const H27Slots sl(lane);
+  const H27Lane L(lane);
+  double pt[3], dt[3], pt2[3], dt2[3];  // the lane's test functions at the 1D points
+#pragma unroll
+  for (int q = 0; q < 3; ++q) {
+    pt[q] = h27_pick(L.l % 3, [&](int i) { return h27_p(q, i); });
+    dt[q] = h27_pick(L.l % 3, [&](int i) { return h27_d(q, i); });
+    pt2[q] = h27_pick(L.l / 3, [&](int i) { return h27_p(q, i); });
+    dt2[q] = h27_pick(L.l / 3, [&](int i) { return h27_d(q, i); });
+  }
+  const int64_t total = ne * 27, groups = (ne + kH27PerWave - 1) / kH27PerWave;
+  int32_t nd[3], dof[3];
+  sl.ids(conn, (int64_t)blockIdx.x * kH27PerWave, total, lane, nd);
+  sl.ids(edofs, (int64_t)blockIdx.x * kH27PerWave, total, lane, dof);
+  for (int64_t gr = blockIdx.x; gr < groups; gr += gridDim.x) {
+    const int64_t e0 = gr * kH27PerWave, e = e0 + L.el;
+#pragma unroll
+    for (int m = 0; m < 3; ++m)
+      if (sl.live[m]) {
+        double *d = s_f + sl.el[m] * ST + sl.lat[m] * NF;
+        const double *x = xyz + 3 * (int64_t)nd[m];
+        d[0] = x[0];
+        d[1] = x[1];
+        d[2] = x[2];
+        d[3] = u[dof[m]];
+      }
+    sl.ids(conn, (gr + gridDim.x) * kH27PerWave, total, lane, nd);
+    sl.ids(edofs, (gr + gridDim.x) * kH27PerWave, total, lane, dof);
+    const bool on = L.el < kH27PerWave && e < ne;
+    h27_sync();
+    if (on) {
+      const double kap = kappa ? kappa[e] : 1.0;
+      double g[3][NF][3], pos[3][FK ? 3 : 1];
+      h27_refgrad<NF, FK ? 3 : 0>(s_f + L.el * ST, L, g, pos);
+      double h[3][3];
+#pragma unroll
+      for (int i = 0; i < 3; ++i) h[i][0] = h[i][1] = h[i][2] = 0.0;
+#pragma unroll
+      for (int q = 0; q < 3; ++q) {
+        double J[3][3], c[3][3];
+#pragma unroll
+        for (int r = 0; r < 3; ++r)
+#pragma unroll
+          for (int k = 0; k < 3; ++k) J[r][k] = g[q][k][r];
+        const double det = cofactors(J, c);
+        if (!(det > 0.0)) atomicOr(err, 1);
+        const double w = L.w12 * h27_w(q), s = kap * w / det;
+        double v[3];  // det * physical gradient of u
+#pragma unroll
+        for (int k = 0; k < 3; ++k) v[k] = g[q][3][0] * c[0][k] + g[q][3][1] * c[1][k] + g[q][3][2] * c[2][k];
+        double fl[3];
+#pragma unroll
+        for (int r = 0; r < 3; ++r) fl[r] = s * (c[r][0] * v[0] + c[r][1] * v[1] + c[r][2] * v[2]);
+        double fj = det * w;
+        if constexpr (FK != 0) fj *= forcing(FK, pos[q][0], pos[q][1], pos[q][2]);
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+          h[i][0] += h27_p(q, i) * fl[0];
+          h[i][1] += h27_p(q, i) * fl[1];
+          h[i][2] += h27_d(q, i) * fl[2] - h27_p(q, i) * fj;
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < 3; ++i)
+#pragma unroll
+        for (int k = 0; k < 3; ++k) s_h[L.el * 81 + (3 * i + k) * 9 + L.l] = h[i][k];
+    }
+    h27_sync();
+    if (on) {
+#pragma unroll
+      for (int i = 0; i < 3; ++i) {
+        const double *H = s_h + L.el * 81 + 27 * i;
+        double s = 0.0;
+#pragma unroll
+        for (int q2 = 0; q2 < 3; ++q2) {
+          double a = 0.0, b = 0.0;
+#pragma unroll
+          for (int q1 = 0; q1 < 3; ++q1) {
+            const int q = 3 * q2 + q1;
+            a += dt[q1] * H[q] + pt[q1] * H[18 + q];
+            b += pt[q1] * H[9 + q];
+          }
+          s += pt2[q2] * a + dt2[q2] * b;
+        }
+        Fe[e * 27 + kH27Node[9 * i + L.l]] = s;
+      }
+    }
+    h27_sync();
+  }
+}
+
+// Q_i = sum over the points inside [lo, hi]^3 of JxW phi_i.
+__global__ __launch_bounds__(64) void k_hex27_qoi(const double *__restrict__ xyz, const int32_t *__restrict__ conn,
+                                                  int64_t ne, double lo, double hi, double *__restrict__ Q,
+                                                  int *__restrict__ err) {
+  constexpr int NF = 3, ST = 27 * NF;
+  __shared__ double s_f[kH27PerWave * ST];
+  __shared__ double s_h[kH27PerWave * 27];
+  const int lane = threadIdx.x;
+  const H27Slots sl(lane);
+  const H27Lane L(lane);
+  double pt[3], pt2[3];
+#pragma unroll
+  for (int q = 0; q < 3; ++q) {
+    pt[q] = h27_pick(L.l % 3, [&](int i) { return h27_p(q, i); });
+    pt2[q] = h27_pick(L.l / 3, [&](int i) { return h27_p(q, i); });
+  }
+  const int64_t total = ne * 27, groups = (ne + kH27PerWave - 1) / kH27PerWave;
+  int32_t nd[3];
+  sl.ids(conn, (int64_t)blockIdx.x * kH27PerWave, total, lane, nd);
+  for (int64_t gr = blockIdx.x; gr < groups; gr += gridDim.x) {
+    const int64_t e = gr * kH27PerWave + L.el;
+#pragma unroll
+    for (int m = 0; m < 3; ++m)
+      if (sl.live[m]) {
+        double *d = s_f + sl.el[m] * ST + sl.lat[m] * NF;
+        const double *x = xyz + 3 * (int64_t)nd[m];
+        d[0] = x[0];
+        d[1] = x[1];
+        d[2] = x[2];
+      }
+    sl.ids(conn, (gr + gridDim.x) * kH27PerWave, total, lane, nd);
+    const bool on = L.el < kH27PerWave && e < ne;
+    h27_sync();
+    if (on) {
+      double g[3][NF][3], pos[3][3], h[3] = {0.0, 0.0, 0.0};
+      h27_refgrad<NF, 3>(s_f + L.el * ST, L, g, pos);
+#pragma unroll
+      for (int q = 0; q < 3; ++q) {
+        double J[3][3], c[3][3];
+#pragma unroll
+        for (int r = 0; r < 3; ++r)
+#pragma unroll
+          for (int k = 0; k < 3; ++k) J[r][k] = g[q][k][r];
+        const double det = cofactors(J, c);
+        if (!(det > 0.0)) atomicOr(err, 1);
+        const double x = pos[q][0], y = pos[q][1], z = pos[q][2];
+        const bool in = x >= lo && x <= hi && y >= lo && y <= hi && z >= lo && z <= hi;
+        const double jc = in ? det * (L.w12 * h27_w(q)) : 0.0;
+#pragma unroll
+        for (int i = 0; i < 3; ++i) h[i] += h27_p(q, i) * jc;
+      }
+#pragma unroll
+      for (int i = 0; i < 3; ++i) s_h[L.el * 27 + 9 * i + L.l] = h[i];
+    }
+    h27_sync();
+    if (on) {
+#pragma unroll
+      for (int i = 0; i < 3; ++i) {
+        const double *H = s_h + L.el * 27 + 9 * i;
+        double s = 0.0;
+#pragma unroll
+        for (int q2 = 0; q2 < 3; ++q2)
+          s += pt2[q2] * (pt[0] * H[3 * q2] + pt[1] * H[3 * q2 + 1] + pt[2] * H[3 * q2 + 2]);
+        Q[e * 27 + kH27Node[9 * i + L.l]] = s;
+      }
+    }
+    h27_sync();
+  }
+}
+
+// dJ/dkappa_e = -sum_q JxW grad(lambda).grad(u), nodal values masked to the
+// free DoFs (see k_adjoint_kappa).
+__global__ __launch_bounds__(64) void k_hex27_adjoint(const double *__restrict__ xyz, const int32_t *__restrict__ conn,
+                                                      const int32_t *__restrict__ edofs,
+                                                      const uint8_t *__restrict__ cons, const double *__restrict__ u,
+                                                      const double *__restrict__ lam, int64_t ne,
+                                                      double *__restrict__ grad, int *__restrict__ err) {
+  constexpr int NF = 5, ST = 27 * NF;
+  __shared__ double s_f[kH27PerWave * ST];
+  const int lane = threadIdx.x;
+  const H27Slots sl(lane);
+  const H27Lane L(lane);
+  const int64_t total = ne * 27, groups = (ne + kH27PerWave - 1) / kH27PerWave;
+  int32_t nd[3], dof[3];
+  sl.ids(conn, (int64_t)blockIdx.x * kH27PerWave, total, lane, nd);
+  sl.ids(edofs, (int64_t)blockIdx.x * kH27PerWave, total, lane, dof);
+  for (int64_t gr = blockIdx.x; gr < groups; gr += gridDim.x) {
+    const int64_t e = gr * kH27PerWave + L.el;
+#pragma unroll
+    for (int m = 0; m < 3; ++m)
+      if (sl.live[m]) {
+        double *d = s_f + sl.el[m] * ST + sl.lat[m] * NF;
+        const double *x = xyz + 3 * (int64_t)nd[m];
+        // all loads issued before the mask is looked at
+        const double um = u[dof[m]], lm = lam[dof[m]];
+        const bool c = cons[dof[m]] != 0;
+        d[0] = x[0];
+        d[1] = x[1];
+        d[2] = x[2];
+        d[3] = c ? 0.0 : um;
+        d[4] = c ? 0.0 : lm;
+      }
+    sl.ids(conn, (gr + gridDim.x) * kH27PerWave, total, lane, nd);
+    sl.ids(edofs, (gr + gridDim.x) * kH27PerWave, total, lane, dof);
+    const bool on = L.el < kH27PerWave && e < ne;
+    h27_sync();
+    double s = 0.0;
+    if (on) {
+      double g[3][NF][3], none[3][1];
+      h27_refgrad<NF, 0>(s_f + L.el * ST, L, g, none);
+#pragma unroll
+      for (int q = 0; q < 3; ++q) {
+        double J[3][3], c[3][3];
+#pragma unroll
+        for (int r = 0; r < 3; ++r)
+#pragma unroll
+          for (int k = 0; k < 3; ++k) J[r][k] = g[q][k][r];
+        const double det = cofactors(J, c);
+        if (!(det > 0.0)) atomicOr(err, 1);
+        double t = 0.0;
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+          const double gu = g[q][3][0] * c[0][k] + g[q][3][1] * c[1][k] + g[q][3][2] * c[2][k];
+          const double gl = g[q][4][0] * c[0][k] + g[q][4][1] * c[1][k] + g[q][4][2] * c[2][k];
+          t += gu * gl;
+        }
+        s += L.w12 * h27_w(q) / det * t;
+      }
+    }
+    // sum of the element's nine columns in a fixed order
+    s += __shfl(s, lane + 3) + __shfl(s, lane + 6);
+    const double s1 = __shfl(s, lane + 1), s2 = __shfl(s, lane + 2);
+    if (on && L.l == 0) grad[e] = -(s + s1 + s2);
+    h27_sync();
+  }
+}
+
+static int h27_grid(lmh_context *ctx, int64_t ne) {
+  return grid_for((ne + kH27PerWave - 1) / kH27PerWave, 1, ctx->cu_count * 32);
+}
+
+int hex27_residual(lmh_context *ctx, const lmh_mesh *m, const lmh_dofmap *dm, const double *kappa, int f_kind,
+                   const double *u, double *Fe) {
+  if (m->n_elem == 0) return LMH_OK;
+  const int g = h27_grid(ctx, m->n_elem);
+  if (f_kind == 0)
+    LMH_LAUNCH(ctx, "element_residual", k_hex27_residual<0>, dim3(g), dim3(64), 0, m->xyz, m->conn, dm->edofs, kappa,
+               u, m->n_elem, Fe, ctx->d_flags);
+  else
+    LMH_LAUNCH(ctx, "element_residual", k_hex27_residual<1>, dim3(g), dim3(64), 0, m->xyz, m->conn, dm->edofs, kappa,
+               u, m->n_elem, Fe, ctx->d_flags);
+  return check_launch("k_hex27_residual");
+}
+
+int hex27_qoi(lmh_context *ctx, const lmh_mesh *m, double lo, double hi, double *Q) {
+  if (m->n_elem == 0) return LMH_OK;
+  LMH_LAUNCH(ctx, "qoi_box", k_hex27_qoi, dim3(h27_grid(ctx, m->n_elem)), dim3(64), 0, m->xyz, m->conn, m->n_elem, lo,
+             hi, Q, ctx->d_flags);
+  return check_launch("k_hex27_qoi");
+}
+
+int hex27_adjoint(lmh_context *ctx, const lmh_mesh *m, const lmh_dofmap *dm, const double *u, const double *lam,
+                  double *grad) {
+  if (m->n_elem == 0) return LMH_OK;
+  LMH_LAUNCH(ctx, "adjoint_kappa", k_hex27_adjoint, dim3(h27_grid(ctx, m->n_elem)), dim3(64), 0, m->xyz, m->conn,
+             dm->edofs, dm->cons, u, lam, m->n_elem, grad, ctx->d_flags);
+  return check_launch("k_hex27_adjoint");
+}
+
+}  // namespace lmh

@@ -58,14 +58,16 @@ int set_error(int code, const char *fmt, ...);
 
 // ---- FE reference tables (QGauss + Lagrange shapes) -------------------------
 // Layout (all FP64): w[nq], phi[n*nq] (phi[a*nq+q]), dref[n*nq*3]
-// (dref[(a*nq+q)*3+r]).
+// (dref[(a*nq+q)*3+r]), then one record of 1 + 4n values per point (w, phi[n],
+// dref[n][3]) for kernels that walk the points with wave-uniform reads.
 struct FETable {
   int type = 0, n = 0, nq = 0, arg = 0;
   std::vector<double> w, phi, dref, qp;
-  double *d_data = nullptr;  // device copy: w | phi | dref
+  double *d_data = nullptr;  // device copy: w | phi | dref | point records
   const double *d_w() const { return d_data; }
   const double *d_phi() const { return d_data + nq; }
   const double *d_dref() const { return d_data + nq + (size_t)n * nq; }
+  const double *d_points() const { return d_data + nq + (size_t)n * nq * 4; }
 };
 // Build the table for an element type; arg = points per direction (hex) or
 // QGauss order (tet).  Returns false for unsupported combinations.
@@ -260,6 +262,27 @@ int release_constraints(lmh_constraints &c);
 __device__ inline double qp_map(const double *X, const double *dref, int n, int nq, int q, double G[3][3]) {
   return lmh_qp_map(X, dref, n, nq, q, G);
 }
+
+// f of the right-hand side (f_kind 0: 1, 1: 3 pi^2 sin(pi x) sin(pi y) sin(pi z));
+// sinpi needs no argument reduction by pi
+__device__ inline double forcing(int f_kind, double x, double y, double z) {
+  if (f_kind == 0) return 1.0;
+  const double pi = 3.14159265358979323846264338327950288;
+  return 3.0 * pi * pi * sinpi(x) * sinpi(y) * sinpi(z);
+}
+
+// ---- element kernels without an element matrix (lmh_hex27.hip: HEX27 with the
+// 3^3 rule; lmh_thread_elem.hip: TET4, TET10, HEX8 with any rule) ----
+int hex27_residual(lmh_context *ctx, const lmh_mesh *m, const lmh_dofmap *dm, const double *kappa, int f_kind,
+                   const double *u, double *Fe);
+int hex27_qoi(lmh_context *ctx, const lmh_mesh *m, double lo, double hi, double *Q);
+int hex27_adjoint(lmh_context *ctx, const lmh_mesh *m, const lmh_dofmap *dm, const double *u, const double *lam,
+                  double *grad);
+int thread_residual(lmh_context *ctx, const FETable *t, const lmh_mesh *m, const lmh_dofmap *dm, const double *kappa,
+                    int f_kind, const double *u, double *Fe);
+int thread_qoi(lmh_context *ctx, const FETable *t, const lmh_mesh *m, double lo, double hi, double *Q);
+int thread_adjoint(lmh_context *ctx, const FETable *t, const lmh_mesh *m, const lmh_dofmap *dm, const double *u,
+                   const double *lam, double *grad);
 
 // MI355X dispatches workgroups round-robin over its 8 XCDs; remap so each XCD
 // owns one contiguous range of logical blocks (its L2 then holds the data its

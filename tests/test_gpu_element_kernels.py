@@ -1,0 +1,65 @@
+"""GPU parity of the element kernels at the edges of their work split, against
+the CPU oracle: residual, QoI derivative and adjoint gradient without an
+element matrix (HEX27: seven elements per wavefront; TET4, TET10, HEX8: one
+element per thread, 64 per workgroup), all quadrature rules they accept.
+
+Bar 1e-12 normwise (max|a - b| / max|b|), as for the other FP64 element
+results: an entry sums at most 27 points x 27 nodes x 9 products, so its
+rounding is below a few hundred ulps (1e-13) of the largest entry.
+"""
+import numpy as np
+import pytest
+
+import libmesh_amd as L
+import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+SEED = 0x5EED0011
+
+
+def rel(a, b):
+    return np.abs(a - b).max() / max(np.abs(b).max(), 1e-300)
+
+
+def problem(ctx, t, box):
+    p = L.Problem(box[0], t, 1, L.ALL_FACES, box[1], box[2])
+    m = O.Mesh(box[0], t, box[1], box[2])
+    frac = 0.2 if t in (L.HEX8, L.HEX27) else 0.02
+    p.perturb(SEED, frac)
+    m.perturb(SEED, frac)
+    return p, O.System(m), L.lognormal(p.n_elem, SEED + 1)
+
+
+# (type, rule, box): one element, whole groups, one over, ragged
+CASES = [(L.HEX27, 3, (1, 1, 1)), (L.HEX27, 3, (7, 1, 1)), (L.HEX27, 3, (2, 2, 2)), (L.HEX27, 3, (5, 3, 7)),
+         (L.HEX27, 2, (3, 1, 2)), (L.HEX8, 2, (1, 1, 1)), (L.HEX8, 2, (8, 8, 1)), (L.HEX8, 2, (13, 5, 1)),
+         (L.HEX8, 3, (3, 4, 5)), (L.TET4, 3, (1, 1, 1)), (L.TET4, 3, (2, 2, 2)), (L.TET4, 5, (3, 1, 1)),
+         (L.TET4, 1, (3, 2, 1)), (L.TET10, 5, (1, 1, 1)), (L.TET10, 5, (3, 2, 1)), (L.TET10, 3, (2, 1, 4)),
+         (L.TET10, 2, (1, 1, 3))]
+
+
+@pytest.mark.parametrize("t,npts,box", CASES)
+def test_matrix_free_element_kernels(ctx, t, npts, box):
+    p, s, kappa = problem(ctx, t, box)
+    g = L.GpuProblem.from_problem(ctx, p)
+    rng = np.random.default_rng(SEED)
+    u, lam = rng.standard_normal(p.n_dofs), rng.standard_normal(p.n_dofs)
+    kd = L.DeviceArray(ctx, p.n_elem, data=kappa)
+    ud, ld = L.DeviceArray(ctx, p.n_dofs, data=u), L.DeviceArray(ctx, p.n_dofs, data=lam)
+    out, grad = L.DeviceArray(ctx, p.n_dofs), L.DeviceArray(ctx, p.n_elem)
+    for f_kind in (0, 1):
+        g.residual_poisson(npts, kd, f_kind, ud, out)
+        assert rel(out.download(), s.residual_poisson(npts, u, kappa, f_kind)) < 1e-12, f_kind
+    g.residual_poisson(npts, None, 0, ud, out)
+    assert rel(out.download(), s.residual_poisson(npts, u)) < 1e-12
+    g.qoi_box_derivative(npts, 0.21, 0.93, out)  # faces away from every rule's points
+    assert rel(out.download(), s.qoi_box_derivative(npts, 0.21, 0.93)) < 1e-12
+    g.adjoint_kappa_gradient(npts, kd, ud, ld, grad)
+    free = p.constrained == 0
+    Ke, _ = s.element_poisson(npts, None, 0, constrain=False)
+    ue, le = (u * free)[p.elem_dofs], (lam * free)[p.elem_dofs]
+    ex = -np.einsum("ei,eij,ej->e", le, Ke, ue)
+    scale = np.einsum("ei,eij,ej->e", np.abs(le), np.abs(Ke), np.abs(ue)).max()
+    assert np.abs(grad.download() - ex).max() <= 1e-12 * scale
+    g.close()
