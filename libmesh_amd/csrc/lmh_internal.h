@@ -278,6 +278,9 @@ int hex27_residual(lmh_context *ctx, const lmh_mesh *m, const lmh_dofmap *dm, co
 int hex27_qoi(lmh_context *ctx, const lmh_mesh *m, double lo, double hi, double *Q);
 int hex27_adjoint(lmh_context *ctx, const lmh_mesh *m, const lmh_dofmap *dm, const double *u, const double *lam,
                   double *grad);
+template <typename CT>
+int thread_poisson(lmh_context *ctx, const FETable *t, const lmh_mesh *m, const lmh_dofmap *dm, const double *kappa,
+                   int f_kind, int constrain, CT *Ke, double *Fe);
 int thread_residual(lmh_context *ctx, const FETable *t, const lmh_mesh *m, const lmh_dofmap *dm, const double *kappa,
                     int f_kind, const double *u, double *Fe);
 int thread_qoi(lmh_context *ctx, const FETable *t, const lmh_mesh *m, double lo, double hi, double *Q);

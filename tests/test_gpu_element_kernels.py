@@ -1,7 +1,8 @@
 """GPU parity of the element kernels at the edges of their work split, against
 the CPU oracle: residual, QoI derivative and adjoint gradient without an
 element matrix (HEX27: seven elements per wavefront; TET4, TET10, HEX8: one
-element per thread, 64 per workgroup), all quadrature rules they accept.
+element per thread, 64 per workgroup) and the element matrices, all quadrature
+rules they accept.
 
 Bar 1e-12 normwise (max|a - b| / max|b|), as for the other FP64 element
 results: an entry sums at most 27 points x 27 nodes x 9 products, so its
@@ -62,4 +63,26 @@ def test_matrix_free_element_kernels(ctx, t, npts, box):
     ex = -np.einsum("ei,eij,ej->e", le, Ke, ue)
     scale = np.einsum("ei,eij,ej->e", np.abs(le), np.abs(Ke), np.abs(ue)).max()
     assert np.abs(grad.download() - ex).max() <= 1e-12 * scale
+    g.close()
+
+
+@pytest.mark.parametrize("t,npts,box", CASES + [(L.HEX8, 2, (26, 26, 25)), (L.HEX8, 2, (33, 1, 1))])
+def test_element_matrices(ctx, t, npts, box):
+    """Element matrices and vectors (constrained and not, with and without
+    kappa, both forcings), and the FP32 operator: each entry rounded once to
+    FP32, then at most 24 of them added in FP32 (24 * 6e-8 < 2e-6)."""
+    p, s, kappa = problem(ctx, t, box)
+    g = L.GpuProblem.from_problem(ctx, p)
+    kd = L.DeviceArray(ctx, p.n_elem, data=kappa)
+    Ke, Fe = L.DeviceArray(ctx, p.n_elem * p.npe ** 2), L.DeviceArray(ctx, p.n_elem * p.npe)
+    for f_kind, k, kh, con in ((0, kd, kappa, True), (1, kd, kappa, False), (1, None, None, True)):
+        g.element_poisson(npts, k, f_kind, Ke, Fe, constrain=con)
+        oK, oF = s.element_poisson(npts, kh, f_kind, constrain=con)
+        assert rel(Ke.download(), oK.ravel()) < 1e-12, (f_kind, con)
+        assert rel(Fe.download(), oF.ravel()) < 1e-12, (f_kind, con)
+    b = L.DeviceArray(ctx, p.n_dofs)
+    vals, rhs = s.assemble_poisson(npts, kappa, 1)
+    g.assemble_poisson(npts, kd, 1, b, L.FP32)
+    assert rel(g.values_fp32().astype(np.float64), vals) < 2e-6
+    assert rel(b.download(), rhs) < 1e-12
     g.close()
