@@ -336,10 +336,10 @@ int lmh_matrix_make_fp32(lmh_matrix *A);
  * 1016 entries and 256 distinct columns (5 bytes per entry with the FP32
  * value instead of 8, 9 with the FP64 value instead of 12), else 16-bit on
  * the 2048-entry blocks, whenever every block fits; x is gathered once per
- * distinct column.  Off keeps the int32 CSR columns.  Built with the matrix;
- * used by the FP32 inner iterations of lmh_mixed_solve and by the iterations
- * of lmh_cg_solve.  Row sums are bit-identical either way; the CG's (p, Ap)
- * partials follow the block partition, so solves agree to rounding.
+ * distinct column.  Off keeps the int32 CSR columns.  Built with the matrix
+ * (one index array for FP64 values and one for FP32); used by every product:
+ * lmh_spmv, lmh_spmv_fp32, lmh_residual and the solvers.  Row blocks and sums
+ * are the same either way, so results are bit-identical.
  * lmh_matrix_fp32_compression reports 1 when the compressed columns are in
  * use, 0 otherwise; lmh_matrix_window_bits their index width (8 or 16, 0 when
  * not in use). */

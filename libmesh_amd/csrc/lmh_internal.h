@@ -178,19 +178,22 @@ struct lmh_matrix {
   double *vals_t = nullptr;
   // Column compression of the SpMV operators (x windows): each row block of
   // the window partition rbw lists its distinct columns once, sorted, as
-  // 16-bit offsets woff16[w0 .. w0+nu), col = off + (off <= s0 ? b0 : base1);
-  // every entry stores the index of its column in that list, 8-bit (blocks of
-  // at most 1024 entries and 256 distinct columns) or else 16-bit (the
-  // 2048-entry SpMV blocks, up to 768 columns).  rbmeta[2bk] = {r0, r1, k0,
-  // cnt} (the block's rows and entries), rbmeta[2bk+1] = {b0, base1, s0 | nu << 16, w0}.
+  // 16-bit offsets, col = off + (off <= s0 ? b0 : base1); every entry stores
+  // the index of its column in that list, 8-bit (blocks of at most 1024
+  // entries and 256 distinct columns) or else 16-bit (the 2048-entry SpMV
+  // blocks, up to 768 columns).  A block's indices fill 1024 (2048) slots of
+  // widx32 / widx64, ordered so that a thread's eight are adjacent: for FP32
+  // values its chunks are 4 entries, for FP64 2.  Offsets start at woff16[w0]:
+  // 8-bit, 256 slots per block, window u at 2 (u % 128) + u / 128; 16-bit, nu
+  // consecutive ones.  rbmeta[2bk] = {r0, r1, k0, cnt} (the block's rows and
+  // entries), rbmeta[2bk+1] = {b0, base1, s0 | nu << 16, w0}.
   int fp32_index = 1;          // 1: use the compressed columns when they fit
   int idx16_state = 0;         // 0 not built, 1 built, -1 does not fit
   int wbits = 0;               // 8 or 16 once built
   int32_t *rbw = nullptr;      // window partition (nrbw + 1 row boundaries)
   int64_t nrbw = 0;
-  uint8_t *widx8 = nullptr;    // nnz: 8-bit window index of each entry's column
-  uint16_t *widx16 = nullptr;  // nnz: 16-bit window index of each entry's column
-  uint16_t *woff16 = nullptr;  // sum of nu over the row blocks
+  void *widx32 = nullptr, *widx64 = nullptr;  // window indices (widx64 with FP64 values only)
+  uint16_t *woff16 = nullptr;  // window offsets
   int4 *rbmeta = nullptr;      // 2 nrbw
   uint16_t *off = nullptr;  // n_elem*dpe*dpe slot offsets within rows
   int32_t *diag = nullptr;  // rows: position of the diagonal entry, -1 if absent
@@ -273,6 +276,9 @@ __device__ inline double forcing(int f_kind, double x, double y, double z) {
 
 // ---- element kernels without an element matrix (lmh_hex27.hip: HEX27 with the
 // 3^3 rule; lmh_thread_elem.hip: TET4, TET10, HEX8 with any rule) ----
+template <typename CT>
+int hex27_poisson(lmh_context *ctx, const lmh_mesh *m, const lmh_dofmap *dm, const double *kappa, int f_kind,
+                  int constrain, CT *Ke, double *Fe);
 int hex27_residual(lmh_context *ctx, const lmh_mesh *m, const lmh_dofmap *dm, const double *kappa, int f_kind,
                    const double *u, double *Fe);
 int hex27_qoi(lmh_context *ctx, const lmh_mesh *m, double lo, double hi, double *Q);

@@ -218,228 +218,299 @@ __device__ inline void rowblock_spmv(const int32_t *__restrict__ rb, int64_t nrb
   }
 }
 
-// FP32 values with x windows.  A row block of ~2000 entries references only a
-// few hundred distinct columns (about 300 for Q2 hexahedra, under 520 for every
-// Lagrange type here), so the block's x values are gathered once, in sorted
-// column order, into an LDS window, and each entry reads its x there through a
-// 16-bit window index.  The sorted gather touches each x cache line about once
-// per block instead of once per entry that uses it.  Values are read as 16-byte
-// chunks and the window indices as 8-entry chunks, both from the block's start
-// rounded down to 8 entries; the indices pass through LDS, so every product
-// lands at its entry's slot and the rows are reduced exactly as in
-// rowblock_spmv (same products, same summation order, bit-identical sums).
-// Row blocks hold at most RB_CAP - 8 entries, so a block's chunks fit one
-// 8-entry index chunk and two 4-entry value chunks per thread.
-// T = double (the FP64 operator) runs the same scheme with 2-entry value
-// chunks; products and sums are formed as in rowblock_spmv<double>, so the
-// FP64 results are bit-identical to the int32-column kernel too.
+// Row sums of an 8-lane group: lanes 0..3 take lane + 4, then pairs and
+// neighbours within the quad (the tree ((0+4)+(2+6))+((1+5)+(3+7))), valid in
+// the group's lane 0.  DPP moves instead of LDS permutes: no wait on LDS.
+template <int CTRL, typename T>
+__device__ inline T dpp_move(T v) {
+  if constexpr (sizeof(T) == 4) {
+    return __builtin_bit_cast(
+        T, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
+  } else {
+    typedef int i32x2 __attribute__((ext_vector_type(2)));
+    i32x2 w = __builtin_bit_cast(i32x2, v);
+    w[0] = __builtin_amdgcn_update_dpp(0, w[0], CTRL, 0xf, 0xf, true);
+    w[1] = __builtin_amdgcn_update_dpp(0, w[1], CTRL, 0xf, 0xf, true);
+    return __builtin_bit_cast(T, w);
+  }
+}
+template <typename T>
+__device__ inline T group8_sum(T s) {
+  s += dpp_move<0x104>(s);  // row_shl:4
+  s += dpp_move<0x4e>(s);   // quad_perm [2,3,0,1]
+  s += dpp_move<0xb1>(s);   // quad_perm [1,0,3,2]
+  return s;
+}
+
+// Streamed row blocks.  A row block of ~1000 entries references only a few
+// hundred distinct columns (about 200 for Q2 hexahedra), so the block's x
+// values are gathered once, in sorted column order, into an LDS window, and
+// each entry reads its x there through an 8- or 16-bit window index: the
+// sorted gather touches each x cache line about once per block instead of once
+// per entry that uses it.  IW = 4 is the same walk with the int32 columns and
+// a gather per entry (no window): same products, same row sums, same partition
+// of rows over threads, so a solve does not depend on which of the two runs.
+// Values are read as 16-byte chunks and the indices of a chunk together, both
+// from the block's start rounded down to 8 entries; the products land at their
+// entry's slot in LDS and every row is summed by 8 lanes, entry t by lane
+// (t - a) % 8, in ascending order, then by the tree of group8_sum -- the sums
+// of rowblock_spmv, bit for bit.  Row blocks hold at most CAPW - 8 entries.
+//
+// What bounds it: the value stream (plain reads of the same arrays reach 6.9
+// TB/s here) and the number of vector memory instructions beside it: a thread's
+// eight window indices are stored adjacent (one load; they took two to four)
+// and its two window offsets too, and the workgroups of an XCD walk its blocks
+// side by side.  64^3 Q2 (135,005,697 entries): FP32 177 -> 155 us, FP64 292 ->
+// 265 us per CG product, FP64 products that used the int32 columns 352 -> 254
+// us, refresh residual 374 -> 264 us.  Without the x gathers the same kernel
+// takes 140 / 235 us; eight consecutive FP64 entries per thread (one index
+// array for both precisions) 300 us.  A block's loads are issued one block
+// ahead: descriptor three ahead (scalar), window offsets two ahead and first in
+// the iteration, so that waiting for them does not wait for the value stream;
+// then the next block's window gathers, values, indices and row data; then the
+// current block's LDS phases.  Two register sets alternate (no copies).
+// Slots a chunk holds outside its block multiply an unread window slot: their
+// products are never read, so no index is masked (8- and 16-bit indices stay
+// inside the window array: it has UC slots and indices below UC).
+//
+// pre(row, out): the NPRE values of a row the epilogue needs, loaded with the
+// block's stream; epi(row, sum, values) consumes each row in one thread.
+// CAPW: block capacity; IW: index bytes; NT: threads per workgroup.
 typedef uint32_t vu4 __attribute__((ext_vector_type(4)));
-constexpr int UCAP = 768;  // distinct columns of one row block (x window)
-// 8-bit windows: blocks of at most W8_CAP - 8 entries and 256 distinct columns
-// (a Q2 hexahedral operator's 1024-entry blocks hold about 200); an entry then
-// costs one index byte instead of two
+constexpr int UCAP = 768;  // distinct columns of one 2048-entry row block (x window)
+// 8-bit windows: blocks of at most W8_CAP - 8 entries and 256 distinct columns;
+// they run on 128-thread workgroups, twice as many of them
 constexpr int W8_CAP = 1024, W8_UCAP = 256;
-// 8-bit blocks run on 128-thread workgroups (8 entries per thread, as the
-// 2048-entry blocks on 256 threads), twice as many of them
 #ifndef LMH_W8_GRID
 #define LMH_W8_GRID 2
 #endif
 constexpr int W8_NT = 128, W8_GRID = LMH_W8_GRID;
 template <int IW>
-using widx_t = typename std::conditional<IW == 1, uint8_t, uint16_t>::type;
-// Pipelining.  Every block's loads are addressed from registers only, so no
-// load waits on another in flight: a 32-byte descriptor per block (rows,
-// entry range, window meta, built with the windows) is loaded three blocks
-// ahead, the block's window offsets two blocks ahead, and its values, window
-// indices, row pointers and x-window gathers one block ahead, while the
-// current block runs its LDS phases.
-// CAPW: the block capacity (RB_CAP with 16-bit indices, W8_CAP with 8-bit);
-// IW: index bytes per entry; NT: threads per workgroup.
-template <typename T, bool DOT, int CAPW = RB_CAP, int IW = 2, int NT = BLK>
-__device__ inline double rowblock_spmv16(int64_t nrb, const int4 *__restrict__ desc, const int32_t *__restrict__ rp,
-                                         const widx_t<IW> *__restrict__ widx, const uint16_t *__restrict__ woff,
-                                         const T *__restrict__ v, const T *__restrict__ x, T *__restrict__ y) {
+using widx_t = typename std::conditional<IW == 1, uint8_t,
+                                         typename std::conditional<IW == 2, uint16_t, int32_t>::type>::type;
+
+template <typename T, int NPRE, int CAPW, int IW, int NT, typename Pre, typename Epi>
+__device__ inline void rowblock_spmv16(int64_t nrb, const int4 *__restrict__ desc, const int32_t *__restrict__ rp,
+                                       const widx_t<IW> *__restrict__ widx, const uint16_t *__restrict__ woff,
+                                       const T *__restrict__ v, const T *__restrict__ x, Pre &&pre, Epi &&epi) {
   constexpr int CH = 16 / sizeof(T);  // entries per 16-byte value chunk
   typedef T vch __attribute__((ext_vector_type(CH)));
-  // the chunk's CH window indices (IW * CH bytes: 8 for FP32 16-bit, 4 for
-  // FP64 16-bit and FP32 8-bit, 2 for FP64 8-bit)
-  typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-  typedef typename std::conditional<
-      IW * CH == 8, u32x2, typename std::conditional<IW * CH == 4, uint32_t, uint16_t>::type>::type ich;
-  constexpr int UC = IW == 1 ? W8_UCAP : UCAP;
-  // products at their chunk positions from the block's start rounded down to 8
-  // entries (slots outside the block hold unread values)
-  __shared__ __attribute__((aligned(16))) T prod[CAPW];
-  __shared__ T xw[UC];
-  // Row offsets and the x of the block's rows (for the (x, Ax) partials).
-  // FP32: double-buffered, written before the first barrier.  FP64: one
-  // buffer, written after it (the previous block's rows are reduced by then),
-  // which keeps the LDS under 32 KB for 5 resident workgroups per CU.
+  typedef widx_t<IW> ich __attribute__((ext_vector_type(IW < 4 ? 8 : CH)));
+  constexpr bool WIN = IW < 4;
+  constexpr int UC = !WIN ? NT : (IW == 1 ? W8_UCAP : UCAP);
+  constexpr int PER = CAPW / NT, UPER = UC / NT, NCH = PER / CH, NP = NPRE > 0 ? NPRE : 1;
+  static_assert(PER == 8 && UC % NT == 0, "eight entries per thread, whole window slots");
+  // entry (from the block's start) of value chunk j; the thread's eight window
+  // indices are stored together in this order (k_build_windows)
+  auto at = [](int j) { return (uint32_t)(CH * threadIdx.x + CH * NT * j); };
+  __shared__ __attribute__((aligned(16))) T prod[CAPW + 32];  // + the reach of an unrolled row sum
+  __shared__ T xw[WIN ? UC : 1];
+  // Row offsets and row values.  FP32: double-buffered, written before the
+  // first barrier.  FP64: one buffer, written after it (the previous block's
+  // rows are summed by then), for more resident workgroups per CU.
   constexpr int NB = sizeof(T) == 8 ? 1 : 2;
   __shared__ int32_t rowbuf[NB][NT];
-  __shared__ T xrow[NB][NT];
-  constexpr int PER = CAPW / NT, UPER = UC / NT, NCH = PER / CH;
-  static_assert(PER % CH == 0 && UC % NT == 0, "whole value chunks and window slots per thread");
-  int64_t lo, hi;
-  block_range(nrb, lo, hi);
-  double acc = 0;
-  if (lo >= hi) return acc;
-  const int tid = threadIdx.x;
-  // descriptor of block bk (clamped to the workgroup's last block): geometry
-  // {r0, r1, k0, cnt} and window {b0, b1, s0 | nu << 16, w0}
-  auto dsc = [&](int64_t bk, int4 &g, int4 &w) {
-    const int64_t b = bk < hi ? bk : hi - 1;
-    g = desc[2 * b];
-    w = desc[2 * b + 1];
+  __shared__ double prebuf[NB][NP][NPRE > 0 ? NT : 1];
+  // this workgroup's blocks: every XCD owns one contiguous range of blocks and
+  // its workgroups walk it side by side (workgroup j takes j, j + step, ...).
+  int64_t lo, hi, step_b;
+  if (gridDim.x % NXCD == 0) {
+    const int64_t xcd = blockIdx.x % NXCD;
+    lo = nrb * xcd / NXCD + blockIdx.x / NXCD;
+    hi = nrb * (xcd + 1) / NXCD;
+    step_b = gridDim.x / NXCD;
+  } else {
+    lo = blockIdx.x;
+    hi = nrb;
+    step_b = gridDim.x;
+  }
+  if (lo >= hi) return;
+  const int tid = threadIdx.x, sub = tid & 7, grp = tid >> 3;
+  struct Blk {
+    int4 G, W;  // {r0, r1, k0, cnt}, {b0, b1, s0 | nu << 16, w0}
+    vch vv[NCH];
+    ich iv[IW < 4 ? 1 : NCH];
+    int32_t b, rpn;
+    T xu[UPER];
+    double pv[NP];
+  };
+  // descriptor of block bk (past the end: the workgroup's first)
+  auto dsc = [&](int64_t bk, int4 &g, int4 &w, int32_t &b) {
+    b = (int32_t)(bk < hi ? bk : lo);
+    g = desc[2 * (int64_t)b];
+    w = desc[2 * (int64_t)b + 1];
   };
   // branch-free loads: out-of-range slots re-read a valid address and are dropped
   auto load_woff = [&](const int4 &W, uint32_t(&uo)[UPER]) {
-    const int32_t nu = W.z >> 16;
+    if constexpr (IW == 1) {  // padded pairs (u, u + NT): one load
+      const uint32_t pr = __builtin_nontemporal_load((const uint32_t *)(woff + W.w) + threadIdx.x);
+      uo[0] = pr & 0xffff;
+      uo[1] = pr >> 16;
+    } else if constexpr (WIN) {
+      const int32_t nu = W.z >> 16;
+      const uint16_t *wo = woff + W.w;
 #pragma unroll
-    for (int j = 0; j < UPER; ++j) {
-      const int32_t u = tid + j * NT;
-      uo[j] = __builtin_nontemporal_load(&woff[W.w + (u < nu ? u : 0)]);
+      for (int j = 0; j < UPER; ++j) {
+        const int32_t u = tid + j * NT;
+        uo[j] = __builtin_nontemporal_load(&wo[(uint32_t)(u < nu ? u : 0)]);
+      }
     }
   };
-  auto gather = [&](const int4 &G, const int4 &W, const uint32_t(&uo)[UPER], T(&xu)[UPER], T &xo) {
-    const int32_t NU = W.z >> 16, S0 = W.z & 0xffff;
+  auto fetch = [&](Blk &B, const uint32_t(&uo)[UPER]) {
+    const int32_t r0 = B.G.x, nr = B.G.y - B.G.x, k0 = B.G.z, cnt = B.G.w;
+    if constexpr (WIN) {
+      const int32_t nu = B.W.z >> 16, s0 = B.W.z & 0xffff;
 #pragma unroll
-    for (int j = 0; j < UPER; ++j) {
-      const int32_t u = tid + j * NT, o = (int32_t)uo[j];
-      xu[j] = x[u < NU ? o + (o <= S0 ? W.x : W.y) : 0];
+      for (int j = 0; j < UPER; ++j) {
+        const int32_t u = tid + j * NT, o = (int32_t)uo[j];
+        // a byte offset below 2^32 (the launch checks the vector's size): one 32-bit register per address
+        const uint32_t off = (uint32_t)(u < nu ? o + (o <= s0 ? B.W.x : B.W.y) : 0) * (uint32_t)sizeof(T);
+        B.xu[j] = *(const T *)((const char *)x + off);
+      }
     }
-    if (DOT) xo = x[G.x + (tid < G.y - G.x ? tid : 0)];
-  };
-  auto fetch = [&](const int4 &G, vch(&vv)[NCH], ich(&iv)[NCH], int32_t &rpn) {
-    const int32_t r0 = G.x, r1 = G.y, k0 = G.z, cnt = G.w;
-    rpn = rp[r0 + (tid <= r1 - r0 ? tid : 0)];
     const int32_t a0 = k0 & ~7, span = (k0 - a0) + cnt;
+    const T *va = v + a0;
 #pragma unroll
     for (int j = 0; j < NCH; ++j) {
-      const int32_t c = CH * tid + CH * NT * j;  // chunks starting past the block re-read chunk 0
-      const int32_t o = c < span ? c : 0;
-      vv[j] = __builtin_nontemporal_load((const vch *)(v + a0 + o));
-      iv[j] = __builtin_nontemporal_load((const ich *)(widx + a0 + o));
+      const uint32_t c = at(j);  // chunks starting past the block re-read chunk 0
+      B.vv[j] = __builtin_nontemporal_load((const vch *)(va + ((int32_t)c < span ? c : 0)));
+    }
+    if constexpr (WIN) {
+      B.iv[0] = __builtin_nontemporal_load((const ich *)(widx + (int64_t)B.b * CAPW) + threadIdx.x);
+    } else {
+#pragma unroll
+      for (int j = 0; j < NCH; ++j) {
+        const uint32_t c = at(j);
+        B.iv[j] = __builtin_nontemporal_load((const ich *)(widx + a0 + ((int32_t)c < span ? c : 0)));
+      }
+    }
+    const int32_t *ra = rp + r0;
+    B.rpn = ra[(uint32_t)(tid <= nr ? tid : 0)];
+    if (NPRE > 0) pre(r0 + (tid < nr ? tid : 0), B.pv);
+  };
+  int buf = 0;
+  // the entries' x without a window: gathered before the next block's loads
+  auto gather = [&](const Blk &B, T(&xs)[PER]) {
+    if constexpr (!WIN) {
+      const int32_t lead = B.G.z & 7, cnt = B.G.w;
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        const int32_t t = (int32_t)at(k / CH) + k % CH - lead;
+        xs[k] = x[t >= 0 && t < cnt ? B.iv[k / CH][k % CH] : 0];
+      }
     }
   };
-  // current block (c), the next (n), the one after (nn)
-  int4 Gc, Wc, Gn, Wn, Gnn, Wnn;
-  vch vvc[NCH], vvn[NCH];
-  ich ivc[NCH], ivn[NCH];
-  int32_t rpnc = 0, rpnn = 0;
-  T xuc[UPER], xun[UPER], xoc = 0, xon = 0;
-  uint32_t uon[UPER], uonn[UPER];
-  dsc(lo, Gc, Wc);
-  dsc(lo + 1, Gn, Wn);
-  dsc(lo + 2, Gnn, Wnn);
-  {
-    uint32_t uoc[UPER];
-    load_woff(Wc, uoc);
-    gather(Gc, Wc, uoc, xuc, xoc);
-  }
-  fetch(Gc, vvc, ivc, rpnc);
-  load_woff(Wn, uon);
-  int buf = 0;
-  // One block from registers: window, indices and row data to LDS, products,
-  // rows reduced in a fixed order.
-  auto compute = [&]() {
+  auto compute = [&](const Blk &B, const T(&xs)[PER]) {
     int32_t *rows = rowbuf[buf];
-    T *xr = xrow[buf];
+    double(*pb)[NPRE > 0 ? NT : 1] = prebuf[buf];
     buf ^= NB - 1;
-    const int32_t R0 = Gc.x, R1 = Gc.y, K0 = Gc.z, CNT = Gc.w, RPN = rpnc, lead = K0 & 7, A0 = K0 - lead;
-    const int32_t NU = Wc.z >> 16;
-    const bool staged = R1 - R0 < NT;
-    if (NB == 2 && staged && tid <= R1 - R0) rows[tid] = RPN - A0;
+    const int32_t R0 = B.G.x, NR = B.G.y - B.G.x, lead = B.G.z & 7, A0 = B.G.z - lead;
+    const bool staged = NR < NT;
+    auto stage_rows = [&]() {
+      if (staged && tid <= NR) rows[tid] = B.rpn - A0;
+      if (NPRE > 0)
 #pragma unroll
-    for (int j = 0; j < UPER; ++j)
-      if (tid + j * NT < NU) xw[tid + j * NT] = xuc[j];
-    if (NB == 2 && DOT) xr[tid] = xoc;
-    __syncthreads();  // window and row data visible; the previous block's rows are reduced
-    if (NB == 1 && staged && tid <= R1 - R0) rows[tid] = RPN - A0;
-    if (NB == 1 && DOT) xr[tid] = xoc;
+        for (int k = 0; k < NP; ++k) pb[k][tid] = B.pv[k];
+    };
+    if (NB == 2) stage_rows();
+    if constexpr (WIN) {
+#pragma unroll
+      for (int j = 0; j < UPER; ++j) xw[tid + j * NT] = B.xu[j];
+    }
+    __syncthreads();  // window and row data visible; the previous block's rows are summed
+    if (NB == 1) stage_rows();
 #pragma unroll
     for (int j = 0; j < NCH; ++j) {
-      vch xs;
+      vch p;
 #pragma unroll
       for (int e = 0; e < CH; ++e) {
-        const int32_t t = CH * tid + CH * NT * j + e - lead;
-        uint32_t word;
-        int sh;
-        if constexpr (IW * CH == 8) {
-          word = ivc[j][e >> 1];
-          sh = 16 * (e & 1);
-        } else {
-          word = (uint32_t)ivc[j];
-          sh = 8 * IW * e;
-        }
-        const int32_t wi = (int32_t)((word >> sh) & (IW == 1 ? 0xffu : 0xffffu));
-        xs[e] = xw[t >= 0 && t < CNT ? wi : 0];
+        if constexpr (WIN)
+          p[e] = B.vv[j][e] * xw[(uint32_t)B.iv[0][j * CH + e]];
+        else
+          p[e] = B.vv[j][e] * xs[j * CH + e];
       }
-      *(vch *)&prod[CH * tid + CH * NT * j] = vvc[j] * xs;
+      *(vch *)&prod[at(j)] = p;
     }
     __syncthreads();
-    const int g = tid >> 3, sub = tid & 7;
     if (staged) {
-      for (int32_t r = R0 + g; r < R1; r += NT / 8) {
-        const int32_t a = rows[r - R0], e = rows[r - R0 + 1];
+      for (int32_t k = grp; k < NR; k += NT / 8) {
+        const int32_t a = rows[k], e = rows[k + 1];
         T s = 0;
-        for (int32_t t = a + sub; t < e; t += 8) s += prod[t];
-        s += __shfl_xor(s, 4, 8);
-        s += __shfl_xor(s, 2, 8);
-        s += __shfl_xor(s, 1, 8);
+        for (int32_t t = a + sub; t < e; t += 32) {
+          const T p0 = prod[t], p1 = prod[t + 8], p2 = prod[t + 16], p3 = prod[t + 24];
+          s += p0;
+          s += t + 8 < e ? p1 : (T)0;
+          s += t + 16 < e ? p2 : (T)0;
+          s += t + 24 < e ? p3 : (T)0;
+        }
+        s = group8_sum(s);
         if (sub == 0) {
-          y[r] = s;
-          if (DOT) acc += (double)xr[r - R0] * (double)s;
+          double p2[NP];
+#pragma unroll
+          for (int m = 0; m < NP; ++m) p2[m] = NPRE > 0 ? pb[m][k] : 0.0;
+          epi(R0 + k, s, p2);
         }
       }
     } else {
-      for (int32_t r = R0 + g; r < R1; r += NT / 8) {
-        const int32_t a = rp[r] - A0, e = rp[r + 1] - A0;
+      for (int32_t k = grp; k < NR; k += NT / 8) {
+        const int32_t a = rp[R0 + k] - A0, e = rp[R0 + k + 1] - A0;
         T s = 0;
         for (int32_t t = a + sub; t < e; t += 8) s += prod[t];
-        s += __shfl_xor(s, 4, 8);
-        s += __shfl_xor(s, 2, 8);
-        s += __shfl_xor(s, 1, 8);
+        s = group8_sum(s);
         if (sub == 0) {
-          y[r] = s;
-          if (DOT) acc += (double)x[r] * (double)s;
+          double p2[NP];
+          pre(R0 + k, p2);
+          epi(R0 + k, s, p2);
         }
       }
     }
   };
-  for (int64_t bk = lo; bk + 1 < hi; ++bk) {
-    // the next block's x window and row x (its offsets arrived with this
-    // block's loads), then its values and indices, the offsets of the block
-    // after it and the descriptor three ahead
-    gather(Gn, Wn, uon, xun, xon);
-    fetch(Gn, vvn, ivn, rpnn);
-    load_woff(Wnn, uonn);
+  Blk A, B;
+  int4 Gnn, Wnn;
+  int32_t bnn;
+  uint32_t uo[UPER], uon[UPER];
+  T xs[PER];
+  dsc(lo, A.G, A.W, A.b);
+  dsc(lo + step_b, B.G, B.W, B.b);
+  dsc(lo + 2 * step_b, Gnn, Wnn, bnn);
+  load_woff(A.W, uo);
+  load_woff(B.W, uon);
+  fetch(A, uo);
+#pragma unroll
+  for (int j = 0; j < UPER; ++j) uo[j] = uon[j];
+  // one block: loads of the next (its offsets are in uo), then this one's LDS phases
+  auto step = [&](int64_t bk, Blk &C, Blk &N) {
+    load_woff(Wnn, uon);
+    __builtin_amdgcn_sched_barrier(0);
+    gather(C, xs);
+    fetch(N, uo);
     int4 G3, W3;
-    dsc(bk + 3, G3, W3);
-    compute();
-    Gc = Gn;
-    Wc = Wn;
+    int32_t b3;
+    dsc(bk + 3 * step_b, G3, W3, b3);
+    compute(C, xs);
 #pragma unroll
-    for (int j = 0; j < NCH; ++j) {
-      vvc[j] = vvn[j];
-      ivc[j] = ivn[j];
-    }
-    rpnc = rpnn;
-#pragma unroll
-    for (int j = 0; j < UPER; ++j) {
-      xuc[j] = xun[j];
-      uon[j] = uonn[j];
-    }
-    xoc = xon;
-    Gn = Gnn;
-    Wn = Wnn;
+    for (int j = 0; j < UPER; ++j) uo[j] = uon[j];
+    C.G = Gnn;
+    C.W = Wnn;
+    C.b = bnn;
     Gnn = G3;
     Wnn = W3;
+    bnn = b3;
+  };
+  int64_t bk = lo;
+  for (; bk + 2 * step_b < hi; bk += 2 * step_b) {
+    step(bk, A, B);
+    step(bk + step_b, B, A);
   }
-  compute();
-  return acc;
+  if (bk + step_b < hi) {
+    step(bk, A, B);
+    gather(B, xs);
+    compute(B, xs);
+  } else {
+    gather(A, xs);
+    compute(A, xs);
+  }
 }
-
 
 // ---------------------------------------------------------------------------
 // plain SpMV y = A x
@@ -469,6 +540,24 @@ __global__ __launch_bounds__(BLK) void k_residual(const int32_t *__restrict__ rb
         acc[1] += bv * bv;
       });
   publish<2>(acc, part);
+}
+
+template <int CAPW, int IW, int NT>
+__global__ __launch_bounds__(NT) void k_residual16(int64_t nrb, const int32_t *__restrict__ rp,
+                                                   const void *__restrict__ widx, const uint16_t *__restrict__ woff,
+                                                   const int4 *__restrict__ desc, const double *__restrict__ v,
+                                                   const double *__restrict__ b, const double *__restrict__ x,
+                                                   double *__restrict__ r, double *__restrict__ part) {
+  double acc[2] = {0, 0};
+  rowblock_spmv16<double, 1, CAPW, IW, NT>(
+      nrb, desc, rp, (const widx_t<IW> *)widx, woff, v, x, [&](int32_t row, double *o) { o[0] = b[row]; },
+      [&](int32_t row, double s, const double *pr) {
+        const double bv = pr[0], rv = bv - s;
+        r[row] = rv;
+        acc[0] += rv * rv;
+        acc[1] += bv * bv;
+      });
+  publish<2, NT>(acc, part);
 }
 
 // out[0] = |r|^2, out[1] = |b|^2
@@ -585,45 +674,30 @@ __global__ __launch_bounds__(BLK) void k_it_spmv(const int32_t *__restrict__ rb,
   publish<1>(acc, part);
 }
 
-// q = A32 p on the x-window FP32 operator (IW-byte window indices on blocks
-// of CAPW entries); partials (p, q).  Held to 64 VGPRs (8 waves per SIMD): the
-// pipelined loop needs every resident wave.
-template <int CAPW, int IW, int NT>
-__global__ __launch_bounds__(NT, 2048 / NT) void k_it_spmv16(int64_t nrb, const int32_t *__restrict__ rp,
-                                                          const void *__restrict__ widx,
-                                                          const uint16_t *__restrict__ woff,
-                                                          const int4 *__restrict__ desc, const float *__restrict__ v,
-                                                          const float *__restrict__ p, float *__restrict__ q,
-                                                          double *__restrict__ part, const double *__restrict__ S,
-                                                          int bank) {
+// The same on the streamed row blocks (see rowblock_spmv16).  FP32 is held to
+// 64 VGPRs (8 waves per SIMD).
+template <typename T, int CAPW, int IW, int NT>
+__global__ __launch_bounds__(NT, sizeof(T) == 4 ? 2048 / NT : 1) void k_it_spmv16(
+    int64_t nrb, const int32_t *__restrict__ rp, const void *__restrict__ widx, const uint16_t *__restrict__ woff,
+    const int4 *__restrict__ desc, const T *__restrict__ v, const T *__restrict__ p, T *__restrict__ q,
+    double *__restrict__ part, const double *__restrict__ S, int bank) {
   if (S[bank * B_SIZE + B_DONE] != 0.0) return;
-  double acc[1] = {
-      rowblock_spmv16<float, true, CAPW, IW, NT>(nrb, desc, rp, (const widx_t<IW> *)widx, woff, v, p, q)};
+  double acc[1] = {0};
+  rowblock_spmv16<T, 1, CAPW, IW, NT>(
+      nrb, desc, rp, (const widx_t<IW> *)widx, woff, v, p, [&](int32_t r, double *o) { o[0] = (double)p[r]; },
+      [&](int32_t r, T s, const double *pr) {
+        q[r] = s;
+        acc[0] += pr[0] * (double)s;
+      });
   publish<1, NT>(acc, part);
 }
 
-// q = A p on the FP64 operator through the same x windows; partials (p, q).
-// Bit-identical to k_it_spmv<double>.
-template <int CAPW, int IW, int NT>
-__global__ __launch_bounds__(NT) void k_it_spmv16d(int64_t nrb, const int32_t *__restrict__ rp,
-                                                   const void *__restrict__ widx, const uint16_t *__restrict__ woff,
-                                                   const int4 *__restrict__ desc, const double *__restrict__ v,
-                                                   const double *__restrict__ p, double *__restrict__ q,
-                                                   double *__restrict__ part, const double *__restrict__ S,
-                                                   int bank) {
-  if (S[bank * B_SIZE + B_DONE] != 0.0) return;
-  double acc[1] = {
-      rowblock_spmv16<double, true, CAPW, IW, NT>(nrb, desc, rp, (const widx_t<IW> *)widx, woff, v, p, q)};
-  publish<1, NT>(acc, part);
-}
-
-template <int CAPW, int IW, int NT>
-__global__ __launch_bounds__(NT, 2048 / NT) void k_spmv16(int64_t nrb, const int32_t *__restrict__ rp,
-                                                       const void *__restrict__ widx,
-                                                       const uint16_t *__restrict__ woff,
-                                                       const int4 *__restrict__ desc, const float *__restrict__ v,
-                                                       const float *__restrict__ x, float *__restrict__ y) {
-  rowblock_spmv16<float, false, CAPW, IW, NT>(nrb, desc, rp, (const widx_t<IW> *)widx, woff, v, x, y);
+template <typename T, int CAPW, int IW, int NT>
+__global__ __launch_bounds__(NT, sizeof(T) == 4 ? 2048 / NT : 1) void k_spmv16(
+    int64_t nrb, const int32_t *__restrict__ rp, const void *__restrict__ widx, const uint16_t *__restrict__ woff,
+    const int4 *__restrict__ desc, const T *__restrict__ v, const T *__restrict__ x, T *__restrict__ y) {
+  rowblock_spmv16<T, 0, CAPW, IW, NT>(nrb, desc, rp, (const widx_t<IW> *)widx, woff, v, x, NoPre{},
+                                      [&](int32_t r, T s, const double *) { y[r] = s; });
 }
 
 // Build the x windows, one row block per workgroup: sort the block's
@@ -642,6 +716,7 @@ template <bool COUNT, int CAP, int IW>
 __global__ __launch_bounds__(BLK) void k_build_windows(const int32_t *__restrict__ rb, int64_t nrb,
                                                        const int32_t *__restrict__ rp, const int32_t *__restrict__ ci,
                                                        int32_t *__restrict__ wsz, widx_t<IW> *__restrict__ widx,
+                                                       widx_t<IW> *__restrict__ widx64,
                                                        uint16_t *__restrict__ woff, int4 *__restrict__ meta,
                                                        int *__restrict__ bad) {
   __shared__ int64_t keys[CAP];
@@ -724,7 +799,7 @@ __global__ __launch_bounds__(BLK) void k_build_windows(const int32_t *__restrict
     } else if (COUNT) {
       if (tid == 0) wsz[bk] = nu;
     } else {
-      const int32_t w0 = wsz[bk];
+      const int32_t w0 = IW == 1 ? (int32_t)(bk * W8_UCAP) : wsz[bk];
       int32_t u = before - 1;  // window index of the last distinct column before this thread's entries
       for (int e = 0; e < PER; ++e) {
         const int i = PER * tid + e;
@@ -732,9 +807,12 @@ __global__ __launch_bounds__(BLK) void k_build_windows(const int32_t *__restrict
           const int32_t c = col(i);
           if (i == 0 || c != col(i - 1)) {
             ++u;
-            woff[w0 + u] = (uint16_t)(c <= split ? c - b0 : c - b1);
+            woff[IW == 1 ? w0 + 2 * (u & (W8_NT - 1)) + u / W8_NT : w0 + u] = (uint16_t)(c <= split ? c - b0 : c - b1);
           }
-          widx[k0 + (int32_t)(keys[i] & 4095)] = (widx_t<IW>)u;
+          // entry o from the block's start rounded down to 8, in the order its thread reads
+          const int32_t o = (int32_t)(keys[i] & 4095) + (k0 & 7), nt = CAP / 8;
+          widx[bk * CAP + 8 * ((o / 4) % nt) + 4 * (o / (4 * nt)) + o % 4] = (widx_t<IW>)u;
+          if (widx64) widx64[bk * CAP + 8 * ((o / 2) % nt) + 2 * (o / (2 * nt)) + o % 2] = (widx_t<IW>)u;
         }
       }
       if (tid == 0) {
@@ -939,6 +1017,35 @@ __global__ __launch_bounds__(BLK) void k_refresh(int init, const int32_t *__rest
   publish<3>(acc, part);
 }
 
+template <int CAPW, int IW, int NT>
+__global__ __launch_bounds__(NT) void k_refresh16(int init, int64_t nrb, const int32_t *__restrict__ rp,
+                                                  const void *__restrict__ widx, const uint16_t *__restrict__ woff,
+                                                  const int4 *__restrict__ desc, const double *__restrict__ v,
+                                                  const double *__restrict__ b, const double *__restrict__ x,
+                                                  const float *__restrict__ dinv32, float *__restrict__ r32,
+                                                  float *__restrict__ p32, double *__restrict__ part,
+                                                  const double *__restrict__ S, int bank) {
+  if (!init && S[bank * B_SIZE + B_DONE] != 0.0) return;
+  double acc[3] = {0, 0, 0};
+  rowblock_spmv16<double, 2, CAPW, IW, NT>(
+      nrb, desc, rp, (const widx_t<IW> *)widx, woff, v, x,
+      [&](int32_t row, double *o) {
+        o[0] = b[row];
+        o[1] = (double)dinv32[row];
+      },
+      [&](int32_t row, double s, const double *pr) {
+        const double bv = pr[0], rv = bv - s;
+        const float rf = (float)rv;
+        r32[row] = rf;
+        const float z = (float)pr[1] * rf;
+        if (init) p32[row] = z;
+        acc[0] += rv * rv;
+        acc[1] += bv * bv;
+        acc[2] += (double)rf * (double)z;
+      });
+  publish<3, NT>(acc, part);
+}
+
 // One block.  init: |b|^2, threshold and the starting bank; otherwise the
 // FP64 convergence test on the true residual and the restart of the FP32
 // recurrence's (r, z) for the next alpha.
@@ -1063,7 +1170,7 @@ static int try_windows(lmh_matrix *A, std::vector<int32_t> rb, bool split, bool 
     LMH_HIP(hipMemcpyAsync(rbd.p, rb.data(), sizeof(int32_t) * rb.size(), hipMemcpyHostToDevice, ctx->stream));
     LMH_HIP(hipMemsetAsync(ctx->d_flags, 0, sizeof(int), ctx->stream));
     LMH_LAUNCH(ctx, "build_windows", (k_build_windows<true, CAP, IW>), dim3(grid_for(nrb, 1, 16384)), dim3(BLK), 0,
-               (const int32_t *)rbd.p, nrb, A->rp, A->ci, (int32_t *)wsz.p, nullptr, nullptr, nullptr,
+               (const int32_t *)rbd.p, nrb, A->rp, A->ci, (int32_t *)wsz.p, nullptr, nullptr, nullptr, nullptr,
                ctx->d_flags);
     LMH_TRY(check_launch("k_build_windows"));
     w0.assign(nrb + 1, 0);
@@ -1096,29 +1203,39 @@ static int try_windows(lmh_matrix *A, std::vector<int32_t> rb, bool split, bool 
   }
   w0[nrb] = (int32_t)total;  // at most nnz < 2^31
   LMH_HIP(hipMemcpyAsync(wsz.p, w0.data(), sizeof(int32_t) * (nrb + 1), hipMemcpyHostToDevice, ctx->stream));
-  widx_t<IW> *widx = nullptr;
+  widx_t<IW> *widx = nullptr, *widx64 = nullptr;
   uint16_t *woff = nullptr;
   int4 *meta = nullptr;
-  LMH_HIP(hipMalloc((void **)&widx, sizeof(widx_t<IW>) * (A->nnz + LMH_PAD)));
+  // every block has CAP index slots (unused ones index window slot 0) and, with
+  // 8-bit indices, a full window of offsets (unused ones 0)
+  if (IW == 1) total = nrb * W8_UCAP;
+  if (total > INT32_MAX) return LMH_OK;
+  const size_t idx_bytes = sizeof(widx_t<IW>) * std::max<int64_t>(1, nrb) * CAP;
+  LMH_HIP(hipMalloc((void **)&widx, idx_bytes));
+  LMH_HIP(hipMemsetAsync(widx, 0, idx_bytes, ctx->stream));
+  if (A->vals) {  // FP64 operator: its chunks hold two entries
+    LMH_HIP(hipMalloc((void **)&widx64, idx_bytes));
+    LMH_HIP(hipMemsetAsync(widx64, 0, idx_bytes, ctx->stream));
+  }
   LMH_HIP(hipMalloc((void **)&woff, sizeof(uint16_t) * (total + LMH_PAD)));
+  LMH_HIP(hipMemsetAsync(woff, 0, sizeof(uint16_t) * (total + LMH_PAD), ctx->stream));
   LMH_HIP(hipMalloc((void **)&meta, sizeof(int4) * 2 * (nrb ? nrb : 1)));
   LMH_HIP(hipMemsetAsync(ctx->d_flags, 0, sizeof(int), ctx->stream));
   LMH_LAUNCH(ctx, "build_windows", (k_build_windows<false, CAP, IW>), dim3(grid_for(nrb, 1, 16384)), dim3(BLK), 0,
-             (const int32_t *)rbd.p, nrb, A->rp, A->ci, (int32_t *)wsz.p, widx, woff, meta, ctx->d_flags);
+             (const int32_t *)rbd.p, nrb, A->rp, A->ci, (int32_t *)wsz.p, widx, widx64, woff, meta, ctx->d_flags);
   LMH_TRY(check_launch("k_build_windows"));
   int bad = 0;
   LMH_HIP(hipMemcpyAsync(&bad, ctx->d_flags, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
   LMH_HIP(hipStreamSynchronize(ctx->stream));
   if (bad) {  // not expected: the counting pass accepted every block
     LMH_HIP(hipFree(widx));
+    LMH_HIP(hipFree(widx64));
     LMH_HIP(hipFree(woff));
     LMH_HIP(hipFree(meta));
     return LMH_OK;
   }
-  if (IW == 1)
-    A->widx8 = (uint8_t *)widx;
-  else
-    A->widx16 = (uint16_t *)widx;
+  A->widx32 = widx;
+  A->widx64 = widx64;
   A->woff16 = woff;
   A->rbmeta = meta;
   A->rbw = (int32_t *)rbd.p;
@@ -1171,6 +1288,54 @@ static int ensure_diag(lmh_matrix *A) {
 
 static bool use_windows(const lmh_matrix *A) { return A->fp32_index && A->idx16_state == 1; }
 
+// How the products of a matrix run.  Matrices whose row blocks fit the windows
+// stream them (rowblock_spmv16) on the window partition: through the 8- or
+// 16-bit windows, or with the int32 columns when the windows are switched off
+// or a vector is too long for their 32-bit byte offsets.  Row blocks and
+// workgroups are the same in both, so the sums and partial sums are too.
+// Others (a row block with more than 768 distinct columns, or a row beyond the
+// block size) run rowblock_spmv.
+struct Stream {
+  bool on = false;
+  int grid = 0, nt = 0;           // workgroups and threads of a product
+  const void *idx = nullptr;
+  int iw = 0;                     // index bytes
+};
+static Stream stream_of(lmh_matrix *A, bool fp32) {
+  Stream s;
+  const int gs = spmv_grid(A->ctx);
+  s.on = A->idx16_state == 1;
+  s.nt = s.on && A->wbits == 8 ? W8_NT : BLK;
+  s.grid = s.on && A->wbits == 8 ? W8_GRID * gs : gs;
+  if (use_windows(A) && A->cols < ((int64_t)1 << 29)) {
+    s.iw = A->wbits / 8;
+    s.idx = fp32 ? A->widx32 : A->widx64;
+  } else {
+    s.iw = 4;
+    s.idx = A->ci;
+  }
+  return s;
+}
+template <int C, int I, int N>
+struct StreamShape {
+  static constexpr int cap = C, iw = I, nt = N;
+};
+// f(StreamShape) for the stream's kernel shape
+template <typename F>
+static void with_stream(const Stream &s, F &&f) {
+  if (s.nt == W8_NT) {
+    if (s.iw == 1)
+      f(StreamShape<W8_CAP, 1, W8_NT>{});
+    else
+      f(StreamShape<W8_CAP, 4, W8_NT>{});
+  } else {
+    if (s.iw == 2)
+      f(StreamShape<RB_CAP, 2, BLK>{});
+    else
+      f(StreamShape<RB_CAP, 4, BLK>{});
+  }
+}
+
 static int ensure_work(lmh_matrix *A, bool mixed) {
   if (!A->w64) LMH_HIP(hipMalloc((void **)&A->w64, sizeof(double) * 4 * work_stride(A->rows)));
   if (mixed && !A->w32) LMH_HIP(hipMalloc((void **)&A->w32, sizeof(float) * 5 * work_stride(A->rows)));
@@ -1187,9 +1352,17 @@ int lmh_spmv(lmh_matrix *A, const double *x_d, double *y_d) {
   LMH_CHECK(A && x_d && y_d, LMH_ERR_INVALID, "null argument");
   LMH_CHECK(A->vals, LMH_ERR_UNSUPPORTED, "matrix holds FP32 values only");
   lmh_context *ctx = A->ctx;
-  const int g = spmv_grid(ctx);
-  LMH_LAUNCH(ctx, "spmv_fp64", (k_spmv<double, double, double, double>), dim3(g),
-                                          dim3(BLK), 0, A->rb, A->nrb, A->rp, A->ci, A->vals, x_d, y_d);
+  LMH_TRY(ensure_windows(A));
+  const Stream st = stream_of(A, false);
+  if (st.on)
+    with_stream(st, [&](auto sh) {
+      typedef decltype(sh) K;
+      LMH_LAUNCH(ctx, "spmv_fp64", (k_spmv16<double, K::cap, K::iw, K::nt>), dim3(st.grid), dim3(K::nt), 0, A->nrbw,
+                 A->rp, st.idx, A->woff16, A->rbmeta, A->vals, x_d, y_d);
+    });
+  else
+    LMH_LAUNCH(ctx, "spmv_fp64", (k_spmv<double, double, double, double>), dim3(st.grid), dim3(BLK), 0, A->rb, A->nrb,
+               A->rp, A->ci, A->vals, x_d, y_d);
   return check_launch("k_spmv");
 }
 
@@ -1197,30 +1370,50 @@ int lmh_spmv_fp32(lmh_matrix *A, const float *x_d, float *y_d) {
   LMH_CHECK(A && x_d && y_d, LMH_ERR_INVALID, "null argument");
   LMH_CHECK(A->have32 && A->vals32, LMH_ERR_INVALID, "matrix has no FP32 operator");
   lmh_context *ctx = A->ctx;
-  const int g = spmv_grid(ctx);
   LMH_TRY(ensure_windows(A));
-  if (use_windows(A)) {
-    if (A->wbits == 8)
-      LMH_LAUNCH(ctx, "spmv_fp32", (k_spmv16<W8_CAP, 1, W8_NT>), dim3(W8_GRID * g), dim3(W8_NT), 0, A->nrbw,
-                 A->rp, A->widx8, A->woff16, A->rbmeta, A->vals32, x_d, y_d);
-    else
-      LMH_LAUNCH(ctx, "spmv_fp32", (k_spmv16<RB_CAP, 2, BLK>), dim3(g), dim3(BLK), 0, A->nrbw, A->rp, A->widx16,
-                 A->woff16, A->rbmeta, A->vals32, x_d, y_d);
-    return check_launch("k_spmv16");
-  }
-  LMH_LAUNCH(ctx, "spmv_fp32", (k_spmv<float, float, float, float>), dim3(g),
-                                          dim3(BLK), 0, A->rb, A->nrb, A->rp, A->ci, A->vals32, x_d, y_d);
+  const Stream st = stream_of(A, true);
+  if (st.on)
+    with_stream(st, [&](auto sh) {
+      typedef decltype(sh) K;
+      LMH_LAUNCH(ctx, "spmv_fp32", (k_spmv16<float, K::cap, K::iw, K::nt>), dim3(st.grid), dim3(K::nt), 0, A->nrbw,
+                 A->rp, st.idx, A->woff16, A->rbmeta, A->vals32, x_d, y_d);
+    });
+  else
+    LMH_LAUNCH(ctx, "spmv_fp32", (k_spmv<float, float, float, float>), dim3(st.grid), dim3(BLK), 0, A->rb, A->nrb,
+               A->rp, A->ci, A->vals32, x_d, y_d);
   return check_launch("k_spmv");
 }
+
+}  // extern "C"
+
+namespace lmh {
+// r = b - A x with the values v on A's pattern; partials (|r|^2, |b|^2) of st.grid workgroups
+static void launch_residual(lmh_matrix *A, const Stream &st, bool prof, const double *v, const double *b_d,
+                            const double *x_d, double *r_d, double *part) {
+  lmh_context *ctx = A->ctx;
+  ProfScope ps(prof ? ctx : nullptr, "residual_fp64");
+  if (st.on)
+    with_stream(st, [&](auto sh) {
+      typedef decltype(sh) K;
+      hipLaunchKernelGGL((k_residual16<K::cap, K::iw, K::nt>), dim3(st.grid), dim3(K::nt), 0, ctx->stream, A->nrbw,
+                         A->rp, st.idx, A->woff16, A->rbmeta, v, b_d, x_d, r_d, part);
+    });
+  else
+    hipLaunchKernelGGL(k_residual, dim3(st.grid), dim3(BLK), 0, ctx->stream, A->rb, A->nrb, A->rp, A->ci, v, b_d, x_d,
+                       r_d, part);
+}
+}  // namespace lmh
+
+extern "C" {
 
 int lmh_residual(lmh_matrix *A, const double *b_d, const double *x_d, double *r_d) {
   LMH_CHECK(A && b_d && x_d && r_d, LMH_ERR_INVALID, "null argument");
   LMH_CHECK(A->vals, LMH_ERR_UNSUPPORTED, "matrix holds FP32 values only");
   lmh_context *ctx = A->ctx;
-  const int g = spmv_grid(ctx);
-  LMH_LAUNCH(ctx, "residual_fp64", k_residual, dim3(g), dim3(BLK), 0, A->rb, A->nrb, A->rp,
-                                          A->ci, A->vals, b_d, x_d, r_d, ctx->d_part);
-  LMH_LAUNCH(ctx, "fin", k_fin_residual, dim3(1), dim3(BLK), 0, ctx->d_part, g, ctx->d_scal + 48);
+  LMH_TRY(ensure_windows(A));
+  const Stream st = stream_of(A, false);
+  launch_residual(A, st, true, A->vals, b_d, x_d, r_d, ctx->d_part);
+  LMH_LAUNCH(ctx, "fin", k_fin_residual, dim3(1), dim3(BLK), 0, ctx->d_part, st.grid, ctx->d_scal + 48);
   return check_launch("k_residual");
 }
 
@@ -1253,6 +1446,10 @@ int lmh_matrix_make_fp32(lmh_matrix *A) {
   A->have32 = true;
   return check_launch("k_round32");
 }
+
+}  // extern "C"
+
+namespace lmh {
 
 // ---------------------------------------------------------------------------
 // BiCGSTAB with the Jacobi preconditioner, FP64 (Eigen BiCGSTAB.h:28-112 as
@@ -1372,6 +1569,24 @@ __global__ __launch_bounds__(BLK) void k_bcg_spmv_v(const int32_t *__restrict__ 
   publish<1>(acc, part);
 }
 
+template <int CAPW, int IW, int NT>
+__global__ __launch_bounds__(NT) void k_bcg_spmv_v16(int64_t nrb, const int32_t *__restrict__ rp,
+                                                     const void *__restrict__ widx, const uint16_t *__restrict__ woff,
+                                                     const int4 *__restrict__ desc, const double *__restrict__ vals,
+                                                     const double *__restrict__ y, const double *__restrict__ r0,
+                                                     double *__restrict__ v, double *__restrict__ part,
+                                                     const double *__restrict__ S, int nbank) {
+  if (S[nbank * B_SIZE + B_DONE] != 0.0) return;
+  double acc[1] = {0};
+  rowblock_spmv16<double, 1, CAPW, IW, NT>(
+      nrb, desc, rp, (const widx_t<IW> *)widx, woff, vals, y, [&](int32_t row, double *o) { o[0] = r0[row]; },
+      [&](int32_t row, double sv, const double *pr) {
+        v[row] = sv;
+        acc[0] += pr[0] * sv;
+      });
+  publish<1, NT>(acc, part);
+}
+
 // alpha = rho / (r0, v); s = r - alpha v; z = dinv s
 __global__ __launch_bounds__(BLK) void k_bcg_s(int64_t n, const double *__restrict__ part_in, int G,
                                                const double *__restrict__ dinv, const double *__restrict__ r,
@@ -1411,6 +1626,25 @@ __global__ __launch_bounds__(BLK) void k_bcg_spmv_t(const int32_t *__restrict__ 
   publish<2>(acc, part);
 }
 
+template <int CAPW, int IW, int NT>
+__global__ __launch_bounds__(NT) void k_bcg_spmv_t16(int64_t nrb, const int32_t *__restrict__ rp,
+                                                     const void *__restrict__ widx, const uint16_t *__restrict__ woff,
+                                                     const int4 *__restrict__ desc, const double *__restrict__ vals,
+                                                     const double *__restrict__ z, const double *__restrict__ s,
+                                                     double *__restrict__ t, double *__restrict__ part,
+                                                     const double *__restrict__ S, int nbank) {
+  if (S[nbank * B_SIZE + B_DONE] != 0.0) return;
+  double acc[2] = {0, 0};
+  rowblock_spmv16<double, 1, CAPW, IW, NT>(
+      nrb, desc, rp, (const widx_t<IW> *)widx, woff, vals, z, [&](int32_t row, double *o) { o[0] = s[row]; },
+      [&](int32_t row, double tv, const double *pr) {
+        t[row] = tv;
+        acc[0] += tv * tv;
+        acc[1] += tv * pr[0];
+      });
+  publish<2, NT>(acc, part);
+}
+
 // w = (t, s) / (t, t) (0 when (t, t) = 0); x += alpha y + w z; r = s - w t;
 // partials |r|^2, (r0, r)
 __global__ __launch_bounds__(BLK) void k_bcg_update(int64_t n, const double *__restrict__ part_in, int G,
@@ -1446,10 +1680,6 @@ struct Poll {
   hipEvent_t ev = nullptr;
   int64_t end = 0;  // iterations launched when the copy was enqueued
 };
-
-}  // extern "C"
-
-namespace lmh {
 
 // Work vectors of the allocation-free CG: r, p, q, 1/a_ii (4 x LMH_CG_NOALLOC_MAX_ROWS
 // doubles), then the diagonal slots (LMH_CG_NOALLOC_MAX_ROWS int32).  Each GPU
@@ -1493,18 +1723,17 @@ static int cg_impl(lmh_matrix *A, const double *b_d, double *x_d, double rtol, i
 #define CG_LAUNCH(name, kernel, grid, ...) CG_LAUNCH_NT(name, kernel, grid, BLK, __VA_ARGS__)
   lmh_context *ctx = A->ctx;
   if (!NA) LMH_TRY(ensure_windows(A));
-  const bool c16 = use_windows(A);
+  const Stream st = stream_of(A, false);
   const int64_t n = A->rows;
   double *S = ctx->d_scal;
   double *part1 = ctx->d_part, *part2 = ctx->d_part + 2 * ctx->n_part;  // 1 and 2 values per block
-  const int g = vec_grid(ctx), gs = spmv_grid(ctx);
-  const int gsp = c16 && A->wbits == 8 ? W8_GRID * gs : gs;  // the iteration SpMV's grid
+  const int g = vec_grid(ctx);
   const int xvec = ((uintptr_t)x_d & 15) == 0;               // the caller's x takes 16-byte chunks
   CG_LAUNCH("invdiag", (k_invdiag<double, double>), dim3(grid_for(n, BLK, 8192)), n, diag, A->vals,
             A->precond == LMH_PRECOND_JACOBI, dinv);
-  CG_LAUNCH("residual_fp64", k_residual, dim3(gs), A->rb, A->nrb, A->rp, A->ci, A->vals, b_d, x_d, r, part2);
+  launch_residual(A, st, !NA, A->vals, b_d, x_d, r, part2);
   CG_LAUNCH("cg_init", k_cg_init, dim3(g), n, dinv, r, p, part1);
-  CG_LAUNCH("cg_init", k_cg_init_fin, dim3(g), part2, gs, part1, g, rtol, S, x_d, n);
+  CG_LAUNCH("cg_init", k_cg_init_fin, dim3(g), part2, st.grid, part1, g, rtol, S, x_d, n);
   LMH_TRY(check_launch("cg setup"));
   // The scalar banks are copied to pinned memory after every batch of
   // iterations; the host reads a batch's copy while the next batch runs.
@@ -1518,16 +1747,16 @@ static int cg_impl(lmh_matrix *A, const double *b_d, double *x_d, double rtol, i
     const int64_t nb = std::min<int64_t>(batch, maxits - K);
     for (int64_t i = 0; i < nb; ++i, ++K) {
       const int bank = (int)(K & 1);
-      if (c16 && A->wbits == 8)
-        CG_LAUNCH_NT("cg_spmv_fp64", (k_it_spmv16d<W8_CAP, 1, W8_NT>), dim3(gsp), W8_NT, A->nrbw, A->rp, A->widx8,
-                     A->woff16, A->rbmeta, A->vals, p, q, part1, S, bank);
-      else if (c16)
-        CG_LAUNCH("cg_spmv_fp64", (k_it_spmv16d<RB_CAP, 2, BLK>), dim3(gs), A->nrbw, A->rp, A->widx16, A->woff16,
-                  A->rbmeta, A->vals, p, q, part1, S, bank);
+      if (st.on)
+        with_stream(st, [&](auto sh) {
+          typedef decltype(sh) K;
+          CG_LAUNCH_NT("cg_spmv_fp64", (k_it_spmv16<double, K::cap, K::iw, K::nt>), dim3(st.grid), K::nt, A->nrbw,
+                       A->rp, st.idx, A->woff16, A->rbmeta, A->vals, p, q, part1, S, bank);
+        });
       else
-        CG_LAUNCH("cg_spmv_fp64", k_it_spmv<double>, dim3(gs), A->rb, A->nrb, A->rp, A->ci, A->vals, p, q, part1, S,
-                  bank);
-      CG_LAUNCH("cg_update_fp64", (k_it_update<double, double>), dim3(g), n, part1, gsp, dinv, p, q, x_d, r, part2, S,
+        CG_LAUNCH("cg_spmv_fp64", k_it_spmv<double>, dim3(st.grid), A->rb, A->nrb, A->rp, A->ci, A->vals, p, q, part1,
+                  S, bank);
+      CG_LAUNCH("cg_update_fp64", (k_it_update<double, double>), dim3(g), n, part1, st.grid, dinv, p, q, x_d, r, part2, S,
                 bank, xvec);
       CG_LAUNCH("cg_pupdate_fp64", k_it_pupdate<double>, dim3(g), n, part2, g, dinv, r, p, S, bank, 0);
     }
@@ -1611,14 +1840,15 @@ static int bicgstab_impl(lmh_matrix *A, const double *vals, const double *b_d, d
          *dinv = tv + n;
   double *S = ctx->d_scal;
   double *part1 = ctx->d_part, *part2 = ctx->d_part + 2 * ctx->n_part;
-  const int g = vec_grid(ctx), gs = spmv_grid(ctx);
+  LMH_TRY(ensure_windows(A));
+  const Stream st = stream_of(A, false);
+  const int g = vec_grid(ctx);
   LMH_TRY(ensure_diag(A));
   LMH_LAUNCH(ctx, "invdiag", (k_invdiag<double, double>), dim3(grid_for(n, 256, 8192)), dim3(256), 0, n, A->diag,
              vals, A->precond == LMH_PRECOND_JACOBI, dinv);
-  LMH_LAUNCH(ctx, "residual_fp64", k_residual, dim3(gs), dim3(BLK), 0, A->rb, A->nrb, A->rp, A->ci, vals, b_d,
-             x_d, r, part2);
+  launch_residual(A, st, true, vals, b_d, x_d, r, part2);
   LMH_LAUNCH(ctx, "bcg_init", k_bcg_init, dim3(g), dim3(BLK), 0, n, (const double *)r, r0, p, v, part1);
-  LMH_LAUNCH(ctx, "bcg_init", k_bcg_init_fin, dim3(g), dim3(BLK), 0, part2, gs, rtol, S, x_d, n);
+  LMH_LAUNCH(ctx, "bcg_init", k_bcg_init_fin, dim3(g), dim3(BLK), 0, part2, st.grid, rtol, S, x_d, n);
   LMH_TRY(check_launch("bicgstab setup"));
   const int batch = 4;
   Poll poll[2];
@@ -1629,12 +1859,26 @@ static int bicgstab_impl(lmh_matrix *A, const double *vals, const double *b_d, d
   auto iteration = [&](int bank) {
     const int nb = bank ^ 1;
     LMH_LAUNCH(ctx, "bcg_p", k_bcg_p, dim3(g), dim3(BLK), 0, n, part1, g, dinv, r, v, p, y, S, bank);
-    LMH_LAUNCH(ctx, "bcg_spmv_fp64", k_bcg_spmv_v, dim3(gs), dim3(BLK), 0, A->rb, A->nrb, A->rp, A->ci, vals, y,
-               r0, v, part1, S, nb);
-    LMH_LAUNCH(ctx, "bcg_s", k_bcg_s, dim3(g), dim3(BLK), 0, n, part1, gs, dinv, r, v, sv, z, S, nb);
-    LMH_LAUNCH(ctx, "bcg_spmv_fp64", k_bcg_spmv_t, dim3(gs), dim3(BLK), 0, A->rb, A->nrb, A->rp, A->ci, vals, z,
-               sv, tv, part2, S, nb);
-    LMH_LAUNCH(ctx, "bcg_update", k_bcg_update, dim3(g), dim3(BLK), 0, n, part2, gs, y, z, sv, tv, r0, x_d, r, part1,
+    if (st.on)
+      with_stream(st, [&](auto sh) {
+        typedef decltype(sh) K;
+        LMH_LAUNCH(ctx, "bcg_spmv_fp64", (k_bcg_spmv_v16<K::cap, K::iw, K::nt>), dim3(st.grid), dim3(K::nt), 0,
+                   A->nrbw, A->rp, st.idx, A->woff16, A->rbmeta, vals, y, r0, v, part1, S, nb);
+      });
+    else
+      LMH_LAUNCH(ctx, "bcg_spmv_fp64", k_bcg_spmv_v, dim3(st.grid), dim3(BLK), 0, A->rb, A->nrb, A->rp, A->ci, vals, y,
+                 r0, v, part1, S, nb);
+    LMH_LAUNCH(ctx, "bcg_s", k_bcg_s, dim3(g), dim3(BLK), 0, n, part1, st.grid, dinv, r, v, sv, z, S, nb);
+    if (st.on)
+      with_stream(st, [&](auto sh) {
+        typedef decltype(sh) K;
+        LMH_LAUNCH(ctx, "bcg_spmv_fp64", (k_bcg_spmv_t16<K::cap, K::iw, K::nt>), dim3(st.grid), dim3(K::nt), 0,
+                   A->nrbw, A->rp, st.idx, A->woff16, A->rbmeta, vals, z, sv, tv, part2, S, nb);
+      });
+    else
+      LMH_LAUNCH(ctx, "bcg_spmv_fp64", k_bcg_spmv_t, dim3(st.grid), dim3(BLK), 0, A->rb, A->nrb, A->rp, A->ci, vals, z,
+                 sv, tv, part2, S, nb);
+    LMH_LAUNCH(ctx, "bcg_update", k_bcg_update, dim3(g), dim3(BLK), 0, n, part2, st.grid, y, z, sv, tv, r0, x_d, r, part1,
                S, nb);
   };
   while (K < maxits && !done) {
@@ -1749,7 +1993,7 @@ int lmh_mixed_solve(lmh_matrix *A, const double *b_d, double *x_d, double rtol, 
   lmh_context *ctx = A->ctx;
   LMH_TRY(ensure_work(A, true));
   LMH_TRY(ensure_windows(A));
-  const bool c16 = use_windows(A);
+  const Stream st = stream_of(A, false), st32 = stream_of(A, true);
   const int64_t n = A->rows;
   // xc: FP32 solution correction accumulated since the last refresh, folded
   // into the FP64 x before each refresh
@@ -1757,8 +2001,19 @@ int lmh_mixed_solve(lmh_matrix *A, const double *b_d, double *x_d, double rtol, 
   float *r32 = A->w32, *p32 = r32 + ns, *q32 = p32 + ns, *d32 = q32 + ns, *xc = d32 + ns;
   double *S = ctx->d_scal;
   double *part1 = ctx->d_part, *part2 = ctx->d_part + 2 * ctx->n_part;
-  const int g = vec_grid(ctx), gs = spmv_grid(ctx);
-  const int gsp = c16 && A->wbits == 8 ? W8_GRID * gs : gs;  // the iteration SpMV's grid
+  const int g = vec_grid(ctx);
+  auto residual32 = [&](int init, int bank) {  // the FP64 residual and the FP32 start of the recurrence
+    if (st.on)
+      with_stream(st, [&](auto sh) {
+        typedef decltype(sh) K;
+        LMH_LAUNCH(ctx, "mx_refresh_fp64", (k_refresh16<K::cap, K::iw, K::nt>), dim3(st.grid), dim3(K::nt), 0, init,
+                   A->nrbw, A->rp, st.idx, A->woff16, A->rbmeta, A->vals, b_d, x_d, d32, r32, p32, part2, S, bank);
+      });
+    else
+      LMH_LAUNCH(ctx, "mx_refresh_fp64", k_refresh, dim3(st.grid), dim3(BLK), 0, init, A->rb, A->nrb, A->rp, A->ci,
+                 A->vals, b_d, x_d, d32, r32, p32, part2, S, bank);
+    LMH_LAUNCH(ctx, "fin", k_refresh_fin, dim3(1), dim3(BLK), 0, part2, st.grid, init, S, bank);
+  };
   double init[40] = {0};
   init[G_THR] = rtol * rtol;
   init[G_DELTA2] = inner_rtol * inner_rtol;
@@ -1768,15 +2023,11 @@ int lmh_mixed_solve(lmh_matrix *A, const double *b_d, double *x_d, double rtol, 
   LMH_LAUNCH(ctx, "invdiag", (k_invdiag<float, float>), dim3(grid_for(n, 256, 8192)), dim3(256), 0, n, A->diag,
              A->vals32, A->precond == LMH_PRECOND_JACOBI, d32);
   LMH_HIP(hipMemsetAsync(xc, 0, sizeof(float) * n, ctx->stream));
-  LMH_LAUNCH(ctx, "mx_refresh_fp64", k_refresh, dim3(gs), dim3(BLK), 0, 1, A->rb, A->nrb, A->rp, A->ci, A->vals,
-             b_d, x_d, d32, r32, p32, part2, S, 0);
-  LMH_LAUNCH(ctx, "fin", k_refresh_fin, dim3(1), dim3(BLK), 0, part2, gs, 1, S, 0);
+  residual32(1, 0);
   LMH_TRY(check_launch("mixed setup"));
   auto refresh = [&](int bank) {
     LMH_LAUNCH(ctx, "mx_fold", k_fold, dim3(g), dim3(BLK), 0, n, xc, x_d);
-    LMH_LAUNCH(ctx, "mx_refresh_fp64", k_refresh, dim3(gs), dim3(BLK), 0, 0, A->rb, A->nrb, A->rp, A->ci, A->vals,
-               b_d, x_d, d32, r32, p32, part2, S, bank);
-    LMH_LAUNCH(ctx, "fin", k_refresh_fin, dim3(1), dim3(BLK), 0, part2, gs, 0, S, bank);
+    residual32(0, bank);
     if (mode == 1) LMH_LAUNCH(ctx, "mx_restart", k_restart_p, dim3(g), dim3(BLK), 0, n, d32, r32, p32, S, bank);
   };
   const int batch = 4;
@@ -1789,16 +2040,16 @@ int lmh_mixed_solve(lmh_matrix *A, const double *b_d, double *x_d, double rtol, 
     const int64_t nb = std::min<int64_t>(batch, maxits - K);
     for (int64_t i = 0; i < nb; ++i, ++K) {
       const int bank = (int)(K & 1);
-      if (c16 && A->wbits == 8)
-        LMH_LAUNCH(ctx, "mx_spmv_fp32", (k_it_spmv16<W8_CAP, 1, W8_NT>), dim3(gsp), dim3(W8_NT), 0, A->nrbw, A->rp,
-                   A->widx8, A->woff16, A->rbmeta, A->vals32, p32, q32, part1, S, bank);
-      else if (c16)
-        LMH_LAUNCH(ctx, "mx_spmv_fp32", (k_it_spmv16<RB_CAP, 2, BLK>), dim3(gs), dim3(BLK), 0, A->nrbw, A->rp,
-                   A->widx16, A->woff16, A->rbmeta, A->vals32, p32, q32, part1, S, bank);
+      if (st.on)
+        with_stream(st32, [&](auto sh) {
+          typedef decltype(sh) K;
+          LMH_LAUNCH(ctx, "mx_spmv_fp32", (k_it_spmv16<float, K::cap, K::iw, K::nt>), dim3(st.grid), dim3(K::nt), 0,
+                     A->nrbw, A->rp, st32.idx, A->woff16, A->rbmeta, A->vals32, p32, q32, part1, S, bank);
+        });
       else
-        LMH_LAUNCH(ctx, "mx_spmv_fp32", k_it_spmv<float>, dim3(gs), dim3(BLK), 0, A->rb, A->nrb, A->rp, A->ci,
+        LMH_LAUNCH(ctx, "mx_spmv_fp32", k_it_spmv<float>, dim3(st.grid), dim3(BLK), 0, A->rb, A->nrb, A->rp, A->ci,
                    A->vals32, p32, q32, part1, S, bank);
-      LMH_LAUNCH(ctx, "mx_update_fp32", (k_it_update<float, float>), dim3(g), dim3(BLK), 0, n, part1, gsp, d32, p32,
+      LMH_LAUNCH(ctx, "mx_update_fp32", (k_it_update<float, float>), dim3(g), dim3(BLK), 0, n, part1, st.grid, d32, p32,
                  q32, xc, r32, part2, S, bank, 1);
       LMH_LAUNCH(ctx, "mx_pupdate_fp32", k_it_pupdate<float>, dim3(g), dim3(BLK), 0, n, part2, g, d32, r32, p32, S,
                  bank, 1);
@@ -1832,9 +2083,8 @@ int lmh_mixed_solve(lmh_matrix *A, const double *b_d, double *x_d, double rtol, 
   bool conv = Bk[B_DONE] != 0.0;
   if (!conv) {
     // iteration limit: report the FP64 true residual of the current x
-    LMH_LAUNCH(ctx, "residual_fp64", k_residual, dim3(gs), dim3(BLK), 0, A->rb, A->nrb, A->rp, A->ci, A->vals, b_d,
-               x_d, A->w64, part2);
-    LMH_LAUNCH(ctx, "fin", k_fin_residual, dim3(1), dim3(BLK), 0, part2, gs, S + G_RRTRUE);
+    launch_residual(A, st, true, A->vals, b_d, x_d, A->w64, part2);
+    LMH_LAUNCH(ctx, "fin", k_fin_residual, dim3(1), dim3(BLK), 0, part2, st.grid, S + G_RRTRUE);
     LMH_TRY(check_launch("mixed finish"));
   }
   LMH_HIP(hipMemcpy(gl, S + G_THR, sizeof(gl), hipMemcpyDeviceToHost));

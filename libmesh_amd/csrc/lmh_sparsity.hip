@@ -354,8 +354,8 @@ int lmh_matrix_destroy(lmh_matrix *A) {
   (void)hipFree(A->rp);
   (void)hipFree(A->ci);
   (void)hipFree(A->rb);
-  (void)hipFree(A->widx16);
-  (void)hipFree(A->widx8);
+  (void)hipFree(A->widx32);
+  (void)hipFree(A->widx64);
   (void)hipFree(A->rbw);
   (void)hipFree(A->woff16);
   (void)hipFree(A->rbmeta);
