@@ -149,7 +149,7 @@ def bench_constrained(args, L, ctx, kappa, log):
     ctx.sync()
     ctx.profile(False)
     kern = {}
-    for k in ("element_hex27_mfma_fp64", "constrain_general_fp64", "scatter_gather_fp64", "scatter_expanded_fp64"):
+    for k in ("element_hex27_fp64", "constrain_general_fp64", "scatter_gather_fp64", "scatter_expanded_fp64"):
         ms, c = ctx.profile_query(k)
         kern[k] = round(ms * c, 4)
     g.assemble_poisson(3, kd, 0, None, L.FP32)
@@ -568,8 +568,8 @@ def main():
     def step(mode):
         """mode fp64: FP64 assembly + FP64 CG.  mixed: FP64 assembly, FP32 inner
         operator rounded from it, mixed solve.  mixed_mfma32: FP64 assembly for
-        the outer residual operator plus an FP32-MFMA assembly of the inner
-        operator, mixed solve."""
+        the outer residual operator plus an FP32 assembly of the inner operator,
+        mixed solve."""
         x.zero()
         ctx.sync()
         ta = time.perf_counter()
@@ -678,7 +678,7 @@ def main():
     ctx.sync()
     ctx.profile(False)
     fem_residual = {k: round(ctx.profile_query(k)[0] * max(ctx.profile_query(k)[1], 1), 4)
-                    for k in ("element_hex27_mfma_fp64", "element_residual", "add_element_vectors")}
+                    for k in ("element_residual", "add_element_vectors")}
     bnorm = float(np.linalg.norm(b.download()))
     fem_residual["rel_residual_at_mixed_solution"] = float(np.linalg.norm(R.download()) / bnorm)
     log(f"fem residual: {fem_residual}")
@@ -690,8 +690,8 @@ def main():
     log(f"condensed: {condensed}")
 
     # assembly kernel timings: mean per assembly over ASM_REPS profiled
-    # assemblies (FP64 path, then the FP32 MFMA contraction + FP32 scatter,
-    # which writes the FP32 operator only)
+    # assemblies (FP64 path, then the FP32 one, which writes the FP32 operator
+    # only)
     ASM_REPS = 10
     asm_k = {}
     for prec, tag in ((L.FP64, "fp64"), (L.FP32, "fp32")):
@@ -701,7 +701,7 @@ def main():
             g.assemble_poisson(3, kd, 0, b, prec, scatter)
         ctx.sync()
         ctx.profile(False)
-        for k in ("element_hex27_mfma_", "scatter_gather_", "scatter_colored_"):
+        for k in ("element_hex27_", "scatter_gather_", "scatter_colored_"):
             ms, c = ctx.profile_query(k + tag)
             if c:
                 asm_k[k + tag] = ms * c / ASM_REPS
@@ -786,7 +786,7 @@ def main():
         "setup_s": round(t_setup, 3),
     }
     for prec in ("fp64", "fp32"):
-        k = f"element_hex27_mfma_{prec}"
+        k = f"element_hex27_{prec}"
         if k in asm_k:
             tf = flops_contract / (asm_k[k] * 1e-3) / 1e12
             out[f"contraction_tflops_{prec}"] = round(tf, 3)

@@ -9,16 +9,14 @@
 //          = sum_q dref_i(q)^T M_q dref_j(q),   M_q = JxW_q kappa_e G_q G_q^T,
 // i.e. Ke = Gref^T H_e with Gref[(q,r)][i] = dref_i(q)[r] constant over elements
 // and H_e[(q,r)][j] = (M_q dref_j(q))[r].  Geometry (J, det, inverse) is FP64.
-// The contraction runs on MFMA for HEX27 (v_mfma_f64_16x16x4f64 / f32), on
-// wavefront FMA for HEX8, and on a generic per-element kernel otherwise.
+// HEX27 with the 3^3 rule runs by sum factorisation (lmh_hex27.hip), TET4,
+// TET10 and many HEX8 with a thread per element (lmh_thread_elem.hip), few HEX8
+// on eight lanes per element, other HEX27 rules on the general kernel.
 #include <cmath>
 
 #include "lmh_internal.h"
 
 namespace lmh {
-
-typedef double double4_t __attribute__((ext_vector_type(4)));
-typedef float float4_t __attribute__((ext_vector_type(4)));
 
 // Geometry at one quadrature point from LDS coordinates X[a*3+c] and the
 // reference derivative table dref[(a*nq+q)*3+r].  Writes M (9, symmetric,
@@ -205,159 +203,6 @@ __global__ __launch_bounds__(256) void k_poisson_hex8(const double *__restrict__
         Ke[(e * 8 + t) * 8 + j] = v;
       }
       Fe[e * 8 + t] = myc ? 0.0 : fe;
-    }
-    __syncthreads();
-  }
-}
-
-// ---------------------------------------------------------------------------
-// Q2 HEX27, 3x3x3 Gauss, MFMA contraction.  One element per wave, 4 waves per
-// block, persistent.  Ke (27x27, padded 32x32) = Gref^T (32x84) * H (84x32):
-// all four 16x16 tiles run on v_mfma_*_16x16x4 (21 k-steps each), so every
-// lane stores its accumulators straight to Ke in row-major order (16
-// consecutive entries per lane group: coalesced), with no LDS staging of Ke.
-// MFMA operand layout (16x16x4): lane l supplies A[l%16][l/16] and
-// B[l/16][l%16]; accumulator element r of lane l holds D[drow(l/16, r)][l%16]
-// (see MfmaT::drow).  The constant Gref^T operand is read per k-step from the
-// LDS derivative table; the shape values for Fe come from the FE table in
-// global memory (27x27, cache resident).  LDS holds the derivative table and
-// per wave the coordinates, the 27 M_q and JxW_q f_q: 29 KB per block, so the
-// occupancy is set by registers, not LDS.  (Measured: per-wave instead of
-// block barriers let the waves drift apart and made the FP64 kernel slower,
-// 1.65 -> 2.22 ms at 64^3.)
-// ---------------------------------------------------------------------------
-template <typename CT>
-struct MfmaT;
-template <>
-struct MfmaT<double> {
-  typedef double4_t acc_t;
-  __device__ static inline acc_t mma(double a, double b, acc_t c) {
-    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-  }
-  // f64 16x16x4: the four accumulator registers of lane group g hold rows g, g+4, g+8, g+12
-  __device__ static inline int drow(int g, int r) { return g + 4 * r; }
-};
-template <>
-struct MfmaT<float> {
-  typedef float4_t acc_t;
-  __device__ static inline acc_t mma(float a, float b, acc_t c) {
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-  }
-  // f32 16x16x4: lane group g holds rows 4g .. 4g+3
-  __device__ static inline int drow(int g, int r) { return 4 * g + r; }
-};
-
-constexpr int Q2N = 27, Q2Q = 27, Q2K = 81, Q2KS = 21;
-
-// The forcing kind is a template argument: the f = 1 launch carries none of
-// the FP64 sine's code or registers.
-template <typename CT, int FK>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(FK ? 2 : 3))) void k_poisson_hex27_mfma(
-    const double *__restrict__ tab, const double *__restrict__ xyz, const int32_t *__restrict__ conn,
-    const int32_t *__restrict__ edofs, const uint8_t *__restrict__ cons, const double *__restrict__ kappa,
-    int constrain, int64_t ne, CT *__restrict__ Ke, double *__restrict__ Fe, int *__restrict__ err) {
-  typedef typename MfmaT<CT>::acc_t acc_t;
-  __shared__ double s_w[Q2Q];
-  __shared__ double s_dref[Q2N * Q2Q * 3];
-  __shared__ double s_X[4][Q2N * 3];
-  __shared__ double s_M[4][Q2Q * 9];
-  __shared__ double s_Jf[4][Q2Q];
-  const double *g_phi = tab + Q2Q;  // phi[a * nq + q]
-  const int tid = threadIdx.x, wv = tid >> 6, lane = tid & 63;
-  for (int i = tid; i < Q2Q; i += 256) s_w[i] = tab[i];
-  for (int i = tid; i < Q2N * Q2Q * 3; i += 256) s_dref[i] = tab[Q2Q + Q2N * Q2Q + i];
-  __syncthreads();
-
-  double *X = s_X[wv];
-  double *M = s_M[wv];
-  double *Jf = s_Jf[wv];
-  const int64_t groups = (ne + 3) / 4;
-  for (int64_t g = blockIdx.x; g < groups; g += gridDim.x) {
-    const int64_t e = g * 4 + wv;
-    const bool valid = e < ne;
-    bool ci = false;
-    double kap = 1.0;
-    if (valid) {
-      if (lane < Q2N) {
-        const int32_t nd = conn[e * Q2N + lane];
-        X[lane * 3] = xyz[3 * (int64_t)nd];
-        X[lane * 3 + 1] = xyz[3 * (int64_t)nd + 1];
-        X[lane * 3 + 2] = xyz[3 * (int64_t)nd + 2];
-        ci = cons[edofs[e * Q2N + lane]] != 0;
-      }
-      if (kappa) kap = kappa[e];
-    }
-    const unsigned long long cmask = constrain ? __ballot(ci) : 0ull;
-    __syncthreads();
-    if (valid && lane < Q2Q) {
-      double Mq[9];
-      double jxw;
-      if (qp_geometry(X, s_dref, Q2N, Q2Q, lane, s_w[lane], kap, Mq, jxw) <= 0.0) atomicOr(err, 1);
-#pragma unroll
-      for (int t = 0; t < 9; ++t) M[lane * 9 + t] = Mq[t];
-      double f = 1.0;
-      if constexpr (FK != 0) {
-        double x = 0, y = 0, z = 0;
-        for (int a = 0; a < Q2N; ++a) {
-          const double p = g_phi[a * Q2Q + lane];
-          x += X[a * 3] * p;
-          y += X[a * 3 + 1] * p;
-          z += X[a * 3 + 2] * p;
-        }
-        f = forcing(FK, x, y, z);
-      }
-      Jf[lane] = jxw * f;
-    }
-    __syncthreads();
-    if (valid) {
-      acc_t c00 = {0, 0, 0, 0}, c01 = {0, 0, 0, 0}, c10 = {0, 0, 0, 0}, c11 = {0, 0, 0, 0};
-      const int li = lane & 15, lk = lane >> 4;
-      const int j0 = li, j1 = 16 + li;
-#pragma unroll 1
-      for (int ks = 0; ks < Q2KS; ++ks) {
-        const int k = 4 * ks + lk;
-        double b0 = 0.0, b1 = 0.0;
-        CT a0 = 0, a1 = 0;
-        if (k < Q2K) {
-          const int q = k / 3, r = k - 3 * (k / 3);
-          const double m0 = M[q * 9 + r * 3], m1 = M[q * 9 + r * 3 + 1], m2 = M[q * 9 + r * 3 + 2];
-          const double *d0 = &s_dref[(j0 * Q2Q + q) * 3];
-          b0 = m0 * d0[0] + m1 * d0[1] + m2 * d0[2];
-          a0 = (CT)d0[r];
-          if (j1 < Q2N) {
-            const double *d1 = &s_dref[(j1 * Q2Q + q) * 3];
-            b1 = m0 * d1[0] + m1 * d1[1] + m2 * d1[2];
-            a1 = (CT)d1[r];
-          }
-        }
-        // A[I][ks] = Gref^T[16I + l%16][4ks + l/16] (the same LDS reads as the B operand's)
-        c00 = MfmaT<CT>::mma(a0, (CT)b0, c00);
-        c01 = MfmaT<CT>::mma(a0, (CT)b1, c01);
-        c10 = MfmaT<CT>::mma(a1, (CT)b0, c10);
-        c11 = MfmaT<CT>::mma(a1, (CT)b1, c11);
-      }
-      CT *Kr = Ke + e * (Q2N * Q2N);
-      const bool cj0 = (cmask >> j0) & 1ull, cj1 = j1 < Q2N && ((cmask >> j1) & 1ull);
-      auto put = [&](int i, int j, bool cj, CT v) {
-        const bool ri = (cmask >> i) & 1ull;
-        if (ri || cj) v = (i == j && ri) ? (CT)1 : (CT)0;
-        Kr[i * Q2N + j] = v;
-      };
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int i0 = MfmaT<CT>::drow(lk, r), i1 = 16 + i0;
-        put(i0, j0, cj0, c00[r]);
-        if (j1 < Q2N) put(i0, j1, cj1, c01[r]);
-        if (i1 < Q2N) {
-          put(i1, j0, cj0, c10[r]);
-          if (j1 < Q2N) put(i1, j1, cj1, c11[r]);
-        }
-      }
-      if (lane < Q2N) {
-        double fe = 0.0;
-        for (int q = 0; q < Q2Q; ++q) fe += Jf[q] * g_phi[lane * Q2Q + q];
-        Fe[e * Q2N + lane] = ((cmask >> lane) & 1ull) ? 0.0 : fe;
-      }
     }
     __syncthreads();
   }
@@ -740,18 +585,7 @@ static int element_poisson_impl(lmh_context *ctx, const lmh_mesh *m, const lmh_d
   LMH_CHECK(t->nq <= 64 && t->n <= 27, LMH_ERR_UNSUPPORTED, "element too large for the generic kernel");
   const int64_t ne = m->n_elem;
   const int maxg = ctx->cu_count * 8;
-  if (m->type == LMH_HEX27 && npts == 3) {
-    // one resident wave of workgroups: 3 per CU at the f = 1 kernel's registers, 2 with the sine
-    const int g = grid_for((ne + 3) / 4, 1, ctx->cu_count * (f_kind == 0 ? 3 : 2));
-    const char *name = sizeof(CT) == 8 ? "element_hex27_mfma_fp64" : "element_hex27_mfma_fp32";
-    if (f_kind == 0)
-      LMH_LAUNCH(ctx, name, (k_poisson_hex27_mfma<CT, 0>), dim3(g), dim3(256), 0, t->d_data, m->xyz, m->conn,
-                 dm->edofs, dm->cons, kappa, constrain, ne, Ke, Fe, ctx->d_flags);
-    else
-      LMH_LAUNCH(ctx, name, (k_poisson_hex27_mfma<CT, 1>), dim3(g), dim3(256), 0, t->d_data, m->xyz, m->conn,
-                 dm->edofs, dm->cons, kappa, constrain, ne, Ke, Fe, ctx->d_flags);
-    return check_launch("k_poisson_hex27_mfma");
-  }
+  if (m->type == LMH_HEX27 && npts == 3) return hex27_poisson<CT>(ctx, m, dm, kappa, f_kind, constrain, Ke, Fe);
   if (m->type == LMH_HEX8 && npts == 2 && sizeof(CT) == 8 && ne < kHex8ThreadMin) {
     const int g = grid_for((ne + 31) / 32, 1, ctx->cu_count * 4);
     LMH_LAUNCH(ctx, "element_hex8_fma", k_poisson_hex8, dim3(g), dim3(256), 0, t->d_data, m->xyz, m->conn, dm->edofs,

@@ -284,9 +284,263 @@ __global__ __launch_bounds__(64) void k_hex27_adjoint(const double *__restrict__
   }
 }
 
+// ---------------------------------------------------------------------------
+// Element matrices of the Poisson operator by sum factorisation, one wavefront
+// per workgroup, up to seven elements of geometry at a time.
+//
+//   K_ij = sum_{r,s} sum_q a_r(q,i) M_rs(q) a_s(q,j),  M = JxW kappa G G^T,
+//
+// with a_r the product of 1D shapes whose direction-r factor is the derivative.
+// Per element, 54 of 64 lanes: lane t = 9 c + k, c one of the six unordered
+// pairs i3 <= j3 (K is symmetric), k first a column (q1, q2), then a pair
+// (i2, j2):
+//   S (8 arrays) = direction 3 contracted, lane (q1, q2) x (i3, j3)
+//   T (4 x 3, by the kind of direction 1's factors: dd, dp, pd, pp)
+//                = direction 2 contracted, lane (i2, j2) x (i3, j3), S through LDS
+//   K = direction 1 contracted in registers, nine entries (i1, j1) per lane,
+// each written with its mirror to an LDS tile that leaves as coalesced stores.
+// 195 multiply-adds per lane instead of the 84 16x16x4 matrix instructions
+// (86,000 multiply-adds with their padding) of the table contraction this
+// replaces, which also formed its operands from nine LDS reads per k-step.
+// FP64 throughout; the FP32 operator is the FP64 entry rounded once.
+// Bound by LDS reads and their latency at two wavefronts per SIMD (248
+// registers, 16.4 KB of LDS); 262,144 elements: FP64 1545 -> 633 us, FP32
+// 1258 -> 600 us.  Three wavefronts per SIMD (168 registers, geometry of five
+// elements) spill: 806 us; the next element's S ahead of this one's T: 256
+// registers and 350 bytes of spills, 913 us.
+// ---------------------------------------------------------------------------
+template <typename CT, int FK>
+__global__ __launch_bounds__(64, 2) void k_hex27_poisson(const double *__restrict__ xyz,
+                                                         const int32_t *__restrict__ conn,
+                                                         const int32_t *__restrict__ edofs,
+                                                         const uint8_t *__restrict__ cons,
+                                                         const double *__restrict__ kappa, int constrain, int per,
+                                                         int64_t ne, CT *__restrict__ Ke, double *__restrict__ Fe,
+                                                         int *__restrict__ err) {
+  constexpr int NF = 3, ST = 27 * NF;
+  // node coordinates of the group; then, per element, S and the matrix tile
+  __shared__ double s_buf[sizeof(CT) == 8 ? 729 : kH27PerWave * ST];
+  __shared__ double s_m[kH27PerWave * 162];  // M[el][6 components][q3][q1q2]
+  __shared__ double s_h[kH27PerWave * 27];
+  const int lane = threadIdx.x;
+  const H27Slots sl(lane);
+  // the matrix lanes: pair (i3, j3) of c, pair (i2, j2) of k
+  const int t54 = lane < 54 ? lane : 0, cc = t54 / 9, kk = t54 - 9 * cc;
+  const int i3 = cc < 3 ? cc : (cc == 5 ? 1 : 0), j3 = cc < 3 ? cc : (cc == 3 ? 1 : 2);
+  const int i2 = kk % 3, j2 = kk / 3;
+  int ni[3], nj[3];  // local nodes of the lane's rows (i1, i2, i3) and columns (j1, j2, j3)
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    ni[i] = kH27Node[9 * i3 + 3 * i2 + i];
+    nj[i] = kH27Node[9 * j3 + 3 * j2 + i];
+  }
+  const int64_t total = ne * 27, groups = (ne + per - 1) / per;
+  int32_t nd[3], dof[3];
+  sl.ids(conn, (int64_t)blockIdx.x * per, total, lane, nd);
+  sl.ids(edofs, (int64_t)blockIdx.x * per, total, lane, dof);
+  for (int64_t gr = blockIdx.x; gr < groups; gr += gridDim.x) {
+    // lane constants of this phase: formed again for every group (the opaque
+    // lane index keeps the compiler from holding both phases' in registers)
+    int lg = lane;
+    asm volatile("" : "+v"(lg));
+    const H27Lane L(lg);
+    double pt[3], pt2[3];
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+      pt[q] = h27_pick(L.l % 3, [&](int i) { return h27_p(q, i); });
+      pt2[q] = h27_pick(L.l / 3, [&](int i) { return h27_p(q, i); });
+    }
+    const int64_t e0 = gr * per;
+    const int cnt = (int)(ne - e0 < per ? ne - e0 : per);
+    unsigned long long bits[3];  // constrained flags, bit 27 el + node of the group
+#pragma unroll
+    for (int m = 0; m < 3; ++m) {
+      const double *x = xyz + 3 * (int64_t)nd[m];
+      const double x0 = x[0], x1 = x[1], x2 = x[2];
+      const bool c = cons[dof[m]] != 0;
+      if (sl.live[m]) {
+        double *d = s_buf + sl.el[m] * ST + sl.lat[m] * NF;
+        d[0] = x0;
+        d[1] = x1;
+        d[2] = x2;
+      }
+      bits[m] = constrain ? __ballot(c && sl.live[m]) : 0ull;
+    }
+    sl.ids(conn, (gr + gridDim.x) * per, total, lane, nd);
+    sl.ids(edofs, (gr + gridDim.x) * per, total, lane, dof);
+    auto mask_of = [&](int el) -> unsigned {  // 27 flags of element el, by local node
+      const int b = 27 * el, w = b >> 6, o = b & 63;
+      unsigned long long v = bits[0];
+      if (w == 1) v = bits[1];
+      if (w == 2) v = bits[2];
+      v >>= o;
+      if (o > 37) v |= (w == 0 ? bits[1] : bits[2]) << (64 - o);
+      return (unsigned)v & 0x7ffffffu;
+    };
+    const bool on = L.el < cnt;
+    h27_sync();
+    if (on) {
+      const double kap = kappa ? kappa[e0 + L.el] : 1.0;
+      double g[3][NF][3], pos[3][FK ? 3 : 1], h[3] = {0.0, 0.0, 0.0};
+      h27_refgrad<NF, FK ? 3 : 0>(s_buf + L.el * ST, L, g, pos);
+#pragma unroll
+      for (int q = 0; q < 3; ++q) {
+        double J[3][3], c[3][3];
+#pragma unroll
+        for (int r = 0; r < 3; ++r)
+#pragma unroll
+          for (int k = 0; k < 3; ++k) J[r][k] = g[q][k][r];
+        const double det = cofactors(J, c);
+        if (!(det > 0.0)) atomicOr(err, 1);
+        const double w = L.w12 * h27_w(q), s = kap * w / det;
+        double *M = s_m + L.el * 162 + 9 * q + L.l;  // components 11, 12, 13, 22, 23, 33
+        int m = 0;
+#pragma unroll
+        for (int r = 0; r < 3; ++r)
+#pragma unroll
+          for (int u = r; u < 3; ++u, ++m)
+            M[27 * m] = s * (c[r][0] * c[u][0] + c[r][1] * c[u][1] + c[r][2] * c[u][2]);
+        double fj = det * w;
+        if constexpr (FK != 0) fj *= forcing(FK, pos[q][0], pos[q][1], pos[q][2]);
+#pragma unroll
+        for (int i = 0; i < 3; ++i) h[i] += h27_p(q, i) * fj;
+      }
+#pragma unroll
+      for (int i = 0; i < 3; ++i) s_h[L.el * 27 + 9 * i + L.l] = h[i];
+    }
+    h27_sync();
+    if (on) {
+      const unsigned cm = mask_of(L.el);
+#pragma unroll
+      for (int i = 0; i < 3; ++i) {
+        const double *H = s_h + L.el * 27 + 9 * i;
+        double s = 0.0;
+#pragma unroll
+        for (int q2 = 0; q2 < 3; ++q2)
+          s += pt2[q2] * (pt[0] * H[3 * q2] + pt[1] * H[3 * q2 + 1] + pt[2] * H[3 * q2 + 2]);
+        const int a = kH27Node[9 * i + L.l];
+        Fe[(e0 + L.el) * 27 + a] = (cm >> a) & 1u ? 0.0 : s;
+      }
+    }
+    int a3 = i3, b3 = j3, a2 = i2, b2 = j2;
+    asm volatile("" : "+v"(a3), "+v"(b3), "+v"(a2), "+v"(b2));
+    double pi3[3], di3[3], pj3[3], dj3[3], pi2[3], di2[3], pj2[3], dj2[3];
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+      pi3[q] = h27_pick(a3, [&](int i) { return h27_p(q, i); });
+      di3[q] = h27_pick(a3, [&](int i) { return h27_d(q, i); });
+      pj3[q] = h27_pick(b3, [&](int i) { return h27_p(q, i); });
+      dj3[q] = h27_pick(b3, [&](int i) { return h27_d(q, i); });
+      pi2[q] = h27_pick(a2, [&](int i) { return h27_p(q, i); });
+      di2[q] = h27_pick(a2, [&](int i) { return h27_d(q, i); });
+      pj2[q] = h27_pick(b2, [&](int i) { return h27_p(q, i); });
+      dj2[q] = h27_pick(b2, [&](int i) { return h27_d(q, i); });
+    }
+    for (int el = 0; el < cnt; ++el) {
+      const unsigned cm = __builtin_amdgcn_readfirstlane(mask_of(el));
+      if (lane < 54) {
+        const double *M = s_m + el * 162 + kk;  // kk: the column (q1, q2)
+        double S[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+          const double m11 = M[9 * q], m12 = M[27 + 9 * q], m13 = M[54 + 9 * q], m22 = M[81 + 9 * q],
+                       m23 = M[108 + 9 * q], m33 = M[135 + 9 * q];
+          const double pp = pi3[q] * pj3[q], pd = pi3[q] * dj3[q], dp = di3[q] * pj3[q], dd = di3[q] * dj3[q];
+          S[0] += pp * m11;
+          S[1] += pp * m12;
+          S[2] += pp * m22;
+          S[3] += pd * m13;
+          S[4] += dp * m13;
+          S[5] += pd * m23;
+          S[6] += dp * m23;
+          S[7] += dd * m33;
+        }
+#pragma unroll
+        for (int k = 0; k < 8; ++k) s_buf[54 * k + lane] = S[k];
+      }
+      h27_sync();
+      double K[3][3];
+      if (lane < 54) {
+        const double *S = s_buf + 9 * cc;
+        double K0[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}};
+#pragma unroll
+        for (int q1 = 0; q1 < 3; ++q1) {
+          double tdd = 0, tdp = 0, tpd = 0, tpp = 0;
+#pragma unroll
+          for (int q2 = 0; q2 < 3; ++q2) {
+            const int q = 3 * q2 + q1;
+            const double pp = pi2[q2] * pj2[q2], pd = pi2[q2] * dj2[q2], dp = di2[q2] * pj2[q2],
+                         dd = di2[q2] * dj2[q2];
+            const double s12 = S[54 + q];
+            tdd += pp * S[q];
+            tdp += pd * s12 + pp * S[162 + q];
+            tpd += dp * s12 + pp * S[216 + q];
+            tpp += dd * S[108 + q] + dp * S[270 + q] + pd * S[324 + q] + pp * S[378 + q];
+          }
+#pragma unroll
+          for (int j = 0; j < 3; ++j) {
+            const double u = h27_d(q1, j) * tdd + h27_p(q1, j) * tdp, v = h27_d(q1, j) * tpd + h27_p(q1, j) * tpp;
+#pragma unroll
+            for (int i = 0; i < 3; ++i) {
+              if (h27_d(q1, i) != 0.0) K0[i][j] += h27_d(q1, i) * u;
+              if (h27_p(q1, i) != 0.0) K0[i][j] += h27_p(q1, i) * v;
+            }
+          }
+        }
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+#pragma unroll
+          for (int j = 0; j < 3; ++j) K[i][j] = K0[i][j];
+      }
+      h27_sync();  // S is read
+      CT *tile = (CT *)s_buf;
+      if (lane < 54) {
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+#pragma unroll
+          for (int j = 0; j < 3; ++j) {
+            double v = K[i][j];
+            if (((cm >> ni[i]) | (cm >> nj[j])) & 1u) v = ni[i] == nj[j] ? 1.0 : 0.0;
+            tile[ni[i] * 27 + nj[j]] = (CT)v;
+            if (cc >= 3) tile[nj[j] * 27 + ni[i]] = (CT)v;
+          }
+      }
+      h27_sync();
+      CT *out = Ke + (e0 + el) * 729;
+#pragma unroll
+      for (int k = 0; k < 12; ++k)
+        if (k < 11 || lane < 729 - 64 * 11) out[64 * k + lane] = tile[64 * k + lane];
+      h27_sync();
+    }
+  }
+}
+
 static int h27_grid(lmh_context *ctx, int64_t ne) {
   return grid_for((ne + kH27PerWave - 1) / kH27PerWave, 1, ctx->cu_count * 32);
 }
+
+template <typename CT>
+int hex27_poisson(lmh_context *ctx, const lmh_mesh *m, const lmh_dofmap *dm, const double *kappa, int f_kind,
+                  int constrain, CT *Ke, double *Fe) {
+  const int64_t ne = m->n_elem;
+  if (ne == 0) return LMH_OK;
+  // seven elements share the geometry lanes; fewer while that leaves wavefronts
+  // unused (8 per CU)
+  const int per = (int)std::min<int64_t>(kH27PerWave, std::max<int64_t>(1, ne / (ctx->cu_count * 8)));
+  const int g = grid_for((ne + per - 1) / per, 1, ctx->cu_count * 9);
+  const char *name = sizeof(CT) == 8 ? "element_hex27_fp64" : "element_hex27_fp32";
+  if (f_kind == 0)
+    LMH_LAUNCH(ctx, name, (k_hex27_poisson<CT, 0>), dim3(g), dim3(64), 0, m->xyz, m->conn, dm->edofs,
+               dm->cons, kappa, constrain, per, ne, Ke, Fe, ctx->d_flags);
+  else
+    LMH_LAUNCH(ctx, name, (k_hex27_poisson<CT, 1>), dim3(g), dim3(64), 0, m->xyz, m->conn, dm->edofs,
+               dm->cons, kappa, constrain, per, ne, Ke, Fe, ctx->d_flags);
+  return check_launch("k_hex27_poisson");
+}
+template int hex27_poisson<double>(lmh_context *, const lmh_mesh *, const lmh_dofmap *, const double *, int, int,
+                                   double *, double *);
+template int hex27_poisson<float>(lmh_context *, const lmh_mesh *, const lmh_dofmap *, const double *, int, int,
+                                  float *, double *);
 
 int hex27_residual(lmh_context *ctx, const lmh_mesh *m, const lmh_dofmap *dm, const double *kappa, int f_kind,
                    const double *u, double *Fe) {
