@@ -196,6 +196,15 @@ struct lmh_matrix {
   uint16_t *woff16 = nullptr;  // window offsets
   int4 *rbmeta = nullptr;      // 2 nrbw
   uint16_t *off = nullptr;  // n_elem*dpe*dpe slot offsets within rows
+  // row tiles of the gather scatter (lmh_scatter.hip): {first row, rows,
+  // sequence start, steps}, incidence sequence, slot offsets (8-bit, 16-bit
+  // when wide), LDS entries of a tile
+  int4 *st_tile = nullptr;
+  int2 *st_seq = nullptr;
+  void *st_map = nullptr;
+  int64_t n_stile = 0;
+  int st_slots = 0;
+  bool st_wide = false;
   int32_t *diag = nullptr;  // rows: position of the diagonal entry, -1 if absent
   int ncolors = 0;
   std::vector<int64_t> color_ptr;  // host, ncolors+1
@@ -248,6 +257,10 @@ int fe_table(lmh_context *ctx, int type, int arg, const FETable **out);
 // CSR pattern, scatter map, (if colour) element colouring and (if fp64) zeroed
 // FP64 values for a DoF map
 int matrix_create_impl(lmh_context *ctx, const lmh_dofmap *dm, bool colour, bool fp64, lmh_matrix **out);
+// row tiles of a matrix's gather scatter, and the scatter on them
+int matrix_build_tiles(lmh_matrix *A, const std::vector<int32_t> &h_rp);
+template <typename T>
+int scatter_tiles(lmh_matrix *A, const T *Ke, const double *Fe, T *vals, double *rhs);
 // general constraints around the scatter: before it, the general elements'
 // matrices are replaced by their constrained, expanded forms (and zeroed in
 // Ke/Fe); after it, those are added into their rows
@@ -308,6 +321,22 @@ __device__ inline void block_range(int64_t n, int64_t &lo, int64_t &hi) {
   const int64_t per = (n + gridDim.x - 1) / gridDim.x;
   lo = (int64_t)lb * per;
   hi = lo + per < n ? lo + per : n;
+}
+
+// Items t, t + step, ... < hi of this workgroup: every XCD owns one contiguous
+// range of the items and its workgroups walk it side by side, so what runs at
+// the same time is adjacent in memory and shares the XCD's L2.
+__device__ inline void xcd_walk(int64_t n, int64_t &t, int64_t &hi, int64_t &step) {
+  if (gridDim.x % NXCD == 0) {
+    const int64_t xcd = blockIdx.x % NXCD;
+    t = n * xcd / NXCD + blockIdx.x / NXCD;
+    hi = n * (xcd + 1) / NXCD;
+    step = gridDim.x / NXCD;
+  } else {
+    t = blockIdx.x;
+    hi = n;
+    step = gridDim.x;
+  }
 }
 
 // the same with lo a multiple of W (the share rounded up to W items)

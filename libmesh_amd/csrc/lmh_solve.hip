@@ -311,19 +311,8 @@ __device__ inline void rowblock_spmv16(int64_t nrb, const int4 *__restrict__ des
   constexpr int NB = sizeof(T) == 8 ? 1 : 2;
   __shared__ int32_t rowbuf[NB][NT];
   __shared__ double prebuf[NB][NP][NPRE > 0 ? NT : 1];
-  // this workgroup's blocks: every XCD owns one contiguous range of blocks and
-  // its workgroups walk it side by side (workgroup j takes j, j + step, ...).
   int64_t lo, hi, step_b;
-  if (gridDim.x % NXCD == 0) {
-    const int64_t xcd = blockIdx.x % NXCD;
-    lo = nrb * xcd / NXCD + blockIdx.x / NXCD;
-    hi = nrb * (xcd + 1) / NXCD;
-    step_b = gridDim.x / NXCD;
-  } else {
-    lo = blockIdx.x;
-    hi = nrb;
-    step_b = gridDim.x;
-  }
+  xcd_walk(nrb, lo, hi, step_b);
   if (lo >= hi) return;
   const int tid = threadIdx.x, sub = tid & 7, grp = tid >> 3;
   struct Blk {
