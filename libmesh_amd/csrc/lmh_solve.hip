@@ -1120,8 +1120,18 @@ __global__ __launch_bounds__(BLK) void k_fin_sum(const double *__restrict__ part
 
 static int vec_grid(lmh_context *ctx) {
   // the partial buffer holds 4 * n_part doubles; publish<3> uses 3 * grid
-  const int g = ctx->cu_count * LMH_GRID_PER_CU;
-  return g < ctx->n_part ? g : ctx->n_part;
+  return std::min(ctx->cu_count * LMH_GRID_PER_CU, ctx->n_part);
+}
+// Small vectors take a workgroup per 512 entries: every consumer sums all
+// workgroups' partials, and empty workgroups cost their dispatch (CG with 1,331
+// rows: update 9.7 -> 6.5 us, p-update 8.0 -> 6.4 us with 3 workgroups for 1024,
+// both with the 5 us of their timing events; BiCGSTAB with 68,921 rows 7.4 ->
+// 6.4 ms a solve).  BiCGSTAB keeps the full grid below kBcgSmall rows: on small
+// systems whose (r0, r) vanishes in exact arithmetic the order of its sums
+// decides between convergence and breakdown, and the launches dominate anyway.
+constexpr int64_t kBcgSmall = 16384;
+static int vec_grid(lmh_context *ctx, int64_t n) {
+  return (int)std::max<int64_t>(1, std::min<int64_t>(vec_grid(ctx), (n + 511) / 512));
 }
 
 // SpMV-type kernels (row-block streams) want more resident waves than the
@@ -1296,6 +1306,8 @@ static Stream stream_of(lmh_matrix *A, bool fp32) {
   s.on = A->idx16_state == 1;
   s.nt = s.on && A->wbits == 8 ? W8_NT : BLK;
   s.grid = s.on && A->wbits == 8 ? W8_GRID * gs : gs;
+  // at most one workgroup per row block (whole XCD rounds)
+  s.grid = (int)std::min<int64_t>(s.grid, ((s.on ? A->nrbw : A->nrb) + NXCD - 1) / NXCD * NXCD);
   if (use_windows(A) && A->cols < ((int64_t)1 << 29)) {
     s.iw = A->wbits / 8;
     s.idx = fp32 ? A->widx32 : A->widx64;
@@ -1408,7 +1420,7 @@ int lmh_residual(lmh_matrix *A, const double *b_d, const double *x_d, double *r_
 
 double lmh_norm2(lmh_context *ctx, const double *x_d, int64_t n) {
   if (!ctx || !x_d) return NAN;
-  const int g = vec_grid(ctx);
+  const int g = vec_grid(ctx, n);
   hipLaunchKernelGGL(k_norm2, dim3(g), dim3(BLK), 0, ctx->stream, n, x_d, ctx->d_part);
   hipLaunchKernelGGL(k_fin_sum, dim3(1), dim3(BLK), 0, ctx->stream, ctx->d_part, g, ctx->d_scal + 56);
   double v = NAN;
@@ -1716,7 +1728,7 @@ static int cg_impl(lmh_matrix *A, const double *b_d, double *x_d, double rtol, i
   const int64_t n = A->rows;
   double *S = ctx->d_scal;
   double *part1 = ctx->d_part, *part2 = ctx->d_part + 2 * ctx->n_part;  // 1 and 2 values per block
-  const int g = vec_grid(ctx);
+  const int g = vec_grid(ctx, n);
   const int xvec = ((uintptr_t)x_d & 15) == 0;               // the caller's x takes 16-byte chunks
   CG_LAUNCH("invdiag", (k_invdiag<double, double>), dim3(grid_for(n, BLK, 8192)), n, diag, A->vals,
             A->precond == LMH_PRECOND_JACOBI, dinv);
@@ -1831,7 +1843,7 @@ static int bicgstab_impl(lmh_matrix *A, const double *vals, const double *b_d, d
   double *part1 = ctx->d_part, *part2 = ctx->d_part + 2 * ctx->n_part;
   LMH_TRY(ensure_windows(A));
   const Stream st = stream_of(A, false);
-  const int g = vec_grid(ctx);
+  const int g = n < kBcgSmall ? vec_grid(ctx) : vec_grid(ctx, n);
   LMH_TRY(ensure_diag(A));
   LMH_LAUNCH(ctx, "invdiag", (k_invdiag<double, double>), dim3(grid_for(n, 256, 8192)), dim3(256), 0, n, A->diag,
              vals, A->precond == LMH_PRECOND_JACOBI, dinv);
@@ -1990,7 +2002,7 @@ int lmh_mixed_solve(lmh_matrix *A, const double *b_d, double *x_d, double rtol, 
   float *r32 = A->w32, *p32 = r32 + ns, *q32 = p32 + ns, *d32 = q32 + ns, *xc = d32 + ns;
   double *S = ctx->d_scal;
   double *part1 = ctx->d_part, *part2 = ctx->d_part + 2 * ctx->n_part;
-  const int g = vec_grid(ctx);
+  const int g = vec_grid(ctx, n);
   auto residual32 = [&](int init, int bank) {  // the FP64 residual and the FP32 start of the recurrence
     if (st.on)
       with_stream(st, [&](auto sh) {
