@@ -241,6 +241,28 @@ __device__ inline T group8_sum(T s) {
   s += dpp_move<0xb1>(s);   // quad_perm [1,0,3,2]
   return s;
 }
+// the sum over each 16 lanes, the same bits in all of them
+__device__ inline double all16_sum(double s) {
+  s += dpp_move<0xb1>(s);   // quad_perm [1,0,3,2]
+  s += dpp_move<0x4e>(s);   // quad_perm [2,3,0,1]
+  s += dpp_move<0x141>(s);  // row_half_mirror
+  s += dpp_move<0x140>(s);  // row_mirror
+  return s;
+}
+// the sum of the values of lanes 0, 16, 32 and 48 in all lanes
+__device__ inline double rows16_sum(double s) {
+  typedef int i32x2 __attribute__((ext_vector_type(2)));
+  const i32x2 w = __builtin_bit_cast(i32x2, s);
+  double t = 0.0;
+#pragma unroll
+  for (int l = 0; l < 64; l += 16) {
+    i32x2 u;
+    u[0] = __builtin_amdgcn_readlane(w[0], l);
+    u[1] = __builtin_amdgcn_readlane(w[1], l);
+    t += __builtin_bit_cast(double, u);
+  }
+  return t;
+}
 
 // Streamed row blocks.  A row block of ~1000 entries references only a few
 // hundred distinct columns (about 200 for Q2 hexahedra), so the block's x
@@ -976,6 +998,222 @@ __global__ __launch_bounds__(BLK) void k_cg_init_fin(const double *__restrict__ 
 }
 
 // ---------------------------------------------------------------------------
+// Whole CG on one workgroup, for matrices whose values and columns fit its
+// registers (1,024 threads with up to 32 entries, kSmallRows rows): no launches,
+// no scalars through memory, one kernel per solve.  Three kernels an iteration
+// take 13-15 us there, most of it launch latency and the wait of each for the
+// last.  Bound by LDS (a random 8-byte read per entry) and the four barriers.
+// Q1 10^3 (1,331 rows, 29,791 entries, 40 iterations) 23 us an iteration, now
+// 6.1; Q2 3^3 (343 rows, 15,625 entries) 24 -> 4.7; TET4 6^3 (1,315 rows, 15,175
+// entries) 23 -> 4.0; Q1 4^3 solve 373 -> 54 us.  Just beyond it, with three
+// kernels an iteration: TET10 4^3 (63,905 entries) 22 -> 14.
+// Thread t holds entries E t .. E t + E - 1 and sums them in order; `ends` marks
+// a row's last entry, whose sum goes to q[row], and what is left of a row that
+// the next thread goes on with goes to tail[t].  Row i's owner (thread i mod
+// 1024) adds the tails of the threads in front of its end.  No row is empty, so
+// a thread's rows count up by one.
+// ---------------------------------------------------------------------------
+constexpr int kSmallNT = 1024, kSmallRows = 4096, kSmallEntries = 32;
+constexpr int64_t kSmallIts = 100000;
+constexpr size_t kSmallLds = sizeof(double) * (3 * kSmallRows + kSmallNT + 256);
+
+template <int E, int K>
+__global__ __launch_bounds__(kSmallNT) void k_cg_small(int n, const int32_t *__restrict__ rp,
+                                                       const int32_t *__restrict__ ci, const double *__restrict__ v,
+                                                       const int32_t *__restrict__ diag, int jacobi,
+                                                       const double *__restrict__ b, double *__restrict__ x,
+                                                       double tol, int64_t maxits, double *__restrict__ S) {
+  extern __shared__ __align__(16) unsigned char sm[];
+  double *p = (double *)sm, *q = p + kSmallRows, *r = q + kSmallRows, *tail = r + kSmallRows, *red = tail + kSmallNT;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int32_t nnz = rp[n], e0 = E * tid;
+  double va[E];
+  uint32_t cx[E / 2], ends = 0;  // 8 x column, two to a register
+  int row0 = 0;                  // the row of entry e0: the last one that starts at or before it
+  for (int step = kSmallRows; step > 0; step >>= 1)
+    if (row0 + step < n && rp[row0 + step] <= e0) row0 += step;
+#pragma unroll
+  for (int j = 0; j < E; j += 2) {
+    const int32_t k = e0 + j;
+    va[j] = k < nnz ? v[k] : 0.0;
+    va[j + 1] = k + 1 < nnz ? v[k + 1] : 0.0;
+    cx[j / 2] = (k < nnz ? 8u * (uint32_t)ci[k] : 0u) | (k + 1 < nnz ? 8u * (uint32_t)ci[k + 1] : 0u) << 16;
+  }
+  for (int i = row0; i < n && e0 < nnz; ++i) {
+    const int32_t last = rp[i + 1] - 1 - e0;
+    if (last >= E) break;
+    ends |= 1u << last;
+  }
+  // totals of up to two values over the workgroup, in every thread; consecutive
+  // calls alternate their LDS slots, so one barrier each is enough
+  int slot = 0;
+  auto total = [&](double s0, double s1, double (&t)[2]) {
+    s0 = all16_sum(s0);
+    s1 = all16_sum(s1);
+    double *rd = red + 128 * slot;
+    slot ^= 1;
+    if ((lane & 15) == 0) {
+      rd[tid >> 4] = s0;
+      rd[64 + (tid >> 4)] = s1;
+    }
+    __syncthreads();
+    s0 = all16_sum(rd[lane]);
+    s1 = all16_sum(rd[64 + lane]);
+    t[0] = rows16_sum(s0);
+    t[1] = rows16_sum(s1);
+  };
+  double xr[K], di[K], t[2];
+  int32_t own[K];  // row i's first thread and, 10 bits up, how many follow it
+  // q = A p (p in LDS): afterwards q[i] is the owner's to read
+  auto product = [&]() {
+    __syncthreads();  // p is written
+    double s = 0.0;
+    double *qr = q + row0;
+#pragma unroll
+    for (int j = 0; j < E; ++j) {
+      const uint32_t c = j & 1 ? cx[j / 2] >> 16 : cx[j / 2] & 0xffffu;
+      s = fma(va[j], *(const double *)(sm + c), s);
+      if (ends >> j & 1) {
+        *qr++ = s;
+        s = 0.0;
+      }
+    }
+    tail[tid] = s;
+    __syncthreads();
+  };
+  auto row_of = [&](int k, int i) {
+    const int t0 = own[k] & 1023, t1 = t0 + (own[k] >> 10);
+    double s = q[i];
+    for (int u = t0; u < t1; ++u) s += tail[u];
+    return s;
+  };
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    const int i = tid + kSmallNT * k;
+    xr[k] = 0.0;
+    di[k] = 1.0;
+    own[k] = 0;
+    if (i < n) {
+      const int32_t d = diag[i], t0 = rp[i] / E, t1 = (rp[i + 1] - 1) / E;
+      own[k] = t0 | (t1 - t0) << 10;
+      if (jacobi && d >= 0 && v[d] != 0.0) di[k] = 1.0 / v[d];
+      p[i] = xr[k] = x[i];
+    }
+  }
+  product();
+  double rr = 0.0, bb = 0.0, rz = 0.0;
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    const int i = tid + kSmallNT * k;
+    if (i < n) {
+      const double bv = b[i], rv = bv - row_of(k, i);
+      r[i] = rv;
+      rr += rv * rv;
+      bb += bv * bv;
+      rz += rv * (di[k] * rv);
+    }
+  }
+  total(rr, bb, t);
+  rr = t[0];
+  bb = t[1];
+  total(rz, 0.0, t);
+  rz = t[0];
+  const double thr = fmax(tol * tol * bb, 2.2250738585072014e-308);
+  bool done = true;
+  int reason = LMH_CONVERGED_RTOL;
+  if (bb == 0.0) {  // x = 0
+    rr = 0.0;
+#pragma unroll
+    for (int k = 0; k < K; ++k) xr[k] = 0.0;
+  } else if (!isfinite(rr) || !isfinite(bb)) {
+    reason = LMH_DIVERGED_NANORINF;
+  } else if (!(rr < thr)) {
+    done = false;
+    reason = 0;
+  }
+  int64_t its = 0;
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    const int i = tid + kSmallNT * k;
+    if (i < n) p[i] = di[k] * r[i];
+  }
+  for (int64_t it = 0; it < maxits && !done; ++it) {
+    product();
+    double pq = 0.0;
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      const int i = tid + kSmallNT * k;
+      if (i < n) {
+        const double s = row_of(k, i);
+        q[i] = s;
+        pq += p[i] * s;
+      }
+    }
+    total(pq, 0.0, t);
+    const double alpha = rz / t[0];
+    if (!(t[0] != 0.0) || !isfinite(alpha)) {
+      done = true;
+      reason = LMH_DIVERGED_BREAKDOWN;
+      break;
+    }
+    double nr = 0.0, nz = 0.0;
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      const int i = tid + kSmallNT * k;
+      if (i < n) {
+        xr[k] += alpha * p[i];
+        const double rv = r[i] - alpha * q[i];
+        r[i] = rv;
+        nr += rv * rv;
+        nz += rv * (di[k] * rv);
+      }
+    }
+    total(nr, nz, t);
+    rr = t[0];
+    if (!isfinite(rr)) {
+      done = true;
+      reason = LMH_DIVERGED_NANORINF;
+    } else if (rr < thr) {
+      done = true;
+      reason = LMH_CONVERGED_RTOL;
+    } else {
+      ++its;
+      const double beta = t[1] / rz;
+      rz = t[1];
+#pragma unroll
+      for (int k = 0; k < K; ++k) {
+        const int i = tid + kSmallNT * k;
+        if (i < n) p[i] = di[k] * r[i] + beta * p[i];
+      }
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    const int i = tid + kSmallNT * k;
+    if (i < n) x[i] = xr[k];
+  }
+  if (tid == 0) {  // both banks: the host reads either
+    for (int bank = 0; bank < 2; ++bank) {
+      double *B = S + bank * B_SIZE;
+      B[B_RZ] = rz;
+      B[B_RR] = rr;
+      B[B_ITS] = (double)its;
+      B[B_DONE] = done ? 1.0 : 0.0;
+      B[B_REASON] = reason;
+    }
+    S[G_THR] = thr;
+    S[G_BB] = bb;
+  }
+}
+
+// the solves k_cg_small takes: whatever fits it (both sides above), with the
+// iterations bounded so that one kernel ends within a second
+static bool cg_small_fits(const lmh_matrix *A, int64_t maxits) {
+  return A->rows == A->cols && A->rows <= kSmallRows && A->nnz <= kSmallNT * kSmallEntries && A->min_row > 0 &&
+         maxits <= kSmallIts;
+}
+
+// ---------------------------------------------------------------------------
 // Mixed precision refresh: r64 = b - A64 x (FP64 operator); r32 = (float) r64;
 // z = dinv32 r32 (p32 = z on the initial call); partials |r|^2, |b|^2, (r32, z).
 // ---------------------------------------------------------------------------
@@ -1708,6 +1946,47 @@ int cg_scratch_setup(lmh_context *ctx) {
   return LMH_OK;
 }
 
+// The outcome of a CG whose last bank is K & 1, read back from the device scalars
+static int cg_result(lmh_matrix *A, int64_t K, int64_t maxits, int64_t *iters, double *rel_res, int *reason) {
+  lmh_context *ctx = A->ctx;
+  double *S = ctx->d_scal, *snap = ctx->h_pinned;
+  // both banks and |b|^2 (G_BB follows the banks) into pinned memory
+  static_assert(G_BB < 64, "scalar slots beyond the pinned copy");
+  LMH_HIP(hipMemcpyAsync(snap, S, sizeof(double) * (G_BB + 1), hipMemcpyDeviceToHost, ctx->stream));
+  LMH_HIP(hipStreamSynchronize(ctx->stream));
+  const double *Bk = snap + (K & 1) * B_SIZE, gbb = snap[G_BB];
+  const bool conv = Bk[B_DONE] != 0.0;
+  if (iters) *iters = conv ? (int64_t)Bk[B_ITS] : maxits;
+  if (rel_res) *rel_res = gbb > 0 ? std::sqrt(Bk[B_RR] / gbb) : 0.0;
+  if (reason) *reason = conv ? (int)Bk[B_REASON] : LMH_DIVERGED_ITS;
+  return LMH_OK;
+}
+
+template <bool NA>
+static int cg_small(lmh_matrix *A, const double *b_d, double *x_d, double rtol, int64_t maxits, const int32_t *diag) {
+  lmh_context *ctx = A->ctx;
+  const int jac = A->precond == LMH_PRECOND_JACOBI;
+  ProfScope ps(NA ? nullptr : ctx, "cg_small");
+  auto launch = [&](auto kern) -> int {
+    LMH_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kSmallLds));
+    hipLaunchKernelGGL(kern, dim3(1), dim3(kSmallNT), kSmallLds, ctx->stream, (int)A->rows, A->rp, A->ci, A->vals, diag,
+                       jac, b_d, x_d, rtol, maxits, ctx->d_scal);
+    return LMH_OK;
+  };
+  const bool two = A->rows > kSmallNT, four = A->rows > 2 * kSmallNT;
+#define CG_SMALL(E) LMH_TRY(four ? launch(k_cg_small<E, 4>) : two ? launch(k_cg_small<E, 2>) : launch(k_cg_small<E, 1>))
+  if (A->nnz <= 8 * kSmallNT)
+    CG_SMALL(8);
+  else if (A->nnz <= 16 * kSmallNT)
+    CG_SMALL(16);
+  else if (A->nnz <= 24 * kSmallNT)
+    CG_SMALL(24);
+  else
+    CG_SMALL(32);
+#undef CG_SMALL
+  return check_launch("k_cg_small");
+}
+
 // Jacobi/identity CG iterations on A (FP64).  r, p, q, dinv: n doubles each;
 // diag: A's diagonal slots.  NA (no allocation): launches without the
 // profiling events and uses the x windows only when they are already built.
@@ -1723,6 +2002,10 @@ static int cg_impl(lmh_matrix *A, const double *b_d, double *x_d, double rtol, i
   } while (0)
 #define CG_LAUNCH(name, kernel, grid, ...) CG_LAUNCH_NT(name, kernel, grid, BLK, __VA_ARGS__)
   lmh_context *ctx = A->ctx;
+  if (cg_small_fits(A, maxits)) {
+    LMH_TRY((cg_small<NA>(A, b_d, x_d, rtol, maxits, diag)));
+    return cg_result(A, 0, maxits, iters, rel_res, reason);
+  }
   if (!NA) LMH_TRY(ensure_windows(A));
   const Stream st = stream_of(A, false);
   const int64_t n = A->rows;
@@ -1774,16 +2057,7 @@ static int cg_impl(lmh_matrix *A, const double *b_d, double *x_d, double rtol, i
   }
 #undef CG_LAUNCH
   LMH_TRY(check_launch("cg iterations"));
-  // both banks and |b|^2 (G_BB follows the banks) into pinned memory
-  static_assert(G_BB < 64, "scalar slots beyond the pinned copy");
-  LMH_HIP(hipMemcpyAsync(snap, S, sizeof(double) * (G_BB + 1), hipMemcpyDeviceToHost, ctx->stream));
-  LMH_HIP(hipStreamSynchronize(ctx->stream));
-  const double *Bk = snap + (K & 1) * B_SIZE, gbb = snap[G_BB];
-  const bool conv = Bk[B_DONE] != 0.0;
-  if (iters) *iters = conv ? (int64_t)Bk[B_ITS] : maxits;
-  if (rel_res) *rel_res = gbb > 0 ? std::sqrt(Bk[B_RR] / gbb) : 0.0;
-  if (reason) *reason = conv ? (int)Bk[B_REASON] : LMH_DIVERGED_ITS;
-  return LMH_OK;
+  return cg_result(A, K, maxits, iters, rel_res, reason);
 }
 
 }  // namespace lmh

@@ -252,7 +252,11 @@ int matrix_create_impl(lmh_context *ctx, const lmh_dofmap *dm, bool colour, bool
   std::vector<int32_t> rp(n + 1);
   LMH_HIP(hipMemcpyAsync(rp.data(), A->rp, sizeof(int32_t) * (n + 1), hipMemcpyDeviceToHost, ctx->stream));
   LMH_HIP(hipStreamSynchronize(ctx->stream));
-  for (int64_t r = 0; r < n; ++r) A->max_row = std::max<int>(A->max_row, rp[r + 1] - rp[r]);
+  A->min_row = INT32_MAX;
+  for (int64_t r = 0; r < n; ++r) {
+    A->max_row = std::max<int>(A->max_row, rp[r + 1] - rp[r]);
+    A->min_row = std::min<int>(A->min_row, rp[r + 1] - rp[r]);
+  }
   LMH_TRY(build_row_blocks(A.get(), rp));
   LMH_HIP(hipFree(rowlen));
   LMH_CHECK(A->max_row <= 65535, LMH_ERR_UNSUPPORTED, "row length %d exceeds 16-bit scatter offsets", A->max_row);
@@ -314,10 +318,11 @@ int lmh_matrix_create_csr2(lmh_context *ctx, int64_t rows, int64_t cols, const i
   const int64_t nnz = row_ptr_h[rows];
   LMH_CHECK(nnz >= 0 && (nnz == 0 || col_idx_h), LMH_ERR_INVALID, "bad nnz");
   std::vector<int32_t> rp(row_ptr_h, row_ptr_h + rows + 1);
-  int max_row = 0;
+  int max_row = 0, min_row = INT32_MAX;
   for (int64_t r = 0; r < rows; ++r) {
     LMH_CHECK(rp[r + 1] >= rp[r], LMH_ERR_INVALID, "row_ptr not monotone at row %lld", (long long)r);
     max_row = std::max<int>(max_row, rp[r + 1] - rp[r]);
+    min_row = std::min<int>(min_row, rp[r + 1] - rp[r]);
     for (int32_t k = rp[r]; k < rp[r + 1]; ++k) {
       LMH_CHECK(col_idx_h[k] >= 0 && col_idx_h[k] < cols, LMH_ERR_INVALID, "column index out of range");
       LMH_CHECK(k == rp[r] || col_idx_h[k] > col_idx_h[k - 1], LMH_ERR_INVALID,
@@ -331,6 +336,7 @@ int lmh_matrix_create_csr2(lmh_context *ctx, int64_t rows, int64_t cols, const i
   A->cols = cols;
   A->nnz = nnz;
   A->max_row = max_row;
+  A->min_row = min_row;
   LMH_HIP(hipMalloc((void **)&A->rp, sizeof(int32_t) * (rows + 1)));
   LMH_HIP(hipMalloc((void **)&A->ci, sizeof(int32_t) * (nnz + LMH_PAD)));
   LMH_HIP(hipMalloc((void **)&A->vals, sizeof(double) * (nnz + LMH_PAD)));
