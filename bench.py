@@ -493,7 +493,7 @@ def bench_batched(args, L, log, ctx, steps, warmup):
                      "element_kernel_ms": dict(zip(["HEX8", "HEX27", "TET4", "TET10"], best.round(4).tolist()))},
         "roofline": {"bound": "hbm", "achieved": round(gbs, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": round(gbs / HBM_PEAK_GBS, 4), "traffic": None, "compulsory_bytes": int(comp),
-                     "kernel": "batch graph (k_batch_elasticity + k_batch_scatter)"},
+                     "kernel": "batch graph (k_batch_elasticity + k_batch_rows)"},
         "setup_s": round(t_setup, 2),
         "mdofs": round(n_dofs / (gms * 1e-3) / 1e6, 3),
     }

@@ -12,19 +12,7 @@
 
 #include <hip/hip_runtime.h>
 
-__device__ inline double lmh_qp_map(const double *X, const double *dref, int n, int nq, int q, double G[3][3]) {
-  double J[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}};  // J[r][c] = d x_c / d xi_r
-#pragma unroll 4
-  for (int a = 0; a < n; ++a) {
-    const double *d = &dref[(a * nq + q) * 3];
-    const double x = X[a * 3], y = X[a * 3 + 1], z = X[a * 3 + 2];
-#pragma unroll
-    for (int r = 0; r < 3; ++r) {
-      J[r][0] += x * d[r];
-      J[r][1] += y * d[r];
-      J[r][2] += z * d[r];
-    }
-  }
+__device__ inline double lmh_map_inverse(const double J[3][3], double G[3][3]) {
   const double dx_dxi = J[0][0], dy_dxi = J[0][1], dz_dxi = J[0][2];
   const double dx_deta = J[1][0], dy_deta = J[1][1], dz_deta = J[1][2];
   const double dx_dzeta = J[2][0], dy_dzeta = J[2][1], dz_dzeta = J[2][2];
@@ -43,6 +31,22 @@ __device__ inline double lmh_qp_map(const double *X, const double *dref, int n, 
   G[2][1] = (dz_dxi * dx_deta - dx_dxi * dz_deta) * inv;
   G[2][2] = (dx_dxi * dy_deta - dy_dxi * dx_deta) * inv;
   return det;
+}
+
+__device__ inline double lmh_qp_map(const double *X, const double *dref, int n, int nq, int q, double G[3][3]) {
+  double J[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}};  // J[r][c] = d x_c / d xi_r
+#pragma unroll 4
+  for (int a = 0; a < n; ++a) {
+    const double *d = &dref[(a * nq + q) * 3];
+    const double x = X[a * 3], y = X[a * 3 + 1], z = X[a * 3 + 2];
+#pragma unroll
+    for (int r = 0; r < 3; ++r) {
+      J[r][0] += x * d[r];
+      J[r][1] += y * d[r];
+      J[r][2] += z * d[r];
+    }
+  }
+  return lmh_map_inverse(J, G);
 }
 
 #endif

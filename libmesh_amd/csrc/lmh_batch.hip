@@ -1,9 +1,9 @@
 // lmh_batch.hip -- FP32 assembly of many independent linear-elasticity problems
-// (uneven sizes, mixed HEX8/HEX27/TET4/TET10) in one hipGraph launch: a
-// persistent element kernel walks a tile list that covers every problem, then
-// a persistent gather-scatter kernel writes every problem's CSR values and
-// right-hand side.  Tile shapes (lanes per element, elements per tile) are
-// chosen per element type by timing candidates on the actual batch.
+// (uneven sizes, mixed HEX8/HEX27/TET4/TET10) in one hipGraph launch: an element
+// kernel takes a tile of elements per workgroup, over every problem, then a row
+// kernel takes a tile of node rows per wave and writes every problem's CSR
+// values and right-hand side.  Tile shapes (lanes per element, elements per
+// tile) are chosen per element type by timing candidates on the actual batch.
 //
 // Element operator (systems_of_equations_ex6.C:127-150, 220-236):
 //   Ke[(i,a),(k,b)] = sum_q JxW_q sum_jl C_ijkl dphi_a(q)_j dphi_b(q)_l,
@@ -12,12 +12,16 @@
 //   Ke[(i,a),(k,b)] = l1 T_ab[i][k] + l2 T_ab[k][i] + d_ik l2 tr T_ab,
 // and Fe[(i,a)] = sum_q JxW_q f_i phi_a(q) with f = (0, 0, fz).  Element DoFs are
 // variable-major as DofMap::dof_indices returns them (all nodes of u, then v,
-// then w).  Geometry (J, det, inverse) is FP64; physical gradients are rounded
-// to FP32 and the contraction accumulates in FP32.  Fe stays FP64.
+// then w); element matrices are kept node-major (row 3a + i, column 3b + k), so
+// that a node pair's 3 x 3 block is three runs of three floats in the element
+// matrix and in the CSR row alike.  Geometry (J, det, inverse) and the gradients
+// scaled by sqrt(JxW) are FP64, then rounded to FP32 once; the contraction
+// accumulates in FP32.  Fe stays FP64 (its z part: the rest is zero).
 #include <algorithm>
 #include <cmath>
 #include <vector>
 
+#include "lmh_hex27.h"
 #include "lmh_internal.h"
 
 namespace lmh {
@@ -28,8 +32,9 @@ struct BProb {
   const int32_t *edofs;
   const uint8_t *cons;
   const double *fe;  // w[nq] | phi[n*nq] | dref[n*nq*3]
-  float *Ke;         // n_elem * dpe * dpe
-  double *Fe;        // n_elem * dpe
+  float *Ke;         // n_elem * dpe * dpe, node-major
+  float4 *rec;       // TET4 with node blocks: sqrt(JxW) grad phi_a and the constraint bits, n_elem * 4
+  double *Fe;        // n_elem * n: the z component
   int64_t n_elem;
   int n, nq;
 };
@@ -42,15 +47,17 @@ struct BScat {
   const int32_t *inc_ptr, *inc, *rp;
   const uint16_t *off;
   const float *Ke;
+  const float4 *rec;
   const double *Fe;
   float *vals;
   double *rhs;
   int64_t rows;
-  int dpe, w;  // element DoFs, lanes per row (16, 32 or 64)
-  int stride;  // LDS accumulator row of each sub-group: the problem's longest row, rounded up to 4
+  int dpe, w;  // element DoFs, lanes per row (16, 32 or 64) of the general row kernel
+  int stride;  // its LDS accumulator row of each sub-group: the problem's longest row, rounded up to 4
   int pad;
 };
 
+// rows r0 .. r1 - 1: node rows (three DoFs each) or, in the general kernel, DoFs
 struct BRTile {
   int32_t p, r0, r1, pad;
 };
@@ -87,127 +94,497 @@ __global__ void k_batch_clear(int *flag) {
   if (threadIdx.x == 0 && blockIdx.x == 0) flag[0] = 0;
 }
 
-__global__ __launch_bounds__(kBatchBlock) void k_batch_elasticity(const BProb *__restrict__ probs,
-                                                                  const BTile *__restrict__ tiles, int ntiles,
-                                                                  float lam1, float lam2, double fz,
-                                                                  int *__restrict__ err) {
-  extern __shared__ __align__(16) unsigned char sm[];
-  for (int t = blockIdx.x; t < ntiles; t += gridDim.x) {
-    const BTile tl = tiles[t];
-    const BProb P = probs[tl.p];
-    const int L = tl.lpe, epp = kBatchBlock / L;
-    const int sub = threadIdx.x / L, l = threadIdx.x - sub * L;
-    const int n = P.n, nq = P.nq, dpe = 3 * n;
-    int gpb = nq * n * 16;
-    if (gpb < n * 24) gpb = n * 24;
-    unsigned char *S = sm + sub * slot_bytes(n, nq);
-    float4 *Gp = (float4 *)S;
-    double *X = (double *)S;
-    double *Gq = (double *)(S + gpb);
-    double *Jw = Gq + nq * 9;
-    double *Fz = Jw + nq;
-    uint8_t *cf = (uint8_t *)(Fz + n);  // constraint flag per element DoF
-    const double *w = P.fe, *phi = P.fe + nq, *dref = P.fe + nq + (size_t)n * nq;
-    for (int64_t eb = tl.e0; eb < tl.e1; eb += epp) {
-      const int64_t e = eb + sub;
-      const bool act = e < tl.e1;
-      if (act)
-        for (int k = l; k < n * 3; k += L) {
-          const int a = k / 3, c = k - a * 3;
-          X[k] = P.xyz[(int64_t)P.conn[e * n + a] * 3 + c];
-          cf[k] = P.cons[P.edofs[e * dpe + k]];
-        }
-      __syncthreads();
-      if (act)
-        for (int q = l; q < nq; q += L) {
-          double G[3][3];
-          const double det = qp_map(X, dref, n, nq, q, G);
-          if (!(det > 0.0)) {
-            atomicOr(err, 1);
-            for (int r = 0; r < 3; ++r)
-              for (int c = 0; c < 3; ++c) G[r][c] = 0.0;
-          }
-          for (int r = 0; r < 3; ++r)
-            for (int c = 0; c < 3; ++c) Gq[q * 9 + r * 3 + c] = G[r][c];
-          Jw[q] = det * w[q];
-        }
-      __syncthreads();
-      if (act) {
-        // dphi_a(q)_c = sum_r dref_a(q)_r G[r][c]  (X is dead from here on)
-        for (int k = l; k < nq * n; k += L) {
-          const int q = k / n, a = k - q * n;
-          const double *d = &dref[(a * nq + q) * 3];
-          const double *G = &Gq[q * 9];
-          float4 g;
-          g.x = (float)(d[0] * G[0] + d[1] * G[3] + d[2] * G[6]);
-          g.y = (float)(d[0] * G[1] + d[1] * G[4] + d[2] * G[7]);
-          g.z = (float)(d[0] * G[2] + d[1] * G[5] + d[2] * G[8]);
-          g.w = 0.f;
-          Gp[q * n + a] = g;
-        }
-        for (int a = l; a < n; a += L) {
-          double s = 0.0;
-          for (int q = 0; q < nq; ++q) s += Jw[q] * (fz * phi[a * nq + q]);
-          Fz[a] = s;
-        }
-      }
-      __syncthreads();
-      if (act) {
-        float *K = P.Ke + e * (int64_t)dpe * dpe;
-        const int npair = n * (n + 1) / 2;
-        for (int k = l; k < npair; k += L) {
-          int a = 0, rem = k;
-          while (rem >= n - a) {
-            rem -= n - a;
-            ++a;
-          }
-          const int b = a + rem;
-          float T[9];
+typedef float f32x3 __attribute__((ext_vector_type(3), aligned(4)));
+
+// row i of the 3 x 3 block of a node pair, after the element constraint
+// (dof_map_constraints.C:2518-2616): zero row and column of a constrained DoF,
+// unit diagonal
+__device__ inline f32x3 elasticity_row(const float (&T)[9], int i, float lam1, float lam2, bool ca, const bool (&cb)[3],
+                                       bool diag) {
+  const float tr = T[0] + T[4] + T[8];
+  f32x3 v;
 #pragma unroll
-          for (int m = 0; m < 9; ++m) T[m] = 0.f;
-          for (int q = 0; q < nq; ++q) {
-            const float wq = (float)Jw[q];
-            const float4 ga = Gp[q * n + a], gb = Gp[q * n + b];
-            const float ax = wq * ga.x, ay = wq * ga.y, az = wq * ga.z;
-            T[0] += ax * gb.x;
-            T[1] += ax * gb.y;
-            T[2] += ax * gb.z;
-            T[3] += ay * gb.x;
-            T[4] += ay * gb.y;
-            T[5] += ay * gb.z;
-            T[6] += az * gb.x;
-            T[7] += az * gb.y;
-            T[8] += az * gb.z;
-          }
-          const float tr = T[0] + T[4] + T[8];
+  for (int c = 0; c < 3; ++c) {
+    float s = lam1 * T[i * 3 + c] + lam2 * T[c * 3 + i];
+    if (i == c) s += lam2 * tr;
+    v[c] = ca || cb[c] ? (diag && i == c ? 1.f : 0.f) : s;
+  }
+  return v;
+}
+
+// TET4 problems with node blocks: no element matrix.  The gradient is constant,
+// so T_ab = h_a h_b^T with h = sqrt(det sum_q w_q) grad phi: 64 bytes an element
+// instead of 576, written by the element's four lanes (one node each, the four
+// corners exchanged by DPP), and the row kernel forms the blocks.
+__device__ inline void elasticity_tet4(const BProb &P, const BTile &tl, double fz, int *__restrict__ err) {
+  const int a = threadIdx.x & 3;
+  double wsum = 0.0;
+  for (int q = 0; q < P.nq; ++q) wsum += P.fe[q];
+  for (int64_t eb = tl.e0; eb < tl.e1; eb += kBatchBlock / 4) {
+    const int64_t ei = eb + (threadIdx.x >> 2);
+    const bool act = ei < tl.e1;
+    const int64_t e = act ? ei : tl.e1 - 1;
+    const double *xp = P.xyz + (int64_t)P.conn[e * 4 + a] * 3;
+    uint32_t bits = 0;
 #pragma unroll
-          for (int i = 0; i < 3; ++i)
+    for (int c = 0; c < 3; ++c) bits |= (P.cons[P.edofs[e * 12 + c * 4 + a]] ? 1u : 0u) << c;
+    const double x[3] = {xp[0], xp[1], xp[2]};
+    double J[3][3], G[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}};
 #pragma unroll
-            for (int c = 0; c < 3; ++c) {
-              float v = lam1 * T[i * 3 + c] + lam2 * T[c * 3 + i];
-              if (i == c) v += lam2 * tr;
-              const int r = i * n + a, s = c * n + b;
-              // element constraint (dof_map_constraints.C:2518-2616): zero row
-              // and column of a constrained DoF, unit diagonal
-              if (cf[r] | cf[s]) v = (r == s) ? 1.f : 0.f;
-              K[(int64_t)r * dpe + s] = v;
-              if (a != b) K[(int64_t)s * dpe + r] = v;
-            }
-        }
-        for (int k = l; k < dpe; k += L) {
-          const int i = k / n, a = k - i * n;
-          double f = (i == 2) ? Fz[a] : 0.0;
-          if (cf[k]) f = 0.0;
-          P.Fe[e * dpe + k] = f;
-        }
-      }
-      __syncthreads();
+    for (int c = 0; c < 3; ++c) {  // quad_perm broadcasts of lanes 0..3
+      const double x0 = dpp_move<0x00>(x[c]);
+      J[0][c] = dpp_move<0x55>(x[c]) - x0;
+      J[1][c] = dpp_move<0xaa>(x[c]) - x0;
+      J[2][c] = dpp_move<0xff>(x[c]) - x0;
+    }
+    const double det = lmh_map_inverse(J, G);
+    if (!(det > 0.0) && act && a == 0) atomicOr(err, 1);
+    const double sc = det > 0.0 ? sqrt(det * wsum) : 0.0;
+    double g[3], f = 0.0;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) g[c] = a == 0 ? -(G[0][c] + G[1][c] + G[2][c]) : a == 1 ? G[0][c] : a == 2 ? G[1][c] : G[2][c];
+    for (int q = 0; q < P.nq; ++q) f += det * P.fe[q] * (fz * P.fe[P.nq + a * P.nq + q]);
+    if (act) {
+      P.rec[e * 4 + a] = make_float4((float)(sc * g[0]), (float)(sc * g[1]), (float)(sc * g[2]), __uint_as_float(bits));
+      P.Fe[e * 4 + a] = bits & 4u ? 0.0 : f;
     }
   }
 }
 
-// Row-gather scatter over all problems (SparseMatrix::add_matrix /
-// NumericVector::add_vector for every element): each CSR row is summed by a
+// Scaled gradients of one pass's elements, X (LDS) -> Gp (LDS, over X), and the z
+// load into P.Fe.  One lane per quadrature point, its row of the reference table
+// in registers (the table read per element and lane cost more than the arithmetic).
+template <int N, int NQ, bool NEG>
+struct TableGrad {
+  static constexpr int W = NQ <= 8 ? 8 : 16, kExtra = 0;
+  double d[N][3], wq;
+  const double *phi;
+  int q, es;
+  __device__ explicit TableGrad(const BProb &P) {
+    q = threadIdx.x % W;
+    es = threadIdx.x / W;
+    const int qc = q < NQ ? q : NQ - 1;
+    const double *dref = P.fe + NQ + N * NQ;
+#pragma unroll
+    for (int a = 0; a < N; ++a)
+#pragma unroll
+      for (int r = 0; r < 3; ++r) d[a][r] = dref[(a * NQ + qc) * 3 + r];
+    wq = P.fe[qc];
+    phi = P.fe + NQ;
+  }
+  static __device__ int position(int a) { return a; }
+  // slot(s): LDS of element s of the pass; n of them
+  template <typename SL>
+  __device__ void operator()(SL slot, int n, int L, int *__restrict__ err) const {
+    (void)L;
+    const bool on = es < n && q < NQ;
+    double J[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}}, G[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}};
+    float4 *Gp = nullptr;
+    double sc = 0.0;
+    float sign = 1.f;
+    if (on) {
+      auto S = slot(es);
+      Gp = S.Gp;
+#pragma unroll
+      for (int a = 0; a < N; ++a)
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+          const double x = S.X[a * 3 + c];
+#pragma unroll
+          for (int r = 0; r < 3; ++r) J[r][c] += x * d[a][r];
+        }
+      const double det = lmh_map_inverse(J, G);
+      if (!(det > 0.0)) atomicOr(err, 1);
+      const double jw = det * wq;
+      sc = det > 0.0 ? sqrt(fabs(jw)) : 0.0;
+      if (NEG && jw < 0.0) sign = -1.f;
+      S.Jw[q] = jw;
+    }
+    __syncthreads();  // X is dead
+    if (on) {
+#pragma unroll
+      for (int r = 0; r < 9; ++r) G[r / 3][r % 3] *= sc;
+#pragma unroll
+      for (int a = 0; a < N; ++a) {
+        float4 g;
+        g.x = (float)(d[a][0] * G[0][0] + d[a][1] * G[1][0] + d[a][2] * G[2][0]);
+        g.y = (float)(d[a][0] * G[0][1] + d[a][1] * G[1][1] + d[a][2] * G[2][1]);
+        g.z = (float)(d[a][0] * G[0][2] + d[a][1] * G[1][2] + d[a][2] * G[2][2]);
+        g.w = sign;
+        Gp[q * N + a] = g;
+      }
+    }
+    __syncthreads();
+  }
+  template <typename S>
+  __device__ double load(const S &s, int a, double fz) const {
+    double f = 0.0;
+#pragma unroll
+    for (int p = 0; p < NQ; ++p) f += s.Jw[p] * (fz * phi[a * NQ + p]);
+    return f;
+  }
+};
+
+// HEX27: the map by sum factorisation, one lane per point (each repeats its
+// column's first two directions: the other lanes would idle), then one lane per
+// node and plane of points, its 1D shapes in registers; no tables read.  The 1D
+// values are picked anew in every pass: held across passes they cost a wave of
+// occupancy.
+struct Hex27Grad {
+  static constexpr int kExtra = 54;  // doubles: the load's other two planes
+  __device__ explicit Hex27Grad(const BProb &) {}
+  static __device__ int position(int a) { return kH27Lat[a]; }
+  template <typename SL>
+  __device__ void operator()(SL slot, int n, int L, int *__restrict__ err) const {
+    const int s = threadIdx.x / L, l = threadIdx.x & (L - 1);
+    if (s < n && l < 27) {
+      auto S = slot(s);
+      int q = l;
+      asm volatile("" : "+v"(q));  // not loop-invariant
+      const int q1 = q % 3, q2 = q / 3 % 3, q3 = q / 9;
+      double p1[3], d1[3];
+#pragma unroll
+      for (int i = 0; i < 3; ++i) {
+        p1[i] = h27_pick(q1, [&](int k) { return h27_p(k, i); });
+        d1[i] = h27_pick(q1, [&](int k) { return h27_d(k, i); });
+      }
+      double J[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}}, G[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}};
+#pragma unroll
+      for (int i3 = 0; i3 < 3; ++i3) {
+        double t0[3] = {0, 0, 0}, t1[3] = {0, 0, 0}, t2[3] = {0, 0, 0};
+#pragma unroll
+        for (int i2 = 0; i2 < 3; ++i2) {
+          const double p2 = h27_pick(q2, [&](int k) { return h27_p(k, i2); });
+          const double d2 = h27_pick(q2, [&](int k) { return h27_d(k, i2); });
+#pragma unroll
+          for (int c = 0; c < 3; ++c) {
+            const double *x = S.X + (9 * i3 + 3 * i2) * 3 + c;
+            const double p = p1[0] * x[0] + p1[1] * x[3] + p1[2] * x[6];
+            const double d = d1[0] * x[0] + d1[1] * x[3] + d1[2] * x[6];
+            t0[c] += p2 * d;
+            t1[c] += d2 * p;
+            t2[c] += p2 * p;
+          }
+        }
+        const double p3 = h27_pick(q3, [&](int k) { return h27_p(k, i3); });
+        const double d3 = h27_pick(q3, [&](int k) { return h27_d(k, i3); });
+#pragma unroll
+        for (int c = 0; c < 3; ++c) {
+          J[0][c] += p3 * t0[c];
+          J[1][c] += p3 * t1[c];
+          J[2][c] += d3 * t2[c];
+        }
+        __builtin_amdgcn_sched_barrier(0);  // one plane's nodes in registers at a time
+      }
+      const double det = lmh_map_inverse(J, G);
+      if (!(det > 0.0)) atomicOr(err, 1);
+      auto w = [](int k) { return h27_w(k); };
+      const double jw = det * (h27_pick(q1, w) * h27_pick(q2, w) * h27_pick(q3, w));
+      const double sc = det > 0.0 ? sqrt(fabs(jw)) : 0.0;
+#pragma unroll
+      for (int r = 0; r < 9; ++r) S.Gq[l * 9 + r] = sc * G[r / 3][r % 3];
+      S.Jw[l] = jw;
+    }
+    __syncthreads();  // X is dead
+    const int node = l & 31, grp = l >> 5;
+    if (s < n && l < 96 && node < 27) {
+      auto S = slot(s);
+      int lat = kH27Lat[node], g3 = grp;
+      asm volatile("" : "+v"(lat), "+v"(g3));
+      const int i1 = lat % 3, i2 = lat / 3 % 3, i3 = lat / 9;
+      double p1[3], d1[3], p3 = 0.0, d3 = 0.0, f = 0.0;
+#pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        p1[k] = h27_pick(i1, [&](int i) { return h27_p(k, i); });
+        d1[k] = h27_pick(i1, [&](int i) { return h27_d(k, i); });
+        const double p = h27_pick(i3, [&](int i) { return h27_p(k, i); });
+        const double d = h27_pick(i3, [&](int i) { return h27_d(k, i); });
+        p3 = k == g3 ? p : p3;
+        d3 = k == g3 ? d : d3;
+      }
+#pragma unroll
+      for (int q2 = 0; q2 < 3; ++q2) {
+        const double p2 = h27_pick(i2, [&](int i) { return h27_p(q2, i); });
+        const double d2 = h27_pick(i2, [&](int i) { return h27_d(q2, i); });
+        const double pp = p2 * p3, dp = d2 * p3, pd = p2 * d3;
+#pragma unroll
+        for (int q1 = 0; q1 < 3; ++q1) {
+          const int q = q1 + 3 * q2 + 9 * grp;
+          const double *G = &S.Gq[q * 9];
+          const double e0 = d1[q1] * pp, e1 = p1[q1] * dp, e2 = p1[q1] * pd;
+          float4 h;
+          h.x = (float)(e0 * G[0] + e1 * G[3] + e2 * G[6]);
+          h.y = (float)(e0 * G[1] + e1 * G[4] + e2 * G[7]);
+          h.z = (float)(e0 * G[2] + e1 * G[5] + e2 * G[8]);
+          h.w = 1.f;
+          S.Gp[q * 27 + node] = h;
+          f += S.Jw[q] * (p1[q1] * pp);
+        }
+      }
+      S.Fz[27 * grp + node] = f;
+    }
+    __syncthreads();
+  }
+  template <typename S>
+  __device__ double load(const S &s, int a, double fz) const {
+    return fz * (s.Fz[a] + s.Fz[27 + a] + s.Fz[54 + a]);
+  }
+};
+
+// One tile of elements.  L lanes per element: coordinates and constraint flags to
+// LDS, the gradients scaled by sqrt(|JxW|) (above), then one node against BG
+// nodes per lane and BG 3 x 3 blocks written as three runs of 3 BG floats.  Both
+// triangles are computed: T_ab[i][k] and T_ba[k][i] are the same products in the
+// same order, so Ke stays symmetric to the bit.  NEG: the rule has a negative
+// weight (its sign goes to the row's side).
+//
+// Bound by the store of Ke, then by the wait of each pass's loads for the last
+// pass's stores (with the stores alone 0.53 of TET10's 0.68 ms; loads one pass
+// ahead cost the registers of more than they hid).  Before, one lane per node
+// pair wrote each triangle's 18 floats one by one and the points' lanes summed
+// the table alone.  32,320 HEX27 elements 0.62 -> 0.46 ms, 375,000 TET10 0.97 ->
+// 0.68, 38,528 HEX8 0.063 -> 0.042, 1,501,416 TET4 (elasticity_tet4) 0.71 -> 0.09.
+struct ElasticitySlot {
+  float4 *Gp;         // [q][a], over X
+  double *X, *Gq, *Jw, *Fz;
+  uint8_t *cf;        // constraint flag per element DoF, variable-major
+};
+template <int N, int NQ, int BG, bool NEG, typename GRAD>
+__device__ inline void elasticity_tile(const BProb &P, const BTile &tl, unsigned char *sm, float lam1, float lam2,
+                                       double fz, int *__restrict__ err) {
+  constexpr int DPE = 3 * N, NG = N / BG;
+  static_assert(NG * BG == N, "node groups");
+  constexpr int gpb = NQ * N * 16 < N * 24 ? N * 24 : NQ * N * 16;
+  const int L = tl.lpe, epp = kBatchBlock / L;
+  const int sub = threadIdx.x / L, l = threadIdx.x & (L - 1);
+  auto slot = [&](int s) {
+    unsigned char *S = sm + s * (slot_bytes(N, NQ) + GRAD::kExtra * 8);
+    ElasticitySlot o;
+    o.Gp = (float4 *)S;
+    o.X = (double *)S;
+    o.Gq = (double *)(S + gpb);
+    o.Jw = o.Gq + NQ * 9;
+    o.Fz = o.Jw + NQ;
+    o.cf = (uint8_t *)(o.Fz + N + GRAD::kExtra);
+    return o;
+  };
+  const ElasticitySlot me = slot(sub);
+  float4 *Gp = me.Gp;
+  uint8_t *cf = me.cf;
+  const GRAD grad(P);
+  for (int64_t eb = tl.e0; eb < tl.e1; eb += epp) {
+    const int64_t e = eb + sub;
+    const bool act = e < tl.e1;
+    if (act)
+      for (int k = l; k < DPE; k += L) {
+        const int a = k / 3, c = k - a * 3;
+        me.X[GRAD::position(a) * 3 + c] = P.xyz[(int64_t)P.conn[e * N + a] * 3 + c];
+        cf[k] = P.cons[P.edofs[e * DPE + k]];
+      }
+    __syncthreads();
+    grad(slot, (int)(tl.e1 - eb < epp ? tl.e1 - eb : epp), L, err);
+    if (act)
+      for (int a = l; a < N; a += L) P.Fe[e * N + a] = cf[2 * N + a] ? 0.0 : grad.load(me, a, fz);
+    if (act) {
+      float *K = P.Ke + e * (int64_t)(DPE * DPE);
+      for (int k = l; k < N * NG; k += L) {
+        const int a = k / NG, b0 = (k - a * NG) * BG;
+        float T[BG][9];
+#pragma unroll
+        for (int u = 0; u < BG; ++u)
+#pragma unroll
+          for (int m = 0; m < 9; ++m) T[u][m] = 0.f;
+#pragma unroll 3
+        for (int q = 0; q < NQ; ++q) {
+          float4 ha = Gp[q * N + a];
+          if (NEG) {
+            ha.x *= ha.w;
+            ha.y *= ha.w;
+            ha.z *= ha.w;
+          }
+#pragma unroll
+          for (int u = 0; u < BG; ++u) {
+            const float4 hb = Gp[q * N + b0 + u];
+            T[u][0] = fmaf(ha.x, hb.x, T[u][0]);
+            T[u][1] = fmaf(ha.x, hb.y, T[u][1]);
+            T[u][2] = fmaf(ha.x, hb.z, T[u][2]);
+            T[u][3] = fmaf(ha.y, hb.x, T[u][3]);
+            T[u][4] = fmaf(ha.y, hb.y, T[u][4]);
+            T[u][5] = fmaf(ha.y, hb.z, T[u][5]);
+            T[u][6] = fmaf(ha.z, hb.x, T[u][6]);
+            T[u][7] = fmaf(ha.z, hb.y, T[u][7]);
+            T[u][8] = fmaf(ha.z, hb.z, T[u][8]);
+          }
+        }
+        bool ca[3], cb[BG][3];
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+          ca[i] = cf[i * N + a];
+#pragma unroll
+          for (int u = 0; u < BG; ++u) cb[u][i] = cf[i * N + b0 + u];
+        }
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+          float *row = K + (3 * a + i) * DPE + 3 * b0;
+#pragma unroll
+          for (int u = 0; u < BG; ++u) {
+            const f32x3 v = elasticity_row(T[u], i, lam1, lam2, ca[i], cb[u], a == b0 + u);
+            *(f32x3 *)(row + 3 * u) = v;
+          }
+        }
+      }
+    }
+    __syncthreads();
+  }
+}
+
+__global__ __launch_bounds__(kBatchBlock, 4) void k_batch_elasticity(const BProb *__restrict__ probs,
+                                                                  const BTile *__restrict__ tiles, float lam1,
+                                                                  float lam2, double fz, int *__restrict__ err) {
+  extern __shared__ __align__(16) unsigned char sm[];
+  const BTile tl = tiles[blockIdx.x];
+  const BProb P = probs[tl.p];
+  if (P.rec)
+    elasticity_tet4(P, tl, fz, err);
+  else if (P.n == 27)
+    elasticity_tile<27, 27, 3, false, Hex27Grad>(P, tl, sm, lam1, lam2, fz, err);
+  else if (P.n == 10)
+    elasticity_tile<10, 14, 2, false, TableGrad<10, 14, false>>(P, tl, sm, lam1, lam2, fz, err);
+  else if (P.n == 8)
+    elasticity_tile<8, 8, 2, false, TableGrad<8, 8, false>>(P, tl, sm, lam1, lam2, fz, err);
+  else
+    elasticity_tile<4, 5, 2, true, TableGrad<4, 5, true>>(P, tl, sm, lam1, lam2, fz, err);
+}
+
+// ---------------------------------------------------------------------------
+// Node rows: when every element's DoFs come in blocks 3B, 3B + 1, 3B + 2 (one
+// block per node), a node's three CSR rows have the same columns, in runs of
+// three.  One wave per tile of node rows: their CSR image is built in LDS (the
+// tile's rows are contiguous there as in memory) and written once.  A sub-group
+// of W lanes takes a node row, lane b the element's node b: per element a column
+// offset (one for nine values) and three runs of three floats (or one gradient),
+// added in element order; U elements' loads are in flight at once.
+//
+// Bound by memory: Ke read once, an eighteenth of it in offsets, the values
+// written once.  The ten problems of the element figures above (3.15 GB of Ke as
+// stored before, 1.3 GB of values): 3.97 -> 1.2 ms; before, one lane per DoF
+// pair read an offset for every value and added through LDS one by one.  Half
+// the image (1,280 floats) +0.1 ms, twice +0.4 ms (fewer waves); U = 2 +0.1 ms.
+// ---------------------------------------------------------------------------
+template <int N, bool REC>
+__device__ inline void elasticity_rows(const BScat &P, const BRTile &tl, float *img, float lam1, float lam2) {
+  constexpr int DPE = 3 * N, W = N <= 4 ? 4 : N <= 8 ? 8 : N <= 16 ? 16 : 32, G = 64 / W, U = 4;
+  const int lane = threadIdx.x, sg = lane / W, b = lane & (W - 1);
+  const int32_t v0 = P.rp[3 * tl.r0], v1 = P.rp[3 * tl.r1];
+  const int sh = v0 & 3;  // the image starts at a 16-byte boundary of vals
+  for (int k = 4 * lane; k < sh + v1 - v0; k += 256) *(float4 *)(img + k) = make_float4(0.f, 0.f, 0.f, 0.f);
+  for (int32_t rb = tl.r0; rb < tl.r1; rb += G) {
+    const int32_t A = rb + sg;
+    int32_t at = 0, len = 0, k0 = 0, cnt = 0;
+    if (A < tl.r1) {
+      at = P.rp[3 * A];
+      len = P.rp[3 * A + 1] - at;
+      at += sh - v0;
+      k0 = P.inc_ptr[3 * A];
+      cnt = P.inc_ptr[3 * A + 1] - k0;
+    }
+    int mx = cnt;
+#pragma unroll
+    for (int o = W; o < 64; o <<= 1) mx = max(mx, __shfl_xor(mx, o, 64));
+    double f = 0.0;
+    for (int c0 = 0; c0 < mx; c0 += U) {
+      int32_t ei[U];
+      uint32_t o[U];
+      f32x3 kv[U][3];
+      float4 ha[U], hb[U];
+      double fe[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) ei[u] = c0 + u < cnt ? P.inc[k0 + c0 + u] : -1;
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (ei[u] >= 0 && b < N) {
+          const int32_t e = ei[u] / DPE, a = ei[u] - e * DPE;
+          o[u] = P.off[(int64_t)ei[u] * DPE + b];
+          fe[u] = P.Fe[(int64_t)e * N + a];
+          if (REC) {
+            ha[u] = P.rec[(int64_t)e * N + a];
+            hb[u] = P.rec[(int64_t)e * N + b];
+          } else {
+            const float *K = P.Ke + ((int64_t)e * DPE + 3 * a) * DPE + 3 * b;
+#pragma unroll
+            for (int i = 0; i < 3; ++i) kv[u][i] = *(const f32x3 *)(K + i * DPE);
+          }
+        }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        if (ei[u] >= 0 && b < N) {
+          if (REC) {
+            const int32_t a = ei[u] % DPE;
+            const float T[9] = {ha[u].x * hb[u].x, ha[u].x * hb[u].y, ha[u].x * hb[u].z,
+                                ha[u].y * hb[u].x, ha[u].y * hb[u].y, ha[u].y * hb[u].z,
+                                ha[u].z * hb[u].x, ha[u].z * hb[u].y, ha[u].z * hb[u].z};
+            const uint32_t ba = __float_as_uint(ha[u].w), bb = __float_as_uint(hb[u].w);
+            const bool cb[3] = {(bb & 1u) != 0, (bb & 2u) != 0, (bb & 4u) != 0};
+#pragma unroll
+            for (int i = 0; i < 3; ++i) kv[u][i] = elasticity_row(T, i, lam1, lam2, (ba >> i & 1u) != 0, cb, a == b);
+          }
+          float *dst = img + at + o[u];
+#pragma unroll
+          for (int i = 0; i < 3; ++i) {
+            f32x3 *d = (f32x3 *)(dst + i * len);
+            *d = *d + kv[u][i];
+          }
+          f += fe[u];
+        }
+        // the next element's lanes read what these wrote: LDS keeps a wave's order
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+      }
+    }
+    if (A < tl.r1 && b < 3) P.rhs[3 * (int64_t)A + b] = b == 2 ? f : 0.0;
+  }
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  float *out = P.vals + (v0 - sh);
+  for (int k = 4 * lane; k < sh + v1 - v0; k += 256) {
+    const float4 v = *(const float4 *)(img + k);
+    if (k >= sh && k + 4 <= sh + v1 - v0) {
+      *(float4 *)(out + k) = v;
+    } else {
+      const float t[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        if (k + u >= sh && k + u < sh + v1 - v0) out[k + u] = t[u];
+    }
+  }
+}
+
+// Workgroups go round-robin over the XCDs: runs of kRunTiles consecutive tiles
+// stay on one XCD, whose L2 then holds the element data its neighbours share.
+constexpr int kRunTiles = 32;
+__global__ __launch_bounds__(64) void k_batch_rows(const BScat *__restrict__ probs, const BRTile *__restrict__ tiles,
+                                                   float lam1, float lam2) {
+  extern __shared__ __align__(16) unsigned char scsm[];
+  constexpr unsigned span = NXCD * kRunTiles;
+  const unsigned base = blockIdx.x / span * span, in = blockIdx.x - base;
+  const unsigned t = base + span <= gridDim.x ? base + in % NXCD * kRunTiles + in / NXCD : blockIdx.x;
+  const BRTile tl = tiles[t];
+  const BScat P = probs[tl.p];
+  float *img = (float *)scsm;
+  if (P.rec)
+    elasticity_rows<4, true>(P, tl, img, lam1, lam2);
+  else if (P.dpe == 81)
+    elasticity_rows<27, false>(P, tl, img, lam1, lam2);
+  else if (P.dpe == 30)
+    elasticity_rows<10, false>(P, tl, img, lam1, lam2);
+  else if (P.dpe == 24)
+    elasticity_rows<8, false>(P, tl, img, lam1, lam2);
+}
+
+// General row gather, for DoFs that do not come in node blocks
+// (SparseMatrix::add_matrix / NumericVector::add_vector for every element): each CSR row is summed by a
 // sub-group of W lanes (W >= the element's DoF count up to 64; 64/W rows per
 // wave) in an LDS accumulator, contributions added in element order, the row
 // written once.  A row's incidences are taken in chunks: the chunk's element
@@ -226,13 +603,13 @@ __global__ __launch_bounds__(64, LMH_BATCH_SCAT_WAVES) void k_batch_scatter(cons
   for (int t = blockIdx.x; t < ntiles; t += gridDim.x) {
     const BRTile tl = tiles[t];
     const BScat P = probs[tl.p];
-    const int dpe = P.dpe, W = P.w, G = 64 / W, stride = P.stride;
+    const int dpe = P.dpe, n = dpe / 3, W = P.w, G = 64 / W, stride = P.stride;
     const int sg = lane / W, l = lane - sg * W;
-    // per sub-group: acc[stride] floats | element ids [kScChunk] | Fe [kScChunk]
-    unsigned char *base = scsm + (size_t)sg * (stride * 4 + kScChunk * 12);
+    // per sub-group: acc[stride] floats | Fe [kScChunk] | element rows [kScChunk], variable- and node-major
+    unsigned char *base = scsm + (size_t)sg * (stride * 4 + kScChunk * 16);
     float *acc = (float *)base;
     double *febuf = (double *)(base + stride * 4);
-    int32_t *incbuf = (int32_t *)(base + stride * 4 + kScChunk * 8);
+    int32_t *incbuf = (int32_t *)(base + stride * 4 + kScChunk * 8), *kbuf = incbuf + kScChunk;
     const int ch = min(min((kScR * W) / dpe, W), kScChunk);  // incidences per chunk
     for (int32_t rb = tl.r0; rb < tl.r1; rb += G) {
       const int32_t r = rb + sg;
@@ -253,8 +630,10 @@ __global__ __launch_bounds__(64, LMH_BATCH_SCAT_WAVES) void k_batch_scatter(cons
         __builtin_amdgcn_wave_barrier();
         if (l < nch) {
           const int32_t ei = P.inc[k0 + c0 + l];
+          const int32_t e = ei / dpe, i = ei - e * dpe, c = i / n, a = i - c * n;
           incbuf[l] = ei;
-          febuf[l] = P.Fe[ei];
+          kbuf[l] = e * dpe + 3 * a + c;
+          febuf[l] = c == 2 ? P.Fe[(int64_t)e * n + a] : 0.0;
         }
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
@@ -268,9 +647,9 @@ __global__ __launch_bounds__(64, LMH_BATCH_SCAT_WAVES) void k_batch_scatter(cons
           oq[q] = 0;
           vq[q] = 0.f;
           if (kk < nch) {
-            const int64_t at = (int64_t)incbuf[kk] * dpe + (tq - kk * dpe);
-            oq[q] = P.off[at];
-            vq[q] = P.Ke[at];
+            const int j = tq - kk * dpe, c = j / n;
+            oq[q] = P.off[(int64_t)incbuf[kk] * dpe + j];
+            vq[q] = P.Ke[(int64_t)kbuf[kk] * dpe + 3 * (j - c * n) + c];
           }
         }
 #pragma unroll
@@ -312,15 +691,17 @@ struct lmh_batch {
   std::vector<int> slot;  // type slot per problem
   BProb *dprob = nullptr;
   BScat *dscat = nullptr;
-  BRTile *drt = nullptr;
-  int nrt = 0;
+  BRTile *drt = nullptr, *dnt = nullptr;  // row tiles of the general kernel and tiles of node rows
+  int nrt = 0, nnt = 0;
+  int *dsplit = nullptr;      // problems whose DoFs are not in node blocks
+  std::vector<float4 *> rec;  // TET4 gradients, per problem
   BTile *dtile = nullptr;
   int ntile = 0, tile_cap = 0;
   int lpe[4] = {16, 128, 16, 32};   // lanes per element
   int ppt[4] = {4, 4, 4, 4};        // passes (groups of concurrent elements) per tile
   int max_row = 0;
-  size_t scat_lds = 0;
-  int grid_elem = 0, grid_scat = 0;
+  size_t scat_lds = 0, rows_lds = 0;
+  int grid_scat = 0;
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
   double gE = 0, gnu = 0, gfz = 0;
@@ -332,7 +713,7 @@ namespace lmh {
 // a multiple of 4) plus a chunk's element ids and Fe values; the launch takes
 // the largest need over the problems
 static int scatter_stride(int max_row) { return (max_row + 3) & ~3; }
-static size_t scatter_lds(const BScat &s) { return (size_t)(64 / s.w) * ((size_t)s.stride * 4 + kScChunk * 12); }
+static size_t scatter_lds(const BScat &s) { return (size_t)(64 / s.w) * ((size_t)s.stride * 4 + kScChunk * 16); }
 
 static bool config_fits(int n, int nq, int L) {
   return L >= 16 && L <= kBatchBlock && (kBatchBlock / L) * slot_bytes(n, nq) <= kBatchLds;
@@ -372,6 +753,39 @@ static void lame(double E, double nu, float &l1, float &l2) {
   l2 = (float)(E / (2. * (1. + nu)));
 }
 
+static void launch_elements(const lmh_batch *b, float l1, float l2, double fz) {
+  hipLaunchKernelGGL(k_batch_elasticity, dim3(b->ntile), dim3(kBatchBlock), kBatchLds, b->ctx->stream,
+                     (const BProb *)b->dprob, (const BTile *)b->dtile, l1, l2, fz, b->ctx->d_flags);
+}
+
+// flags the problems whose element DoFs do not come in node blocks
+__global__ void k_node_blocks(const int32_t *__restrict__ edofs, int64_t n_elem, int n, int *__restrict__ flag) {
+  for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < n_elem * n; t += (int64_t)gridDim.x * blockDim.x) {
+    const int64_t e = t / n, at = e * 3 * n + (t - e * n);
+    const int32_t d = edofs[at];
+    if (d % 3 != 0 || edofs[at + n] != d + 1 || edofs[at + 2 * n] != d + 2) *flag = 1;
+  }
+}
+
+// Tiles of consecutive node rows whose CSR image stays within kImage floats (one
+// longer row has a tile to itself, up to kImageMax).  8 KB an image: twenty waves
+// fit a CU and a tile's loads, adds and stores overlap with the others'.
+constexpr int kImage = 2048, kImageMax = 12288, kTileNodes = 64;
+static bool node_tiles(int p, const std::vector<int32_t> &rp, std::vector<BRTile> &out, int &image) {
+  const int64_t nodes = (int64_t)(rp.size() - 1) / 3;
+  for (int64_t A = 0; A < nodes; ++A) {
+    const int32_t *r = &rp[3 * A], len = r[1] - r[0];
+    if (r[2] - r[1] != len || r[3] - r[2] != len || len % 3 || 3 * len > kImageMax) return false;
+  }
+  for (int64_t r0 = 0, r1; r0 < nodes; r0 = r1) {
+    r1 = r0 + 1;
+    while (r1 < nodes && r1 - r0 < kTileNodes && rp[3 * r1 + 3] - rp[3 * r0] <= kImage) ++r1;
+    image = std::max(image, rp[3 * r1] - rp[3 * r0]);
+    out.push_back(BRTile{p, (int32_t)r0, (int32_t)r1, 0});
+  }
+  return true;
+}
+
 static int build_graph(lmh_batch *b, double E, double nu, double fz) {
   lmh_context *ctx = b->ctx;
   if (b->exec) LMH_HIP(hipGraphExecDestroy(b->exec));
@@ -383,9 +797,10 @@ static int build_graph(lmh_batch *b, double E, double nu, double fz) {
   LMH_HIP(hipStreamSynchronize(ctx->stream));
   LMH_HIP(hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
   hipLaunchKernelGGL(k_batch_clear, dim3(1), dim3(64), 0, ctx->stream, ctx->d_flags);
-  if (b->ntile > 0)
-    hipLaunchKernelGGL(k_batch_elasticity, dim3(b->grid_elem), dim3(kBatchBlock), kBatchLds, ctx->stream,
-                       (const BProb *)b->dprob, (const BTile *)b->dtile, b->ntile, l1, l2, fz, ctx->d_flags);
+  if (b->ntile > 0) launch_elements(b, l1, l2, fz);
+  if (b->nnt > 0)
+    hipLaunchKernelGGL(k_batch_rows, dim3(b->nnt), dim3(64), b->rows_lds, ctx->stream, (const BScat *)b->dscat,
+                       (const BRTile *)b->dnt, l1, l2);
   if (b->nrt > 0)
     hipLaunchKernelGGL(k_batch_scatter, dim3(b->grid_scat), dim3(64), b->scat_lds, ctx->stream,
                        (const BScat *)b->dscat, (const BRTile *)b->drt, b->nrt);
@@ -406,6 +821,11 @@ int lmh_batch_destroy(lmh_batch *b);
 
 static int batch_setup(lmh_batch *b, lmh_context *ctx, int n_prob, const lmh_dofmap *const *dms) {
   LMH_HIP(hipSetDevice(ctx->device));
+  std::vector<std::vector<int32_t>> rp(n_prob);
+  int *split_d = nullptr;  // DoFs not in node blocks, per problem
+  LMH_HIP(hipMalloc((void **)&split_d, sizeof(int) * n_prob));
+  b->dsplit = split_d;
+  LMH_HIP(hipMemsetAsync(split_d, 0, sizeof(int) * n_prob, ctx->stream));
   for (int p = 0; p < n_prob; ++p) {
     const lmh_dofmap *dm = dms[p];
     LMH_CHECK(dm && dm->ctx == ctx, LMH_ERR_INVALID, "problem %d: null DoF map or other context", p);
@@ -419,14 +839,13 @@ static int batch_setup(lmh_batch *b, lmh_context *ctx, int n_prob, const lmh_dof
     const FETable *t = nullptr;
     LMH_TRY(fe_table(ctx, dm->mesh->type, arg, &t));
     lmh_matrix *A = nullptr;
-    LMH_TRY(matrix_create_impl(ctx, dm, false, false, &A));
+    LMH_TRY(matrix_create_impl(ctx, dm, false, false, &A, &rp[p]));
     b->mats.push_back(A);
     b->dms.push_back(dm);
     b->slot.push_back(s);
     b->max_row = std::max(b->max_row, A->max_row);
     const int64_t ne = dm->mesh->n_elem;
     const int dpe = dm->dpe;
-    LMH_HIP(hipMalloc((void **)&A->Ke32, sizeof(float) * std::max<int64_t>(1, ne * dpe * dpe)));
     LMH_HIP(hipMalloc((void **)&A->Fe, sizeof(double) * std::max<int64_t>(1, ne * dpe)));
     LMH_HIP(hipMalloc((void **)&A->vals32, sizeof(float) * (A->nnz + LMH_PAD)));
     LMH_HIP(hipMemsetAsync(A->vals32, 0, sizeof(float) * (A->nnz + LMH_PAD), ctx->stream));
@@ -440,15 +859,45 @@ static int batch_setup(lmh_batch *b, lmh_context *ctx, int n_prob, const lmh_dof
     bp.edofs = dm->edofs;
     bp.cons = dm->cons;
     bp.fe = t->d_data;
-    bp.Ke = A->Ke32;
+    bp.Ke = nullptr;
+    bp.rec = nullptr;
     bp.Fe = A->Fe;
     bp.n_elem = ne;
     bp.n = t->n;
     bp.nq = t->nq;
+    const int rule[4] = {8, 27, 5, 14};  // the point counts the element kernels are built for
+    LMH_CHECK(bp.nq == rule[s], LMH_ERR_UNSUPPORTED, "element type %d: %d quadrature points", dm->mesh->type, bp.nq);
     LMH_CHECK(config_fits(bp.n, bp.nq, kBatchBlock), LMH_ERR_UNSUPPORTED, "element type %d does not fit in LDS",
               dm->mesh->type);
     b->hprob.push_back(bp);
+    if (ne)
+      hipLaunchKernelGGL(k_node_blocks, dim3(grid_for(ne * t->n, 256, 4096)), dim3(256), 0, ctx->stream, dm->edofs, ne,
+                         t->n, split_d + p);
   }
+  LMH_TRY(check_launch("k_node_blocks"));
+  std::vector<int> split(n_prob);
+  LMH_HIP(hipMemcpyAsync(split.data(), split_d, sizeof(int) * n_prob, hipMemcpyDeviceToHost, ctx->stream));
+  LMH_HIP(hipStreamSynchronize(ctx->stream));
+  // row tiles; what the element kernel writes for them
+  std::vector<BRTile> rt, nt;
+  int image = 0;
+  for (int p = 0; p < n_prob; ++p) {
+    lmh_matrix *A = b->mats[p];
+    BProb &bp = b->hprob[p];
+    const bool blocks = !split[p] && A->rows % 3 == 0 && node_tiles(p, rp[p], nt, image);
+    if (!blocks)
+      for (int64_t r = 0; r < A->rows; r += kRowsPerTile)
+        rt.push_back(BRTile{p, (int32_t)r, (int32_t)std::min<int64_t>(A->rows, r + kRowsPerTile), 0});
+    if (blocks && bp.n == 4) {
+      LMH_HIP(hipMalloc((void **)&bp.rec, sizeof(float4) * std::max<int64_t>(1, bp.n_elem * 4)));
+      b->rec.push_back(bp.rec);
+    } else {
+      const int64_t dpe = 3 * bp.n;
+      LMH_HIP(hipMalloc((void **)&A->Ke32, sizeof(float) * std::max<int64_t>(1, bp.n_elem * dpe * dpe)));
+      bp.Ke = A->Ke32;
+    }
+  }
+  b->rows_lds = sizeof(float) * (size_t)((image + 11) & ~3);
   // default tile shapes: the smallest lanes-per-element that fits the LDS budget
   for (int p = 0; p < n_prob; ++p) {
     const int s = b->slot[p];
@@ -459,16 +908,13 @@ static int batch_setup(lmh_batch *b, lmh_context *ctx, int n_prob, const lmh_dof
   LMH_HIP(hipMalloc((void **)&b->dprob, sizeof(BProb) * n_prob));
   LMH_HIP(hipMemcpy(b->dprob, b->hprob.data(), sizeof(BProb) * n_prob, hipMemcpyHostToDevice));
   std::vector<BScat> sc(n_prob);
-  std::vector<BRTile> rt;
   for (int p = 0; p < n_prob; ++p) {
     lmh_matrix *A = b->mats[p];
     const int dpe = b->dms[p]->dpe;
-    sc[p] = BScat{b->dms[p]->inc_ptr, b->dms[p]->inc, A->rp, A->off, A->Ke32, A->Fe, A->vals32, b->rhs[p],
-                  A->rows, dpe, dpe <= 16 ? 16 : dpe <= 32 ? 32 : 64, scatter_stride(A->max_row), 0};
-    b->scat_lds = std::max(b->scat_lds, scatter_lds(sc[p]));
-    for (int64_t r = 0; r < A->rows; r += kRowsPerTile)
-      rt.push_back(BRTile{p, (int32_t)r, (int32_t)std::min<int64_t>(A->rows, r + kRowsPerTile), 0});
+    sc[p] = BScat{b->dms[p]->inc_ptr, b->dms[p]->inc, A->rp, A->off, A->Ke32, b->hprob[p].rec, A->Fe, A->vals32,
+                  b->rhs[p], A->rows, dpe, dpe <= 16 ? 16 : dpe <= 32 ? 32 : 64, scatter_stride(A->max_row), 0};
   }
+  for (const BRTile &t : rt) b->scat_lds = std::max(b->scat_lds, scatter_lds(sc[t.p]));
   // interleave row tiles of different problems so each part of the grid sees a mix
   std::vector<BRTile> rt2;
   rt2.reserve(rt.size());
@@ -492,13 +938,13 @@ static int batch_setup(lmh_batch *b, lmh_context *ctx, int n_prob, const lmh_dof
   LMH_HIP(hipMemcpy(b->dscat, sc.data(), sizeof(BScat) * n_prob, hipMemcpyHostToDevice));
   LMH_HIP(hipMalloc((void **)&b->drt, sizeof(BRTile) * std::max(1, b->nrt)));
   if (b->nrt) LMH_HIP(hipMemcpy(b->drt, rt2.data(), sizeof(BRTile) * b->nrt, hipMemcpyHostToDevice));
-  int occ = 0;
-  LMH_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, k_batch_elasticity, kBatchBlock, kBatchLds));
-  b->grid_elem = ctx->cu_count * std::max(1, occ);
+  b->nnt = (int)nt.size();
+  LMH_HIP(hipMalloc((void **)&b->dnt, sizeof(BRTile) * std::max(1, b->nnt)));
+  if (b->nnt) LMH_HIP(hipMemcpy(b->dnt, nt.data(), sizeof(BRTile) * b->nnt, hipMemcpyHostToDevice));
   // one-wave workgroups, as many per CU as can be resident at once (registers
   // and LDS): the tiles are dealt round-robin, so a second round of
   // workgroups would only wait (measured: 24 resident per CU 71 ms, 32 launched 84 ms)
-  {
+  if (b->nrt) {
     int socc = 0;
     LMH_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&socc, k_batch_scatter, 64, b->scat_lds));
     b->grid_scat = ctx->cu_count * std::max(1, std::min(socc, (int)LMH_BATCH_SCAT_PER_CU));
@@ -535,6 +981,9 @@ int lmh_batch_destroy(lmh_batch *b) {
   (void)hipFree(b->dprob);
   (void)hipFree(b->dscat);
   (void)hipFree(b->drt);
+  (void)hipFree(b->dnt);
+  (void)hipFree(b->dsplit);
+  for (float4 *r : b->rec) (void)hipFree(r);
   (void)hipFree(b->dtile);
   delete b;
   return LMH_OK;
@@ -629,8 +1078,7 @@ int lmh_batch_autotune(lmh_batch *b, double E, double nu, double fz, int reps, d
         float ms_min = 1e30f;
         for (int r = 0; r <= reps; ++r) {
           LMH_HIP(hipEventRecord(e0, ctx->stream));
-          hipLaunchKernelGGL(k_batch_elasticity, dim3(b->grid_elem), dim3(kBatchBlock), kBatchLds, ctx->stream,
-                             (const BProb *)b->dprob, (const BTile *)b->dtile, b->ntile, l1, l2, fz, ctx->d_flags);
+          if (b->ntile > 0) launch_elements(b, l1, l2, fz);
           LMH_HIP(hipEventRecord(e1, ctx->stream));
           LMH_HIP(hipEventSynchronize(e1));
           float ms = 0;

@@ -256,7 +256,8 @@ int build_incidence(lmh_context *ctx, const int32_t *edofs, int64_t n_elem, int 
 int fe_table(lmh_context *ctx, int type, int arg, const FETable **out);
 // CSR pattern, scatter map, (if colour) element colouring and (if fp64) zeroed
 // FP64 values for a DoF map
-int matrix_create_impl(lmh_context *ctx, const lmh_dofmap *dm, bool colour, bool fp64, lmh_matrix **out);
+int matrix_create_impl(lmh_context *ctx, const lmh_dofmap *dm, bool colour, bool fp64, lmh_matrix **out,
+                       std::vector<int32_t> *row_ptr = nullptr);
 // row tiles of a matrix's gather scatter, and the scatter on them
 int matrix_build_tiles(lmh_matrix *A, const std::vector<int32_t> &h_rp);
 template <typename T>
@@ -305,6 +306,21 @@ int thread_residual(lmh_context *ctx, const FETable *t, const lmh_mesh *m, const
 int thread_qoi(lmh_context *ctx, const FETable *t, const lmh_mesh *m, double lo, double hi, double *Q);
 int thread_adjoint(lmh_context *ctx, const FETable *t, const lmh_mesh *m, const lmh_dofmap *dm, const double *u,
                    const double *lam, double *grad);
+
+// a value moved between lanes by a DPP control word
+template <int CTRL, typename T>
+__device__ inline T dpp_move(T v) {
+  if constexpr (sizeof(T) == 4) {
+    return __builtin_bit_cast(
+        T, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
+  } else {
+    typedef int i32x2 __attribute__((ext_vector_type(2)));
+    i32x2 w = __builtin_bit_cast(i32x2, v);
+    w[0] = __builtin_amdgcn_update_dpp(0, w[0], CTRL, 0xf, 0xf, true);
+    w[1] = __builtin_amdgcn_update_dpp(0, w[1], CTRL, 0xf, 0xf, true);
+    return __builtin_bit_cast(T, w);
+  }
+}
 
 // MI355X dispatches workgroups round-robin over its 8 XCDs; remap so each XCD
 // owns one contiguous range of logical blocks (its L2 then holds the data its

@@ -221,19 +221,6 @@ __device__ inline void rowblock_spmv(const int32_t *__restrict__ rb, int64_t nrb
 // Row sums of an 8-lane group: lanes 0..3 take lane + 4, then pairs and
 // neighbours within the quad (the tree ((0+4)+(2+6))+((1+5)+(3+7))), valid in
 // the group's lane 0.  DPP moves instead of LDS permutes: no wait on LDS.
-template <int CTRL, typename T>
-__device__ inline T dpp_move(T v) {
-  if constexpr (sizeof(T) == 4) {
-    return __builtin_bit_cast(
-        T, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
-  } else {
-    typedef int i32x2 __attribute__((ext_vector_type(2)));
-    i32x2 w = __builtin_bit_cast(i32x2, v);
-    w[0] = __builtin_amdgcn_update_dpp(0, w[0], CTRL, 0xf, 0xf, true);
-    w[1] = __builtin_amdgcn_update_dpp(0, w[1], CTRL, 0xf, 0xf, true);
-    return __builtin_bit_cast(T, w);
-  }
-}
 template <typename T>
 __device__ inline T group8_sum(T s) {
   s += dpp_move<0x104>(s);  // row_shl:4

@@ -204,7 +204,8 @@ using namespace lmh;
 
 namespace lmh {
 
-int matrix_create_impl(lmh_context *ctx, const lmh_dofmap *dm, bool colour, bool fp64, lmh_matrix **out) {
+int matrix_create_impl(lmh_context *ctx, const lmh_dofmap *dm, bool colour, bool fp64, lmh_matrix **out,
+                       std::vector<int32_t> *row_ptr) {
   LMH_CHECK(ctx && dm && out, LMH_ERR_INVALID, "null argument");
   LMH_HIP(hipSetDevice(ctx->device));
   const int64_t n = dm->n_dofs, ne = dm->mesh->n_elem;
@@ -258,6 +259,7 @@ int matrix_create_impl(lmh_context *ctx, const lmh_dofmap *dm, bool colour, bool
     A->min_row = std::min<int>(A->min_row, rp[r + 1] - rp[r]);
   }
   LMH_TRY(build_row_blocks(A.get(), rp));
+  if (row_ptr) *row_ptr = rp;
   LMH_HIP(hipFree(rowlen));
   LMH_CHECK(A->max_row <= 65535, LMH_ERR_UNSUPPORTED, "row length %d exceeds 16-bit scatter offsets", A->max_row);
 
