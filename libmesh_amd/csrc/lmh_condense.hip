@@ -33,13 +33,18 @@ struct lmh_condensation {
   int32_t *cdof = nullptr;   // n_cond: condensed DoFs, ascending
   int32_t *dpos = nullptr;   // n_cond: position of K_cc in A's row c
   double *g = nullptr, *y = nullptr;  // reduced right-hand side and solution
-  bool pattern_checked = false;       // k_sc_values found no fill-in (then k_sc_values_wave is used)
-  // Position map (pattern only, built after the fill check): for reduced row r
-  // and each structurally condensed column c of its full row i (ascending),
-  // the full-row-i position of every entry of row c, -1 for condensed or
-  // absent columns.  pmoff[r] .. pmoff[r + 1] are row r's entries.
-  int64_t *pmoff = nullptr;
-  int16_t *pmap = nullptr;
+  bool pattern_checked = false;       // k_sc_values found no fill-in (refreshes then skip the check)
+  // Refresh plan (pattern only, built after the fill check).  rec[r]: start of
+  // A's row, its length | n << 16, start in lst, start of reduced row r.  Its n
+  // condensed columns, ascending, in lst: position in A's row | length of row c
+  // << 16, start of row c, position of K_cc, start of row c's slots in pmap; and
+  // c in lcol.  A slot is the place of row c's entry in reduced row r; all ones
+  // for condensed columns.  Slots have 8 or 16 bits.
+  uint4 *rec = nullptr, *lst = nullptr;
+  int32_t *lcol = nullptr;
+  void *pmap = nullptr;
+  bool wide = false;     // 16-bit slots
+  bool coupled = false;  // a condensed row has another condensed column
 };
 
 namespace lmh {
@@ -254,35 +259,61 @@ __global__ __launch_bounds__(256) void k_sc_forward(int64_t n_red, const int32_t
   }
 }
 
-// y_r = x_{rfull[r]} (TO_RED) or x_{rfull[r]} = y_r
-template <bool TO_RED>
-__global__ __launch_bounds__(256) void k_sc_map(int64_t n_red, const int32_t *__restrict__ rfull, double *__restrict__ x,
-                                                double *__restrict__ y) {
+// The same from the plan's lists: one thread per reduced row, no walk over its
+// columns.  33 x 35 x 31 Q2 elements (270,000 rows): 156 -> 33 us, two thirds of it
+// the cache line each K_ic drags in.
+__global__ __launch_bounds__(256) void k_sc_forward_list(int64_t n_red, const int32_t *__restrict__ rfull,
+                                                         const double *__restrict__ v, const uint4 *__restrict__ rec,
+                                                         const uint4 *__restrict__ lst,
+                                                         const int32_t *__restrict__ lcol,
+                                                         const double *__restrict__ b, double *__restrict__ g) {
   for (int64_t r = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; r < n_red; r += (int64_t)gridDim.x * blockDim.x) {
-    if (TO_RED)
-      y[r] = x[rfull[r]];
-    else
-      x[rfull[r]] = y[r];
+    const uint4 q = rec[r];
+    const uint32_t n = q.y >> 16;
+    double s = 0.0;
+#pragma unroll 4
+    for (uint32_t e = q.z; e < q.z + n; ++e) {
+      const uint4 l = lst[e];
+      s += v[q.x + (l.x & 0xffffu)] * (b[lcol[e]] / v[l.z]);
+    }
+    g[r] = b[rfull[r]] - s;
   }
 }
 
-// x_c = (b_c - sum_{j uncondensed} K_cj x_j) / K_cc, after the uncondensed x_j
-// are in place.  Columns of other condensed DoFs are skipped: k_sc_check
-// admits them only as exact zeros, and those x_j are being written by other
-// threads of this launch (their old contents may even be NaN).
-__global__ __launch_bounds__(256) void k_sc_backward(int64_t n_cond, const int32_t *__restrict__ cdof,
+// y_r = x_{rfull[r]}
+__global__ __launch_bounds__(256) void k_sc_map(int64_t n_red, const int32_t *__restrict__ rfull,
+                                                const double *__restrict__ x, double *__restrict__ y) {
+  for (int64_t r = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; r < n_red; r += (int64_t)gridDim.x * blockDim.x)
+    y[r] = x[rfull[r]];
+}
+
+// x_{rfull[r]} = y_r, and x_c = (b_c - sum_{j uncondensed} K_cj x_j) / K_cc with
+// x_j read from y, so both go in one launch: the first nbc workgroups take the
+// condensed DoFs, 32 lanes to a row (coalesced), the others copy (33 x 35 x 31 Q2: two launches 24
+// us, now 14).  Columns of
+// other condensed DoFs are skipped: k_sc_check admits them only as exact zeros.
+__global__ __launch_bounds__(256) void k_sc_backward(int nbc, int64_t n_cond, const int32_t *__restrict__ cdof,
                                                      const int32_t *__restrict__ rp, const int32_t *__restrict__ ci,
                                                      const double *__restrict__ v, const int32_t *__restrict__ ridx,
                                                      const int32_t *__restrict__ dpos, const double *__restrict__ b,
-                                                     double *__restrict__ x) {
-  for (int64_t q = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; q < n_cond; q += (int64_t)gridDim.x * blockDim.x) {
-    const int32_t c = cdof[q], d = dpos[q];
-    double s = b[c];
-    for (int32_t k = rp[c]; k < rp[c + 1]; ++k) {
-      const int32_t j = ci[k];
-      if (ridx[j] >= 0) s -= v[k] * x[j];
+                                                     int64_t n_red, const int32_t *__restrict__ rfull,
+                                                     const double *__restrict__ y, double *__restrict__ x) {
+  if ((int)blockIdx.x >= nbc) {
+    const int64_t step = (int64_t)(gridDim.x - nbc) * 256;
+    for (int64_t r = (int64_t)(blockIdx.x - nbc) * 256 + threadIdx.x; r < n_red; r += step) x[rfull[r]] = y[r];
+    return;
+  }
+  const int sl = threadIdx.x & 31;
+  for (int64_t q = blockIdx.x * (int64_t)8 + (threadIdx.x >> 5); q < n_cond; q += (int64_t)nbc * 8) {
+    const int32_t c = cdof[q], k1 = rp[c + 1];
+    double s = 0.0;
+    for (int32_t k = rp[c] + sl; k < k1; k += 32) {
+      const int32_t j = ridx[ci[k]];
+      if (j >= 0) s += v[k] * y[j];
     }
-    x[c] = s / v[d];
+#pragma unroll
+    for (int o = 16; o > 0; o >>= 1) s += __shfl_xor(s, o, 32);
+    if (sl == 0) x[c] = (b[c] - s) / v[dpos[q]];
   }
 }
 
@@ -297,41 +328,71 @@ __device__ inline int32_t sc_wave_scan(int32_t x) {
   return x;
 }
 
-// Position-map sizes: per reduced row, the entries of all rows c of its
-// structurally condensed columns.  One wavefront per reduced row.
-__global__ __launch_bounds__(256) void k_sc_map_count(int64_t n_red, const int32_t *__restrict__ rfull,
-                                                      const int32_t *__restrict__ rp, const int32_t *__restrict__ ci,
-                                                      const int32_t *__restrict__ ridx, int64_t *__restrict__ cnt) {
+// Plan sizes: per reduced row its structurally condensed columns and the entries
+// of their rows.  One wavefront per reduced row.
+__global__ __launch_bounds__(256) void k_sc_plan_count(int64_t n_red, const int32_t *__restrict__ rfull,
+                                                       const int32_t *__restrict__ rp, const int32_t *__restrict__ ci,
+                                                       const int32_t *__restrict__ ridx, int2 *__restrict__ cnt) {
   const int lane = threadIdx.x & 63;
   const int64_t nw = (int64_t)gridDim.x * (blockDim.x >> 6);
   for (int64_t r = blockIdx.x * (int64_t)(blockDim.x >> 6) + (threadIdx.x >> 6); r < n_red; r += nw) {
     const int32_t i = rfull[r], k1 = rp[i + 1];
-    int64_t tot = 0;
+    int n = 0, tot = 0;
     for (int32_t cb = rp[i]; cb < k1; cb += 64) {
       const int32_t kc = cb + lane;
       const int32_t cc = kc < k1 ? ci[kc] : 0;
-      const int32_t lenc = kc < k1 && ridx[cc] < 0 ? rp[cc + 1] - rp[cc] : 0;
-      tot += __shfl(sc_wave_scan(lenc), 63);
+      const bool isc = kc < k1 && ridx[cc] < 0;
+      n += __popcll(__ballot(isc));
+      tot += __shfl(sc_wave_scan(isc ? rp[cc + 1] - rp[cc] : 0), 63);
     }
-    if (lane == 0) cnt[r] = tot;
+    if (lane == 0) cnt[r] = make_int2(n, tot);
   }
 }
 
-// Position-map entries (same walk as k_sc_values_lds, positions instead of
-// updates).  LDS: max_row int32 per wavefront.
-__global__ __launch_bounds__(256) void k_sc_map_fill(int64_t n_red, const int32_t *__restrict__ rfull,
-                                                     const int32_t *__restrict__ rp, const int32_t *__restrict__ ci,
-                                                     const int32_t *__restrict__ ridx, const int64_t *__restrict__ pmoff,
-                                                     int16_t *__restrict__ pmap, int max_row) {
+// flag: a condensed row has a condensed column besides its own
+__global__ __launch_bounds__(256) void k_sc_coupled(int64_t n_cond, const int32_t *__restrict__ cdof,
+                                                    const int32_t *__restrict__ rp, const int32_t *__restrict__ ci,
+                                                    const int32_t *__restrict__ ridx, int *__restrict__ flag) {
+  for (int64_t q = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; q < n_cond; q += (int64_t)gridDim.x * blockDim.x) {
+    const int32_t c = cdof[q];
+    for (int32_t k = rp[c]; k < rp[c + 1]; ++k)
+      if (ci[k] != c && ridx[ci[k]] < 0) *flag = 1;
+  }
+}
+
+// Plan entries (the walk of k_sc_values_lds, places instead of updates).  LDS: 2
+// max_row int32 per wavefront: the row's columns and their places in the reduced
+// row.
+template <typename MT>
+__global__ __launch_bounds__(256) void k_sc_plan_fill(int64_t n_red, const int32_t *__restrict__ rfull,
+                                                      const int32_t *__restrict__ rp, const int32_t *__restrict__ ci,
+                                                      const int32_t *__restrict__ ridx,
+                                                      const int32_t *__restrict__ dpos, const int32_t *__restrict__ srp,
+                                                      const int2 *__restrict__ start, uint4 *__restrict__ rec,
+                                                      uint4 *__restrict__ lst, int32_t *__restrict__ lcol,
+                                                      MT *__restrict__ pmap, int max_row) {
   extern __shared__ int32_t sc_cols[];
   const int lane = threadIdx.x & 63;
-  int32_t *cols = sc_cols + (size_t)(threadIdx.x >> 6) * max_row;
+  int32_t *cols = sc_cols + (size_t)(threadIdx.x >> 6) * 2 * max_row, *place = cols + max_row;
   const int64_t nw = (int64_t)gridDim.x * (blockDim.x >> 6);
   for (int64_t r = blockIdx.x * (int64_t)(blockDim.x >> 6) + (threadIdx.x >> 6); r < n_red; r += nw) {
     const int32_t i = rfull[r], k0 = rp[i], k1 = rp[i + 1], len = k1 - k0;
-    for (int32_t t = lane; t < len; t += 64) cols[t] = ci[k0 + t];
+    int32_t kept = 0;
+    for (int32_t tb = 0; tb < len; tb += 64) {
+      const int32_t t = tb + lane, j = t < len ? ci[k0 + t] : 0;
+      const bool keep = t < len && ridx[j] >= 0;
+      const uint64_t km = __ballot(keep);
+      if (t < len) {
+        cols[t] = j;
+        place[t] = keep ? kept + __popcll(km & ((1ull << lane) - 1)) : -1;
+      }
+      kept += __popcll(km);
+    }
     sc_wave_lds_sync();
-    int64_t base = pmoff[r];
+    uint32_t base = (uint32_t)start[r].y;
+    int32_t e = start[r].x;
+    if (lane == 0)
+      rec[r] = make_uint4((uint32_t)k0, (uint32_t)len | (uint32_t)(len - kept) << 16, (uint32_t)e, (uint32_t)srp[r]);
     for (int32_t cb = k0; cb < k1; cb += 64) {
       const int32_t kc = cb + lane;
       const int32_t cc = kc < k1 ? ci[kc] : 0;
@@ -339,6 +400,12 @@ __global__ __launch_bounds__(256) void k_sc_map_fill(int64_t n_red, const int32_
       const int32_t lenc = isc ? rp[cc + 1] - rp[cc] : 0;
       const int32_t inc = sc_wave_scan(lenc), moff = inc - lenc;
       uint64_t m = __ballot(isc);
+      if (isc) {
+        const int32_t at = e + __popcll(m & ((1ull << lane) - 1));
+        lst[at] = make_uint4((uint32_t)(kc - k0) | (uint32_t)lenc << 16, rp[cc], dpos[-1 - ridx[cc]], base + moff);
+        lcol[at] = cc;
+      }
+      e += __popcll(m);
       while (m) {
         const int b = __builtin_ctzll(m);
         m &= m - 1;
@@ -355,9 +422,9 @@ __global__ __launch_bounds__(256) void k_sc_map_fill(int64_t n_red, const int32_
               else
                 hi = mid;
             }
-            if (lo < len && cols[lo] == j) pos = lo;
+            if (lo < len && cols[lo] == j) pos = place[lo];
           }
-          pmap[base + mo + (mm - rp[c])] = (int16_t)pos;
+          pmap[base + mo + (mm - rp[c])] = (MT)pos;
         }
       }
       base += __shfl(inc, 63);
@@ -366,120 +433,198 @@ __global__ __launch_bounds__(256) void k_sc_map_fill(int64_t n_red, const int32_
   }
 }
 
-// Inclusive prefix sum over the 16 lanes of a lane group.
-__device__ inline int32_t sc_group_scan(int32_t x) {
-  const int sl = threadIdx.x & 15;
+// Reduced values from the plan: the same subtractions in the same order as
+// k_sc_values_lds (condensed columns of row i ascending, those with a zero K_ic
+// skipped, f_c = K_ic / K_cc), so the values are bit-identical.  One workgroup per
+// row block of the reduced matrix, whose values are built in LDS and written once;
+// 32 lanes take a row: lane u holds the row's u-th condensed column, the row's
+// values land at their reduced places (a count of the condensed positions before
+// them), then the columns' rows are subtracted in turn.  The grid's threads also
+// check the pivots (n_cond = 0: k_sc_check ran instead).
+// Bound by memory: the matrix read and the reduced values written once, a byte of
+// slot per condensed coupling's entry; short of that by the chain of loads, so a
+// row's record and list are read one and two rows ahead and its values, pivots and
+// the first kScU columns' rows and slots are in flight at once.  33 x 35 x 31 Q2
+// elements: 343 us (16 lanes to a row, columns tested again, 16-bit map) -> 178
+// without the reading ahead -> 116, 2.9 TB/s of the 340 MB it cannot do without.
+constexpr int kScU = 4, kScC = 4, kScRow = LMH_RB_CAP;
+template <typename MT>
+__global__ __launch_bounds__(256) void k_sc_values_plan(int nrb, const int32_t *__restrict__ rb,
+                                                        const double *__restrict__ v, const uint4 *__restrict__ rec,
+                                                        const uint4 *__restrict__ lst, const MT *__restrict__ pmap,
+                                                        const int32_t *__restrict__ srp, double *__restrict__ sv,
+                                                        int64_t n_cond, const int32_t *__restrict__ dpos,
+                                                        int *__restrict__ flags) {
+  __shared__ __align__(16) double img[kScRow + 2];
+  const int sl = threadIdx.x & 31, sg = threadIdx.x >> 5;
+  for (int64_t q = blockIdx.x * (int64_t)256 + threadIdx.x; q < n_cond; q += (int64_t)gridDim.x * 256)
+    if (v[dpos[q]] == 0.0) atomicOr(flags, SC_ZEROPIVOT);
+  const int blk = logical_block();
+  if (blk >= nrb) return;
+  const int32_t r0 = rb[blk], r1 = rb[blk + 1], s0 = srp[r0], s1 = srp[r1], sh = s0 & 1;
+  auto record = [&](int32_t r) { return r + sg < r1 ? rec[r + sg] : make_uint4(0, 0, 0, (uint32_t)s0); };
+  auto entry = [&](const uint4 &q) {
+    return sl < (int)(q.y >> 16) ? lst[q.z + sl] : make_uint4(0xffffu, 0, 0, 0);
+  };
+  uint4 q0 = record(r0), q1 = record(r0 + 8), l0 = entry(q0);
+  for (int32_t rr = r0; rr < r1; rr += 8) {
+    const uint4 q = q0, l = l0;
+    q0 = q1;
+    q1 = record(rr + 16);
+    l0 = entry(q0);
+    const int32_t len = q.y & 0xffffu, n = q.y >> 16, pos = l.x & 0xffffu, lenc = l.x >> 16;
+    const double *row = v + q.x;
+    double *acc = img + sh + (int32_t)(q.w - (uint32_t)s0);
+    const int nmax = max(n, __shfl_xor(n, 32)), lmax = max(len, __shfl_xor(len, 32));
+    const double kic = sl < n ? row[pos] : 0.0, kcc = sl < n ? v[l.z] : 1.0;
+    double xr[kScC];
 #pragma unroll
-  for (int d = 1; d < 16; d <<= 1) {
-    const int32_t y = __shfl_up(x, d, 16);
-    if (sl >= d) x += y;
-  }
-  return x;
-}
-
-// Reduced values through the position map: the same subtractions in the same
-// order as k_sc_values_lds (condensed columns of row i ascending, those with a
-// zero K_ic skipped, f_c = K_ic / K_cc), so the values are bit-identical.
-// Each row c is walked with coalesced loads of its values and map entries, no
-// searches.  A wavefront runs four reduced rows, one per 16-lane group, so
-// four rows' chains of dependent loads are in flight at once.  LDS: max_row
-// doubles per row (16 per workgroup).
-__global__ __launch_bounds__(256) void k_sc_values_map(int64_t n_red, const int32_t *__restrict__ rfull,
-                                                       const int32_t *__restrict__ rp, const int32_t *__restrict__ ci,
-                                                       const double *__restrict__ v, const int32_t *__restrict__ ridx,
-                                                       const int32_t *__restrict__ dpos,
-                                                       const int64_t *__restrict__ pmoff,
-                                                       const int16_t *__restrict__ pmap,
-                                                       const int32_t *__restrict__ srp, double *__restrict__ sv,
-                                                       int max_row) {
-  extern __shared__ double sc_sm[];
-  const int lane = threadIdx.x & 63, sl = lane & 15, gb = lane & 48;
-  const int slot = (threadIdx.x >> 6) * 4 + (lane >> 4);
-  double *acc = sc_sm + (size_t)slot * max_row;
-  const uint32_t below = (1u << sl) - 1;
-  auto gballot = [&](bool p) { return (uint32_t)(__ballot(p) >> gb) & 0xffffu; };
-  const int64_t ng = (int64_t)gridDim.x * (blockDim.x >> 4);
-  for (int64_t r = blockIdx.x * (int64_t)(blockDim.x >> 4) + slot; r < n_red; r += ng) {
-    const int32_t i = rfull[r], k0 = rp[i], k1 = rp[i + 1], len = k1 - k0;
-    for (int32_t t = sl; t < len; t += 16) acc[t] = v[k0 + t];
-    sc_wave_lds_sync();
-    int64_t base = pmoff[r];
-    for (int32_t cb = k0; cb < k1; cb += 16) {
-      const int32_t kc = cb + sl;
-      const int32_t cc = kc < k1 ? ci[kc] : 0;
-      const int32_t qc = kc < k1 ? ridx[cc] : 0;
-      const bool isc = kc < k1 && qc < 0;
-      const int32_t c0 = isc ? rp[cc] : 0, lenc = isc ? rp[cc + 1] - c0 : 0;
-      const double vic = isc ? v[kc] : 0.0;
-      const double fl = vic != 0.0 ? vic / v[dpos[-1 - qc]] : 0.0;
-      const int32_t inc = sc_group_scan(lenc), moff = inc - lenc;
-      uint32_t m = gballot(vic != 0.0);
-      while (m) {
-        const int b = __builtin_ctz(m);
-        m &= m - 1;
-        const double f = __shfl(fl, b, 16);
-        const int32_t cs = __shfl(c0, b, 16), L = __shfl(lenc, b, 16);
-        const int16_t *mp = pmap + base + __shfl(moff, b, 16);
-        for (int32_t t = sl; t < L; t += 16) {
-          const int32_t pos = mp[t];
-          if (pos >= 0) acc[pos] -= f * v[cs + t];
-        }
-        sc_wave_lds_sync();  // this condensed column's updates land before the next one's
+    for (int c = 0; c < kScC; ++c) xr[c] = 32 * c + sl < len ? row[32 * c + sl] : 0.0;
+    MT at[kScU];
+    double xc[kScU];
+    auto column = [&](int u0) {  // rows and slots of columns u0 .. u0 + kScU - 1
+#pragma unroll
+      for (int u = 0; u < kScU; ++u) {
+        const int src = u0 + u < 32 ? u0 + u : 31;
+        const int32_t L = __shfl(lenc, src, 32);
+        const uint32_t c0 = __shfl(l.y, src, 32), m0 = __shfl(l.w, src, 32);
+        const bool on = u0 + u < n && sl < L;
+        at[u] = on ? pmap[m0 + sl] : (MT)-1;
+        xc[u] = on ? v[c0 + sl] : 0.0;
       }
-      base += __shfl(inc, 15, 16);
+    };
+    column(0);
+    int before[kScC];
+    bool cond[kScC];
+#pragma unroll
+    for (int c = 0; c < kScC; ++c) {
+      before[c] = 0;
+      cond[c] = false;
     }
-    int32_t out = srp[r];
-    for (int32_t t0 = 0; t0 < len; t0 += 16) {
-      const int32_t t = t0 + sl;
-      const bool keep = t < len && ridx[ci[k0 + t]] >= 0;
-      const uint32_t km = gballot(keep);
-      if (keep) sv[out + __popc(km & below)] = acc[t];
-      out += __popc(km);
+    for (int u = 0; u < nmax; ++u) {
+      const int32_t p = __shfl(pos, u, 32);
+#pragma unroll
+      for (int c = 0; c < kScC; ++c) {
+        before[c] += p < 32 * c + sl;
+        cond[c] |= p == 32 * c + sl;
+      }
     }
-    sc_wave_lds_sync();  // the staged row is read before the next row overwrites it
+#pragma unroll
+    for (int c = 0; c < kScC; ++c)
+      if (32 * c + sl < len && !cond[c]) acc[32 * c + sl - before[c]] = xr[c];
+    for (int tb = 32 * kScC; tb < lmax; tb += 32) {  // longer rows: the rest of them
+      const int32_t t = tb + sl;
+      const double x = t < len ? row[t] : 0.0;
+      int bf = 0;
+      bool cn = false;
+      for (int u = 0; u < nmax; ++u) {
+        const int32_t p = __shfl(pos, u, 32);
+        bf += p < t;
+        cn |= p == t;
+      }
+      if (t < len && !cn) acc[t - bf] = x;
+    }
+    const double f = kic != 0.0 ? kic / kcc : 0.0;
+    for (int u0 = 0; u0 < nmax; u0 += kScU) {
+      if (u0) column(u0);
+#pragma unroll
+      for (int u = 0; u < kScU; ++u) {
+        const int src = u0 + u < 32 ? u0 + u : 31;
+        const double fu = __shfl(f, src, 32), ku = __shfl(kic, src, 32);
+        sc_wave_lds_sync();  // the last column's updates land before this one's
+        if (at[u] != (MT)-1 && ku != 0.0) acc[at[u]] -= fu * xc[u];
+        const int32_t L = __shfl(lenc, src, 32);
+        if (__any(u0 + u < n && L > 32)) {  // longer condensed rows: the rest of them
+          const uint32_t c0 = __shfl(l.y, src, 32), m0 = __shfl(l.w, src, 32);
+          if (u0 + u < n && ku != 0.0)
+            for (int32_t t = sl + 32; t < L; t += 32) {
+              const MT p = pmap[m0 + t];
+              if (p != (MT)-1) acc[p] -= fu * v[c0 + t];
+            }
+        }
+      }
+    }
+  }
+  __syncthreads();
+  double *out = sv + (s0 - sh);
+  for (int32_t t = 2 * threadIdx.x; t < sh + s1 - s0; t += 512) {
+    const double2 w = *(const double2 *)(img + t);
+    if (t >= sh && t + 2 <= sh + s1 - s0)
+      *(double2 *)(out + t) = w;
+    else if (t >= sh)
+      out[t] = w.x;
+    else if (t + 1 < sh + s1 - s0)
+      out[t + 1] = w.y;
   }
 }
 
-// Position map, built once the pattern has passed the fill check; skipped
-// (the refresh keeps k_sc_values_lds) when rows are too long for int16
-// positions or the map would exceed 4 GiB.
-static int sc_build_map(lmh_condensation *sc) {
+// The plan, built once the pattern has passed the fill check; skipped (the
+// refresh keeps k_sc_values_lds, the forward step k_sc_forward) when a row is
+// longer than a row block, has more condensed columns than lanes, or the slots
+// would exceed 4 GiB.
+static int sc_build_plan(lmh_condensation *sc) {
   lmh_matrix *A = sc->A;
   lmh_context *ctx = A->ctx;
-  // the refresh stages max_row doubles per reduced row (16 per workgroup)
-  if (!sc->n_cond || A->max_row >= 32768 || (size_t)A->max_row * 8 * 16 > 48 * 1024) return LMH_OK;
+  if (!sc->n_cond || A->max_row > kScRow) return LMH_OK;
   const int64_t nr = sc->n_red;
-  if (hipMalloc((void **)&sc->pmoff, sizeof(int64_t) * (nr + 1)) != hipSuccess) {
-    (void)hipGetLastError();
-    sc->pmoff = nullptr;
-    return LMH_OK;  // no room: the refresh keeps the search kernel
-  }
-  LMH_LAUNCH(ctx, "sc_map_count", k_sc_map_count, dim3(grid_for(nr, 4, 65536)), dim3(256), 0, nr, sc->rfull, A->rp,
-             A->ci, sc->ridx, sc->pmoff);
-  std::vector<int64_t> h(nr + 1);
-  LMH_HIP(hipMemcpyAsync(h.data(), sc->pmoff, sizeof(int64_t) * nr, hipMemcpyDeviceToHost, ctx->stream));
-  LMH_HIP(hipStreamSynchronize(ctx->stream));
-  int64_t tot = 0;
+  int2 *cnt = nullptr;  // sizes, then starts
+  auto give_up = [&](int rc) {
+    (void)hipFree(cnt);
+    if (rc != LMH_OK || !sc->pmap) {
+      (void)hipGetLastError();
+      (void)hipFree(sc->rec);
+      (void)hipFree(sc->lst);
+      (void)hipFree(sc->lcol);
+      (void)hipFree(sc->pmap);
+      sc->rec = sc->lst = nullptr;
+      sc->lcol = nullptr;
+      sc->pmap = nullptr;
+    }
+    return rc;
+  };
+  if (hipMalloc((void **)&cnt, sizeof(int2) * nr) != hipSuccess) return give_up(LMH_OK);
+  LMH_HIP(hipMemsetAsync(ctx->d_flags, 0, sizeof(int), ctx->stream));
+  LMH_LAUNCH(ctx, "sc_map_count", k_sc_plan_count, dim3(grid_for(nr, 4, 65536)), dim3(256), 0, nr, sc->rfull, A->rp,
+             A->ci, sc->ridx, cnt);
+  LMH_LAUNCH(ctx, "sc_map_count", k_sc_coupled, dim3(grid_for(sc->n_cond, 256, 8192)), dim3(256), 0, sc->n_cond,
+             sc->cdof, A->rp, A->ci, sc->ridx, ctx->d_flags);
+  std::vector<int2> h(nr);
+  int coupled = 0;
+  if (hipMemcpyAsync(h.data(), cnt, sizeof(int2) * nr, hipMemcpyDeviceToHost, ctx->stream) != hipSuccess ||
+      hipMemcpyAsync(&coupled, ctx->d_flags, sizeof(int), hipMemcpyDeviceToHost, ctx->stream) != hipSuccess ||
+      hipStreamSynchronize(ctx->stream) != hipSuccess)
+    return give_up(set_error(LMH_ERR_HIP, "condensation plan"));
+  int64_t tl = 0, tm = 0;
+  int most = 0;
   for (int64_t r = 0; r < nr; ++r) {
-    const int64_t c = h[r];
-    h[r] = tot;
-    tot += c;
+    const int2 c = h[r];
+    h[r] = make_int2((int)tl, (int)(uint32_t)tm);
+    tl += c.x;
+    tm += c.y;
+    most = std::max(most, c.x);
   }
-  h[nr] = tot;
-  if (tot * (int64_t)sizeof(int16_t) > (int64_t(4) << 30) ||
-      hipMalloc((void **)&sc->pmap, sizeof(int16_t) * std::max<int64_t>(1, tot)) != hipSuccess) {
-    (void)hipGetLastError();
-    (void)hipFree(sc->pmoff);
-    sc->pmoff = nullptr;
-    sc->pmap = nullptr;
-    return LMH_OK;
-  }
-  LMH_HIP(hipMemcpyAsync(sc->pmoff, h.data(), sizeof(int64_t) * (nr + 1), hipMemcpyHostToDevice, ctx->stream));
-  LMH_LAUNCH(ctx, "sc_map_fill", k_sc_map_fill, dim3(grid_for(nr, 4, 65536)), dim3(256), (size_t)A->max_row * 4 * 4,
-             nr, sc->rfull, A->rp, A->ci, sc->ridx, sc->pmoff, sc->pmap, A->max_row);
-  LMH_TRY(check_launch("k_sc_map_fill"));
-  LMH_HIP(hipStreamSynchronize(ctx->stream));  // h is read by the copy above
-  return LMH_OK;
+  sc->wide = A->max_row > 255;
+  const int64_t bytes = tm * (sc->wide ? 2 : 1);
+  if (most > 32 || tl > INT32_MAX || bytes >= (int64_t(4) << 30) ||
+      hipMalloc((void **)&sc->rec, sizeof(uint4) * nr) != hipSuccess ||
+      hipMalloc((void **)&sc->lst, sizeof(uint4) * std::max<int64_t>(1, tl)) != hipSuccess ||
+      hipMalloc((void **)&sc->lcol, sizeof(int32_t) * std::max<int64_t>(1, tl)) != hipSuccess ||
+      hipMalloc((void **)&sc->pmap, std::max<int64_t>(16, bytes)) != hipSuccess)
+    return give_up(LMH_OK);
+  if (hipMemcpy(cnt, h.data(), sizeof(int2) * nr, hipMemcpyHostToDevice) != hipSuccess)
+    return give_up(set_error(LMH_ERR_HIP, "condensation plan"));
+  const dim3 grid(grid_for(nr, 4, 65536));
+  const size_t lds = (size_t)A->max_row * 4 * 2 * 4;
+  if (sc->wide)
+    LMH_LAUNCH(ctx, "sc_map_fill", k_sc_plan_fill<uint16_t>, grid, dim3(256), lds, nr, sc->rfull, A->rp, A->ci,
+               sc->ridx, sc->dpos, sc->R->rp, cnt, sc->rec, sc->lst, sc->lcol, (uint16_t *)sc->pmap, A->max_row);
+  else
+    LMH_LAUNCH(ctx, "sc_map_fill", k_sc_plan_fill<uint8_t>, grid, dim3(256), lds, nr, sc->rfull, A->rp, A->ci,
+               sc->ridx, sc->dpos, sc->R->rp, cnt, sc->rec, sc->lst, sc->lcol, (uint8_t *)sc->pmap, A->max_row);
+  if (check_launch("k_sc_plan_fill") != LMH_OK || hipStreamSynchronize(ctx->stream) != hipSuccess)
+    return give_up(set_error(LMH_ERR_HIP, "condensation plan"));
+  sc->coupled = coupled != 0;
+  return give_up(LMH_OK);
 }
 
 static int sc_setup(lmh_condensation *sc) {
@@ -487,7 +632,7 @@ static int sc_setup(lmh_condensation *sc) {
   lmh_context *ctx = A->ctx;
   LMH_HIP(hipSetDevice(ctx->device));
   LMH_HIP(hipMemsetAsync(ctx->d_flags, 0, sizeof(int), ctx->stream));
-  if (sc->n_cond) {
+  if (sc->n_cond && (!sc->pmap || sc->coupled)) {
     LMH_LAUNCH(ctx, "sc_check", k_sc_check, dim3(grid_for(sc->n_cond, 256, 8192)), dim3(256), 0, sc->n_cond, sc->cdof,
                A->rp, A->ci, A->vals, sc->ridx, sc->dpos, ctx->d_flags);
     LMH_TRY(check_launch("k_sc_check"));
@@ -497,10 +642,15 @@ static int sc_setup(lmh_condensation *sc) {
                sc->rfull, A->rp, A->ci, A->vals, sc->ridx, sc->dpos, R->rp, R->ci, R->vals, ctx->d_flags);
     LMH_TRY(check_launch("k_sc_values"));
   } else if (sc->pmap) {
-    LMH_LAUNCH(ctx, "sc_values", k_sc_values_map, dim3(grid_for(sc->n_red, 16, 65536)), dim3(256),
-               (size_t)A->max_row * 8 * 16, sc->n_red, sc->rfull, A->rp, A->ci, A->vals, sc->ridx, sc->dpos, sc->pmoff,
-               sc->pmap, R->rp, R->vals, A->max_row);
-    LMH_TRY(check_launch("k_sc_values_map"));
+    const dim3 grid((unsigned)((R->nrb + NXCD - 1) / NXCD * NXCD));
+    const int64_t pivots = sc->coupled ? 0 : sc->n_cond;
+    if (sc->wide)
+      LMH_LAUNCH(ctx, "sc_values", k_sc_values_plan<uint16_t>, grid, dim3(256), 0, (int)R->nrb, R->rb, A->vals,
+                 sc->rec, sc->lst, (const uint16_t *)sc->pmap, R->rp, R->vals, pivots, sc->dpos, ctx->d_flags);
+    else
+      LMH_LAUNCH(ctx, "sc_values", k_sc_values_plan<uint8_t>, grid, dim3(256), 0, (int)R->nrb, R->rb, A->vals,
+                 sc->rec, sc->lst, (const uint8_t *)sc->pmap, R->rp, R->vals, pivots, sc->dpos, ctx->d_flags);
+    LMH_TRY(check_launch("k_sc_values_plan"));
   } else if ((size_t)A->max_row * 12 * 4 <= 48 * 1024) {
     LMH_LAUNCH(ctx, "sc_values", k_sc_values_lds, dim3(grid_for(sc->n_red, 4, 65536)), dim3(256),
                (size_t)A->max_row * 12 * 4, sc->n_red, sc->rfull, A->rp, A->ci, A->vals, sc->ridx, sc->dpos, R->rp,
@@ -523,7 +673,7 @@ static int sc_setup(lmh_condensation *sc) {
             "condensation needs an entry outside the matrix pattern (the condensed DoF is not element-interior)");
   if (!sc->pattern_checked) {
     sc->pattern_checked = true;
-    LMH_TRY(sc_build_map(sc));
+    LMH_TRY(sc_build_plan(sc));
   }
   return LMH_OK;
 }
@@ -618,6 +768,11 @@ int lmh_condensation_forward(lmh_condensation *sc, const double *full_rhs_d, dou
   LMH_CHECK(sc && full_rhs_d && reduced_rhs_d, LMH_ERR_INVALID, "null argument");
   lmh_matrix *A = sc->A;
   lmh_context *ctx = A->ctx;
+  if (sc->pmap) {
+    LMH_LAUNCH(ctx, "sc_forward", k_sc_forward_list, dim3(grid_for(sc->n_red, 256, 16384)), dim3(256), 0, sc->n_red,
+               sc->rfull, A->vals, sc->rec, sc->lst, sc->lcol, full_rhs_d, reduced_rhs_d);
+    return check_launch("k_sc_forward_list");
+  }
   LMH_LAUNCH(ctx, "sc_forward", k_sc_forward, dim3(grid_for(sc->n_red, 4, 65536)), dim3(256), 0, sc->n_red,
              sc->rfull, A->rp, A->ci, A->vals, sc->ridx, sc->dpos, full_rhs_d, reduced_rhs_d);
   return check_launch("k_sc_forward");
@@ -628,12 +783,10 @@ int lmh_condensation_backward(lmh_condensation *sc, const double *full_rhs_d, co
   LMH_CHECK(sc && full_rhs_d && reduced_sol_d && full_sol_d, LMH_ERR_INVALID, "null argument");
   lmh_matrix *A = sc->A;
   lmh_context *ctx = A->ctx;
-  LMH_LAUNCH(ctx, "sc_map", k_sc_map<false>, dim3(grid_for(sc->n_red, 256, 16384)), dim3(256), 0, sc->n_red,
-             sc->rfull, full_sol_d, const_cast<double *>(reduced_sol_d));
-  LMH_TRY(check_launch("k_sc_map"));
-  if (!sc->n_cond) return LMH_OK;
-  LMH_LAUNCH(ctx, "sc_backward", k_sc_backward, dim3(grid_for(sc->n_cond, 256, 8192)), dim3(256), 0, sc->n_cond,
-             sc->cdof, A->rp, A->ci, A->vals, sc->ridx, sc->dpos, full_rhs_d, full_sol_d);
+  const int nbc = sc->n_cond ? grid_for(sc->n_cond, 8, 4096) : 0;
+  LMH_LAUNCH(ctx, "sc_backward", k_sc_backward, dim3(nbc + grid_for(sc->n_red, 256, 4096)), dim3(256), 0, nbc,
+             sc->n_cond, sc->cdof, A->rp, A->ci, A->vals, sc->ridx, sc->dpos, full_rhs_d, sc->n_red, sc->rfull,
+             reduced_sol_d, full_sol_d);
   return check_launch("k_sc_backward");
 }
 
@@ -642,7 +795,7 @@ int lmh_condensation_solve(lmh_condensation *sc, const double *b_d, double *x_d,
   LMH_CHECK(sc && b_d && x_d, LMH_ERR_INVALID, "null argument");
   lmh_context *ctx = sc->A->ctx;
   LMH_TRY(lmh_condensation_forward(sc, b_d, sc->g));
-  LMH_LAUNCH(ctx, "sc_map", k_sc_map<true>, dim3(grid_for(sc->n_red, 256, 16384)), dim3(256), 0, sc->n_red, sc->rfull,
+  LMH_LAUNCH(ctx, "sc_map", k_sc_map, dim3(grid_for(sc->n_red, 256, 16384)), dim3(256), 0, sc->n_red, sc->rfull,
              x_d, sc->y);
   LMH_TRY(check_launch("k_sc_map"));
   LMH_TRY(lmh_cg_solve(sc->R, sc->g, sc->y, rtol, maxits, iters, rel_res, reason));
@@ -660,7 +813,9 @@ int lmh_condensation_destroy(lmh_condensation *sc) {
   (void)hipFree(sc->dpos);
   (void)hipFree(sc->g);
   (void)hipFree(sc->y);
-  (void)hipFree(sc->pmoff);
+  (void)hipFree(sc->rec);
+  (void)hipFree(sc->lst);
+  (void)hipFree(sc->lcol);
   (void)hipFree(sc->pmap);
   delete sc;
   return LMH_OK;
