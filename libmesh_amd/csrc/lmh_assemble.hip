@@ -77,7 +77,7 @@ __global__ __launch_bounds__(64) void k_poisson_generic(const double *__restrict
     if (lane < nq) {
       double Mq[9];
       double jxw;
-      if (qp_geometry(X, dref, n, nq, lane, w[lane], kap, Mq, jxw) <= 0.0) atomicOr(err, 1);
+      if (qp_geometry(X, dref, n, nq, lane, w[lane], kap, Mq, jxw) <= 0.0) raise_flag(err);
       for (int t = 0; t < 9; ++t) M[lane * 9 + t] = Mq[t];
       double f = 1.0;
       if (f_kind != 0) {
@@ -160,7 +160,7 @@ __global__ __launch_bounds__(256) void k_poisson_hex8(const double *__restrict__
     if (valid) {
       double Mq[9];
       double jxw;
-      if (qp_geometry(X, dref, 8, 8, t, w[t], kap, Mq, jxw) <= 0.0) atomicOr(err, 1);
+      if (qp_geometry(X, dref, 8, 8, t, w[t], kap, Mq, jxw) <= 0.0) raise_flag(err);
       for (int k = 0; k < 9; ++k) s_M[wv][el][t * 9 + k] = Mq[k];
       double f = 1.0;
       if (f_kind != 0) {
@@ -397,7 +397,7 @@ __global__ __launch_bounds__(64) void k_qoi_box(const double *__restrict__ tab, 
     if (lane < nq) {
       double Mq[9];
       double jxw;
-      if (qp_geometry(X, dref, n, nq, lane, w[lane], 1.0, Mq, jxw) <= 0.0) atomicOr(err, 1);
+      if (qp_geometry(X, dref, n, nq, lane, w[lane], 1.0, Mq, jxw) <= 0.0) raise_flag(err);
       double x = 0, y = 0, z = 0;
       for (int a = 0; a < n; ++a) {
         const double p = phi[a * nq + lane];
@@ -453,7 +453,7 @@ __global__ __launch_bounds__(64) void k_adjoint_kappa(const double *__restrict__
     if (lane < nq) {
       double Mq[9];
       double jxw;
-      if (qp_geometry(X, dref, n, nq, lane, w[lane], 1.0, Mq, jxw) <= 0.0) atomicOr(err, 1);
+      if (qp_geometry(X, dref, n, nq, lane, w[lane], 1.0, Mq, jxw) <= 0.0) raise_flag(err);
       double gu[3] = {0, 0, 0}, gl[3] = {0, 0, 0};
       for (int a = 0; a < n; ++a) {
         const double *d = &dref[(a * nq + lane) * 3];
@@ -486,10 +486,8 @@ static int matrix_free_path(int type, int npts) {
 }
 
 static int read_flag(lmh_context *ctx, const char *what) {
-  int flag = 0;
-  LMH_HIP(hipMemcpyAsync(&flag, ctx->d_flags, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
   LMH_HIP(hipStreamSynchronize(ctx->stream));
-  if (flag) return set_error(LMH_ERR_DEGENERATE, "%s: Jacobian determinant <= 0 (degenerate map)", what);
+  if (*(volatile int *)ctx->h_flag) return set_error(LMH_ERR_DEGENERATE, "%s: Jacobian determinant <= 0 (degenerate map)", what);
   return LMH_OK;
 }
 
@@ -534,14 +532,14 @@ static int element_poisson_impl(lmh_context *ctx, const lmh_mesh *m, const lmh_d
   if (m->type == LMH_HEX8 && npts == 2 && sizeof(CT) == 8 && ne < kHex8ThreadMin) {
     const int g = grid_for((ne + 31) / 32, 1, ctx->cu_count * 4);
     LMH_LAUNCH(ctx, "element_hex8_fma", k_poisson_hex8, dim3(g), dim3(256), 0, t->d_data, m->xyz, m->conn, dm->edofs,
-               dm->cons, kappa, f_kind, constrain, ne, (double *)Ke, Fe, ctx->d_flags);
+               dm->cons, kappa, f_kind, constrain, ne, (double *)Ke, Fe, ctx->g_flag);
     return check_launch("k_poisson_hex8");
   }
   if (m->type != LMH_HEX27) return thread_poisson<CT>(ctx, t, m, dm, kappa, f_kind, constrain, Ke, Fe);
   const size_t shm = sizeof(double) * (t->nq + (size_t)t->n * t->nq * 4 + 81 + 9 * t->nq + t->nq);
   const int g = grid_for(ne, 1, maxg);
   LMH_LAUNCH(ctx, "element_generic", k_poisson_generic<CT>, dim3(g), dim3(64), shm, t->d_data, t->n, t->nq, m->xyz,
-             m->conn, dm->edofs, dm->cons, kappa, f_kind, constrain, ne, Ke, Fe, ctx->d_flags);
+             m->conn, dm->edofs, dm->cons, kappa, f_kind, constrain, ne, Ke, Fe, ctx->g_flag);
   return check_launch("k_poisson_generic");
 }
 
@@ -585,7 +583,7 @@ int lmh_element_poisson(lmh_context *ctx, const lmh_mesh *m, const lmh_dofmap *d
   LMH_CHECK(ctx && m && dm && Ke_d && Fe_d, LMH_ERR_INVALID, "null argument");
   LMH_CHECK(!constrain || dm->cr.n_general == 0, LMH_ERR_UNSUPPORTED,
             "element matrices with general constraint rows grow past the element's DoFs: assemble the matrix");
-  LMH_HIP(hipMemsetAsync(ctx->d_flags, 0, sizeof(int), ctx->stream));
+  *(volatile int *)ctx->h_flag = 0;
   LMH_TRY(element_poisson_impl<double>(ctx, m, dm, npts, kappa_d, f_kind, constrain, Ke_d, Fe_d));
   return read_flag(ctx, "lmh_element_poisson");
 }
@@ -600,7 +598,7 @@ int lmh_assemble_poisson(lmh_matrix *A, const lmh_mesh *m, const lmh_dofmap *dm,
   lmh_context *ctx = A->ctx;
   const int64_t ne = m->n_elem, dd = (int64_t)dm->dpe * dm->dpe;
   if (!A->Fe) LMH_HIP(hipMalloc((void **)&A->Fe, sizeof(double) * ne * dm->dpe));
-  LMH_HIP(hipMemsetAsync(ctx->d_flags, 0, sizeof(int), ctx->stream));
+  *(volatile int *)ctx->h_flag = 0;
   if (precision == LMH_FP64) {
     if (!A->Ke) LMH_HIP(hipMalloc((void **)&A->Ke, sizeof(double) * ne * dd));
     LMH_TRY(element_poisson_impl<double>(ctx, m, dm, npts, kappa_d, f_kind, 1, A->Ke, A->Fe));
@@ -694,7 +692,7 @@ int lmh_assemble_residual_poisson(lmh_matrix *A, const lmh_mesh *m, const lmh_do
   LMH_CHECK(dm->nv == 1, LMH_ERR_UNSUPPORTED, "Poisson assembly needs one variable");
   const FETable *t = nullptr;
   LMH_TRY(fe_table(ctx, m->type, npts, &t));
-  LMH_HIP(hipMemsetAsync(ctx->d_flags, 0, sizeof(int), ctx->stream));
+  *(volatile int *)ctx->h_flag = 0;
   const int path = matrix_free_path(m->type, npts);
   if (path == 1) {
     LMH_TRY(hex27_residual(ctx, m, dm, kappa_d, f_kind, u_d, A->Fe));
@@ -724,7 +722,7 @@ int lmh_qoi_box_derivative(const lmh_mesh *m, const lmh_dofmap *dm, int npts, do
   LMH_TRY(fe_table(ctx, m->type, npts, &t));
   double *Q = nullptr;
   LMH_HIP(hipMallocAsync((void **)&Q, sizeof(double) * m->n_elem * t->n, ctx->stream));
-  LMH_HIP(hipMemsetAsync(ctx->d_flags, 0, sizeof(int), ctx->stream));
+  *(volatile int *)ctx->h_flag = 0;
   const int path = matrix_free_path(m->type, npts);
   if (path == 1) {
     LMH_TRY(hex27_qoi(ctx, m, lo, hi, Q));
@@ -733,7 +731,7 @@ int lmh_qoi_box_derivative(const lmh_mesh *m, const lmh_dofmap *dm, int npts, do
   } else {
     const size_t shm = sizeof(double) * (t->nq + (size_t)t->n * t->nq * 4 + 81 + t->nq);
     LMH_LAUNCH(ctx, "qoi_box", k_qoi_box, dim3(grid_for(m->n_elem, 1, ctx->cu_count * 8)), dim3(64), shm, t->d_data,
-               t->n, t->nq, m->xyz, m->conn, m->n_elem, lo, hi, Q, ctx->d_flags);
+               t->n, t->nq, m->xyz, m->conn, m->n_elem, lo, hi, Q, ctx->g_flag);
     LMH_TRY(check_launch("k_qoi_box"));
   }
   LMH_LAUNCH(ctx, "add_element_vectors", k_sum_vec_gather<true>, dim3(grid_for(dm->n_dofs, 256, 8192)), dim3(256), 0,
@@ -758,7 +756,7 @@ int lmh_adjoint_kappa_gradient(const lmh_mesh *m, const lmh_dofmap *dm, int npts
   const FETable *t = nullptr;
   LMH_TRY(fe_table(ctx, m->type, npts, &t));
   LMH_CHECK(t->nq <= 64 && t->n <= 27, LMH_ERR_UNSUPPORTED, "element too large");
-  LMH_HIP(hipMemsetAsync(ctx->d_flags, 0, sizeof(int), ctx->stream));
+  *(volatile int *)ctx->h_flag = 0;
   const int path = matrix_free_path(m->type, npts);
   if (path != 0) {
     LMH_TRY(path == 1 ? hex27_adjoint(ctx, m, dm, u_d, lambda_d, grad_d)
@@ -768,7 +766,7 @@ int lmh_adjoint_kappa_gradient(const lmh_mesh *m, const lmh_dofmap *dm, int npts
   const size_t shm = sizeof(double) * (t->nq + (size_t)t->n * t->nq * 4 + 81 + 27 + 27 + 64);
   LMH_LAUNCH(ctx, "adjoint_kappa", k_adjoint_kappa, dim3(grid_for(m->n_elem, 1, ctx->cu_count * 8)), dim3(64), shm,
              t->d_data, t->n, t->nq, m->xyz, m->conn, dm->edofs, dm->cons, u_d, lambda_d, m->n_elem, grad_d,
-             ctx->d_flags);
+             ctx->g_flag);
   LMH_TRY(check_launch("k_adjoint_kappa"));
   return read_flag(ctx, "lmh_adjoint_kappa_gradient");
 }

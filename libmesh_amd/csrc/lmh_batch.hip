@@ -90,10 +90,6 @@ __host__ __device__ inline int slot_bytes(int n, int nq) {
   return (s + 15) & ~15;
 }
 
-__global__ void k_batch_clear(int *flag) {
-  if (threadIdx.x == 0 && blockIdx.x == 0) flag[0] = 0;
-}
-
 typedef float f32x3 __attribute__((ext_vector_type(3), aligned(4)));
 
 // row i of the 3 x 3 block of a node pair, after the element constraint
@@ -138,7 +134,7 @@ __device__ inline void elasticity_tet4(const BProb &P, const BTile &tl, double f
       J[2][c] = dpp_move<0xff>(x[c]) - x0;
     }
     const double det = lmh_map_inverse(J, G);
-    if (!(det > 0.0) && act && a == 0) atomicOr(err, 1);
+    if (!(det > 0.0) && act && a == 0) raise_flag(err);
     const double sc = det > 0.0 ? sqrt(det * wsum) : 0.0;
     double g[3], f = 0.0;
 #pragma unroll
@@ -194,7 +190,7 @@ struct TableGrad {
           for (int r = 0; r < 3; ++r) J[r][c] += x * d[a][r];
         }
       const double det = lmh_map_inverse(J, G);
-      if (!(det > 0.0)) atomicOr(err, 1);
+      if (!(det > 0.0)) raise_flag(err);
       const double jw = det * wq;
       sc = det > 0.0 ? sqrt(fabs(jw)) : 0.0;
       if (NEG && jw < 0.0) sign = -1.f;
@@ -277,7 +273,7 @@ struct Hex27Grad {
         __builtin_amdgcn_sched_barrier(0);  // one plane's nodes in registers at a time
       }
       const double det = lmh_map_inverse(J, G);
-      if (!(det > 0.0)) atomicOr(err, 1);
+      if (!(det > 0.0)) raise_flag(err);
       auto w = [](int k) { return h27_w(k); };
       const double jw = det * (h27_pick(q1, w) * h27_pick(q2, w) * h27_pick(q3, w));
       const double sc = det > 0.0 ? sqrt(fabs(jw)) : 0.0;
@@ -755,7 +751,7 @@ static void lame(double E, double nu, float &l1, float &l2) {
 
 static void launch_elements(const lmh_batch *b, float l1, float l2, double fz) {
   hipLaunchKernelGGL(k_batch_elasticity, dim3(b->ntile), dim3(kBatchBlock), kBatchLds, b->ctx->stream,
-                     (const BProb *)b->dprob, (const BTile *)b->dtile, l1, l2, fz, b->ctx->d_flags);
+                     (const BProb *)b->dprob, (const BTile *)b->dtile, l1, l2, fz, b->ctx->g_flag);
 }
 
 // flags the problems whose element DoFs do not come in node blocks
@@ -796,7 +792,6 @@ static int build_graph(lmh_batch *b, double E, double nu, double fz) {
   lame(E, nu, l1, l2);
   LMH_HIP(hipStreamSynchronize(ctx->stream));
   LMH_HIP(hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
-  hipLaunchKernelGGL(k_batch_clear, dim3(1), dim3(64), 0, ctx->stream, ctx->d_flags);
   if (b->ntile > 0) launch_elements(b, l1, l2, fz);
   if (b->nnt > 0)
     hipLaunchKernelGGL(k_batch_rows, dim3(b->nnt), dim3(64), b->rows_lds, ctx->stream, (const BScat *)b->dscat,
@@ -1114,14 +1109,13 @@ int lmh_batch_assemble_elasticity(lmh_batch *b, double E, double nu, double fz) 
   LMH_CHECK(E > 0 && nu > -1.0 && nu < 0.5, LMH_ERR_INVALID, "need E > 0 and -1 < nu < 1/2");
   lmh_context *ctx = b->ctx;
   if (!b->exec || E != b->gE || nu != b->gnu || fz != b->gfz) LMH_TRY(build_graph(b, E, nu, fz));
+  *(volatile int *)ctx->h_flag = 0;
   {
     ProfScope ps(ctx, "batch_graph");
     LMH_HIP(hipGraphLaunch(b->exec, ctx->stream));
   }
-  int bad = 0;
-  LMH_HIP(hipMemcpyAsync(&bad, ctx->d_flags, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
   LMH_HIP(hipStreamSynchronize(ctx->stream));
-  LMH_CHECK(!bad, LMH_ERR_DEGENERATE, "degenerate element map (det J <= 0) in the batch");
+  LMH_CHECK(!*(volatile int *)ctx->h_flag, LMH_ERR_DEGENERATE, "degenerate element map (det J <= 0) in the batch");
   for (lmh_matrix *A : b->mats) A->have32 = true;
   return LMH_OK;
 }

@@ -454,11 +454,11 @@ __global__ __launch_bounds__(256) void k_sc_values_plan(int nrb, const int32_t *
                                                         const uint4 *__restrict__ lst, const MT *__restrict__ pmap,
                                                         const int32_t *__restrict__ srp, double *__restrict__ sv,
                                                         int64_t n_cond, const int32_t *__restrict__ dpos,
-                                                        int *__restrict__ flags) {
+                                                        int *__restrict__ flag) {
   __shared__ __align__(16) double img[kScRow + 2];
   const int sl = threadIdx.x & 31, sg = threadIdx.x >> 5;
   for (int64_t q = blockIdx.x * (int64_t)256 + threadIdx.x; q < n_cond; q += (int64_t)gridDim.x * 256)
-    if (v[dpos[q]] == 0.0) atomicOr(flags, SC_ZEROPIVOT);
+    if (v[dpos[q]] == 0.0) raise_flag(flag);
   const int blk = logical_block();
   if (blk >= nrb) return;
   const int32_t r0 = rb[blk], r1 = rb[blk + 1], s0 = srp[r0], s1 = srp[r1], sh = s0 & 1;
@@ -631,8 +631,10 @@ static int sc_setup(lmh_condensation *sc) {
   lmh_matrix *A = sc->A, *R = sc->R;
   lmh_context *ctx = A->ctx;
   LMH_HIP(hipSetDevice(ctx->device));
-  LMH_HIP(hipMemsetAsync(ctx->d_flags, 0, sizeof(int), ctx->stream));
-  if (sc->n_cond && (!sc->pmap || sc->coupled)) {
+  const bool pivots_only = sc->pmap && !sc->coupled;  // k_sc_values_plan checks them
+  *(volatile int *)ctx->h_flag = 0;
+  if (!pivots_only) LMH_HIP(hipMemsetAsync(ctx->d_flags, 0, sizeof(int), ctx->stream));
+  if (sc->n_cond && !pivots_only) {
     LMH_LAUNCH(ctx, "sc_check", k_sc_check, dim3(grid_for(sc->n_cond, 256, 8192)), dim3(256), 0, sc->n_cond, sc->cdof,
                A->rp, A->ci, A->vals, sc->ridx, sc->dpos, ctx->d_flags);
     LMH_TRY(check_launch("k_sc_check"));
@@ -643,13 +645,13 @@ static int sc_setup(lmh_condensation *sc) {
     LMH_TRY(check_launch("k_sc_values"));
   } else if (sc->pmap) {
     const dim3 grid((unsigned)((R->nrb + NXCD - 1) / NXCD * NXCD));
-    const int64_t pivots = sc->coupled ? 0 : sc->n_cond;
+    const int64_t pivots = pivots_only ? sc->n_cond : 0;
     if (sc->wide)
       LMH_LAUNCH(ctx, "sc_values", k_sc_values_plan<uint16_t>, grid, dim3(256), 0, (int)R->nrb, R->rb, A->vals,
-                 sc->rec, sc->lst, (const uint16_t *)sc->pmap, R->rp, R->vals, pivots, sc->dpos, ctx->d_flags);
+                 sc->rec, sc->lst, (const uint16_t *)sc->pmap, R->rp, R->vals, pivots, sc->dpos, ctx->g_flag);
     else
       LMH_LAUNCH(ctx, "sc_values", k_sc_values_plan<uint8_t>, grid, dim3(256), 0, (int)R->nrb, R->rb, A->vals,
-                 sc->rec, sc->lst, (const uint8_t *)sc->pmap, R->rp, R->vals, pivots, sc->dpos, ctx->d_flags);
+                 sc->rec, sc->lst, (const uint8_t *)sc->pmap, R->rp, R->vals, pivots, sc->dpos, ctx->g_flag);
     LMH_TRY(check_launch("k_sc_values_plan"));
   } else if ((size_t)A->max_row * 12 * 4 <= 48 * 1024) {
     LMH_LAUNCH(ctx, "sc_values", k_sc_values_lds, dim3(grid_for(sc->n_red, 4, 65536)), dim3(256),
@@ -662,8 +664,9 @@ static int sc_setup(lmh_condensation *sc) {
     LMH_TRY(check_launch("k_sc_values_wave"));
   }
   int flags = 0;
-  LMH_HIP(hipMemcpyAsync(&flags, ctx->d_flags, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
+  if (!pivots_only) LMH_HIP(hipMemcpyAsync(&flags, ctx->d_flags, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
   LMH_HIP(hipStreamSynchronize(ctx->stream));
+  if (*(volatile int *)ctx->h_flag) flags |= SC_ZEROPIVOT;
   R->have32 = false;
   LMH_CHECK(!(flags & SC_OFFDIAG), LMH_ERR_UNSUPPORTED,
             "condensed DoFs couple to each other: only a diagonal condensed block is supported");

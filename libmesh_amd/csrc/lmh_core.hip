@@ -355,6 +355,10 @@ int lmh_context_create(int device, lmh_context **out) {
   LMH_HIP(hipMalloc((void **)&c->d_flags, 16 * sizeof(int)));
   LMH_HIP(hipMemset(c->d_flags, 0, 16 * sizeof(int)));
   LMH_HIP(hipHostMalloc((void **)&c->h_pinned, 64 * sizeof(double), hipHostMallocDefault));
+  LMH_HIP(hipHostGetDevicePointer((void **)&c->g_pinned, c->h_pinned, 0));
+  LMH_HIP(hipHostMalloc((void **)&c->h_flag, 64, hipHostMallocDefault));
+  LMH_HIP(hipHostGetDevicePointer((void **)&c->g_flag, c->h_flag, 0));
+  *c->h_flag = 0;
   LMH_HIP(hipEventCreateWithFlags(&c->ev_poll[0], hipEventDisableTiming));
   LMH_HIP(hipEventCreateWithFlags(&c->ev_poll[1], hipEventDisableTiming));
   LMH_TRY(cg_scratch_setup(c.get()));
@@ -380,6 +384,7 @@ int lmh_context_destroy(lmh_context *ctx) {
   (void)hipFree(ctx->d_count);
   (void)hipFree(ctx->d_flags);
   (void)hipHostFree(ctx->h_pinned);
+  (void)hipHostFree(ctx->h_flag);
   (void)hipStreamDestroy(ctx->stream);
   delete ctx;
   return LMH_OK;

@@ -101,7 +101,7 @@ __global__ __launch_bounds__(64) void k_hex27_residual(const double *__restrict_
 #pragma unroll
           for (int k = 0; k < 3; ++k) J[r][k] = g[q][k][r];
         const double det = cofactors(J, c);
-        if (!(det > 0.0)) atomicOr(err, 1);
+        if (!(det > 0.0)) raise_flag(err);
         const double w = L.w12 * h27_w(q), s = kap * w / det;
         double v[3];  // det * physical gradient of u
 #pragma unroll
@@ -191,7 +191,7 @@ __global__ __launch_bounds__(64) void k_hex27_qoi(const double *__restrict__ xyz
 #pragma unroll
           for (int k = 0; k < 3; ++k) J[r][k] = g[q][k][r];
         const double det = cofactors(J, c);
-        if (!(det > 0.0)) atomicOr(err, 1);
+        if (!(det > 0.0)) raise_flag(err);
         const double x = pos[q][0], y = pos[q][1], z = pos[q][2];
         const bool in = x >= lo && x <= hi && y >= lo && y <= hi && z >= lo && z <= hi;
         const double jc = in ? det * (L.w12 * h27_w(q)) : 0.0;
@@ -265,7 +265,7 @@ __global__ __launch_bounds__(64) void k_hex27_adjoint(const double *__restrict__
 #pragma unroll
           for (int k = 0; k < 3; ++k) J[r][k] = g[q][k][r];
         const double det = cofactors(J, c);
-        if (!(det > 0.0)) atomicOr(err, 1);
+        if (!(det > 0.0)) raise_flag(err);
         double t = 0.0;
 #pragma unroll
         for (int k = 0; k < 3; ++k) {
@@ -391,7 +391,7 @@ __global__ __launch_bounds__(64, 2) void k_hex27_poisson(const double *__restric
 #pragma unroll
           for (int k = 0; k < 3; ++k) J[r][k] = g[q][k][r];
         const double det = cofactors(J, c);
-        if (!(det > 0.0)) atomicOr(err, 1);
+        if (!(det > 0.0)) raise_flag(err);
         const double w = L.w12 * h27_w(q), s = kap * w / det;
         double *M = s_m + L.el * 162 + 9 * q + L.l;  // components 11, 12, 13, 22, 23, 33
         int m = 0;
@@ -531,10 +531,10 @@ int hex27_poisson(lmh_context *ctx, const lmh_mesh *m, const lmh_dofmap *dm, con
   const char *name = sizeof(CT) == 8 ? "element_hex27_fp64" : "element_hex27_fp32";
   if (f_kind == 0)
     LMH_LAUNCH(ctx, name, (k_hex27_poisson<CT, 0>), dim3(g), dim3(64), 0, m->xyz, m->conn, dm->edofs,
-               dm->cons, kappa, constrain, per, ne, Ke, Fe, ctx->d_flags);
+               dm->cons, kappa, constrain, per, ne, Ke, Fe, ctx->g_flag);
   else
     LMH_LAUNCH(ctx, name, (k_hex27_poisson<CT, 1>), dim3(g), dim3(64), 0, m->xyz, m->conn, dm->edofs,
-               dm->cons, kappa, constrain, per, ne, Ke, Fe, ctx->d_flags);
+               dm->cons, kappa, constrain, per, ne, Ke, Fe, ctx->g_flag);
   return check_launch("k_hex27_poisson");
 }
 template int hex27_poisson<double>(lmh_context *, const lmh_mesh *, const lmh_dofmap *, const double *, int, int,
@@ -548,17 +548,17 @@ int hex27_residual(lmh_context *ctx, const lmh_mesh *m, const lmh_dofmap *dm, co
   const int g = h27_grid(ctx, m->n_elem);
   if (f_kind == 0)
     LMH_LAUNCH(ctx, "element_residual", k_hex27_residual<0>, dim3(g), dim3(64), 0, m->xyz, m->conn, dm->edofs, kappa,
-               u, m->n_elem, Fe, ctx->d_flags);
+               u, m->n_elem, Fe, ctx->g_flag);
   else
     LMH_LAUNCH(ctx, "element_residual", k_hex27_residual<1>, dim3(g), dim3(64), 0, m->xyz, m->conn, dm->edofs, kappa,
-               u, m->n_elem, Fe, ctx->d_flags);
+               u, m->n_elem, Fe, ctx->g_flag);
   return check_launch("k_hex27_residual");
 }
 
 int hex27_qoi(lmh_context *ctx, const lmh_mesh *m, double lo, double hi, double *Q) {
   if (m->n_elem == 0) return LMH_OK;
   LMH_LAUNCH(ctx, "qoi_box", k_hex27_qoi, dim3(h27_grid(ctx, m->n_elem)), dim3(64), 0, m->xyz, m->conn, m->n_elem, lo,
-             hi, Q, ctx->d_flags);
+             hi, Q, ctx->g_flag);
   return check_launch("k_hex27_qoi");
 }
 
@@ -566,7 +566,7 @@ int hex27_adjoint(lmh_context *ctx, const lmh_mesh *m, const lmh_dofmap *dm, con
                   double *grad) {
   if (m->n_elem == 0) return LMH_OK;
   LMH_LAUNCH(ctx, "adjoint_kappa", k_hex27_adjoint, dim3(h27_grid(ctx, m->n_elem)), dim3(64), 0, m->xyz, m->conn,
-             dm->edofs, dm->cons, u, lam, m->n_elem, grad, ctx->d_flags);
+             dm->edofs, dm->cons, u, lam, m->n_elem, grad, ctx->g_flag);
   return check_launch("k_hex27_adjoint");
 }
 

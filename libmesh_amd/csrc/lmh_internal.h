@@ -95,7 +95,12 @@ struct lmh_context {
   double *d_part = nullptr;     // reduction partials
   unsigned *d_count = nullptr;  // last-block counters (zeroed, self-resetting)
   int *d_flags = nullptr;       // error flags
-  double *h_pinned = nullptr;   // pinned host scalars
+  // The map kernels' error flag, in pinned host memory: the host clears it before
+  // the launch (the stream is idle then: every call that uses it waits) and reads
+  // it after the wait, without a clear and a copy on the stream (Q1 10^3 assembly
+  // 34 -> 21 us, three Q2 40^3 gradient calls 240 -> 189 us).
+  int *h_flag = nullptr, *g_flag = nullptr;  // its host and device addresses
+  double *h_pinned = nullptr, *g_pinned = nullptr;  // pinned host scalars: host and device addresses
   hipEvent_t ev_poll[2] = {nullptr, nullptr};  // solver convergence polls
   void *cg_scratch = nullptr;   // this device's address of the allocation-free CG's scratch
   int n_part = 0;
@@ -306,6 +311,9 @@ int thread_residual(lmh_context *ctx, const FETable *t, const lmh_mesh *m, const
 int thread_qoi(lmh_context *ctx, const FETable *t, const lmh_mesh *m, double lo, double hi, double *Q);
 int thread_adjoint(lmh_context *ctx, const FETable *t, const lmh_mesh *m, const lmh_dofmap *dm, const double *u,
                    const double *lam, double *grad);
+
+// sets the host-memory error flag: a plain store, as host memory takes no atomic or
+__device__ inline void raise_flag(int *flag) { *(volatile int *)flag = 1; }
 
 // a value moved between lanes by a DPP control word
 template <int CTRL, typename T>

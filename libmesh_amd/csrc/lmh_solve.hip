@@ -1934,12 +1934,13 @@ int cg_scratch_setup(lmh_context *ctx) {
 }
 
 // The outcome of a CG whose last bank is K & 1, read back from the device scalars
-static int cg_result(lmh_matrix *A, int64_t K, int64_t maxits, int64_t *iters, double *rel_res, int *reason) {
+static int cg_result(lmh_matrix *A, int64_t K, int64_t maxits, int64_t *iters, double *rel_res, int *reason,
+                     bool copy = true) {
   lmh_context *ctx = A->ctx;
   double *S = ctx->d_scal, *snap = ctx->h_pinned;
-  // both banks and |b|^2 (G_BB follows the banks) into pinned memory
+  // (copy = false: the kernel wrote them there) both banks and |b|^2 (G_BB follows the banks) into pinned memory
   static_assert(G_BB < 64, "scalar slots beyond the pinned copy");
-  LMH_HIP(hipMemcpyAsync(snap, S, sizeof(double) * (G_BB + 1), hipMemcpyDeviceToHost, ctx->stream));
+  if (copy) LMH_HIP(hipMemcpyAsync(snap, S, sizeof(double) * (G_BB + 1), hipMemcpyDeviceToHost, ctx->stream));
   LMH_HIP(hipStreamSynchronize(ctx->stream));
   const double *Bk = snap + (K & 1) * B_SIZE, gbb = snap[G_BB];
   const bool conv = Bk[B_DONE] != 0.0;
@@ -1957,7 +1958,7 @@ static int cg_small(lmh_matrix *A, const double *b_d, double *x_d, double rtol, 
   auto launch = [&](auto kern) -> int {
     LMH_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kSmallLds));
     hipLaunchKernelGGL(kern, dim3(1), dim3(kSmallNT), kSmallLds, ctx->stream, (int)A->rows, A->rp, A->ci, A->vals, diag,
-                       jac, b_d, x_d, rtol, maxits, ctx->d_scal);
+                       jac, b_d, x_d, rtol, maxits, ctx->g_pinned);
     return LMH_OK;
   };
   const bool two = A->rows > kSmallNT, four = A->rows > 2 * kSmallNT;
@@ -1991,7 +1992,7 @@ static int cg_impl(lmh_matrix *A, const double *b_d, double *x_d, double rtol, i
   lmh_context *ctx = A->ctx;
   if (cg_small_fits(A, maxits)) {
     LMH_TRY((cg_small<NA>(A, b_d, x_d, rtol, maxits, diag)));
-    return cg_result(A, 0, maxits, iters, rel_res, reason);
+    return cg_result(A, 0, maxits, iters, rel_res, reason, false);
   }
   if (!NA) LMH_TRY(ensure_windows(A));
   const Stream st = stream_of(A, false);

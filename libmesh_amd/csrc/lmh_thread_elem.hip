@@ -101,7 +101,7 @@ __global__ __launch_bounds__(kTB) void k_thread_residual(const double *__restric
     for (int a = 0; a < N; ++a)
       R[a] += fl[0] * d[3 * a] + fl[1] * d[3 * a + 1] + fl[2] * d[3 * a + 2] - fj * phi[a];
   }
-  if (bad) atomicOr(err, 1);
+  if (bad) raise_flag(err);
 #pragma unroll
   for (int a = 0; a < N; ++a) Fe[e * N + a] = R[a];
 }
@@ -131,7 +131,7 @@ __global__ __launch_bounds__(kTB) void k_thread_qoi(const double *__restrict__ p
 #pragma unroll
     for (int a = 0; a < N; ++a) R[a] += jc * phi[a];
   }
-  if (bad) atomicOr(err, 1);
+  if (bad) raise_flag(err);
 #pragma unroll
   for (int a = 0; a < N; ++a) Q[e * N + a] = R[a];
 }
@@ -177,7 +177,7 @@ __global__ __launch_bounds__(kTB) void k_thread_adjoint(const double *__restrict
            (gl[0] * c[0][k] + gl[1] * c[1][k] + gl[2] * c[2][k]);
     s += P[0] / det * t;
   }
-  if (bad) atomicOr(err, 1);
+  if (bad) raise_flag(err);
   grad[e] = -s;
 }
 
@@ -242,7 +242,7 @@ __global__ __launch_bounds__(kTB) __attribute__((amdgpu_waves_per_eu(2))) void k
       for (int j = i; j < N; ++j, ++k) K[k] += v[0] * d[3 * j] + v[1] * d[3 * j + 1] + v[2] * d[3 * j + 2];
     }
   }
-  if (bad && live) atomicOr(err, 1);
+  if (bad && live) raise_flag(err);
   const int64_t left = (ne - e0 < kTB ? ne - e0 : kTB) * W;  // entries of this block of rows
 #pragma unroll
   for (int i0 = 0; i0 < N; i0 += R) {
@@ -274,10 +274,10 @@ static int residual_n(lmh_context *ctx, const FETable *t, const lmh_mesh *m, con
                       const double *kappa, int f_kind, const double *u, double *Fe) {
   if (f_kind == 0)
     LMH_LAUNCH(ctx, "element_residual", (k_thread_residual<N, 0>), te_grid(m->n_elem), dim3(kTB), 0, t->d_points(),
-               t->nq, m->xyz, m->conn, dm->edofs, kappa, u, m->n_elem, Fe, ctx->d_flags);
+               t->nq, m->xyz, m->conn, dm->edofs, kappa, u, m->n_elem, Fe, ctx->g_flag);
   else
     LMH_LAUNCH(ctx, "element_residual", (k_thread_residual<N, 1>), te_grid(m->n_elem), dim3(kTB), 0, t->d_points(),
-               t->nq, m->xyz, m->conn, dm->edofs, kappa, u, m->n_elem, Fe, ctx->d_flags);
+               t->nq, m->xyz, m->conn, dm->edofs, kappa, u, m->n_elem, Fe, ctx->g_flag);
   return check_launch("k_thread_residual");
 }
 
@@ -296,7 +296,7 @@ int thread_qoi(lmh_context *ctx, const FETable *t, const lmh_mesh *m, double lo,
   if (m->n_elem == 0) return LMH_OK;
 #define TE_QOI(N)                                                                                                   \
   LMH_LAUNCH(ctx, "qoi_box", k_thread_qoi<N>, te_grid(m->n_elem), dim3(kTB), 0, t->d_points(), t->nq, m->xyz, m->conn, \
-             m->n_elem, lo, hi, Q, ctx->d_flags)
+             m->n_elem, lo, hi, Q, ctx->g_flag)
   switch (t->n) {
     case 4: TE_QOI(4); break;
     case 8: TE_QOI(8); break;
@@ -312,7 +312,7 @@ int thread_adjoint(lmh_context *ctx, const FETable *t, const lmh_mesh *m, const 
   if (m->n_elem == 0) return LMH_OK;
 #define TE_ADJ(N)                                                                                                     \
   LMH_LAUNCH(ctx, "adjoint_kappa", k_thread_adjoint<N>, te_grid(m->n_elem), dim3(kTB), 0, t->d_points(), t->nq, m->xyz, \
-             m->conn, dm->edofs, dm->cons, u, lam, m->n_elem, grad, ctx->d_flags)
+             m->conn, dm->edofs, dm->cons, u, lam, m->n_elem, grad, ctx->g_flag)
   switch (t->n) {
     case 4: TE_ADJ(4); break;
     case 8: TE_ADJ(8); break;
@@ -329,11 +329,11 @@ static int poisson_n(lmh_context *ctx, const FETable *t, const lmh_mesh *m, cons
   if (f_kind == 0)
     LMH_LAUNCH(ctx, "element_thread", (k_thread_poisson<N, R, CT, 0>), te_grid(m->n_elem), dim3(kTB), 0,
                t->d_points(), t->nq, m->xyz, m->conn, dm->edofs, dm->cons, kappa, constrain, m->n_elem, Ke, Fe,
-               ctx->d_flags);
+               ctx->g_flag);
   else
     LMH_LAUNCH(ctx, "element_thread", (k_thread_poisson<N, R, CT, 1>), te_grid(m->n_elem), dim3(kTB), 0,
                t->d_points(), t->nq, m->xyz, m->conn, dm->edofs, dm->cons, kappa, constrain, m->n_elem, Ke, Fe,
-               ctx->d_flags);
+               ctx->g_flag);
   return check_launch("k_thread_poisson");
 }
 
