@@ -28,60 +28,65 @@ namespace lmh {
 
 constexpr int kTileSlots = 512, kTileRows = 64, kTileSteps = 16;  // steps whose loads are in flight together
 
-// Walks the incidence sequence of a tile: put(step slot, incidence, row) for
-// every entry in order, gaps skipped over; returns the padded length, whole
-// groups of kTileQuad steps.
+// Walks the incidence sequence of a tile, one wavefront with a row per lane:
+// put(step slot, incidence, row) in the lane of every entry, gap(slot) for every
+// gap; returns the padded length, whole groups of kTileQuad steps.  In round k the
+// rows that have a k-th incidence follow each other; where one of them is already
+// in the step that the last round left open, the rest begin the next step.
 constexpr int kTileQuad = 4;  // steps whose offsets a lane reads at once
-template <typename F>
-__device__ inline int tile_walk(const int32_t *__restrict__ inc_ptr, int32_t r0, int nr, int pi, F &&put) {
+template <typename F, typename H>
+__device__ inline int tile_walk(const int32_t *__restrict__ inc_ptr, int32_t r0, int nr, int pi, F &&put, H &&gap) {
+  const int lane = threadIdx.x & 63;
+  const uint64_t below = (1ull << lane) - 1;
+  const int32_t b = lane < nr ? inc_ptr[r0 + lane] : 0, cnt = lane < nr ? inc_ptr[r0 + lane + 1] - b : 0;
   int pos = 0;
-  int32_t recent[16];  // rows of the current step (pi <= 16)
-  int nrec = 0;
+  uint64_t open = 0;  // rows of the step that pos is in
   for (int k = 0;; ++k) {
-    bool any = false;
-    for (int r = 0; r < nr; ++r) {
-      const int32_t b = inc_ptr[r0 + r];
-      if (b + k >= inc_ptr[r0 + r + 1]) continue;
-      any = true;
-      if (pos % pi == 0) nrec = 0;
-      bool clash = false;
-      for (int c = 0; c < nrec; ++c) clash |= recent[c] == r;
-      if (clash) {  // next step
-        pos = (pos / pi + 1) * pi;
-        nrec = 0;
-      }
-      put(pos, b + k, r);
-      recent[nrec++] = r;
-      ++pos;
+    const bool on = cnt > k;
+    const uint64_t m = __ballot(on);
+    if (!m) break;
+    const int n = __popcll(m), rank = __popcll(m & below), left = pos % pi ? pi - pos % pi : pi;
+    const uint64_t clash = __ballot(on && rank < left && (open >> lane & 1));
+    int mine = pos + rank, next = pos + n;
+    if (clash) {
+      const int c = __popcll(m & ((clash & -clash) - 1)), step = (pos / pi + 1) * pi;
+      if (rank >= c) mine = step + rank - c;
+      next = step + n - c;
+      if (pos + c + lane < step) gap(pos + c + lane);
     }
-    if (!any) break;
+    if (on) put(mine, b + k, lane);
+    const uint64_t same = __ballot(on && mine / pi == next / pi);
+    open = next % pi == 0 ? 0 : pos / pi == next / pi ? open | same : same;
+    pos = next;
   }
-  const int q = pi * kTileQuad;
-  return (pos + q - 1) / q * q;
+  const int q = pi * kTileQuad, len = (pos + q - 1) / q * q;
+  if (pos + lane < len) gap(pos + lane);  // q <= 64
+  return len;
 }
 
-__global__ __launch_bounds__(64) void k_tile_count(const int32_t *__restrict__ inc_ptr,
-                                                   const int32_t *__restrict__ tr, int64_t nt, int pi,
-                                                   int32_t *__restrict__ len) {
-  for (int64_t t = blockIdx.x * (int64_t)64 + threadIdx.x; t < nt; t += (int64_t)gridDim.x * 64)
-    len[t] = tile_walk(inc_ptr, tr[t], tr[t + 1] - tr[t], pi, [](int, int32_t, int) {});
+__global__ __launch_bounds__(256) void k_tile_count(const int32_t *__restrict__ inc_ptr,
+                                                    const int32_t *__restrict__ tr, int64_t nt, int pi,
+                                                    int32_t *__restrict__ len) {
+  for (int64_t t = blockIdx.x * (int64_t)4 + (threadIdx.x >> 6); t < nt; t += (int64_t)gridDim.x * 4) {
+    const int l = tile_walk(
+        inc_ptr, tr[t], tr[t + 1] - tr[t], pi, [](int, int32_t, int) {}, [](int) {});
+    if ((threadIdx.x & 63) == 0) len[t] = l;
+  }
 }
 
 // seq: {incidence (element * dpe + local row) or -1, entry base | row << 16}, within the tile
-__global__ __launch_bounds__(64) void k_tile_fill(const int32_t *__restrict__ inc_ptr,
-                                                  const int32_t *__restrict__ inc, const int32_t *__restrict__ rp,
-                                                  const int32_t *__restrict__ tr, const int32_t *__restrict__ start,
-                                                  int64_t nt, int pi, int2 *__restrict__ seq,
-                                                  int4 *__restrict__ tile) {
-  for (int64_t t = blockIdx.x * (int64_t)64 + threadIdx.x; t < nt; t += (int64_t)gridDim.x * 64) {
+__global__ __launch_bounds__(256) void k_tile_fill(const int32_t *__restrict__ inc_ptr,
+                                                   const int32_t *__restrict__ inc, const int32_t *__restrict__ rp,
+                                                   const int32_t *__restrict__ tr, const int32_t *__restrict__ start,
+                                                   int64_t nt, int pi, int2 *__restrict__ seq,
+                                                   int4 *__restrict__ tile) {
+  for (int64_t t = blockIdx.x * (int64_t)4 + (threadIdx.x >> 6); t < nt; t += (int64_t)gridDim.x * 4) {
     const int32_t r0 = tr[t], nr = tr[t + 1] - r0, s0 = start[t], b0 = rp[r0];
-    int at = 0;
-    const int len = tile_walk(inc_ptr, r0, nr, pi, [&](int pos, int32_t k, int r) {
-      for (; at < pos; ++at) seq[s0 + at] = make_int2(-1, 0);
-      seq[s0 + at++] = make_int2(inc[k], (rp[r0 + r] - b0) | (r << 16));
-    });
-    for (; at < len; ++at) seq[s0 + at] = make_int2(-1, 0);
-    tile[t] = make_int4(r0, nr, s0, len / pi);
+    const int len = tile_walk(
+        inc_ptr, r0, nr, pi,
+        [&](int pos, int32_t k, int r) { seq[s0 + pos] = make_int2(inc[k], (rp[r0 + r] - b0) | (r << 16)); },
+        [&](int pos) { seq[s0 + pos] = make_int2(-1, 0); });
+    if ((threadIdx.x & 63) == 0) tile[t] = make_int4(r0, nr, s0, len / pi);
   }
 }
 
@@ -209,15 +214,15 @@ int matrix_build_tiles(lmh_matrix *A, const std::vector<int32_t> &h_rp) {
   int32_t *dtr = tmp, *len = tmp + nt + 1, *start = len + nt + 1;
   LMH_HIP(hipMemcpyAsync(dtr, tr.data(), sizeof(int32_t) * tr.size(), hipMemcpyHostToDevice, ctx->stream));
   LMH_HIP(hipMemsetAsync(len, 0, sizeof(int32_t) * (nt + 1), ctx->stream));
-  const int g = grid_for(nt, 64, 16384);
-  LMH_LAUNCH(ctx, "tile_plan", k_tile_count, dim3(g), dim3(64), 0, dm->inc_ptr, (const int32_t *)dtr, nt, pi,
+  const int g = grid_for(nt, 4, 16384);
+  LMH_LAUNCH(ctx, "tile_plan", k_tile_count, dim3(g), dim3(256), 0, dm->inc_ptr, (const int32_t *)dtr, nt, pi,
              len);
   LMH_TRY(check_launch("k_tile_count"));
   int64_t total = 0;
   LMH_TRY(exclusive_scan_i32(ctx, len, start, nt, &total));
   LMH_HIP(hipMalloc((void **)&A->st_tile, sizeof(int4) * nt));
   LMH_HIP(hipMalloc((void **)&A->st_seq, sizeof(int2) * std::max<int64_t>(1, total)));
-  LMH_LAUNCH(ctx, "tile_plan", k_tile_fill, dim3(g), dim3(64), 0, dm->inc_ptr, dm->inc, A->rp,
+  LMH_LAUNCH(ctx, "tile_plan", k_tile_fill, dim3(g), dim3(256), 0, dm->inc_ptr, dm->inc, A->rp,
              (const int32_t *)dtr, (const int32_t *)start, nt, pi, A->st_seq, A->st_tile);
   LMH_TRY(check_launch("k_tile_fill"));
   const bool wide = A->max_row > 256;
