@@ -1541,8 +1541,20 @@ static Stream stream_of(lmh_matrix *A, bool fp32) {
   s.on = A->idx16_state == 1;
   s.nt = s.on && A->wbits == 8 ? W8_NT : BLK;
   s.grid = s.on && A->wbits == 8 ? W8_GRID * gs : gs;
-  // at most one workgroup per row block (whole XCD rounds)
-  s.grid = (int)std::min<int64_t>(s.grid, ((s.on ? A->nrbw : A->nrb) + NXCD - 1) / NXCD * NXCD);
+  // At most one workgroup per row block (whole XCD rounds).  Up to four rounds of
+  // what a GPU holds at once, a workgroup takes as many blocks as there are
+  // rounds: it loads one while it sums the last, and its consumers read fewer
+  // partial sums.  Q2 20^3 (4,050 blocks) BiCGSTAB 6.8 -> 6.4 ms a solve, Q2 24^3 CG
+  // 7.69 -> 7.32, mixed 7.68 -> 7.37, Q1 50^3 CG 4.82 -> 4.63, TET4 40^3 products 49 ->
+  // 43 us; one round (Q2 12^3) 2.6 ms either way, and two rounds for it 2.8;
+  // beyond four rounds (Q2 30^3 and up) the full grid measures the same.
+  const int64_t nb = s.on ? A->nrbw : A->nrb, resident = (int64_t)A->ctx->cu_count * (s.nt == W8_NT ? 10 : 5);
+  int64_t want = nb;
+  if (nb <= 4 * resident) {
+    const int64_t rounds = std::max<int64_t>(1, (nb + resident - 1) / resident);
+    want = (nb + rounds - 1) / rounds;
+  }
+  s.grid = (int)std::min<int64_t>(s.grid, (want + NXCD - 1) / NXCD * NXCD);
   if (use_windows(A) && A->cols < ((int64_t)1 << 29)) {
     s.iw = A->wbits / 8;
     s.idx = fp32 ? A->widx32 : A->widx64;
