@@ -298,19 +298,28 @@ __global__ __launch_bounds__(64) void k_hex27_adjoint(const double *__restrict__
 //   T (4 x 3, by the kind of direction 1's factors: dd, dp, pd, pp)
 //                = direction 2 contracted, lane (i2, j2) x (i3, j3), S through LDS
 //   K = direction 1 contracted in registers, nine entries (i1, j1) per lane,
-// each written with its mirror to an LDS tile that leaves as coalesced stores.
+// each written with its mirror to an LDS tile that leaves as 16-byte stores.
 // 195 multiply-adds per lane instead of the 84 16x16x4 matrix instructions
 // (86,000 multiply-adds with their padding) of the table contraction this
 // replaces, which also formed its operands from nine LDS reads per k-step.
 // FP64 throughout; the FP32 operator is the FP64 entry rounded once.
-// Bound by LDS reads and their latency at two wavefronts per SIMD (248
-// registers, 16.4 KB of LDS); 262,144 elements: FP64 1545 -> 633 us, FP32
-// 1258 -> 600 us.  Three wavefronts per SIMD (168 registers, geometry of five
-// elements) spill: 806 us; the next element's S ahead of this one's T: 256
-// registers and 350 bytes of spills, 913 us.
+// Bound by LDS reads and their latency: S is read array by array, a column set in
+// five 16-byte reads (nine 8-byte reads of all arrays held at once took 250
+// registers, two wavefronts per SIMD: FP64 633, FP32 600 us).  262,144 elements:
+// FP64 1545 -> 577 us, FP32 1258 -> 473 us.  The next element's S ahead of this
+// one's T: 256 registers and 350 bytes of spills, 913 us.
 // ---------------------------------------------------------------------------
+// Elements whose geometry a wavefront forms together and wavefronts per CU that
+// fit (168 registers, LDS).  FP64: 7 and 9; six elements let twelve in, whose
+// stores then get in each other's way (64^3 724 us against 577).  FP32: 6 and 12
+// (473 us; 491 with 7 and 10).
+template <typename CT>
+struct H27Group {
+  static constexpr int per = sizeof(CT) == 8 ? 7 : 6, waves = sizeof(CT) == 8 ? 9 : 12,
+                       grid = sizeof(CT) == 8 ? 20 : 12;  // workgroups per CU
+};
 template <typename CT, int FK>
-__global__ __launch_bounds__(64, 2) void k_hex27_poisson(const double *__restrict__ xyz,
+__global__ __launch_bounds__(64, 3) void k_hex27_poisson(const double *__restrict__ xyz,
                                                          const int32_t *__restrict__ conn,
                                                          const int32_t *__restrict__ edofs,
                                                          const uint8_t *__restrict__ cons,
@@ -319,9 +328,9 @@ __global__ __launch_bounds__(64, 2) void k_hex27_poisson(const double *__restric
                                                          int *__restrict__ err) {
   constexpr int NF = 3, ST = 27 * NF;
   // node coordinates of the group; then, per element, S and the matrix tile
-  __shared__ double s_buf[sizeof(CT) == 8 ? 729 : kH27PerWave * ST];
-  __shared__ double s_m[kH27PerWave * 162];  // M[el][6 components][q3][q1q2]
-  __shared__ double s_h[kH27PerWave * 27];
+  __shared__ __attribute__((aligned(16))) double s_buf[sizeof(CT) == 8 ? 730 : kH27PerWave * ST];
+  __shared__ double s_m[H27Group<CT>::per * 162];  // M[el][6 components][q3][q1q2]
+  double *s_h = s_buf;  // over the coordinates: a wavefront's lanes have all read them by then
   const int lane = threadIdx.x;
   const H27Slots sl(lane);
   // the matrix lanes: pair (i3, j3) of c, pair (i2, j2) of k
@@ -456,27 +465,42 @@ __global__ __launch_bounds__(64, 2) void k_hex27_poisson(const double *__restric
           S[7] += dd * m33;
         }
 #pragma unroll
-        for (int k = 0; k < 8; ++k) s_buf[54 * k + lane] = S[k];
+        for (int k = 0; k < 8; ++k) s_buf[60 * k + 10 * cc + kk] = S[k];
       }
       h27_sync();
       double K[3][3];
       if (lane < 54) {
-        const double *S = s_buf + 9 * cc;
+        // an array's nine columns (and a pad) in five 16-byte reads, array by array
+        typedef double d2 __attribute__((ext_vector_type(2)));
+        double T[3][4] = {{0, 0, 0, 0}, {0, 0, 0, 0}, {0, 0, 0, 0}};  // [q1][dd, dp, pd, pp]
+        auto array = [&](int k, auto &&add) {
+          double S[10];
+#pragma unroll
+          for (int u = 0; u < 5; ++u) {
+            const d2 w = *(const d2 *)(s_buf + 60 * k + 10 * cc + 2 * u);
+            S[2 * u] = w[0];
+            S[2 * u + 1] = w[1];
+          }
+#pragma unroll
+          for (int q2 = 0; q2 < 3; ++q2)
+#pragma unroll
+            for (int q1 = 0; q1 < 3; ++q1) add(T[q1], q2, S[3 * q2 + q1]);
+        };
+        array(0, [&](double(&t)[4], int q, double s) { t[0] += pi2[q] * pj2[q] * s; });
+        array(1, [&](double(&t)[4], int q, double s) {
+          t[1] += pi2[q] * dj2[q] * s;
+          t[2] += di2[q] * pj2[q] * s;
+        });
+        array(2, [&](double(&t)[4], int q, double s) { t[3] += di2[q] * dj2[q] * s; });
+        array(3, [&](double(&t)[4], int q, double s) { t[1] += pi2[q] * pj2[q] * s; });
+        array(4, [&](double(&t)[4], int q, double s) { t[2] += pi2[q] * pj2[q] * s; });
+        array(5, [&](double(&t)[4], int q, double s) { t[3] += di2[q] * pj2[q] * s; });
+        array(6, [&](double(&t)[4], int q, double s) { t[3] += pi2[q] * dj2[q] * s; });
+        array(7, [&](double(&t)[4], int q, double s) { t[3] += pi2[q] * pj2[q] * s; });
         double K0[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}};
 #pragma unroll
         for (int q1 = 0; q1 < 3; ++q1) {
-          double tdd = 0, tdp = 0, tpd = 0, tpp = 0;
-#pragma unroll
-          for (int q2 = 0; q2 < 3; ++q2) {
-            const int q = 3 * q2 + q1;
-            const double pp = pi2[q2] * pj2[q2], pd = pi2[q2] * dj2[q2], dp = di2[q2] * pj2[q2],
-                         dd = di2[q2] * dj2[q2];
-            const double s12 = S[54 + q];
-            tdd += pp * S[q];
-            tdp += pd * s12 + pp * S[162 + q];
-            tpd += dp * s12 + pp * S[216 + q];
-            tpp += dd * S[108 + q] + dp * S[270 + q] + pd * S[324 + q] + pp * S[378 + q];
-          }
+          const double tdd = T[q1][0], tdp = T[q1][1], tpd = T[q1][2], tpp = T[q1][3];
 #pragma unroll
           for (int j = 0; j < 3; ++j) {
             const double u = h27_d(q1, j) * tdd + h27_p(q1, j) * tdp, v = h27_d(q1, j) * tpd + h27_p(q1, j) * tpp;
@@ -507,9 +531,14 @@ __global__ __launch_bounds__(64, 2) void k_hex27_poisson(const double *__restric
       }
       h27_sync();
       CT *out = Ke + (e0 + el) * 729;
+      constexpr int V = 16 / sizeof(CT), NV = 729 / V;  // 16-byte pieces, and the last entry
+      typedef CT vt __attribute__((ext_vector_type(V)));
+      typedef vt vtu __attribute__((aligned(sizeof(CT))));
 #pragma unroll
-      for (int k = 0; k < 12; ++k)
-        if (k < 11 || lane < 729 - 64 * 11) out[64 * k + lane] = tile[64 * k + lane];
+      for (int k = 0; k < (NV + 63) / 64; ++k)
+        if (64 * k + 63 < NV || 64 * k + lane < NV)
+          *(vtu *)(out + V * (64 * k + lane)) = *(const vt *)(tile + V * (64 * k + lane));
+      if (lane == 0) out[728] = tile[728];
       h27_sync();
     }
   }
@@ -524,10 +553,11 @@ int hex27_poisson(lmh_context *ctx, const lmh_mesh *m, const lmh_dofmap *dm, con
                   int constrain, CT *Ke, double *Fe) {
   const int64_t ne = m->n_elem;
   if (ne == 0) return LMH_OK;
-  // seven elements share the geometry lanes; fewer while that leaves wavefronts
-  // unused (8 per CU)
-  const int per = (int)std::min<int64_t>(kH27PerWave, std::max<int64_t>(1, ne / (ctx->cu_count * 8)));
-  const int g = grid_for((ne + per - 1) / per, 1, ctx->cu_count * 9);
+  // as many elements share the geometry lanes as one round of wavefronts takes (Q2
+  // 20^3: 36 us with whole groups in two rounds, 30 in one)
+  const int64_t waves = (int64_t)ctx->cu_count * H27Group<CT>::waves;
+  const int per = (int)std::min<int64_t>(H27Group<CT>::per, (ne + waves - 1) / waves);
+  const int g = grid_for((ne + per - 1) / per, 1, ctx->cu_count * H27Group<CT>::grid);
   const char *name = sizeof(CT) == 8 ? "element_hex27_fp64" : "element_hex27_fp32";
   if (f_kind == 0)
     LMH_LAUNCH(ctx, name, (k_hex27_poisson<CT, 0>), dim3(g), dim3(64), 0, m->xyz, m->conn, dm->edofs,
