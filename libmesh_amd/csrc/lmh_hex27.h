@@ -112,6 +112,7 @@ __device__ inline void h27_refgrad(const double *F, const H27Lane &L, double (&g
         }
         if (h27_d(q, i3) != 0.0) g[q][f][2] += h27_d(q, i3) * a2[f];
       }
+    __builtin_amdgcn_sched_barrier(0);  // one plane's nodes in registers at a time
   }
 }
 

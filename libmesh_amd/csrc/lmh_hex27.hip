@@ -305,14 +305,16 @@ __global__ __launch_bounds__(64) void k_hex27_adjoint(const double *__restrict__
 // FP64 throughout; the FP32 operator is the FP64 entry rounded once.
 // Bound by LDS reads and their latency: S is read array by array, a column set in
 // five 16-byte reads (nine 8-byte reads of all arrays held at once took 250
-// registers, two wavefronts per SIMD: FP64 633, FP32 600 us).  262,144 elements:
-// FP64 1545 -> 577 us, FP32 1258 -> 473 us.  The next element's S ahead of this
-// one's T: 256 registers and 350 bytes of spills, 913 us.
+// registers, two wavefronts per SIMD: FP64 633, FP32 600 us), and what a phase
+// needs is formed in it, not kept across (lane constants and the next group's
+// indices in registers spilled 116 bytes a lane: 580 and 480 us; 28 bytes are
+// left).  262,144 elements: FP64 1545 -> 543 us, FP32 1258 -> 448 us.  The next
+// element's S ahead of this one's T: 256 registers and 350 bytes of spills, 913 us.
 // ---------------------------------------------------------------------------
 // Elements whose geometry a wavefront forms together and wavefronts per CU that
 // fit (168 registers, LDS).  FP64: 7 and 9; six elements let twelve in, whose
 // stores then get in each other's way (64^3 724 us against 577).  FP32: 6 and 12
-// (473 us; 491 with 7 and 10).
+// (64^3 473 us; 491 with 7 and 10).
 template <typename CT>
 struct H27Group {
   static constexpr int per = sizeof(CT) == 8 ? 7 : 6, waves = sizeof(CT) == 8 ? 9 : 12,
@@ -332,33 +334,21 @@ __global__ __launch_bounds__(64, 3) void k_hex27_poisson(const double *__restric
   __shared__ double s_m[H27Group<CT>::per * 162];  // M[el][6 components][q3][q1q2]
   double *s_h = s_buf;  // over the coordinates: a wavefront's lanes have all read them by then
   const int lane = threadIdx.x;
-  const H27Slots sl(lane);
   // the matrix lanes: pair (i3, j3) of c, pair (i2, j2) of k
   const int t54 = lane < 54 ? lane : 0, cc = t54 / 9, kk = t54 - 9 * cc;
   const int i3 = cc < 3 ? cc : (cc == 5 ? 1 : 0), j3 = cc < 3 ? cc : (cc == 3 ? 1 : 2);
   const int i2 = kk % 3, j2 = kk / 3;
-  int ni[3], nj[3];  // local nodes of the lane's rows (i1, i2, i3) and columns (j1, j2, j3)
-#pragma unroll
-  for (int i = 0; i < 3; ++i) {
-    ni[i] = kH27Node[9 * i3 + 3 * i2 + i];
-    nj[i] = kH27Node[9 * j3 + 3 * j2 + i];
-  }
   const int64_t total = ne * 27, groups = (ne + per - 1) / per;
-  int32_t nd[3], dof[3];
-  sl.ids(conn, (int64_t)blockIdx.x * per, total, lane, nd);
-  sl.ids(edofs, (int64_t)blockIdx.x * per, total, lane, dof);
   for (int64_t gr = blockIdx.x; gr < groups; gr += gridDim.x) {
     // lane constants of this phase: formed again for every group (the opaque
     // lane index keeps the compiler from holding both phases' in registers)
     int lg = lane;
     asm volatile("" : "+v"(lg));
+    const H27Slots sl(lg);
+    int32_t nd[3], dof[3];
+    sl.ids(conn, gr * per, total, lane, nd);
+    sl.ids(edofs, gr * per, total, lane, dof);
     const H27Lane L(lg);
-    double pt[3], pt2[3];
-#pragma unroll
-    for (int q = 0; q < 3; ++q) {
-      pt[q] = h27_pick(L.l % 3, [&](int i) { return h27_p(q, i); });
-      pt2[q] = h27_pick(L.l / 3, [&](int i) { return h27_p(q, i); });
-    }
     const int64_t e0 = gr * per;
     const int cnt = (int)(ne - e0 < per ? ne - e0 : per);
     unsigned long long bits[3];  // constrained flags, bit 27 el + node of the group
@@ -375,8 +365,6 @@ __global__ __launch_bounds__(64, 3) void k_hex27_poisson(const double *__restric
       }
       bits[m] = constrain ? __ballot(c && sl.live[m]) : 0ull;
     }
-    sl.ids(conn, (gr + gridDim.x) * per, total, lane, nd);
-    sl.ids(edofs, (gr + gridDim.x) * per, total, lane, dof);
     auto mask_of = [&](int el) -> unsigned {  // 27 flags of element el, by local node
       const int b = 27 * el, w = b >> 6, o = b & 63;
       unsigned long long v = bits[0];
@@ -413,6 +401,7 @@ __global__ __launch_bounds__(64, 3) void k_hex27_poisson(const double *__restric
         if constexpr (FK != 0) fj *= forcing(FK, pos[q][0], pos[q][1], pos[q][2]);
 #pragma unroll
         for (int i = 0; i < 3; ++i) h[i] += h27_p(q, i) * fj;
+        __builtin_amdgcn_sched_barrier(0);
       }
 #pragma unroll
       for (int i = 0; i < 3; ++i) s_h[L.el * 27 + 9 * i + L.l] = h[i];
@@ -420,6 +409,12 @@ __global__ __launch_bounds__(64, 3) void k_hex27_poisson(const double *__restric
     h27_sync();
     if (on) {
       const unsigned cm = mask_of(L.el);
+      double pt[3], pt2[3];
+#pragma unroll
+      for (int q = 0; q < 3; ++q) {
+        pt[q] = h27_pick(L.l % 3, [&](int i) { return h27_p(q, i); });
+        pt2[q] = h27_pick(L.l / 3, [&](int i) { return h27_p(q, i); });
+      }
 #pragma unroll
       for (int i = 0; i < 3; ++i) {
         const double *H = s_h + L.el * 27 + 9 * i;
@@ -433,6 +428,12 @@ __global__ __launch_bounds__(64, 3) void k_hex27_poisson(const double *__restric
     }
     int a3 = i3, b3 = j3, a2 = i2, b2 = j2;
     asm volatile("" : "+v"(a3), "+v"(b3), "+v"(a2), "+v"(b2));
+  int ni[3], nj[3];  // local nodes of the lane's rows (i1, i2, i3) and columns (j1, j2, j3)
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      ni[i] = kH27Node[9 * a3 + 3 * a2 + i];
+      nj[i] = kH27Node[9 * b3 + 3 * b2 + i];
+    }
     double pi3[3], di3[3], pj3[3], dj3[3], pi2[3], di2[3], pj2[3], dj2[3];
 #pragma unroll
     for (int q = 0; q < 3; ++q) {
