@@ -30,7 +30,6 @@ METRIC = "Mdof/s assembly + CG time to 1e-10 (mixed vs FP64), Q2 hex 2.1M dof, 1
 SEED_PERTURB = 0x5EED0001
 SEED_KAPPA = 0x5EED0002
 HBM_PEAK_GBS = 8000.0
-MFMA_PEAK_TFLOPS = {"fp64": 78.6, "fp32": 157.3}
 # hardware-counter summary of the dominant kernel at the 64^3 workload
 TRAFFIC_SUMMARY = os.path.join(ROOT, "profiles", "k_it_spmv16_hex27_64cube_pmc.txt")
 
@@ -56,9 +55,9 @@ def spmv_symbol(L, g, fp64):
     windows with 8- or 16-bit indices, or int32 columns)."""
     bits = L.hip().lmh_matrix_window_bits(g.matrix)
     if bits == 8:
-        return f"lmh::k_it_spmv16{'d' if fp64 else ''}<1024, 1, 128>"
+        return f"lmh::k_it_spmv16<{'double' if fp64 else 'float'}, 1024, 1, 128>"
     if bits == 16:
-        return f"lmh::k_it_spmv16{'d' if fp64 else ''}<2048, 2, 256>"
+        return f"lmh::k_it_spmv16<{'double' if fp64 else 'float'}, 2048, 2, 256>"
     return f"lmh::k_it_spmv<{'double' if fp64 else 'float'}>"
 
 
@@ -567,9 +566,9 @@ def main():
 
     def step(mode):
         """mode fp64: FP64 assembly + FP64 CG.  mixed: FP64 assembly, FP32 inner
-        operator rounded from it, mixed solve.  mixed_mfma32: FP64 assembly for
-        the outer residual operator plus an FP32 assembly of the inner operator,
-        mixed solve."""
+        operator rounded from it, mixed solve.  mixed_mfma32 (its name
+        from earlier lines): FP64 assembly for the outer residual operator plus an
+        FP32 assembly of the inner operator, mixed solve."""
         x.zero()
         ctx.sync()
         ta = time.perf_counter()
@@ -661,7 +660,6 @@ def main():
         "qoi_derivative_ms": round(qd_ms, 4),
         "adjoint_solve_iterations": int(a_its),
         "backward_kernel_ms": round(gk_ms, 4),
-        "backward_kernel_tflops_fp64": round(9.7e9 / (gk_ms * 1e-3) / 1e12, 3),
         "J": J,
         "homogeneity_rel_err": abs(float(kappa @ gh) + J) / abs(J),
     }
@@ -723,8 +721,8 @@ def main():
     alg = spmv_bytes(nnz, N, 4)
     achieved = alg / (working_ms(mx) * 1e-3) / 1e9
     alg64 = spmv_bytes(nnz, N, 8)
-    ach64 = alg64 / (working_ms(results["fp64"]) * 1e-3) / 1e9
-    flops_contract = 27 * 27 * 27 * 3 * 2 * p.n_elem
+    w64 = working_ms(results["fp64"])  # 0: a system solved by one kernel has no product launches
+    ach64 = alg64 / (w64 * 1e-3) / 1e9 if w64 else 0.0
     traffic = read_traffic(TRAFFIC_SUMMARY) if args.n == 64 else None
     out = {
         "metric": METRIC,
@@ -776,21 +774,21 @@ def main():
         "fp64_spmv_roofline": {"kernel_symbol": spmv_symbol(L, g, fp64=True), "achieved": round(ach64, 1),
                                "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(ach64 / HBM_PEAK_GBS, 4),
                                "algorithmic_bytes": alg64,
-                               "avg_working_launch_ms": round(working_ms(results["fp64"]), 5)},
+                               "avg_working_launch_ms": round(w64, 5)},
         "assembly_kernels_ms": {k: round(v, 4) for k, v in asm_k.items()},
         "adjoint": adjoint,
         "constrained": constrained,
         "condensed": condensed,
         "fem_residual_ms": fem_residual,
-        "contraction_gflop": flops_contract / 1e9,
         "setup_s": round(t_setup, 3),
     }
-    for prec in ("fp64", "fp32"):
+    for prec, vb in (("fp64", 8), ("fp32", 4)):
         k = f"element_hex27_{prec}"
-        if k in asm_k:
-            tf = flops_contract / (asm_k[k] * 1e-3) / 1e12
-            out[f"contraction_tflops_{prec}"] = round(tf, 3)
-            out[f"contraction_frac_of_{prec}_peak"] = round(tf / MFMA_PEAK_TFLOPS[prec], 4)
+        if k in asm_k:  # element matrices and vectors written, nodes and DoFs read
+            eb = (27 * 27 * vb + 27 * 8 + 2 * 27 * 4) * p.n_elem + 24 * p.n_nodes
+            gbs = eb / (asm_k[k] * 1e-3) / 1e9
+            out[f"element_roofline_{prec}"] = {"achieved": round(gbs, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
+                                               "frac": round(gbs / HBM_PEAK_GBS, 4), "compulsory_bytes": eb}
     for prec, vb in (("fp64", 8), ("fp32", 4)):
         k = f"scatter_{'gather' if args.scatter == 'gather' else 'colored'}_{prec}"
         if k in asm_k:

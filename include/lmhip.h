@@ -178,8 +178,8 @@ int lmh_vector_add_element_vectors(lmh_context *ctx, double *v_d, int64_t n_elem
  * numeric_vector.C:690-697).  Overwrites the matrix values and rhs_d.
  * kappa_d: per-element coefficient (NULL -> 1); f_kind 0: f = 1, 1: f =
  * 3 pi^2 sin(pi x) sin(pi y) sin(pi z).  precision LMH_FP64 builds the FP64
- * CSR; LMH_FP32 runs the element contraction in FP32 on MFMA and writes the
- * FP32 operator used by the mixed-precision inner solver (geometry stays FP64).
+ * CSR; LMH_FP32 writes the FP32 operator used by the mixed-precision inner
+ * solver (geometry stays FP64).
  * scatter: LMH_SCATTER_COLORED or LMH_SCATTER_GATHER.  rhs_d may be NULL
  * (matrix only).  The rhs of an FP32 assembly equals the FP64 one except for
  * the K H terms of nonzero constraint values, formed from the FP32 element
