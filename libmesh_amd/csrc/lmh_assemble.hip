@@ -316,14 +316,32 @@ __global__ void k_check_range(const int32_t *__restrict__ v, int64_t n, int64_t 
     if (v[t] < 0 || v[t] >= hi) atomicOr(err, 2);
 }
 
+// s + Fe over the incidences k0 .. k1 - 1, in order: four at a time, so that a
+// row waits for its list and its values once per four (40^3 Q2, 531,441 rows of 1
+// to 8 incidences: 17.0 us one by one, now 11.3).  Past the end the last one
+// is read again and dropped.
+__device__ inline double incidence_sum(const int32_t *__restrict__ inc, const double *__restrict__ Fe, int32_t k0,
+                                       int32_t k1, double s) {
+  constexpr int U = 4;
+  for (int32_t k = k0; k < k1; k += U) {
+    int32_t at[U];
+    double f[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) at[u] = inc[k + u < k1 ? k + u : k1 - 1];
+#pragma unroll
+    for (int u = 0; u < U; ++u) f[u] = Fe[at[u]];
+#pragma unroll
+    for (int u = 0; u < U; ++u) s = k + u < k1 ? s + f[u] : s;
+  }
+  return s;
+}
+
 __global__ void k_add_vec_gather(const int32_t *__restrict__ inc_ptr, const int32_t *__restrict__ inc, int64_t n_rows,
                                  const double *__restrict__ Fe, double *__restrict__ v) {
   for (int64_t r = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; r < n_rows; r += (int64_t)gridDim.x * blockDim.x) {
     const int32_t k0 = inc_ptr[r], k1 = inc_ptr[r + 1];
     if (k0 == k1) continue;
-    double s = v[r];
-    for (int32_t k = k0; k < k1; ++k) s += Fe[inc[k]];
-    v[r] = s;
+    v[r] = incidence_sum(inc, Fe, k0, k1, v[r]);
   }
 }
 
@@ -336,8 +354,7 @@ __global__ __launch_bounds__(256) void k_sum_vec_gather(const int32_t *__restric
                                                         const double *__restrict__ Fe, double *__restrict__ v) {
   for (int64_t r = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; r < n_rows; r += (int64_t)gridDim.x * blockDim.x) {
     const int32_t k0 = inc_ptr[r], k1 = inc_ptr[r + 1];
-    double s = 0.0;
-    for (int32_t k = k0; k < k1; ++k) s += Fe[inc[k]];
+    const double s = incidence_sum(inc, Fe, k0, k1, 0.0);
     v[r] = MASK && cons[r] ? 0.0 : s;
   }
 }
