@@ -72,8 +72,8 @@ struct H27Lane {
 
 // Reference gradients of NF nodal fields at the lane's three points:
 // g[q3][f][r] = sum_a F_a dphi_a/dxi_r, fields in lattice order in LDS
-// (F[lat * NF + f]); with NV > 0 also the values v[q3][f] of the first NV.
-template <int NF, int NV>
+// (F[lat * ST + f]); with NV > 0 also the values v[q3][f] of the first NV.
+template <int NF, int NV, int ST = NF>
 __device__ inline void h27_refgrad(const double *F, const H27Lane &L, double (&g)[3][NF][3],
                                    double (&v)[3][NV > 0 ? NV : 1]) {
 #pragma unroll
@@ -94,9 +94,9 @@ __device__ inline void h27_refgrad(const double *F, const H27Lane &L, double (&g
     for (int i2 = 0; i2 < 3; ++i2)
 #pragma unroll
       for (int f = 0; f < NF; ++f) {
-        const double *x = F + (9 * i3 + 3 * i2) * NF + f;
-        const double p = L.p1[0] * x[0] + L.p1[1] * x[NF] + L.p1[2] * x[2 * NF];
-        const double d = L.d1[0] * x[0] + L.d1[1] * x[NF] + L.d1[2] * x[2 * NF];
+        const double *x = F + (9 * i3 + 3 * i2) * ST + f;
+        const double p = L.p1[0] * x[0] + L.p1[1] * x[ST] + L.p1[2] * x[2 * ST];
+        const double d = L.d1[0] * x[0] + L.d1[1] * x[ST] + L.d1[2] * x[2 * ST];
         a0[f] += L.p2[i2] * d;
         a1[f] += L.d2[i2] * p;
         a2[f] += L.p2[i2] * p;
@@ -127,6 +127,35 @@ __device__ inline double cofactors(const double (&J)[3][3], double (&c)[3][3]) {
     c[r][2] = a[0] * b[1] - a[1] * b[0];
   }
   return J[0][0] * c[0][0] + J[0][1] * c[0][1] + J[0][2] * c[0][2];
+}
+
+// M[q3] = w / det C C^T (components 11, 12, 13, 22, 23, 33; C the cofactor rows) and
+// det at the lane's three points, from the coordinates' reference gradients; w(q3)
+// is the point's factor.  The gradients need not outlive it.
+template <typename W>
+__device__ inline void h27_metric(const double (&g)[3][3][3], W &&w, double (&M)[3][6], double (&det)[3], int *err) {
+#pragma unroll
+  for (int q = 0; q < 3; ++q) {
+    double J[3][3], c[3][3];
+#pragma unroll
+    for (int r = 0; r < 3; ++r)
+#pragma unroll
+      for (int k = 0; k < 3; ++k) J[r][k] = g[q][k][r];
+    det[q] = cofactors(J, c);
+    if (!(det[q] > 0.0)) raise_flag(err);
+    const double s = w(q) / det[q];
+    int m = 0;
+#pragma unroll
+    for (int r = 0; r < 3; ++r)
+#pragma unroll
+      for (int k = r; k < 3; ++k, ++m) M[q][m] = s * (c[r][0] * c[k][0] + c[r][1] * c[k][1] + c[r][2] * c[k][2]);
+  }
+}
+// M v for such a point
+__device__ inline void h27_apply(const double (&M)[6], const double (&v)[3], double (&y)[3]) {
+  y[0] = M[0] * v[0] + M[1] * v[1] + M[2] * v[2];
+  y[1] = M[1] * v[0] + M[3] * v[1] + M[4] * v[2];
+  y[2] = M[2] * v[0] + M[4] * v[1] + M[5] * v[2];
 }
 
 }  // namespace lmh

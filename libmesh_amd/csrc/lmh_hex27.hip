@@ -7,18 +7,21 @@
 // wavefront and a lane per point, 27 of 64 lanes worked and every point summed
 // 27 nodes against a 17 KB table in LDS (three workgroups per CU).  Here seven
 // elements share a wavefront, each lane forms three points by sum factorisation
-// and no table is read.  64,000 elements (40^3), before -> now: residual
-// element stage 555 (element matrices, then K_e u_e) -> 35 us, QoI 290 -> 21 us,
-// adjoint gradient 326 -> 52 us; the three calls with their gathers and host
-// waits 1288 -> 240 us.
+// and no table is read.  Residual and adjoint form the metric (six values a
+// point) from the coordinates first and only then the other fields' gradients,
+// and form their lane constants anew in every group: 168 registers and three
+// wavefronts per SIMD instead of 242 and two (residual) or more than 256 and one
+// (adjoint); four spill (45 and 38 us).  64,000 elements (40^3), before -> now:
+// residual element stage 555 (element matrices, then K_e u_e) -> 36 -> 33.7 us, QoI
+// 290 -> 22 us, adjoint gradient 326 -> 44 -> 30.5 us; the three calls with their
+// gathers and host waits 1290 -> 161 us.
 #include <algorithm>
 
 #include "lmh_hex27.h"
 
 namespace lmh {
 
-// Nodal data of the wavefront's seven elements: ids of the next group are
-// fetched while the current one is computed.
+// Nodal data of the wavefront's seven elements.
 struct H27Slots {
   int el[3], lat[3];
   bool live[3];
@@ -48,29 +51,24 @@ struct H27Slots {
 // functions direction 3 first (in registers), then directions 1 and 2 through
 // LDS, lane l owning the test functions (i1, i2) = (l % 3, l / 3).
 template <int FK>
-__global__ __launch_bounds__(64) void k_hex27_residual(const double *__restrict__ xyz, const int32_t *__restrict__ conn,
-                                                       const int32_t *__restrict__ edofs,
-                                                       const double *__restrict__ kappa, const double *__restrict__ u,
-                                                       int64_t ne, double *__restrict__ Fe, int *__restrict__ err) {
+__global__ __launch_bounds__(64, 3) void k_hex27_residual(const double *__restrict__ xyz,
+                                                          const int32_t *__restrict__ conn,
+                                                          const int32_t *__restrict__ edofs,
+                                                          const double *__restrict__ kappa, const double *__restrict__ u,
+                                                          int64_t ne, double *__restrict__ Fe, int *__restrict__ err) {
   constexpr int NF = 4, ST = 27 * NF + 1;  // odd stride: the elements' broadcasts fall in different banks
   __shared__ double s_f[kH27PerWave * ST];
   __shared__ double s_h[kH27PerWave * 81];
   const int lane = threadIdx.x;
-  const H27Slots sl(lane);
-  const H27Lane L(lane);
-  double pt[3], dt[3], pt2[3], dt2[3];  // the lane's test functions at the 1D points
-#pragma unroll
-  for (int q = 0; q < 3; ++q) {
-    pt[q] = h27_pick(L.l % 3, [&](int i) { return h27_p(q, i); });
-    dt[q] = h27_pick(L.l % 3, [&](int i) { return h27_d(q, i); });
-    pt2[q] = h27_pick(L.l / 3, [&](int i) { return h27_p(q, i); });
-    dt2[q] = h27_pick(L.l / 3, [&](int i) { return h27_d(q, i); });
-  }
   const int64_t total = ne * 27, groups = (ne + kH27PerWave - 1) / kH27PerWave;
-  int32_t nd[3], dof[3];
-  sl.ids(conn, (int64_t)blockIdx.x * kH27PerWave, total, lane, nd);
-  sl.ids(edofs, (int64_t)blockIdx.x * kH27PerWave, total, lane, dof);
   for (int64_t gr = blockIdx.x; gr < groups; gr += gridDim.x) {
+    int lg = lane;
+    asm volatile("" : "+v"(lg));  // lane constants formed again for every group, not held
+    const H27Slots sl(lg);
+    int32_t nd[3], dof[3];
+    sl.ids(conn, gr * kH27PerWave, total, lane, nd);
+    sl.ids(edofs, gr * kH27PerWave, total, lane, dof);
+    const H27Lane L(lg);
     const int64_t e0 = gr * kH27PerWave, e = e0 + L.el;
 #pragma unroll
     for (int m = 0; m < 3; ++m)
@@ -82,34 +80,27 @@ __global__ __launch_bounds__(64) void k_hex27_residual(const double *__restrict_
         d[2] = x[2];
         d[3] = u[dof[m]];
       }
-    sl.ids(conn, (gr + gridDim.x) * kH27PerWave, total, lane, nd);
-    sl.ids(edofs, (gr + gridDim.x) * kH27PerWave, total, lane, dof);
     const bool on = L.el < kH27PerWave && e < ne;
     h27_sync();
     if (on) {
       const double kap = kappa ? kappa[e] : 1.0;
-      double g[3][NF][3], pos[3][FK ? 3 : 1];
-      h27_refgrad<NF, FK ? 3 : 0>(s_f + L.el * ST, L, g, pos);
+      double M[3][6], det[3], pos[3][FK ? 3 : 1], none[3][1];
+      {
+        double g[3][3][3];
+        h27_refgrad<3, FK ? 3 : 0, NF>(s_f + L.el * ST, L, g, pos);
+        h27_metric(g, [&](int q) { return kap * (L.w12 * h27_w(q)); }, M, det, err);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      double g[3][1][3];
+      h27_refgrad<1, 0, NF>(s_f + L.el * ST + 3, L, g, none);
       double h[3][3];
 #pragma unroll
       for (int i = 0; i < 3; ++i) h[i][0] = h[i][1] = h[i][2] = 0.0;
 #pragma unroll
       for (int q = 0; q < 3; ++q) {
-        double J[3][3], c[3][3];
-#pragma unroll
-        for (int r = 0; r < 3; ++r)
-#pragma unroll
-          for (int k = 0; k < 3; ++k) J[r][k] = g[q][k][r];
-        const double det = cofactors(J, c);
-        if (!(det > 0.0)) raise_flag(err);
-        const double w = L.w12 * h27_w(q), s = kap * w / det;
-        double v[3];  // det * physical gradient of u
-#pragma unroll
-        for (int k = 0; k < 3; ++k) v[k] = g[q][3][0] * c[0][k] + g[q][3][1] * c[1][k] + g[q][3][2] * c[2][k];
         double fl[3];
-#pragma unroll
-        for (int r = 0; r < 3; ++r) fl[r] = s * (c[r][0] * v[0] + c[r][1] * v[1] + c[r][2] * v[2]);
-        double fj = det * w;
+        h27_apply(M[q], g[q][0], fl);
+        double fj = det[q] * (L.w12 * h27_w(q));
         if constexpr (FK != 0) fj *= forcing(FK, pos[q][0], pos[q][1], pos[q][2]);
 #pragma unroll
         for (int i = 0; i < 3; ++i) {
@@ -125,6 +116,14 @@ __global__ __launch_bounds__(64) void k_hex27_residual(const double *__restrict_
     }
     h27_sync();
     if (on) {
+      double pt[3], dt[3], pt2[3], dt2[3];  // the lane's test functions at the 1D points
+#pragma unroll
+      for (int q = 0; q < 3; ++q) {
+        pt[q] = h27_pick(L.l % 3, [&](int i) { return h27_p(q, i); });
+        dt[q] = h27_pick(L.l % 3, [&](int i) { return h27_d(q, i); });
+        pt2[q] = h27_pick(L.l / 3, [&](int i) { return h27_p(q, i); });
+        dt2[q] = h27_pick(L.l / 3, [&](int i) { return h27_d(q, i); });
+      }
 #pragma unroll
       for (int i = 0; i < 3; ++i) {
         const double *H = s_h + L.el * 81 + 27 * i;
@@ -219,21 +218,24 @@ __global__ __launch_bounds__(64) void k_hex27_qoi(const double *__restrict__ xyz
 
 // dJ/dkappa_e = -sum_q JxW grad(lambda).grad(u), nodal values masked to the
 // free DoFs (see k_adjoint_kappa).
-__global__ __launch_bounds__(64) void k_hex27_adjoint(const double *__restrict__ xyz, const int32_t *__restrict__ conn,
-                                                      const int32_t *__restrict__ edofs,
-                                                      const uint8_t *__restrict__ cons, const double *__restrict__ u,
-                                                      const double *__restrict__ lam, int64_t ne,
-                                                      double *__restrict__ grad, int *__restrict__ err) {
+__global__ __launch_bounds__(64, 3) void k_hex27_adjoint(const double *__restrict__ xyz,
+                                                         const int32_t *__restrict__ conn,
+                                                         const int32_t *__restrict__ edofs,
+                                                         const uint8_t *__restrict__ cons, const double *__restrict__ u,
+                                                         const double *__restrict__ lam, int64_t ne,
+                                                         double *__restrict__ grad, int *__restrict__ err) {
   constexpr int NF = 5, ST = 27 * NF;
   __shared__ double s_f[kH27PerWave * ST];
   const int lane = threadIdx.x;
-  const H27Slots sl(lane);
-  const H27Lane L(lane);
   const int64_t total = ne * 27, groups = (ne + kH27PerWave - 1) / kH27PerWave;
-  int32_t nd[3], dof[3];
-  sl.ids(conn, (int64_t)blockIdx.x * kH27PerWave, total, lane, nd);
-  sl.ids(edofs, (int64_t)blockIdx.x * kH27PerWave, total, lane, dof);
   for (int64_t gr = blockIdx.x; gr < groups; gr += gridDim.x) {
+    int lg = lane;
+    asm volatile("" : "+v"(lg));  // lane constants formed again for every group, not held
+    const H27Slots sl(lg);
+    int32_t nd[3], dof[3];
+    sl.ids(conn, gr * kH27PerWave, total, lane, nd);
+    sl.ids(edofs, gr * kH27PerWave, total, lane, dof);
+    const H27Lane L(lg);
     const int64_t e = gr * kH27PerWave + L.el;
 #pragma unroll
     for (int m = 0; m < 3; ++m)
@@ -249,31 +251,24 @@ __global__ __launch_bounds__(64) void k_hex27_adjoint(const double *__restrict__
         d[3] = c ? 0.0 : um;
         d[4] = c ? 0.0 : lm;
       }
-    sl.ids(conn, (gr + gridDim.x) * kH27PerWave, total, lane, nd);
-    sl.ids(edofs, (gr + gridDim.x) * kH27PerWave, total, lane, dof);
     const bool on = L.el < kH27PerWave && e < ne;
     h27_sync();
     double s = 0.0;
     if (on) {
-      double g[3][NF][3], none[3][1];
-      h27_refgrad<NF, 0>(s_f + L.el * ST, L, g, none);
+      double M[3][6], det[3], none[3][1];
+      {
+        double g[3][3][3];
+        h27_refgrad<3, 0, NF>(s_f + L.el * ST, L, g, none);
+        h27_metric(g, [&](int q) { return L.w12 * h27_w(q); }, M, det, err);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      double g[3][2][3];
+      h27_refgrad<2, 0, NF>(s_f + L.el * ST + 3, L, g, none);
 #pragma unroll
       for (int q = 0; q < 3; ++q) {
-        double J[3][3], c[3][3];
-#pragma unroll
-        for (int r = 0; r < 3; ++r)
-#pragma unroll
-          for (int k = 0; k < 3; ++k) J[r][k] = g[q][k][r];
-        const double det = cofactors(J, c);
-        if (!(det > 0.0)) raise_flag(err);
-        double t = 0.0;
-#pragma unroll
-        for (int k = 0; k < 3; ++k) {
-          const double gu = g[q][3][0] * c[0][k] + g[q][3][1] * c[1][k] + g[q][3][2] * c[2][k];
-          const double gl = g[q][4][0] * c[0][k] + g[q][4][1] * c[1][k] + g[q][4][2] * c[2][k];
-          t += gu * gl;
-        }
-        s += L.w12 * h27_w(q) / det * t;
+        double y[3];
+        h27_apply(M[q], g[q][0], y);
+        s += y[0] * g[q][1][0] + y[1] * g[q][1][1] + y[2] * g[q][1][2];
       }
     }
     // sum of the element's nine columns in a fixed order
