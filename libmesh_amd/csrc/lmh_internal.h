@@ -12,6 +12,7 @@
 
 #include "../../include/lmhip.h"
 #include "../../include/lmh_fe_map.h"
+#include "lmh_grids.h"
 
 namespace lmh {
 
@@ -330,10 +331,9 @@ __device__ inline T dpp_move(T v) {
   }
 }
 
-// MI355X dispatches workgroups round-robin over its 8 XCDs; remap so each XCD
-// owns one contiguous range of logical blocks (its L2 then holds the data its
-// neighbouring rows share).
-constexpr int NXCD = 8;
+// Workgroups go round-robin over the XCDs; remap so each XCD owns one contiguous
+// range of logical blocks (its L2 then holds the data its neighbouring rows
+// share).
 __device__ inline int logical_block() {
   const int G = gridDim.x, b = blockIdx.x;
   if (G % NXCD) return b;

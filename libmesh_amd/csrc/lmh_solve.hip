@@ -1354,7 +1354,7 @@ __global__ __launch_bounds__(BLK) void k_fin_sum(const double *__restrict__ part
 }
 
 static int vec_grid(lmh_context *ctx) {
-  // the partial buffer holds 4 * n_part doubles; publish<3> uses 3 * grid
+  // up to two partials per workgroup in half the partial buffer (2 * n_part doubles)
   return std::min(ctx->cu_count * LMH_GRID_PER_CU, ctx->n_part);
 }
 // Small vectors take a workgroup per 512 entries: every consumer sums all
@@ -1367,15 +1367,6 @@ static int vec_grid(lmh_context *ctx) {
 constexpr int64_t kBcgSmall = 16384;
 static int vec_grid(lmh_context *ctx, int64_t n) {
   return (int)std::max<int64_t>(1, std::min<int64_t>(vec_grid(ctx), (n + 511) / 512));
-}
-
-// SpMV-type kernels (row-block streams) want more resident waves than the
-// vector kernels: their grid is sized separately; every kernel that reduces
-// partials is told the producer's grid.
-static int spmv_grid(lmh_context *ctx) {
-  // k_refresh publishes 3 values per workgroup into the second half (2 * n_part)
-  const int g = ctx->cu_count * LMH_SPMV_GRID_PER_CU, cap = 2 * ctx->n_part / 3;
-  return g < cap ? g : cap;
 }
 
 // x windows of the SpMV operators, built once per pattern on the row
@@ -1537,24 +1528,14 @@ struct Stream {
 };
 static Stream stream_of(lmh_matrix *A, bool fp32) {
   Stream s;
-  const int gs = spmv_grid(A->ctx);
   s.on = A->idx16_state == 1;
-  s.nt = s.on && A->wbits == 8 ? W8_NT : BLK;
-  s.grid = s.on && A->wbits == 8 ? W8_GRID * gs : gs;
-  // At most one workgroup per row block (whole XCD rounds).  Up to four rounds of
-  // what a GPU holds at once, a workgroup takes as many blocks as there are
-  // rounds: it loads one while it sums the last, and its consumers read fewer
-  // partial sums.  Q2 20^3 (4,050 blocks) BiCGSTAB 6.8 -> 6.4 ms a solve, Q2 24^3 CG
-  // 7.69 -> 7.32, mixed 7.68 -> 7.37, Q1 50^3 CG 4.82 -> 4.63, TET4 40^3 products 49 ->
-  // 43 us; one round (Q2 12^3) 2.6 ms either way, and two rounds for it 2.8;
-  // beyond four rounds (Q2 30^3 and up) the full grid measures the same.
-  const int64_t nb = s.on ? A->nrbw : A->nrb, resident = (int64_t)A->ctx->cu_count * (s.nt == W8_NT ? 10 : 5);
-  int64_t want = nb;
-  if (nb <= 4 * resident) {
-    const int64_t rounds = std::max<int64_t>(1, (nb + resident - 1) / resident);
-    want = (nb + rounds - 1) / rounds;
-  }
-  s.grid = (int)std::min<int64_t>(s.grid, (want + NXCD - 1) / NXCD * NXCD);
+  const bool small = s.on && A->wbits == 8;  // 1024-entry blocks on 128 threads
+  s.nt = small ? W8_NT : BLK;
+  // SpMV-type kernels want more resident waves than the vector kernels: their
+  // grid is sized separately; every kernel that reduces partials is told the
+  // producer's grid
+  s.grid = product_grid(A->ctx->cu_count, LMH_SPMV_GRID_PER_CU * (small ? W8_GRID : 1), small ? 10 : 5,
+                        A->ctx->n_part, s.on ? A->nrbw : A->nrb);
   if (use_windows(A) && A->cols < ((int64_t)1 << 29)) {
     s.iw = A->wbits / 8;
     s.idx = fp32 ? A->widx32 : A->widx64;
