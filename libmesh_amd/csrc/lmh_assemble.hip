@@ -502,9 +502,10 @@ static int matrix_free_path(int type, int npts) {
   return type == LMH_TET4 || type == LMH_TET10 || type == LMH_HEX8 ? 2 : 0;
 }
 
-static int read_flag(lmh_context *ctx, const char *what) {
-  LMH_HIP(hipStreamSynchronize(ctx->stream));
-  if (*(volatile int *)ctx->h_flag) return set_error(LMH_ERR_DEGENERATE, "%s: Jacobian determinant <= 0 (degenerate map)", what);
+static int read_flag(MapFlag &flag, const char *what) {
+  bool raised = false;
+  LMH_TRY(flag.wait(&raised));
+  if (raised) return set_error(LMH_ERR_DEGENERATE, "%s: Jacobian determinant <= 0 (degenerate map)", what);
   return LMH_OK;
 }
 
@@ -600,9 +601,9 @@ int lmh_element_poisson(lmh_context *ctx, const lmh_mesh *m, const lmh_dofmap *d
   LMH_CHECK(ctx && m && dm && Ke_d && Fe_d, LMH_ERR_INVALID, "null argument");
   LMH_CHECK(!constrain || dm->cr.n_general == 0, LMH_ERR_UNSUPPORTED,
             "element matrices with general constraint rows grow past the element's DoFs: assemble the matrix");
-  *(volatile int *)ctx->h_flag = 0;
+  MapFlag flag(ctx);
   LMH_TRY(element_poisson_impl<double>(ctx, m, dm, npts, kappa_d, f_kind, constrain, Ke_d, Fe_d));
-  return read_flag(ctx, "lmh_element_poisson");
+  return read_flag(flag, "lmh_element_poisson");
 }
 
 int lmh_assemble_poisson(lmh_matrix *A, const lmh_mesh *m, const lmh_dofmap *dm, int npts, const double *kappa_d,
@@ -615,7 +616,7 @@ int lmh_assemble_poisson(lmh_matrix *A, const lmh_mesh *m, const lmh_dofmap *dm,
   lmh_context *ctx = A->ctx;
   const int64_t ne = m->n_elem, dd = (int64_t)dm->dpe * dm->dpe;
   if (!A->Fe) LMH_HIP(hipMalloc((void **)&A->Fe, sizeof(double) * ne * dm->dpe));
-  *(volatile int *)ctx->h_flag = 0;
+  MapFlag flag(ctx);
   if (precision == LMH_FP64) {
     if (!A->Ke) LMH_HIP(hipMalloc((void **)&A->Ke, sizeof(double) * ne * dd));
     LMH_TRY(element_poisson_impl<double>(ctx, m, dm, npts, kappa_d, f_kind, 1, A->Ke, A->Fe));
@@ -633,7 +634,7 @@ int lmh_assemble_poisson(lmh_matrix *A, const lmh_mesh *m, const lmh_dofmap *dm,
     LMH_TRY(scatter_extra_impl<float>(A, A->vals32, rhs_d));
     A->have32 = true;
   }
-  return read_flag(ctx, "lmh_assemble_poisson");
+  return read_flag(flag, "lmh_assemble_poisson");
 }
 
 int lmh_matrix_get_values_fp32(const lmh_matrix *A, float *vals_h) {
@@ -709,7 +710,7 @@ int lmh_assemble_residual_poisson(lmh_matrix *A, const lmh_mesh *m, const lmh_do
   LMH_CHECK(dm->nv == 1, LMH_ERR_UNSUPPORTED, "Poisson assembly needs one variable");
   const FETable *t = nullptr;
   LMH_TRY(fe_table(ctx, m->type, npts, &t));
-  *(volatile int *)ctx->h_flag = 0;
+  MapFlag flag(ctx);
   const int path = matrix_free_path(m->type, npts);
   if (path == 1) {
     LMH_TRY(hex27_residual(ctx, m, dm, kappa_d, f_kind, u_d, A->Fe));
@@ -725,7 +726,7 @@ int lmh_assemble_residual_poisson(lmh_matrix *A, const lmh_mesh *m, const lmh_do
   LMH_LAUNCH(ctx, "add_element_vectors", k_sum_vec_gather<true>, dim3(grid_for(dm->n_dofs, 256, 8192)), dim3(256), 0,
              dm->inc_ptr, dm->inc, dm->cons, dm->n_dofs, (const double *)A->Fe, R_d);
   LMH_TRY(check_launch("residual"));
-  LMH_TRY(read_flag(ctx, "lmh_assemble_residual_poisson"));
+  LMH_TRY(read_flag(flag, "lmh_assemble_residual_poisson"));
   // general rows: u holds the enforced values (C u + H), so the summed element
   // residuals get C^T, as constrain_element_residual does per element
   return apply_constraint_transpose(ctx, dm, R_d);
@@ -739,7 +740,7 @@ int lmh_qoi_box_derivative(const lmh_mesh *m, const lmh_dofmap *dm, int npts, do
   LMH_TRY(fe_table(ctx, m->type, npts, &t));
   double *Q = nullptr;
   LMH_HIP(hipMallocAsync((void **)&Q, sizeof(double) * m->n_elem * t->n, ctx->stream));
-  *(volatile int *)ctx->h_flag = 0;
+  MapFlag flag(ctx);
   const int path = matrix_free_path(m->type, npts);
   if (path == 1) {
     LMH_TRY(hex27_qoi(ctx, m, lo, hi, Q));
@@ -755,7 +756,7 @@ int lmh_qoi_box_derivative(const lmh_mesh *m, const lmh_dofmap *dm, int npts, do
              dm->inc_ptr, dm->inc, dm->cons, dm->n_dofs, (const double *)Q, dq_d);
   LMH_TRY(check_launch("qoi"));
   LMH_HIP(hipFreeAsync(Q, ctx->stream));
-  LMH_TRY(read_flag(ctx, "lmh_qoi_box_derivative"));
+  LMH_TRY(read_flag(flag, "lmh_qoi_box_derivative"));
   // what assemble_qoi_derivative with apply_constraints = true gives
   return apply_constraint_transpose(ctx, dm, dq_d);
 }
@@ -773,19 +774,19 @@ int lmh_adjoint_kappa_gradient(const lmh_mesh *m, const lmh_dofmap *dm, int npts
   const FETable *t = nullptr;
   LMH_TRY(fe_table(ctx, m->type, npts, &t));
   LMH_CHECK(t->nq <= 64 && t->n <= 27, LMH_ERR_UNSUPPORTED, "element too large");
-  *(volatile int *)ctx->h_flag = 0;
+  MapFlag flag(ctx);
   const int path = matrix_free_path(m->type, npts);
   if (path != 0) {
     LMH_TRY(path == 1 ? hex27_adjoint(ctx, m, dm, u_d, lambda_d, grad_d)
                       : thread_adjoint(ctx, t, m, dm, u_d, lambda_d, grad_d));
-    return read_flag(ctx, "lmh_adjoint_kappa_gradient");
+    return read_flag(flag, "lmh_adjoint_kappa_gradient");
   }
   const size_t shm = sizeof(double) * (t->nq + (size_t)t->n * t->nq * 4 + 81 + 27 + 27 + 64);
   LMH_LAUNCH(ctx, "adjoint_kappa", k_adjoint_kappa, dim3(grid_for(m->n_elem, 1, ctx->cu_count * 8)), dim3(64), shm,
              t->d_data, t->n, t->nq, m->xyz, m->conn, dm->edofs, dm->cons, u_d, lambda_d, m->n_elem, grad_d,
              ctx->g_flag);
   LMH_TRY(check_launch("k_adjoint_kappa"));
-  return read_flag(ctx, "lmh_adjoint_kappa_gradient");
+  return read_flag(flag, "lmh_adjoint_kappa_gradient");
 }
 
 // ---------------------------------------------------------------------------

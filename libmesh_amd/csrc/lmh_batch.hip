@@ -1034,6 +1034,7 @@ int lmh_batch_get_tiles(const lmh_batch *b, int *lpe, int *passes) {
 int lmh_batch_autotune(lmh_batch *b, double E, double nu, double fz, int reps, double *best_ms) {
   LMH_CHECK(b && reps >= 1, LMH_ERR_INVALID, "bad argument");
   lmh_context *ctx = b->ctx;
+  MapFlag flag(ctx);  // raised by the timed launches, not read: a degenerate map is the assembly's to report
   float l1, l2;
   lame(E, nu, l1, l2);
   const int cand_l[5] = {16, 32, 64, 128, 256};
@@ -1109,13 +1110,14 @@ int lmh_batch_assemble_elasticity(lmh_batch *b, double E, double nu, double fz) 
   LMH_CHECK(E > 0 && nu > -1.0 && nu < 0.5, LMH_ERR_INVALID, "need E > 0 and -1 < nu < 1/2");
   lmh_context *ctx = b->ctx;
   if (!b->exec || E != b->gE || nu != b->gnu || fz != b->gfz) LMH_TRY(build_graph(b, E, nu, fz));
-  *(volatile int *)ctx->h_flag = 0;
+  MapFlag flag(ctx);
   {
     ProfScope ps(ctx, "batch_graph");
     LMH_HIP(hipGraphLaunch(b->exec, ctx->stream));
   }
-  LMH_HIP(hipStreamSynchronize(ctx->stream));
-  LMH_CHECK(!*(volatile int *)ctx->h_flag, LMH_ERR_DEGENERATE, "degenerate element map (det J <= 0) in the batch");
+  bool raised = false;
+  LMH_TRY(flag.wait(&raised));
+  LMH_CHECK(!raised, LMH_ERR_DEGENERATE, "degenerate element map (det J <= 0) in the batch");
   for (lmh_matrix *A : b->mats) A->have32 = true;
   return LMH_OK;
 }

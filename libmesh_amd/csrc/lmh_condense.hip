@@ -632,7 +632,7 @@ static int sc_setup(lmh_condensation *sc) {
   lmh_context *ctx = A->ctx;
   LMH_HIP(hipSetDevice(ctx->device));
   const bool pivots_only = sc->pmap && !sc->coupled;  // k_sc_values_plan checks them
-  *(volatile int *)ctx->h_flag = 0;
+  MapFlag pivot(ctx);
   if (!pivots_only) LMH_HIP(hipMemsetAsync(ctx->d_flags, 0, sizeof(int), ctx->stream));
   if (sc->n_cond && !pivots_only) {
     LMH_LAUNCH(ctx, "sc_check", k_sc_check, dim3(grid_for(sc->n_cond, 256, 8192)), dim3(256), 0, sc->n_cond, sc->cdof,
@@ -665,8 +665,9 @@ static int sc_setup(lmh_condensation *sc) {
   }
   int flags = 0;
   if (!pivots_only) LMH_HIP(hipMemcpyAsync(&flags, ctx->d_flags, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
-  LMH_HIP(hipStreamSynchronize(ctx->stream));
-  if (*(volatile int *)ctx->h_flag) flags |= SC_ZEROPIVOT;
+  bool zero_pivot = false;
+  LMH_TRY(pivot.wait(&zero_pivot));
+  if (zero_pivot) flags |= SC_ZEROPIVOT;
   R->have32 = false;
   LMH_CHECK(!(flags & SC_OFFDIAG), LMH_ERR_UNSUPPORTED,
             "condensed DoFs couple to each other: only a diagonal condensed block is supported");

@@ -97,9 +97,9 @@ struct lmh_context {
   unsigned *d_count = nullptr;  // last-block counters (zeroed, self-resetting)
   int *d_flags = nullptr;       // error flags
   // The map kernels' error flag, in pinned host memory: the host clears it before
-  // the launch (the stream is idle then: every call that uses it waits) and reads
-  // it after the wait, without a clear and a copy on the stream (Q1 10^3 assembly
-  // 34 -> 21 us, three Q2 40^3 gradient calls 240 -> 189 us).
+  // the launch and reads it after the wait, without a clear and a copy on the
+  // stream (Q1 8^3 assembly 34 -> 21 us, three Q2 40^3 gradient calls 240 -> 189
+  // us).  Only through MapFlag, which leaves no kernel behind that may still set it.
   int *h_flag = nullptr, *g_flag = nullptr;  // its host and device addresses
   double *h_pinned = nullptr, *g_pinned = nullptr;  // pinned host scalars: host and device addresses
   hipEvent_t ev_poll[2] = {nullptr, nullptr};  // solver convergence polls
@@ -107,6 +107,31 @@ struct lmh_context {
   int n_part = 0;
   int cu_count = 256;
 };
+
+namespace lmh {
+// One use of the context's map flag: cleared here, raised by the kernels launched
+// meanwhile, read by wait().  A call that returns without wait() (an error after a
+// launch) waits on the way out, or its kernels could raise the next call's flag.
+class MapFlag {
+ public:
+  explicit MapFlag(lmh_context *ctx) : ctx_(ctx) { *(volatile int *)ctx_->h_flag = 0; }
+  ~MapFlag() {
+    if (!waited_) (void)hipStreamSynchronize(ctx_->stream);
+  }
+  MapFlag(const MapFlag &) = delete;
+  MapFlag &operator=(const MapFlag &) = delete;
+  int wait(bool *raised) {
+    LMH_HIP(hipStreamSynchronize(ctx_->stream));
+    waited_ = true;
+    *raised = *(volatile int *)ctx_->h_flag != 0;
+    return LMH_OK;
+  }
+
+ private:
+  lmh_context *ctx_;
+  bool waited_ = false;
+};
+}  // namespace lmh
 
 struct lmh_mesh {
   lmh_context *ctx = nullptr;
