@@ -303,8 +303,11 @@ int lmh_cg_solve_noalloc(lmh_matrix *A, const double *b_d, double *x_d, double r
  * BICGSTAB + JACOBI_PRECOND -> Eigen::BiCGSTAB, eigen_sparse_linear_solver.C:175-205,
  * BiCGSTAB.h:28-112), for nonsymmetric matrices such as those with asymmetric
  * constraint rows.  Same contract as lmh_cg_solve: stops when
- * |r|^2 <= rtol^2 |b|^2; b = 0 gives x = 0.  Eigen's restart when (r0, r)
- * vanishes relative to |r0|^2 is reported as LMH_DIVERGED_BREAKDOWN. */
+ * |r|^2 <= rtol^2 |b|^2; b = 0 gives x = 0.  Where (r0, r) vanishes relative to
+ * |r0|^2 it restarts with r0 = r and counts from 0 after the first restart, as
+ * Eigen's loop does; so it does where (r0, A y) = 0, by which that loop would
+ * divide.  maxits bounds the iterations in all.  A restart after omega = 0 would
+ * get nowhere: LMH_DIVERGED_BREAKDOWN. */
 int lmh_bicgstab_solve(lmh_matrix *A, const double *b_d, double *x_d, double rtol, int64_t maxits, int64_t *iters,
                        double *rel_res, int *reason);
 /* The same BiCGSTAB on the transpose, A^T x = b: what LinearSolver::

@@ -1361,10 +1361,7 @@ static int vec_grid(lmh_context *ctx) {
 // workgroups' partials, and empty workgroups cost their dispatch (CG with 1,331
 // rows: update 9.7 -> 6.5 us, p-update 8.0 -> 6.4 us with 3 workgroups for 1024,
 // both with the 5 us of their timing events; BiCGSTAB with 68,921 rows 7.4 ->
-// 6.4 ms a solve).  BiCGSTAB keeps the full grid below kBcgSmall rows: on small
-// systems whose (r0, r) vanishes in exact arithmetic the order of its sums
-// decides between convergence and breakdown, and the launches dominate anyway.
-constexpr int64_t kBcgSmall = 16384;
+// 6.4 ms a solve).
 static int vec_grid(lmh_context *ctx, int64_t n) {
   return (int)std::max<int64_t>(1, std::min<int64_t>(vec_grid(ctx), (n + 511) / 512));
 }
@@ -1685,11 +1682,11 @@ namespace lmh {
 // EigenSparseLinearSolver::solve runs it for BICGSTAB + JACOBI_PRECOND).  One
 // iteration is five kernels: p/y update (reduces |r|^2 and (r0, r), tests
 // convergence) | v = A y + (r0, v) | s, z | t = A z + (t, t), (t, s) | x, r
-// update + |r|^2, (r0, r).  rho, alpha, w live in the banks next to the CG
-// fields; each is written by block 0 of one kernel and read by later kernels.
+// update + |r|^2, (r0, r).  rho, alpha, w and |r0|^2 live in the banks next to
+// the CG fields; each is written by block 0 of one kernel and read by later
+// kernels.
 // ---------------------------------------------------------------------------
-enum { B_RHO = 8, B_ALPHA, B_W };
-enum { G_R0SQ = 40 };
+enum { B_RHO = 8, B_ALPHA, B_W, B_R0SQ, B_RESTARTS, B_LOST };
 
 // r0 = r, p = v = 0; partials (r.r, r0.r)
 __global__ __launch_bounds__(BLK) void k_bcg_init(int64_t n, const double *__restrict__ r, double *__restrict__ r0,
@@ -1720,11 +1717,10 @@ __global__ __launch_bounds__(BLK) void k_bcg_init_fin(const double *__restrict__
   if (blockIdx.x != 0 || threadIdx.x != 0) return;
   S[G_THR] = tol * tol * bb;
   S[G_BB] = bb;
-  S[G_R0SQ] = rr;
   double *B0 = S;
   for (int k = 0; k < B_SIZE; ++k) B0[k] = 0.0;
   B0[B_RHO] = B0[B_ALPHA] = B0[B_W] = 1.0;
-  B0[B_RR] = rr;
+  B0[B_RR] = B0[B_R0SQ] = rr;
   if (bb == 0.0) {
     B0[B_RR] = 0.0;
     B0[B_DONE] = 1;
@@ -1735,13 +1731,18 @@ __global__ __launch_bounds__(BLK) void k_bcg_init_fin(const double *__restrict__
   }
 }
 
-// top of the loop: rr = |r|^2, rho = (r0, r); stop when rr <= tol2; the
-// restart of Eigen's loop (|rho| < eps^2 |r0|^2) is reported as a breakdown;
-// else beta = (rho / rho_old)(alpha / w), p = r + beta (p - w v), y = dinv p
+// top of the loop: rr = |r|^2, rho = (r0, r); stop when rr <= tol2; where r has
+// become orthogonal to r0 (|rho| < eps^2 |r0|^2) restart with r0 = r, rho = |r|^2,
+// the count from 0 after the first restart (BiCGSTAB.h:68-77; r is the recursion's,
+// not formed again from x); beta = (rho / rho_old)(alpha / w), p = r + beta (p - w
+// v), y = dinv p.  w = 0 makes rho vanish too and leaves no beta: a breakdown.
+// (r0, v) = 0 (k_bcg_s) restarts as well, with p = r: Eigen's loop divides by it,
+// and on small systems the order of the sums decides whether it comes up.
 __global__ __launch_bounds__(BLK) void k_bcg_p(int64_t n, const double *__restrict__ part_in, int G,
                                                const double *__restrict__ dinv, const double *__restrict__ r,
-                                               const double *__restrict__ v, double *__restrict__ p,
-                                               double *__restrict__ y, double *__restrict__ S, int bank) {
+                                               const double *__restrict__ v, double *__restrict__ r0,
+                                               double *__restrict__ p, double *__restrict__ y,
+                                               double *__restrict__ S, int bank) {
   const double *Sb = S + bank * B_SIZE;
   double *Sn = S + (bank ^ 1) * B_SIZE;
   if (Sb[B_DONE] != 0.0) {
@@ -1750,15 +1751,16 @@ __global__ __launch_bounds__(BLK) void k_bcg_p(int64_t n, const double *__restri
   }
   double t[2];
   reduce_all<2>(part_in, G, t);
-  const double rr = t[0], rho = t[1];
-  const double eps = 2.220446049250313e-16;
+  const double rr = t[0], eps = 2.220446049250313e-16;
+  const bool restart = Sb[B_LOST] != 0.0 || fabs(t[1]) < eps * eps * Sb[B_R0SQ];
+  const double rho = restart ? rr : t[1];
   bool done = true;
   int reason = 0;
   if (!isfinite(rr))
     reason = LMH_DIVERGED_NANORINF;
   else if (rr <= S[G_THR])
     reason = LMH_CONVERGED_RTOL;
-  else if (fabs(rho) < eps * eps * S[G_R0SQ])
+  else if (restart && Sb[B_W] == 0.0)
     reason = LMH_DIVERGED_BREAKDOWN;
   else
     done = false;
@@ -1768,13 +1770,19 @@ __global__ __launch_bounds__(BLK) void k_bcg_p(int64_t n, const double *__restri
     Sn[B_DONE] = done ? 1.0 : 0.0;
     Sn[B_REASON] = reason;
     Sn[B_RHO] = done ? Sb[B_RHO] : rho;
+    if (restart && !done) {
+      Sn[B_R0SQ] = rr;
+      if (Sb[B_RESTARTS] == 0.0) Sn[B_ITS] = 0.0;
+      Sn[B_RESTARTS] = Sb[B_RESTARTS] + 1.0;
+    }
   }
   if (done) return;
   const double beta = (rho / Sb[B_RHO]) * (Sb[B_ALPHA] / Sb[B_W]), w = Sb[B_W];
   int64_t lo, hi;
   block_range(n, lo, hi);
   for (int64_t i = lo + threadIdx.x; i < hi; i += BLK) {
-    const double pi = r[i] + beta * (p[i] - w * v[i]);
+    const double ri = r[i], pi = ri + beta * (p[i] - w * v[i]);
+    if (restart) r0[i] = ri;
     p[i] = pi;
     y[i] = dinv[i] * pi;
   }
@@ -1816,7 +1824,9 @@ __global__ __launch_bounds__(NT) void k_bcg_spmv_v16(int64_t nrb, const int32_t 
   publish<1, NT>(acc, part);
 }
 
-// alpha = rho / (r0, v); s = r - alpha v; z = dinv s
+// alpha = rho / (r0, v); s = r - alpha v; z = dinv s.  (r0, v) = 0 gives no alpha:
+// the iteration goes on with s = r, its w the one that makes |r| smallest, and the
+// next one restarts.
 __global__ __launch_bounds__(BLK) void k_bcg_s(int64_t n, const double *__restrict__ part_in, int G,
                                                const double *__restrict__ dinv, const double *__restrict__ r,
                                                const double *__restrict__ v, double *__restrict__ s,
@@ -1825,8 +1835,13 @@ __global__ __launch_bounds__(BLK) void k_bcg_s(int64_t n, const double *__restri
   if (Sn[B_DONE] != 0.0) return;
   double t[1];
   reduce_all<1>(part_in, G, t);
-  const double alpha = Sn[B_RHO] / t[0];
-  if (blockIdx.x == 0 && threadIdx.x == 0) Sn[B_ALPHA] = alpha;
+  const double ratio = Sn[B_RHO] / t[0];
+  const bool lost = isinf(ratio);
+  const double alpha = lost ? 0.0 : ratio;
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    Sn[B_ALPHA] = alpha;
+    Sn[B_LOST] = lost ? 1.0 : 0.0;
+  }
   int64_t lo, hi;
   block_range(n, lo, hi);
   for (int64_t i = lo + threadIdx.x; i < hi; i += BLK) {
@@ -2108,7 +2123,7 @@ static int bicgstab_impl(lmh_matrix *A, const double *vals, const double *b_d, d
   double *part1 = ctx->d_part, *part2 = ctx->d_part + 2 * ctx->n_part;
   LMH_TRY(ensure_windows(A));
   const Stream st = stream_of(A, false);
-  const int g = n < kBcgSmall ? vec_grid(ctx) : vec_grid(ctx, n);
+  const int g = vec_grid(ctx, n);
   LMH_TRY(ensure_diag(A));
   LMH_LAUNCH(ctx, "invdiag", (k_invdiag<double, double>), dim3(grid_for(n, 256, 8192)), dim3(256), 0, n, A->diag,
              vals, A->precond == LMH_PRECOND_JACOBI, dinv);
@@ -2124,7 +2139,7 @@ static int bicgstab_impl(lmh_matrix *A, const double *vals, const double *b_d, d
   bool pending = false, done = false;
   auto iteration = [&](int bank) {
     const int nb = bank ^ 1;
-    LMH_LAUNCH(ctx, "bcg_p", k_bcg_p, dim3(g), dim3(BLK), 0, n, part1, g, dinv, r, v, p, y, S, bank);
+    LMH_LAUNCH(ctx, "bcg_p", k_bcg_p, dim3(g), dim3(BLK), 0, n, part1, g, dinv, r, v, r0, p, y, S, bank);
     if (st.on)
       with_stream(st, [&](auto sh) {
         typedef decltype(sh) K;
@@ -2163,7 +2178,7 @@ static int bicgstab_impl(lmh_matrix *A, const double *vals, const double *b_d, d
     slot ^= 1;
   }
   // the loop test after the last iteration (Eigen: while (|r|^2 > tol2 && i < maxIters))
-  LMH_LAUNCH(ctx, "bcg_p", k_bcg_p, dim3(g), dim3(BLK), 0, n, part1, g, dinv, r, v, p, y, S, (int)(K & 1));
+  LMH_LAUNCH(ctx, "bcg_p", k_bcg_p, dim3(g), dim3(BLK), 0, n, part1, g, dinv, r, v, r0, p, y, S, (int)(K & 1));
   LMH_HIP(hipStreamSynchronize(ctx->stream));
   LMH_TRY(check_launch("bicgstab iterations"));
   for (auto &pl : poll)
@@ -2173,7 +2188,7 @@ static int bicgstab_impl(lmh_matrix *A, const double *vals, const double *b_d, d
   LMH_HIP(hipMemcpy(&gbb, S + G_BB, sizeof(double), hipMemcpyDeviceToHost));
   const double *Bk = h + ((K + 1) & 1) * B_SIZE;
   const bool conv = Bk[B_DONE] != 0.0;
-  if (iters) *iters = (int64_t)Bk[B_ITS];
+  if (iters) *iters = conv ? (int64_t)Bk[B_ITS] : maxits;
   if (rel_res) *rel_res = gbb > 0 ? std::sqrt(Bk[B_RR] / gbb) : 0.0;
   if (reason) *reason = conv ? (int)Bk[B_REASON] : LMH_DIVERGED_ITS;
   return LMH_OK;
