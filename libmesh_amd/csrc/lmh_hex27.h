@@ -129,7 +129,21 @@ __device__ inline double cofactors(const double (&J)[3][3], double (&c)[3][3]) {
   return J[0][0] * c[0][0] + J[0][1] * c[0][1] + J[0][2] * c[0][2];
 }
 
-// M[q3] = w / det C C^T (components 11, 12, 13, 22, 23, 33; C the cofactor rows) and
+// M = s C C^T, C the cofactor rows: put(m, value) for the components 11, 12, 13,
+// 22, 23, 33.  s is on one factor, not on the product: C C^T alone leaves the range
+// of FP64 for elements smaller than 1e-77 or larger than 1e77, M at 1e-102 and 1e102.
+template <typename P>
+__device__ inline void cofactor_metric(const double (&c)[3][3], double s, P &&put) {
+  int m = 0;
+#pragma unroll
+  for (int r = 0; r < 3; ++r) {
+    const double a = s * c[r][0], b = s * c[r][1], d = s * c[r][2];
+#pragma unroll
+    for (int k = r; k < 3; ++k, ++m) put(m, a * c[k][0] + b * c[k][1] + d * c[k][2]);
+  }
+}
+
+// M[q3] = w / det C C^T (components as above) and
 // det at the lane's three points, from the coordinates' reference gradients; w(q3)
 // is the point's factor.  The gradients need not outlive it.
 template <typename W>
@@ -143,12 +157,7 @@ __device__ inline void h27_metric(const double (&g)[3][3][3], W &&w, double (&M)
       for (int k = 0; k < 3; ++k) J[r][k] = g[q][k][r];
     det[q] = cofactors(J, c);
     if (!(det[q] > 0.0)) raise_flag(err);
-    const double s = w(q) / det[q];
-    int m = 0;
-#pragma unroll
-    for (int r = 0; r < 3; ++r)
-#pragma unroll
-      for (int k = r; k < 3; ++k, ++m) M[q][m] = s * (c[r][0] * c[k][0] + c[r][1] * c[k][1] + c[r][2] * c[k][2]);
+    cofactor_metric(c, w(q) / det[q], [&](int m, double v) { M[q][m] = v; });
   }
 }
 // M v for such a point

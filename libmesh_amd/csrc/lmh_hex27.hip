@@ -408,14 +408,9 @@ __global__ __launch_bounds__(64, 3) void k_hex27_poisson(const double *__restric
           for (int k = 0; k < 3; ++k) J[r][k] = g[q][k][r];
         const double det = cofactors(J, c);
         if (!(det > 0.0)) raise_flag(err);
-        const double w = L.w12 * h27_w(q), s = kap * w / det;
+        const double w = L.w12 * h27_w(q);
         double *M = s_m + L.el * 162 + 9 * q + L.l;  // components 11, 12, 13, 22, 23, 33
-        int m = 0;
-#pragma unroll
-        for (int r = 0; r < 3; ++r)
-#pragma unroll
-          for (int u = r; u < 3; ++u, ++m)
-            M[27 * m] = s * (c[r][0] * c[u][0] + c[r][1] * c[u][1] + c[r][2] * c[u][2]);
+        cofactor_metric(c, kap * w / det, [&](int m, double v) { M[27 * m] = v; });
         double fj = det * w;
         if constexpr (FK != 0) {
           const double *o = s_c + L.el * 4;

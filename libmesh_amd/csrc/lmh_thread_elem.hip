@@ -100,11 +100,15 @@ __global__ __launch_bounds__(kTB) void k_thread_residual(const double *__restric
       for (int a = 0; a < N; ++a)
 #pragma unroll
         for (int r = 0; r < 3; ++r) g[r] += U[a] * d[3 * a + r];
-#pragma unroll
-      for (int k = 0; k < 3; ++k) v[k] = g[0] * c[0][k] + g[1] * c[1][k] + g[2] * c[2][k];
+      // on one factor, not on the product: c c^T alone leaves the range of FP64 for
+      // elements smaller than 1e-77 or larger than 1e77
       const double s = kap * (N == 4 ? wsum : P[0]) / det;
 #pragma unroll
-      for (int r = 0; r < 3; ++r) fl[r] = s * (c[r][0] * v[0] + c[r][1] * v[1] + c[r][2] * v[2]);
+      for (int r = 0; r < 3; ++r) g[r] *= s;
+#pragma unroll
+      for (int k = 0; k < 3; ++k) v[k] = g[0] * c[0][k] + g[1] * c[1][k] + g[2] * c[2][k];
+#pragma unroll
+      for (int r = 0; r < 3; ++r) fl[r] = c[r][0] * v[0] + c[r][1] * v[1] + c[r][2] * v[2];
 #pragma unroll
       for (int a = 0; a < N; ++a) R[a] += fl[0] * d[3 * a] + fl[1] * d[3 * a + 1] + fl[2] * d[3 * a + 2];
     }
@@ -188,12 +192,13 @@ __global__ __launch_bounds__(kTB) void k_thread_adjoint(const double *__restrict
         gu[r] += U[a] * d[3 * a + r];
         gl[r] += W[a] * d[3 * a + r];
       }
-    double t = 0.0;
+    const double f = (N == 4 ? wsum : P[0]) / det;
+#pragma unroll
+    for (int r = 0; r < 3; ++r) gu[r] *= f;
 #pragma unroll
     for (int k = 0; k < 3; ++k)
-      t += (gu[0] * c[0][k] + gu[1] * c[1][k] + gu[2] * c[2][k]) *
+      s += (gu[0] * c[0][k] + gu[1] * c[1][k] + gu[2] * c[2][k]) *
            (gl[0] * c[0][k] + gl[1] * c[1][k] + gl[2] * c[2][k]);
-    s += (N == 4 ? wsum : P[0]) / det * t;
   }
   if (bad) raise_flag(err);
   grad[e] = -s;
@@ -241,10 +246,11 @@ __global__ __launch_bounds__(kTB) __attribute__((amdgpu_waves_per_eu(2))) void k
       bad |= !(det > 0.0);
       const double s = kap * (N == 4 ? wsum : P[0]) / det;
 #pragma unroll
-      for (int r = 0; r < 3; ++r)
+      for (int r = 0; r < 3; ++r) {
+        const double a = s * c[r][0], b = s * c[r][1], f = s * c[r][2];
 #pragma unroll
-        for (int t = r; t < 3; ++t)
-          M[r][t] = M[t][r] = s * (c[r][0] * c[t][0] + c[r][1] * c[t][1] + c[r][2] * c[t][2]);
+        for (int t = r; t < 3; ++t) M[r][t] = M[t][r] = a * c[t][0] + b * c[t][1] + f * c[t][2];
+      }
       int k = 0;
 #pragma unroll
       for (int i = 0; i < N; ++i) {

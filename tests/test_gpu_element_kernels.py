@@ -86,3 +86,32 @@ def test_element_matrices(ctx, t, npts, box):
     assert rel(g.values_fp32().astype(np.float64), vals) < 2e-6
     assert rel(b.download(), rhs) < 1e-12
     g.close()
+
+
+@pytest.mark.parametrize("power", [-300, 300])
+@pytest.mark.parametrize("t,npts,box", [(L.HEX27, 3, (3, 2, 1)), (L.HEX27, 2, (2, 1, 1)), (L.HEX8, 2, (3, 2, 2)),
+                                        (L.HEX8, 2, (26, 26, 25)), (L.HEX8, 3, (3, 2, 2)), (L.TET4, 3, (2, 1, 1)),
+                                        (L.TET10, 5, (1, 2, 1))])
+def test_any_size_of_element(ctx, t, npts, box, power):
+    """Coordinates times 2^power (elements of edge 1e-91 and 1e90): every product on
+    the way is exact, so the results scale exactly, K and the gradient by 2^power,
+    F, the residual (of u times 4^power) and the QoI derivative by 8^power."""
+    p, s, kappa = problem(ctx, t, box)
+    rng = np.random.default_rng(SEED + 2)
+    u, lam = rng.standard_normal(p.n_dofs), rng.standard_normal(p.n_dofs)
+    kd, ld = L.DeviceArray(ctx, p.n_elem, data=kappa), L.DeviceArray(ctx, p.n_dofs, data=lam)
+    dpe = p.elem_dofs.shape[1]
+    got = []
+    for k in (0, power):
+        g = L.GpuProblem(ctx, np.ldexp(p.coords, k), p.conn, p.elem_type, p.elem_dofs, p.n_dofs, p.constrained)
+        ud, us = L.DeviceArray(ctx, p.n_dofs, data=u), L.DeviceArray(ctx, p.n_dofs, data=np.ldexp(u, 2 * k))
+        K, F = L.DeviceArray(ctx, p.n_elem * dpe * dpe), L.DeviceArray(ctx, p.n_elem * dpe)
+        R, q, grad = L.DeviceArray(ctx, p.n_dofs), L.DeviceArray(ctx, p.n_dofs), L.DeviceArray(ctx, p.n_elem)
+        L.check(L.hip().lmh_element_poisson(ctx.h, g.mesh, g.dofmap, npts, kd.ptr, 0, 0, K.ptr, F.ptr))
+        g.residual_poisson(npts, kd, 0, us, R)
+        g.qoi_box_derivative(npts, -1e300, 1e300, q)
+        g.adjoint_kappa_gradient(npts, kd, ud, ld, grad)
+        got.append([np.ldexp(a.download(), -e * k) for a, e in ((K, 1), (F, 3), (R, 3), (q, 3), (grad, 1))])
+        g.close()
+    for name, a, b in zip(("K", "F", "residual", "qoi", "gradient"), *got):
+        assert np.array_equal(a, b), name
