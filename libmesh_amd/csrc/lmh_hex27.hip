@@ -51,7 +51,10 @@ struct H27Slots {
 // nodal coordinates: formed from absolute ones it loses the digits that the
 // element's place takes.  64^3 matrices against 80-bit arithmetic, largest error of
 // an entry over the largest entry, mean of 24 elements: absolute 3.7e-15 (sums over
-// a table 3.1e-15), relative 2.0e-16; as fast (536-545 us, 541).
+// a table 3.1e-15), relative 2.0e-16.  The matrix kernel takes 453 -> 466 us for
+// 64^3 with f = 1, 74 -> 70 for 31 x 29 x 37 with the sine; 40^3 residual 32.2 ->
+// 33.8, QoI 21.4 -> 20.9, adjoint 30.3 -> 30.5, every load issued before the first
+// use (one after the other: residual 34.9, adjoint 33.2).
 template <int NF, int ST>
 __device__ inline void h27_store_nodes(const H27Slots &sl, const double (&x)[3][3], double *s_f, double *s_c) {
 #pragma unroll
@@ -61,12 +64,17 @@ __device__ inline void h27_store_nodes(const H27Slots &sl, const double (&x)[3][
       for (int c = 0; c < 3; ++c) s_c[sl.el[m] * 4 + c] = x[m][c];
     }
   h27_sync();
+  double r[3][3];  // idle slots' too: no branch between the reads
+#pragma unroll
+  for (int m = 0; m < 3; ++m)
+#pragma unroll
+    for (int c = 0; c < 3; ++c) r[m][c] = x[m][c] - s_c[sl.el[m] * 4 + c];
 #pragma unroll
   for (int m = 0; m < 3; ++m)
     if (sl.live[m]) {
       double *d = s_f + sl.el[m] * ST + sl.lat[m] * NF;
 #pragma unroll
-      for (int c = 0; c < 3; ++c) d[c] = x[m][c] - s_c[sl.el[m] * 4 + c];
+      for (int c = 0; c < 3; ++c) d[c] = r[m][c];
     }
 }
 
@@ -95,14 +103,17 @@ __global__ __launch_bounds__(64, 3) void k_hex27_residual(const double *__restri
     sl.ids(edofs, gr * kH27PerWave, total, lane, dof);
     const H27Lane L(lg);
     const int64_t e0 = gr * kH27PerWave, e = e0 + L.el;
-    double x[3][3];
+    double x[3][3], um[3];
 #pragma unroll
     for (int m = 0; m < 3; ++m) {
 #pragma unroll
       for (int c = 0; c < 3; ++c) x[m][c] = xyz[3 * (int64_t)nd[m] + c];
-      if (sl.live[m]) s_f[sl.el[m] * ST + sl.lat[m] * NF + 3] = u[dof[m]];
+      um[m] = u[dof[m]];
     }
     h27_store_nodes<NF, ST>(sl, x, s_f, s_c);
+#pragma unroll
+    for (int m = 0; m < 3; ++m)
+      if (sl.live[m]) s_f[sl.el[m] * ST + sl.lat[m] * NF + 3] = um[m];
     const bool on = L.el < kH27PerWave && e < ne;
     h27_sync();
     if (on) {
@@ -263,21 +274,25 @@ __global__ __launch_bounds__(64, 3) void k_hex27_adjoint(const double *__restric
     sl.ids(edofs, gr * kH27PerWave, total, lane, dof);
     const H27Lane L(lg);
     const int64_t e = gr * kH27PerWave + L.el;
-    double x[3][3];
+    // all loads issued before any is looked at
+    double x[3][3], um[3], lm[3];
+    int cv[3];
 #pragma unroll
     for (int m = 0; m < 3; ++m) {
 #pragma unroll
       for (int c = 0; c < 3; ++c) x[m][c] = xyz[3 * (int64_t)nd[m] + c];
-      // all loads issued before the mask is looked at
-      const double um = u[dof[m]], lm = lam[dof[m]];
-      const bool c = cons[dof[m]] != 0;
-      if (sl.live[m]) {
-        double *d = s_f + sl.el[m] * ST + sl.lat[m] * NF;
-        d[3] = c ? 0.0 : um;
-        d[4] = c ? 0.0 : lm;
-      }
+      cv[m] = cons[dof[m]];
+      um[m] = u[dof[m]];
+      lm[m] = lam[dof[m]];
     }
     h27_store_nodes<NF, ST>(sl, x, s_f, s_c);
+#pragma unroll
+    for (int m = 0; m < 3; ++m)
+      if (sl.live[m]) {
+        double *d = s_f + sl.el[m] * ST + sl.lat[m] * NF;
+        d[3] = cv[m] ? 0.0 : um[m];
+        d[4] = cv[m] ? 0.0 : lm[m];
+      }
     const bool on = L.el < kH27PerWave && e < ne;
     h27_sync();
     double s = 0.0;
@@ -376,14 +391,18 @@ __global__ __launch_bounds__(64, 3) void k_hex27_poisson(const double *__restric
     const int cnt = (int)(ne - e0 < per ? ne - e0 : per);
     unsigned long long bits[3];  // constrained flags, bit 27 el + node of the group
     double x[3][3];
+    int cv[3];
 #pragma unroll
-    for (int m = 0; m < 3; ++m) {
+    for (int m = 0; m < 3; ++m) cv[m] = cons[dof[m]];
+#pragma unroll
+    for (int m = 0; m < 3; ++m)
 #pragma unroll
       for (int c = 0; c < 3; ++c) x[m][c] = xyz[3 * (int64_t)nd[m] + c];
-      const bool c = cons[dof[m]] != 0;
-      bits[m] = constrain ? __ballot(c && sl.live[m]) : 0ull;
-    }
+    // loaded with the rest, not one after the other where they are used
+    asm volatile("" : "+v"(cv[0]), "+v"(cv[1]), "+v"(cv[2]));
     h27_store_nodes<NF, ST>(sl, x, s_buf, s_c);
+#pragma unroll
+    for (int m = 0; m < 3; ++m) bits[m] = constrain ? __ballot(cv[m] != 0 && sl.live[m]) : 0ull;
     auto mask_of = [&](int el) -> unsigned {  // 27 flags of element el, by local node
       const int b = 27 * el, w = b >> 6, o = b & 63;
       unsigned long long v = bits[0];
