@@ -229,7 +229,7 @@ struct lmh_matrix {
   uint16_t *off = nullptr;  // n_elem*dpe*dpe slot offsets within rows
   // row tiles of the gather scatter (lmh_scatter.hip): {first row, rows,
   // sequence start, steps}, incidence sequence, slot offsets (8-bit, 16-bit
-  // when wide), LDS entries of a tile
+  // when wide), LDS entries of a tile; one allocation at st_tile
   int4 *st_tile = nullptr;
   int2 *st_seq = nullptr;
   void *st_map = nullptr;
@@ -290,7 +290,7 @@ int fe_table(lmh_context *ctx, int type, int arg, const FETable **out);
 int matrix_create_impl(lmh_context *ctx, const lmh_dofmap *dm, bool colour, bool fp64, lmh_matrix **out,
                        std::vector<int32_t> *row_ptr = nullptr);
 // row tiles of a matrix's gather scatter, and the scatter on them
-int matrix_build_tiles(lmh_matrix *A, const std::vector<int32_t> &h_rp);
+int matrix_build_tiles(lmh_matrix *A, const std::vector<int32_t> &h_rp, std::vector<int32_t> &rows);
 template <typename T>
 int scatter_tiles(lmh_matrix *A, const T *Ke, const double *Fe, T *vals, double *rhs);
 // general constraints around the scatter: before it, the general elements'

@@ -75,35 +75,67 @@ __global__ __launch_bounds__(256) void k_tile_count(const int32_t *__restrict__ 
 }
 
 // seq: {incidence (element * dpe + local row) or -1, entry base | row << 16}, within the tile
+__device__ inline void tile_fill(const int32_t *__restrict__ inc_ptr, const int32_t *__restrict__ inc,
+                                 const int32_t *__restrict__ rp, int32_t r0, int32_t nr, int32_t s0, int pi,
+                                 int2 *seq, int4 *__restrict__ tile) {
+  const int32_t b0 = rp[r0];
+  const int len = tile_walk(
+      inc_ptr, r0, nr, pi,
+      [&](int pos, int32_t k, int r) { seq[s0 + pos] = make_int2(inc[k], (rp[r0 + r] - b0) | (r << 16)); },
+      [&](int pos) { seq[s0 + pos] = make_int2(-1, 0); });
+  if ((threadIdx.x & 63) == 0) *tile = make_int4(r0, nr, s0, len / pi);
+}
+
 __global__ __launch_bounds__(256) void k_tile_fill(const int32_t *__restrict__ inc_ptr,
                                                    const int32_t *__restrict__ inc, const int32_t *__restrict__ rp,
                                                    const int32_t *__restrict__ tr, const int32_t *__restrict__ start,
                                                    int64_t nt, int pi, int2 *__restrict__ seq,
                                                    int4 *__restrict__ tile) {
-  for (int64_t t = blockIdx.x * (int64_t)4 + (threadIdx.x >> 6); t < nt; t += (int64_t)gridDim.x * 4) {
-    const int32_t r0 = tr[t], nr = tr[t + 1] - r0, s0 = start[t], b0 = rp[r0];
-    const int len = tile_walk(
-        inc_ptr, r0, nr, pi,
-        [&](int pos, int32_t k, int r) { seq[s0 + pos] = make_int2(inc[k], (rp[r0 + r] - b0) | (r << 16)); },
-        [&](int pos) { seq[s0 + pos] = make_int2(-1, 0); });
-    if ((threadIdx.x & 63) == 0) tile[t] = make_int4(r0, nr, s0, len / pi);
-  }
+  for (int64_t t = blockIdx.x * (int64_t)4 + (threadIdx.x >> 6); t < nt; t += (int64_t)gridDim.x * 4)
+    tile_fill(inc_ptr, inc, rp, tr[t], tr[t + 1] - tr[t], start[t], pi, seq, tile + t);
 }
 
-// Offsets of every sequence entry: lane (g, j) of step I reads its kTileQuad
+// Offset j of sequence entry s: lane (g, j) of step I reads its kTileQuad
 // consecutive steps' offsets at once, at ((I / quad) * 64 + lane) * quad + I % quad.
+template <typename OT>
+__device__ inline void tile_offset(const int2 *seq, int64_t s, int j, int dpe, int gs, int pi,
+                                   const uint16_t *__restrict__ off, OT *__restrict__ map) {
+  const int64_t I = s / pi;
+  const int lane = (int)(s - I * pi) * gs + j;
+  const int32_t ei = seq[s].x;
+  map[((I / kTileQuad) * 64 + lane) * kTileQuad + I % kTileQuad] =
+      ei >= 0 && j < dpe ? (OT)off[(int64_t)ei * dpe + j] : (OT)0;
+}
+
 template <typename OT>
 __global__ __launch_bounds__(256) void k_tile_map(const int2 *__restrict__ seq, int64_t total, int dpe, int gs,
                                                   const uint16_t *__restrict__ off, OT *__restrict__ map) {
   const int pi = 64 / gs;
   for (int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; t < total * gs;
-       t += (int64_t)gridDim.x * blockDim.x) {
-    const int64_t s = t / gs, I = s / pi;
-    const int j = (int)(t - s * gs), lane = (int)(s - I * pi) * gs + j;
-    const int32_t ei = seq[s].x;
-    const OT o = ei >= 0 && j < dpe ? (OT)off[(int64_t)ei * dpe + j] : (OT)0;
-    map[((I / kTileQuad) * 64 + lane) * kTileQuad + I % kTileQuad] = o;
-  }
+       t += (int64_t)gridDim.x * blockDim.x)
+    tile_offset(seq, t / gs, (int)(t % gs), dpe, gs, pi, off, map);
+}
+
+// The whole plan of a small matrix in one launch: a wavefront per tile, whose place
+// in the sequence comes from a counter (which tile comes first makes no difference).
+template <typename OT>
+__global__ __launch_bounds__(256) void k_tile_plan(const int32_t *__restrict__ inc_ptr,
+                                                   const int32_t *__restrict__ inc, const int32_t *__restrict__ rp,
+                                                   const int32_t *__restrict__ tr, int64_t nt, int dpe, int gs,
+                                                   const uint16_t *__restrict__ off, int32_t *__restrict__ count,
+                                                   int2 *seq, int4 *__restrict__ tile, OT *__restrict__ map) {
+  const int64_t t = blockIdx.x * (int64_t)4 + (threadIdx.x >> 6);
+  if (t >= nt) return;
+  const int lane = threadIdx.x & 63, pi = 64 / gs;
+  const int32_t r0 = tr[t], nr = tr[t + 1] - r0;
+  const int len = tile_walk(
+      inc_ptr, r0, nr, pi, [](int, int32_t, int) {}, [](int) {});
+  int32_t s0 = 0;
+  if (lane == 0) s0 = atomicAdd(count, len);
+  s0 = __shfl(s0, 0);
+  tile_fill(inc_ptr, inc, rp, r0, nr, s0, pi, seq, tile + t);
+  __threadfence_block();  // the lanes read each other's entries
+  for (int u = lane; u < len * gs; u += 64) tile_offset(seq, s0 + u / gs, u % gs, dpe, gs, pi, off, map);
 }
 
 // FP64: the LDS adder (no value returns to the wavefront, so a step does not
@@ -191,10 +223,21 @@ __global__ __launch_bounds__(64) void k_scatter_tiles(const int4 *__restrict__ t
 
 static int group_lanes(int dpe) { return dpe <= 4 ? 4 : dpe <= 8 ? 8 : dpe <= 16 ? 16 : 32; }
 
+// Small matrices: the plan in one launch and one allocation, whose sequence is sized
+// for the worst case (every incidence alone in its step) instead of counted first
+// and waited for.  Matrix creation, without a plan / counted first / this way: Q1
+// 8^3 383, 467, 390 us, Q2 4^3 385, 468, 394, TET10 3^3 462, 559, 468.  Up to 2 MB, of
+// which a Q1 matrix uses a fifth, or 8 MB where the matrix's values take as much (Q2,
+// whose plan fills half of it).
+static bool plan_worst_case(size_t bytes, size_t values) {
+  return bytes <= (2 << 20) || (bytes <= (8 << 20) && bytes <= values);
+}
+
 // Tiles of the matrix's rows; h_rp: its row pointers.  Patterns the tiles do
-// not take (more than 32 element DoFs, a row beyond 4096 entries) keep the
-// row-at-a-time kernel.
-int matrix_build_tiles(lmh_matrix *A, const std::vector<int32_t> &h_rp) {
+// not take (more than 32 element DoFs, a row beyond 4096 entries) and matrices
+// without room for the plan keep the row-at-a-time kernel.  `rows` holds what a
+// copy on the stream may still read: for the caller to keep until it has waited.
+int matrix_build_tiles(lmh_matrix *A, const std::vector<int32_t> &h_rp, std::vector<int32_t> &rows) {
   const lmh_dofmap *dm = A->dm;
   lmh_context *ctx = A->ctx;
   if (!dm || dm->dpe > 32 || A->max_row > 4096 || A->rows == 0) return LMH_OK;
@@ -202,42 +245,81 @@ int matrix_build_tiles(lmh_matrix *A, const std::vector<int32_t> &h_rp) {
   // small matrices: fewer entries per tile, so that every CU has several
   const int64_t want = A->nnz / ((int64_t)ctx->cu_count * 8);
   const int cap = (int)std::min<int64_t>(kTileSlots, std::max<int64_t>(64, want));
-  std::vector<int32_t> tr{0};
+  rows.assign(1, 0);
   for (int64_t r = 0; r < A->rows; ++r) {
-    const int32_t f = tr.back();
-    if (r > f && (h_rp[r + 1] - h_rp[f] > cap || r - f >= kTileRows)) tr.push_back((int32_t)r);
+    const int32_t f = rows.back();
+    if (r > f && (h_rp[r + 1] - h_rp[f] > cap || r - f >= kTileRows)) rows.push_back((int32_t)r);
   }
-  tr.push_back((int32_t)A->rows);
-  const int64_t nt = (int64_t)tr.size() - 1;
-  int32_t *tmp = nullptr;  // tile rows, lengths, starts: nt + 1 each
-  LMH_HIP(hipMallocAsync((void **)&tmp, sizeof(int32_t) * 3 * (nt + 1), ctx->stream));
-  int32_t *dtr = tmp, *len = tmp + nt + 1, *start = len + nt + 1;
-  LMH_HIP(hipMemcpyAsync(dtr, tr.data(), sizeof(int32_t) * tr.size(), hipMemcpyHostToDevice, ctx->stream));
-  LMH_HIP(hipMemsetAsync(len, 0, sizeof(int32_t) * (nt + 1), ctx->stream));
-  const int g = grid_for(nt, 4, 16384);
-  LMH_LAUNCH(ctx, "tile_plan", k_tile_count, dim3(g), dim3(256), 0, dm->inc_ptr, (const int32_t *)dtr, nt, pi,
-             len);
-  LMH_TRY(check_launch("k_tile_count"));
-  int64_t total = 0;
-  LMH_TRY(exclusive_scan_i32(ctx, len, start, nt, &total));
-  LMH_HIP(hipMalloc((void **)&A->st_tile, sizeof(int4) * nt));
-  LMH_HIP(hipMalloc((void **)&A->st_seq, sizeof(int2) * std::max<int64_t>(1, total)));
-  LMH_LAUNCH(ctx, "tile_plan", k_tile_fill, dim3(g), dim3(256), 0, dm->inc_ptr, dm->inc, A->rp,
-             (const int32_t *)dtr, (const int32_t *)start, nt, pi, A->st_seq, A->st_tile);
-  LMH_TRY(check_launch("k_tile_fill"));
+  rows.push_back((int32_t)A->rows);
+  const int64_t nt = (int64_t)rows.size() - 1;
+  rows.push_back(0);  // k_tile_plan's counter
   const bool wide = A->max_row > 256;
-  LMH_HIP(hipMalloc(&A->st_map, (wide ? 2 : 1) * (size_t)std::max<int64_t>(1, total) * gs));
-  if (total > 0) {
-    const int gm = grid_for(total * gs, 256, 16384);
+  // tiles, sequence, offsets and `more` bytes in one allocation
+  auto allocate = [&](int64_t total, size_t more) {
+    const size_t seq = sizeof(int4) * nt, map = seq + ((sizeof(int2) * total + 15) & ~(size_t)15),
+                 end = map + (((wide ? 2 : 1) * (size_t)total * gs + 15) & ~(size_t)15);
+    if (hipMalloc((void **)&A->st_tile, end + more) != hipSuccess) {
+      (void)hipGetLastError();
+      A->st_tile = nullptr;
+      return (unsigned char *)nullptr;
+    }
+    unsigned char *m = (unsigned char *)A->st_tile;
+    A->st_seq = (int2 *)(m + seq);
+    A->st_map = m + map;
+    return m + end;
+  };
+  const int64_t most = dm->mesh->n_elem * dm->dpe * pi + nt * (int64_t)(pi * kTileQuad);
+  if (plan_worst_case((size_t)most * (8 + gs * (wide ? 2 : 1)), sizeof(double) * (size_t)A->nnz)) {
+    int32_t *dtr = (int32_t *)allocate(most, sizeof(int32_t) * rows.size());
+    if (!dtr) return LMH_OK;
+    LMH_HIP(hipMemcpyAsync(dtr, rows.data(), sizeof(int32_t) * rows.size(), hipMemcpyHostToDevice, ctx->stream));
+    const dim3 g((unsigned)((nt + 3) / 4));
     if (wide)
-      LMH_LAUNCH(ctx, "tile_plan", k_tile_map<uint16_t>, dim3(gm), dim3(256), 0, A->st_seq, total, dm->dpe, gs, A->off,
+      LMH_LAUNCH(ctx, "tile_plan", k_tile_plan<uint16_t>, g, dim3(256), 0, dm->inc_ptr, dm->inc, A->rp,
+                 (const int32_t *)dtr, nt, dm->dpe, gs, A->off, dtr + nt + 1, A->st_seq, A->st_tile,
                  (uint16_t *)A->st_map);
     else
-      LMH_LAUNCH(ctx, "tile_plan", k_tile_map<uint8_t>, dim3(gm), dim3(256), 0, A->st_seq, total, dm->dpe, gs, A->off,
+      LMH_LAUNCH(ctx, "tile_plan", k_tile_plan<uint8_t>, g, dim3(256), 0, dm->inc_ptr, dm->inc, A->rp,
+                 (const int32_t *)dtr, nt, dm->dpe, gs, A->off, dtr + nt + 1, A->st_seq, A->st_tile,
                  (uint8_t *)A->st_map);
-    LMH_TRY(check_launch("k_tile_map"));
+    LMH_TRY(check_launch("k_tile_plan"));
+  } else {
+    int32_t *tmp = nullptr;  // tile rows, lengths, starts: nt + 1 each
+    if (hipMallocAsync((void **)&tmp, sizeof(int32_t) * 3 * (nt + 1), ctx->stream) != hipSuccess) {
+      (void)hipGetLastError();
+      return LMH_OK;
+    }
+    int32_t *dtr = tmp, *len = tmp + nt + 1, *start = len + nt + 1;
+    auto plan = [&]() -> int {
+      LMH_HIP(hipMemcpyAsync(dtr, rows.data(), sizeof(int32_t) * (nt + 1), hipMemcpyHostToDevice, ctx->stream));
+      LMH_HIP(hipMemsetAsync(len, 0, sizeof(int32_t) * (nt + 1), ctx->stream));
+      const int g = grid_for(nt, 4, 16384);
+      LMH_LAUNCH(ctx, "tile_plan", k_tile_count, dim3(g), dim3(256), 0, dm->inc_ptr, (const int32_t *)dtr, nt, pi,
+                 len);
+      LMH_TRY(check_launch("k_tile_count"));
+      int64_t total = 0;
+      const int rc = exclusive_scan_i32(ctx, len, start, nt, &total);
+      if (rc == LMH_ERR_UNSUPPORTED) return LMH_OK;  // a sequence beyond 32-bit places
+      LMH_TRY(rc);
+      if (!allocate(total, 0)) return LMH_OK;
+      LMH_LAUNCH(ctx, "tile_plan", k_tile_fill, dim3(g), dim3(256), 0, dm->inc_ptr, dm->inc, A->rp,
+                 (const int32_t *)dtr, (const int32_t *)start, nt, pi, A->st_seq, A->st_tile);
+      LMH_TRY(check_launch("k_tile_fill"));
+      if (total == 0) return LMH_OK;
+      const int gm = grid_for(total * gs, 256, 16384);
+      if (wide)
+        LMH_LAUNCH(ctx, "tile_plan", k_tile_map<uint16_t>, dim3(gm), dim3(256), 0, A->st_seq, total, dm->dpe, gs,
+                   A->off, (uint16_t *)A->st_map);
+      else
+        LMH_LAUNCH(ctx, "tile_plan", k_tile_map<uint8_t>, dim3(gm), dim3(256), 0, A->st_seq, total, dm->dpe, gs,
+                   A->off, (uint8_t *)A->st_map);
+      return check_launch("k_tile_map");
+    };
+    const int rc = plan();
+    (void)hipFreeAsync(tmp, ctx->stream);
+    LMH_TRY(rc);
+    if (!A->st_tile) return LMH_OK;
   }
-  LMH_HIP(hipFreeAsync(tmp, ctx->stream));
   A->st_wide = wide;
   A->st_slots = std::max(cap, A->max_row);
   A->n_stile = nt;

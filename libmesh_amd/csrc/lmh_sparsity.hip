@@ -283,7 +283,8 @@ int matrix_create_impl(lmh_context *ctx, const lmh_dofmap *dm, bool colour, bool
     LMH_CHECK(!bad, LMH_ERR_INVALID, "internal: expanded DoF pair missing from the sparsity pattern");
   }
 
-  if (fp64) LMH_TRY(matrix_build_tiles(A.get(), rp));
+  std::vector<int32_t> tile_rows;  // read by a copy until the wait below
+  if (fp64) LMH_TRY(matrix_build_tiles(A.get(), rp, tile_rows));
   if (fp64) {
     LMH_HIP(hipMalloc((void **)&A->vals, sizeof(double) * (nnz + LMH_PAD)));
     LMH_HIP(hipMemsetAsync(A->vals, 0, sizeof(double) * (nnz + LMH_PAD), ctx->stream));
@@ -374,8 +375,6 @@ int lmh_matrix_destroy(lmh_matrix *A) {
   (void)hipFree(A->vals_t);
   (void)hipFree(A->off);
   (void)hipFree(A->st_tile);
-  (void)hipFree(A->st_seq);
-  (void)hipFree(A->st_map);
   (void)hipFree(A->diag);
   (void)hipFree(A->color_elems);
   (void)hipFree(A->Ke);

@@ -41,3 +41,12 @@ def test_scatter_is_the_sequential_sum(ctx, t, nv, box):
     L.check(L.hip().lmh_matrix_scatter_elements(g.matrix, None, Fd.ptr, R.ptr))
     assert np.array_equal(R.download(), rhs)
     g.close()
+
+
+@pytest.mark.parametrize("t,nv,box", [
+    (L.HEX8, 1, (11, 11, 11)), (L.HEX8, 1, (12, 12, 12)), (L.HEX27, 1, (13, 13, 13)), (L.HEX27, 1, (15, 15, 15)),
+    (L.TET4, 1, (4, 4, 4)), (L.TET4, 1, (5, 5, 6)), (L.TET10, 1, (3, 3, 3)), (L.TET10, 1, (5, 5, 5)),
+    (L.TET10, 3, (2, 2, 2)), (L.TET10, 3, (3, 3, 3))])
+def test_both_ways_to_the_plan(ctx, t, nv, box):
+    """On each side of the size to which the plan is made in one launch"""
+    test_scatter_is_the_sequential_sum(ctx, t, nv, box)
