@@ -1433,15 +1433,25 @@ static int try_windows(lmh_matrix *A, std::vector<int32_t> rb, bool split, bool 
   if (IW == 1) total = nrb * W8_UCAP;
   if (total > INT32_MAX) return LMH_OK;
   const size_t idx_bytes = sizeof(widx_t<IW>) * std::max<int64_t>(1, nrb) * CAP;
-  LMH_HIP(hipMalloc((void **)&widx, idx_bytes));
-  LMH_HIP(hipMemsetAsync(widx, 0, idx_bytes, ctx->stream));
-  if (A->vals) {  // FP64 operator: its chunks hold two entries
-    LMH_HIP(hipMalloc((void **)&widx64, idx_bytes));
-    LMH_HIP(hipMemsetAsync(widx64, 0, idx_bytes, ctx->stream));
+  auto drop = [&] {
+    (void)hipFree(widx);
+    (void)hipFree(widx64);
+    (void)hipFree(woff);
+    (void)hipFree(meta);
+  };
+  // without room for the windows the products use the int32 columns
+  if (hipMalloc((void **)&widx, idx_bytes) != hipSuccess ||
+      (A->vals && hipMalloc((void **)&widx64, idx_bytes) != hipSuccess) ||  // FP64 chunks hold two entries
+      hipMalloc((void **)&woff, sizeof(uint16_t) * (total + LMH_PAD)) != hipSuccess ||
+      hipMalloc((void **)&meta, sizeof(int4) * 2 * (nrb ? nrb : 1)) != hipSuccess) {
+    (void)hipGetLastError();
+    drop();
+    LMH_HIP(hipStreamSynchronize(ctx->stream));  // w0 is read by the copy above
+    return LMH_OK;
   }
-  LMH_HIP(hipMalloc((void **)&woff, sizeof(uint16_t) * (total + LMH_PAD)));
+  LMH_HIP(hipMemsetAsync(widx, 0, idx_bytes, ctx->stream));
+  if (widx64) LMH_HIP(hipMemsetAsync(widx64, 0, idx_bytes, ctx->stream));
   LMH_HIP(hipMemsetAsync(woff, 0, sizeof(uint16_t) * (total + LMH_PAD), ctx->stream));
-  LMH_HIP(hipMalloc((void **)&meta, sizeof(int4) * 2 * (nrb ? nrb : 1)));
   LMH_HIP(hipMemsetAsync(ctx->d_flags, 0, sizeof(int), ctx->stream));
   LMH_LAUNCH(ctx, "build_windows", (k_build_windows<false, CAP, IW>), dim3(grid_for(nrb, 1, 16384)), dim3(BLK), 0,
              (const int32_t *)rbd.p, nrb, A->rp, A->ci, (int32_t *)wsz.p, widx, widx64, woff, meta, ctx->d_flags);
@@ -1450,10 +1460,7 @@ static int try_windows(lmh_matrix *A, std::vector<int32_t> rb, bool split, bool 
   LMH_HIP(hipMemcpyAsync(&bad, ctx->d_flags, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
   LMH_HIP(hipStreamSynchronize(ctx->stream));
   if (bad) {  // not expected: the counting pass accepted every block
-    LMH_HIP(hipFree(widx));
-    LMH_HIP(hipFree(widx64));
-    LMH_HIP(hipFree(woff));
-    LMH_HIP(hipFree(meta));
+    drop();
     return LMH_OK;
   }
   A->widx32 = widx;
