@@ -28,3 +28,24 @@ def test_degenerate_flag_of_a_failed_call(ctx, precision):
     good.assemble_poisson(2, None, 0, c, precision)
     bad.close()
     good.close()
+
+
+@pytest.mark.parametrize("t,npts,box", [(L.HEX8, 2, (2, 2, 2)), (L.HEX8, 2, (26, 26, 25)), (L.HEX8, 3, (2, 2, 2)),
+                                        (L.HEX27, 3, (2, 2, 2)), (L.HEX27, 2, (2, 2, 2)), (L.TET4, 3, (2, 2, 2)),
+                                        (L.TET10, 5, (2, 2, 2))])
+def test_nan_coordinate_is_refused(ctx, t, npts, box):
+    """By every element kernel alike: a determinant that is not a number is not positive"""
+    p = L.Problem(box[0], t, 1, L.ALL_FACES, box[1], box[2])
+    xyz = p.coords.copy()
+    xyz[p.conn[p.n_elem // 2, 0], 1] = float("nan")
+    g = L.GpuProblem(ctx, xyz, p.conn, p.elem_type, p.elem_dofs, p.n_dofs, p.constrained)
+    b, u = L.DeviceArray(ctx, p.n_dofs), L.DeviceArray(ctx, p.n_dofs)
+    k, grad = L.DeviceArray(ctx, p.n_elem), L.DeviceArray(ctx, p.n_elem)
+    u.zero()
+    k.zero()
+    for call in (lambda: g.assemble_poisson(npts, None, 0, b), lambda: g.assemble_poisson(npts, None, 1, b, L.FP32),
+                 lambda: g.residual_poisson(npts, None, 0, u, b), lambda: g.qoi_box_derivative(npts, 0.0, 1.0, b),
+                 lambda: g.adjoint_kappa_gradient(npts, k, u, u, grad)):
+        with pytest.raises(L.LmhError, match="degenerate"):
+            call()
+    g.close()

@@ -131,3 +131,29 @@ def test_empty_row(ctx):
         assert np.linalg.norm(x.download() - ref) <= 4e-11 * np.sqrt(300) * np.linalg.norm(ref)
     finally:
         L.hip().lmh_matrix_destroy(h)
+
+
+@pytest.mark.parametrize("n,length", [(2100, 2048), (4096, 4096)])
+def test_longest_rows(ctx, n, length):
+    """A row over 256 threads of the workgroup, whose pieces its owner adds alone"""
+    rng = np.random.default_rng(7)
+    A = arrow(rng, n, length)
+    b = rng.standard_normal(n)
+    rp, ci = A.indptr.astype(np.int32), A.indices.astype(np.int32)
+    h = C.c_void_p()
+    L.check(L.hip().lmh_matrix_create_csr(ctx.h, n, L._ptr(rp), L._ptr(ci), C.byref(h)))
+    try:
+        L.check(L.hip().lmh_matrix_set_values(h, L._ptr(A.data)))
+        ref, ref_its = reference(A, b, True, 1e-11)
+        bd, x = L.DeviceArray(ctx, n, data=b), L.DeviceArray(ctx, n)
+        x.zero()
+        its, res, why = C.c_int64(), C.c_double(), C.c_int()
+        ctx.profile_reset()
+        ctx.profile(True)
+        L.check(L.hip().lmh_cg_solve(h, bd.ptr, x.ptr, 1e-11, 5000, C.byref(its), C.byref(res), C.byref(why)))
+        ctx.profile(False)
+        assert ctx.profile_query("cg_small")[1] == 1
+        assert why.value == L.CONVERGED_RTOL and abs(its.value - ref_its) <= 1
+        assert np.linalg.norm(x.download() - ref) <= 4e-11 * np.sqrt(n) * np.linalg.norm(ref)
+    finally:
+        L.hip().lmh_matrix_destroy(h)
