@@ -210,8 +210,8 @@ __global__ __launch_bounds__(256) void k_poisson_hex8(const double *__restrict__
 
 // ---------------------------------------------------------------------------
 // Scatter Ke/Fe -> CSR values / rhs.
-// Gather form: tiles of rows (lmh_scatter.hip), or for elements they do not
-// take (more than 32 DoFs) one wave per row; the row's slots accumulate in LDS over the
+// Gather form: tiles of rows (lmh_scatter.hip), or without them a half-wave per
+// row (up to 32 element DoFs) or one wave per row; the row's slots accumulate in LDS over the
 // row's incidences in ascending (element, local index) order -- the same
 // summation order as the element loop of the reference -- then the row is
 // written once.  Coloured form: one launch per colour, every (element, i, j)
@@ -244,6 +244,67 @@ __global__ __launch_bounds__(64) void k_scatter_gather(const int32_t *__restrict
     for (int t = lane; t < len; t += 64) vals[b + t] = acc[t];
     if (rhs && lane == 0) rhs[r] = f;
     __syncthreads();
+  }
+}
+
+// The same gather for element DoF counts up to 32: each half-wave owns a row
+// (two rows per wave), and a row's incidences are taken in chunks of GC
+// whose element matrix rows and slot offsets are all loaded before any is
+// added, so a row waits on one round of loads instead of one per incidence.
+// The adds still go in ascending incidence order (one wave executes its LDS
+// operations in program order, so no barrier is needed between them): the
+// sums are bit-identical to k_scatter_gather's.  For small tetrahedral matrices and
+// where there is no plan for tiles (matrix_build_tiles).
+template <typename T>
+__global__ __launch_bounds__(64) void k_scatter_rows(const int32_t *__restrict__ inc_ptr,
+                                                     const int32_t *__restrict__ inc, int dpe, int64_t n_rows,
+                                                     const int32_t *__restrict__ rp,
+                                                     const uint16_t *__restrict__ off, const T *__restrict__ Ke,
+                                                     const double *__restrict__ Fe, T *__restrict__ vals,
+                                                     double *__restrict__ rhs, int stride) {
+  constexpr int GC = 8;
+  extern __shared__ unsigned char smraw[];
+  const int lane = threadIdx.x, h = lane >> 5, hl = lane & 31;
+  T *acc = (T *)smraw + h * stride;
+  int64_t rlo, rhi;
+  block_range(n_rows, rlo, rhi);
+  for (int64_t rb = rlo; rb < rhi; rb += 2) {
+    const int64_t r = rb + h;
+    const bool live = r < rhi;
+    const int32_t b = live ? rp[r] : 0, len = live ? rp[r + 1] - b : 0;
+    for (int t = hl; t < len; t += 32) acc[t] = (T)0;
+    const int32_t k0 = live ? inc_ptr[r] : 0, k1 = live ? inc_ptr[r + 1] : 0;
+    double f = 0.0;
+    for (int32_t kc = k0; kc < k1; kc += GC) {
+      const int nc = k1 - kc < GC ? k1 - kc : GC;
+      int64_t ei[GC];
+      T v[GC];
+      uint16_t o[GC];
+#pragma unroll
+      for (int c = 0; c < GC; ++c) ei[c] = inc[kc + (c < nc ? c : 0)];
+#pragma unroll
+      for (int c = 0; c < GC; ++c) {
+        const int64_t at = ei[c] * dpe + (hl < dpe ? hl : 0);
+        v[c] = Ke[at];
+        o[c] = off[at];
+      }
+      double fv[GC];
+      if (rhs)
+#pragma unroll
+        for (int c = 0; c < GC; ++c) fv[c] = Fe[ei[c]];
+#pragma unroll
+      for (int c = 0; c < GC; ++c)
+        if (c < nc) {
+          if (hl < dpe) acc[o[c]] += v[c];
+          if (rhs) f += fv[c];
+          // the next incidence's lanes read what these wrote: LDS keeps a wave's order
+          __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+          __builtin_amdgcn_wave_barrier();
+          __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        }
+    }
+    for (int t = hl; t < len; t += 32) vals[b + t] = acc[t];
+    if (rhs && live && hl == 0) rhs[r] = f;
   }
 }
 
@@ -569,6 +630,14 @@ static int scatter_impl(lmh_matrix *A, const T *Ke, const double *Fe, T *vals, d
   lmh_context *ctx = A->ctx;
   const lmh_dofmap *dm = A->dm;
   if (scatter == LMH_SCATTER_GATHER && A->n_stile > 0) return scatter_tiles<T>(A, Ke, Fe, vals, rhs);
+  const int stride = (int)((A->max_row + 1) & ~1);
+  if (scatter == LMH_SCATTER_GATHER && dm->dpe <= 32 && sizeof(T) * 2 * (size_t)stride <= 32768) {
+    const int g = (int)std::min<int64_t>((A->rows + 1) / 2, (int64_t)ctx->cu_count * LMH_SCATTER_PER_CU);
+    LMH_LAUNCH(ctx, sizeof(T) == 8 ? "scatter_gather_fp64" : "scatter_gather_fp32", k_scatter_rows<T>, dim3(g),
+               dim3(64), sizeof(T) * 2 * stride, dm->inc_ptr, dm->inc, dm->dpe, A->rows, A->rp, A->off, Ke, Fe, vals,
+               rhs, stride);
+    return check_launch("k_scatter_rows");
+  }
   if (scatter == LMH_SCATTER_GATHER) {
     const int g = (int)std::min<int64_t>(A->rows, (int64_t)ctx->cu_count * LMH_SCATTER_PER_CU);
     LMH_LAUNCH(ctx, sizeof(T) == 8 ? "scatter_gather_fp64" : "scatter_gather_fp32", k_scatter_gather<T>, dim3(g),

@@ -233,14 +233,26 @@ static bool plan_worst_case(size_t bytes, size_t values) {
   return bytes <= (2 << 20) || (bytes <= (8 << 20) && bytes <= values);
 }
 
+// Below this many rows a tetrahedral matrix has no tiles.  Its rows have up to 24
+// incidences and a few entries, so a tile's steps are a long chain with most of
+// their lane groups idle; two rows to a wavefront (k_scatter_rows) end sooner while
+// the GPU holds all of them.  A scatter among others, rows / tiles: TET4 1,315 rows
+// 8.2 / 10.4 us, 5,631 11.1 / 11.2, 9,541 16.5 / 13.4; three variables 2,373 rows 8.5 /
+// 9.9, 6,093 12.3 / 11.7; TET10 4,881 rows 9.4 / 9.8, 8,245 10.9 / 10.2; three variables
+// 3,459 9.3 / 10.3, 7,755 12.5 / 11.2.  Hexahedra (at most 8 incidences) 3.9 / 3.6 at
+// the smallest sizes.
+constexpr int64_t kTetTileRows = 5500;
+
 // Tiles of the matrix's rows; h_rp: its row pointers.  Patterns the tiles do
-// not take (more than 32 element DoFs, a row beyond 4096 entries) and matrices
-// without room for the plan keep the row-at-a-time kernel.  `rows` holds what a
+// not take (more than 32 element DoFs, a row beyond 4096 entries, small tetrahedral
+// ones) and matrices without room for the plan keep the row kernels.  `rows` holds what a
 // copy on the stream may still read: for the caller to keep until it has waited.
 int matrix_build_tiles(lmh_matrix *A, const std::vector<int32_t> &h_rp, std::vector<int32_t> &rows) {
   const lmh_dofmap *dm = A->dm;
   lmh_context *ctx = A->ctx;
   if (!dm || dm->dpe > 32 || A->max_row > 4096 || A->rows == 0) return LMH_OK;
+  const bool tet = dm->mesh->type == LMH_TET4 || dm->mesh->type == LMH_TET10;
+  if (tet && A->rows < kTetTileRows) return LMH_OK;
   const int gs = group_lanes(dm->dpe), pi = 64 / gs;
   // small matrices: fewer entries per tile, so that every CU has several
   const int64_t want = A->nnz / ((int64_t)ctx->cu_count * 8);

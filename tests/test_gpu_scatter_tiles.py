@@ -45,8 +45,9 @@ def test_scatter_is_the_sequential_sum(ctx, t, nv, box):
 
 @pytest.mark.parametrize("t,nv,box", [
     (L.HEX8, 1, (11, 11, 11)), (L.HEX8, 1, (12, 12, 12)), (L.HEX27, 1, (13, 13, 13)), (L.HEX27, 1, (15, 15, 15)),
-    (L.TET4, 1, (4, 4, 4)), (L.TET4, 1, (5, 5, 6)), (L.TET10, 1, (3, 3, 3)), (L.TET10, 1, (5, 5, 5)),
-    (L.TET10, 3, (2, 2, 2)), (L.TET10, 3, (3, 3, 3))])
+    (L.TET4, 1, (10, 10, 9)), (L.TET4, 1, (10, 10, 10)), (L.TET10, 1, (5, 5, 5)), (L.TET10, 1, (6, 5, 5)),
+    (L.TET4, 3, (7, 6, 6)), (L.TET4, 3, (7, 7, 7)), (L.TET10, 3, (3, 3, 4)), (L.TET10, 3, (4, 4, 3))])
 def test_both_ways_to_the_plan(ctx, t, nv, box):
-    """On each side of the size to which the plan is made in one launch"""
+    """On each side of the size to which the plan is made in one launch (hexahedra), and
+    of the one from which tetrahedral matrices have a plan (5,500 rows)"""
     test_scatter_is_the_sequential_sum(ctx, t, nv, box)
