@@ -2374,6 +2374,7 @@ int lmh_mixed_solve(lmh_matrix *A, const double *b_d, double *x_d, double rtol, 
     launch_residual(A, st, true, A->vals, b_d, x_d, A->w64, part2);
     LMH_LAUNCH(ctx, "fin", k_fin_residual, dim3(1), dim3(BLK), 0, part2, st.grid, S + G_RRTRUE);
     LMH_TRY(check_launch("mixed finish"));
+    LMH_HIP(hipStreamSynchronize(ctx->stream));  // a plain copy does not wait for the context's stream
   }
   LMH_HIP(hipMemcpy(gl, S + G_THR, sizeof(gl), hipMemcpyDeviceToHost));
   const double bb = gl[G_BB - G_THR], rrt = gl[G_RRTRUE - G_THR];
