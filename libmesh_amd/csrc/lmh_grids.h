@@ -10,7 +10,8 @@ namespace lmh {
 constexpr int NXCD = 8;
 
 // Workgroups of a product over `blocks` row blocks on a GPU of `cus` CUs: `per_cu`
-// on every CU at most, of which `resident` are there at once.
+// on every CU at most, of which `resident` are there at once (0: no rounds, see
+// below).
 //
 // Each publishes up to three partial sums (k_refresh, k_refresh16) into the
 // second half of the partial buffer, 2 n_part doubles: no more than fit there,

@@ -142,3 +142,39 @@ def test_transpose_solve_needs_symmetric_pattern(ctx):
         assert rel(x.download(), np.linalg.solve(A.toarray(), np.ones(n))) < 1e-10
     finally:
         L.hip().lmh_matrix_destroy(h)
+
+
+def test_rows_longer_than_a_block(ctx):
+    """3,000 rows of 1,500 to 2,999 entries, most a row block of their own: FP32
+    products run one workgroup a row, FP64 ones several rows a workgroup, and the
+    mixed solve both."""
+    n, k = 3000, 1499
+    rng = np.random.default_rng(13)
+    A = sp.diags([rng.uniform(-1, 1) * np.ones(n - d) for d in range(1, k + 1)], list(range(1, k + 1)), format="csr")
+    A = A + A.T
+    A = (A + sp.diags(np.asarray(abs(A).sum(1)).ravel() + 1.0)).tocsr()
+    h, A, rp, ci, v = make(ctx, A)
+    try:
+        assert A.nnz > 2048 * n and L.hip().lmh_matrix_window_bits(h) == 0
+        xh, bh = rng.standard_normal(n), rng.standard_normal(n)
+        x, b, y = L.DeviceArray(ctx, n, data=xh), L.DeviceArray(ctx, n, data=bh), L.DeviceArray(ctx, n)
+        L.check(L.hip().lmh_spmv(h, x.ptr, y.ptr))
+        assert rel(y.download(), A @ xh) < 1e-13
+        L.check(L.hip().lmh_matrix_make_fp32(h))
+        x32, y32 = L.DeviceArray(ctx, n, np.float32, data=xh.astype(np.float32)), L.DeviceArray(ctx, n, np.float32)
+        L.check(L.hip().lmh_spmv_fp32(h, x32.ptr, y32.ptr))
+        A32 = sp.csr_matrix((v.astype(np.float32).astype(np.float64), ci, rp), shape=(n, n))
+        # a lane sums 12 entries, a wave 64 lanes in FP64: 16 roundings of 6e-8 at most
+        assert rel(y32.download().astype(np.float64), A32 @ xh.astype(np.float32).astype(np.float64)) < 1e-6
+        its, res, reason, stats = C.c_int64(), C.c_double(), C.c_int(), np.zeros(3)
+        exact = np.linalg.solve(A.toarray(), bh)
+        # (an iteration gains a factor of 20, FP32 has seven digits: a loose limit)
+        x.zero()
+        L.check(L.hip().lmh_mixed_solve(h, b.ptr, x.ptr, 1e-4, 0.1, 0, 1000, C.byref(its), C.byref(res),
+                                        C.byref(reason), L._ptr(stats)))
+        assert reason.value == L.CONVERGED_RTOL and res.value <= 1e-4 and rel(x.download(), exact) < 1e-3
+        x.zero()
+        L.check(L.hip().lmh_cg_solve(h, b.ptr, x.ptr, 1e-10, 1000, C.byref(its), C.byref(res), C.byref(reason)))
+        assert reason.value == L.CONVERGED_RTOL and rel(x.download(), exact) < 1e-8
+    finally:
+        L.hip().lmh_matrix_destroy(h)

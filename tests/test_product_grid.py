@@ -14,7 +14,7 @@ int main() {
   int bad = 0;
   for (int cus : {1, 8, 64, 255, 256, 304, 341, 342, 512, 1024})
     for (int per_cu : {1, 4, 16, 32, 64, 128})
-      for (int resident : {5, 10})
+      for (int resident : {0, 5, 10})
         for (int n_part : {256, 4096, 16384})
           for (int64_t blocks : {1, 7, 8, 9, 1000, 2561, 10241, 24576, 140203, 1 << 30}) {
             const int64_t g = product_grid(cus, per_cu, resident, n_part, blocks);
@@ -28,6 +28,8 @@ int main() {
   if (product_grid(256, 32, 10, 16384, 140203) != 8192 || product_grid(256, 32, 10, 16384, 4050) != 2032 ||
       product_grid(256, 32, 10, 16384, 3) != 8 || product_grid(256, 16, 5, 16384, 70000) != 4096)
     ++bad, std::printf("256-CU grids differ\n");
+  // without rounds: a workgroup per block
+  if (product_grid(256, 16, 0, 16384, 4000) != 4000) ++bad, std::printf("rounds where none are asked for\\n");
   return bad != 0;
 }
 """
