@@ -268,8 +268,9 @@ int matrix_build_tiles(lmh_matrix *A, const std::vector<int32_t> &h_rp, std::vec
   const bool wide = A->max_row > 256;
   // tiles, sequence, offsets and `more` bytes in one allocation
   auto allocate = [&](int64_t total, size_t more) {
-    const size_t seq = sizeof(int4) * nt, map = seq + ((sizeof(int2) * total + 15) & ~(size_t)15),
-                 end = map + (((wide ? 2 : 1) * (size_t)total * gs + 15) & ~(size_t)15);
+    auto line = [](size_t bytes) { return (bytes + 255) & ~(size_t)255; };  // a wavefront's reads start on a line
+    const size_t seq = line(sizeof(int4) * nt), map = seq + line(sizeof(int2) * total),
+                 end = map + line((wide ? 2 : 1) * (size_t)total * gs);
     if (hipMalloc((void **)&A->st_tile, end + more) != hipSuccess) {
       (void)hipGetLastError();
       A->st_tile = nullptr;
