@@ -600,16 +600,16 @@ def main():
 
     def step(mode):
         """mode fp64: FP64 assembly + FP64 CG.  mixed: FP64 assembly, FP32 inner
-        operator rounded from it, mixed solve.  mixed_mfma32 (its name
-        from earlier lines): FP64 assembly for the outer residual operator plus an
-        FP32 assembly of the inner operator, mixed solve."""
+        operator rounded from it, mixed solve.  mixed_fp32_assembly:
+        FP64 assembly for the outer residual operator plus an FP32 assembly of the
+        inner operator, mixed solve."""
         x.zero()
         ctx.sync()
         ta = time.perf_counter()
         g.assemble_poisson(3, kd, 0, b, L.FP64, scatter)
         if mode == "mixed":
             g.make_fp32()
-        elif mode == "mixed_mfma32":
+        elif mode == "mixed_fp32_assembly":
             g.assemble_poisson(3, kd, 0, b, L.FP32, scatter)
         ctx.sync()
         tb = time.perf_counter()
@@ -626,7 +626,7 @@ def main():
         return tb - ta, tc - tb, its, res, nref
 
     results = {}
-    for mode in ("fp64", "mixed_mfma32", "mixed"):
+    for mode in ("fp64", "mixed_fp32_assembly", "mixed"):
         mixed = mode != "fp64"
         for _ in range(args.warmup):
             step(mode)
@@ -742,8 +742,8 @@ def main():
     x64 = results["fp64"].pop("x")
     xmx = results["mixed"].pop("x")
     err_mixed_vs_fp64 = float(np.linalg.norm(xmx - x64) / np.linalg.norm(x64))
-    x32m = results["mixed_mfma32"].pop("x")
-    err_mfma32_vs_fp64 = float(np.linalg.norm(x32m - x64) / np.linalg.norm(x64))
+    x32m = results["mixed_fp32_assembly"].pop("x")
+    err_fp32_assembly_vs_fp64 = float(np.linalg.norm(x32m - x64) / np.linalg.norm(x64))
 
     mx = results["mixed"]
 
@@ -800,9 +800,10 @@ def main():
         },
         "fp64": results["fp64"],
         "mixed": results["mixed"],
-        "mixed_mfma32": results["mixed_mfma32"],
-        "speedup_mixed_mfma32_vs_fp64": round(results["mixed_mfma32"]["mdofs"] / results["fp64"]["mdofs"], 4),
-        "mixed_mfma32_rel_diff_vs_fp64_solution": err_mfma32_vs_fp64,
+        "mixed_fp32_assembly": results["mixed_fp32_assembly"],
+        "speedup_mixed_fp32_assembly_vs_fp64": round(results["mixed_fp32_assembly"]["mdofs"]
+                                                     / results["fp64"]["mdofs"], 4),
+        "mixed_fp32_assembly_rel_diff_vs_fp64_solution": err_fp32_assembly_vs_fp64,
         "speedup_mixed_vs_fp64": round(mx["mdofs"] / results["fp64"]["mdofs"], 4),
         "mixed_rel_diff_vs_fp64_solution": err_mixed_vs_fp64,
         "fp64_spmv_roofline": {"kernel_symbol": spmv_symbol(L, g, fp64=True), "achieved": round(ach64, 1),
@@ -842,7 +843,8 @@ def main():
                           if k not in ("n_gpus", "higher_is_better", "scaling", "vs_baseline", "data")}
     if args.cpu == "run":
         log("cpu baseline (reference path on the full workload) ...")
-        out.update(cpu_block(args.n, args.rtol, {"fp64": x64, "mixed": xmx, "mixed_mfma32": x32m}, gvals, rhs_h, log))
+        solutions = {"fp64": x64, "mixed": xmx, "mixed_fp32_assembly": x32m}
+        out.update(cpu_block(args.n, args.rtol, solutions, gvals, rhs_h, log))
     print(json.dumps(sig(out)), flush=True)
 
 

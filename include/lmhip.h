@@ -290,9 +290,8 @@ int lmh_cg_solve(lmh_matrix *A, const double *b_d, double *x_d, double rtol, int
  * array of the library sized for LMH_CG_NOALLOC_MAX_ROWS rows (4 doubles and
  * one int32 per row: 144 MiB), which every GPU the library runs on holds from
  * its first context until the process ends.  A matrix with more rows:
- * LMH_ERR_INVALID.  A's compressed column windows are used when an earlier
- * lmh_cg_solve or lmh_mixed_solve on A built them (the iterates are the same
- * either way).  All calls on one GPU share the array and keep the last call's
+ * LMH_ERR_INVALID.  A's compressed column windows, built with the matrix, are
+ * used as in lmh_cg_solve (the iterates are the same either way).  All calls on one GPU share the array and keep the last call's
  * contents: calls that overlap on one GPU (from several contexts or threads)
  * race.  Not recorded by lmh_profile_enable. */
 #define LMH_CG_NOALLOC_MAX_ROWS 4194304

@@ -12,9 +12,9 @@
 // and form their lane constants anew in every group: 168 registers and three
 // wavefronts per SIMD instead of 242 and two (residual) or more than 256 and one
 // (adjoint); four spill (45 and 38 us).  64,000 elements (40^3), before -> now:
-// residual element stage 555 (element matrices, then K_e u_e) -> 36 -> 33.7 us, QoI
-// 290 -> 22 us, adjoint gradient 326 -> 44 -> 30.5 us; the three calls with their
-// gathers and host waits 1290 -> 161 us.
+// residual element stage 555 (element matrices, then K_e u_e) -> 33.8 us, QoI 290 ->
+// 20.9 us, adjoint gradient 326 -> 30.5 us; the three calls with their gathers and
+// host waits 1290 -> 159 us.
 #include <algorithm>
 
 #include "lmh_hex27.h"
@@ -464,7 +464,7 @@ __global__ __launch_bounds__(64, 3) void k_hex27_poisson(const double *__restric
     }
     int a3 = i3, b3 = j3, a2 = i2, b2 = j2;
     asm volatile("" : "+v"(a3), "+v"(b3), "+v"(a2), "+v"(b2));
-  int ni[3], nj[3];  // local nodes of the lane's rows (i1, i2, i3) and columns (j1, j2, j3)
+    int ni[3], nj[3];  // local nodes of the lane's rows (i1, i2, i3) and columns (j1, j2, j3)
 #pragma unroll
     for (int i = 0; i < 3; ++i) {
       ni[i] = kH27Node[9 * a3 + 3 * a2 + i];
